@@ -104,6 +104,11 @@ __global__ __launch_bounds__(256) void fp8_gemm_rowscaled_kernel(
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
+    if (sizeof(OUT) == 2 && N % 8 == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0) {
+        __syncthreads();     // the operand panels are free: 8 KB of results per wave
+        store_rows<4, 4>(acc, &lds_a[0][0] + wave * 8192, reinterpret_cast<uint16_t*>(c), N, nullptr, m0 + wm * 64, n0 + wn * 64, M, N, lane);
+        return;
+    }
     const bool vec_ok = (N % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
