@@ -216,11 +216,12 @@ __global__ __launch_bounds__(256) void act_quant_typed_kernel(const void* __rest
     }
 }
 
-// x_dtype: 0 bf16, 1 fp16, 2 fp32; block_size: 8 x a power of two, 8..512.  bf16 with block_size 128 is launch_act_quant.
+// x_dtype: 0 bf16, 1 fp16, 2 fp32; block_size: 8 x a power of two, 8..512.  bf16 with block_size 128 is launch_act_quant, in
+// every dialect (e5m2 bytes, 8192x4096: 23.7 us here with a division per element, 17 us there).
 int launch_act_quant_typed(const void* x, int x_dtype, int block_size, void* y, float* s, int64_t M, int64_t K,
                            int64_t x_row_stride, int64_t PM, int64_t PK, int64_t s_row_stride, int64_t s_col_stride, int mode,
                            hipStream_t stream) {
-    if (x_dtype == 0 && block_size == 128 && mode != 2)
+    if (x_dtype == 0 && block_size == 128)
         return launch_act_quant(x, y, s, M, K, x_row_stride, PM, PK, s_row_stride, s_col_stride, mode, stream);
     if (PM == 0 || PK == 0) return 0;
     const int esz = x_dtype == 2 ? 4 : 2;
@@ -259,6 +260,8 @@ int launch_act_quant(const void* x, void* y, float* s, int64_t M, int64_t K, int
                        (int)PM, (int)PK, s_col_stride)
         if (mode == 0) {
             if (vec) MDY_CM(0, true); else MDY_CM(0, false);
+        } else if (mode == 2) {
+            if (vec) MDY_CM(2, true); else MDY_CM(2, false);
         } else {
             if (vec) MDY_CM(1, true); else MDY_CM(1, false);
         }
@@ -283,6 +286,8 @@ int launch_act_quant(const void* x, void* y, float* s, int64_t M, int64_t K, int
                        x_row_stride, (int)pm, (int)PK, s_row_stride, s_col_stride, by_xcd)
         if (mode == 0) {
             if (vec) MDY_AQ(0, true); else MDY_AQ(0, false);
+        } else if (mode == 2) {
+            if (vec) MDY_AQ(2, true); else MDY_AQ(2, false);
         } else {
             if (vec) MDY_AQ(1, true); else MDY_AQ(1, false);
         }

@@ -24,6 +24,8 @@ constexpr int kGroup = 128;  // quantization group / block edge
 // residual underflows.  The DeepLinear dialect (eps keeps s normal) is clean for
 // every finite amax.
 constexpr uint32_t kFastQuotientMinExp = 23;
+// The same for e5m2 bytes (s = amax / 57344, 2^7 smaller: the residual underflows earlier), proven in the same walk.
+constexpr uint32_t kFastQuotientMinExpE5m2 = 37;
 
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
@@ -43,7 +45,7 @@ __device__ __forceinline__ float group_scale(float amax) {
 template <int MODE>
 __device__ __forceinline__ bool fast_quotient_ok(float amax) {
     uint32_t b = __float_as_uint(amax);
-    if (MODE == 2) return false;            // the exhaustive proof covers e4m3fn bytes only
+    if (MODE == 2) return b >= (kFastQuotientMinExpE5m2 << 23) && b < 0x7F800000u;
     if (MODE == 0) return b >= (kFastQuotientMinExp << 23) && b < 0x7F800000u;
     return b < 0x7F800000u;
 }
@@ -105,7 +107,7 @@ __device__ __forceinline__ uint2 quantize8_scaled(const float (&f)[8], float s, 
 // needs |x / s| <= 448 without the saturating clamp, i.e. an absmax within the 1e4 clamp).
 template <int MODE>
 __device__ __forceinline__ bool group_is_fast(float amax) {
-    return MODE == 0 ? fast_quotient_ok<0>(amax) : MODE == 2 ? false : (amax <= 1e4f);
+    return MODE == 1 ? (amax <= 1e4f) : fast_quotient_ok<MODE>(amax);
 }
 template <int MODE>
 __device__ __forceinline__ uint2 quantize8(const float (&f)[8], float amax, float& scale_out) {

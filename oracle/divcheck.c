@@ -19,9 +19,10 @@
  * e4m3fn byte would be lost)
  *
  * x and amax are bfloat16, so there are only 2^15 possible amax values and 2^16
- * possible x: this program walks every pair with |x| <= amax, both dialects, and
- * counts where q differs from x / s as an fp32 pattern and as an e4m3fn byte.
- * It prints, per dialect, the set of amax biased exponents for which any e4m3fn
+ * possible x: this program walks every pair with |x| <= amax, both dialects (modes
+ * 0 and 1) and the first one with e5m2 bytes (mode 2: s = amax / 57344), and
+ * counts where q differs from x / s as an fp32 pattern and as an fp8 byte.
+ * It prints, per mode, the set of amax biased exponents for which any fp8
  * byte differs; the kernels take the plain-division path for exponents outside
  * the clean range that is hard-coded there, and the test asserts that range.
  *
@@ -64,6 +65,22 @@ static uint8_t e4m3_encode(float f) {
     return sign | (uint8_t)code;
 }
 
+/* fp32 -> e5m2, round-to-nearest-even, overflow -> inf, NaN -> 0x7F. */
+static uint8_t e5m2_encode(float f) {
+    uint32_t u = f32_bits(f);
+    uint8_t sign = (uint8_t)((u >> 24) & 0x80);
+    uint32_t mag = u & 0x7FFFFFFFu;
+    if (mag > 0x7F800000u) return sign | 0x7F;
+    if (mag < 0x38800000u) /* below 2^-14: multiples of 2^-16 */
+        return sign | (uint8_t)nearbyint(fabs((double)f) * 65536.0);
+    uint32_t lsb = (mag >> 21) & 1u;
+    uint32_t rounded = (mag + 0xFFFFFu + lsb) & 0xFFE00000u;
+    int e = (int)(rounded >> 23) - 127;
+    int code = ((e + 15) << 2) | (int)((rounded >> 21) & 3u);
+    if (mag == 0x7F800000u || code > 0x7B) return sign | 0x7C;
+    return sign | (uint8_t)code;
+}
+
 static inline float sat448(float q) {
     if (q != q) return q;
     return q > 448.0f ? 448.0f : (q < -448.0f ? -448.0f : q);
@@ -72,7 +89,7 @@ static inline float sat448(float q) {
 int main(int argc, char** argv) {
     int verbose = argc > 1;
     int rc = 0;
-    for (int mode = 0; mode < 2; ++mode) {
+    for (int mode = 0; mode < 3; ++mode) {
         long long n_pairs = 0, n_f32 = 0, n_fp8 = 0;
         long long fp8_by_exp[256];
         long long f32_by_exp[256];
@@ -84,6 +101,8 @@ int main(int argc, char** argv) {
             float s;
             if (mode == 0) {
                 s = amax / 448.0f;
+            } else if (mode == 2) {
+                s = amax / 57344.0f;
             } else {
                 float c = amax > 1e4f ? 1e4f : amax;
                 s = (c + 1e-8f) / 448.0f;
@@ -102,12 +121,15 @@ int main(int argc, char** argv) {
                     if (mode == 0) {
                         bref = e4m3_encode(ref);
                         bq = e4m3_encode(q);
+                    } else if (mode == 2) {
+                        bref = e5m2_encode(ref);
+                        bq = e5m2_encode(q);
                     } else {
                         bref = e4m3_encode(sat448(ref));
                         bq = e4m3_encode(sat448(q));
                     }
                     /* NaN bytes compare equal whatever their sign */
-                    int nan_both = ((bref & 0x7F) == 0x7F) && ((bq & 0x7F) == 0x7F);
+                    int nan_both = mode == 2 ? (bref & 0x7F) > 0x7C && (bq & 0x7F) > 0x7C : ((bref & 0x7F) == 0x7F) && ((bq & 0x7F) == 0x7F);
                     if (f32_bits(ref) != f32_bits(q) && !(ref != ref && q != q)) ++lf32;
                     if (bref != bq && !nan_both) ++lfp8;
                     ++n_pairs;
