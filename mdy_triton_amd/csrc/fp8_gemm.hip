@@ -723,7 +723,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_scalar_kernel(const uint8_t* __r
 
 // Compute units of the current device (workgroups of the big tile that run at once, one per CU): read from the
 // device properties once per device and thread, 256 on a full MI355X, fewer on a partitioned part.
-static int cu_count() {
+int cu_count() {
     static thread_local int cached_dev = -1, cached_cus = 256;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return cached_cus;

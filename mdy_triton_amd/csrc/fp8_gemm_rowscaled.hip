@@ -7,10 +7,12 @@
 // dimension (fp8_matmul_bwd, :254-257).
 //
 // The combined scale differs for each of a lane's four results of an MFMA (four consecutive n of one m), so the
-// fold is 4 multiplies + 4 FMAs per MFMA instead of 4 FMAs.  Two kernels: the scheduled tile body of fp8_gemm_tile.h in its
-// row-scaled-weight form (128x256 tiles; the 256x256 tile has no registers left for the per-column scales) for problems
-// that fill the CUs, and a plain loop (128x128 tile, four waves of 64x64, the K block's two panels and two scale vectors
-// copied global -> LDS by `buffer_load ... lds`, double buffered, one barrier per K block) for the rest.  K % 128 == 0 (the callers contract over a padded token count).
+// fold is 4 multiplies + 4 FMAs per MFMA instead of 4 FMAs: the VALU is as busy as the matrix cores, and what is left to
+// save is everything else a wave issues.  So the scheduled tile body of fp8_gemm_tile.h in its row-scaled-weight form takes
+// 256x256 tiles where their rounds come out ahead (a quarter fewer LDS reads and a third fewer copies per MFMA than 128x256:
+// 4096x7168x4096 154 -> 130 us = 1.85 PFLOP/s, 4096x4096x8192 159 -> 136 us = 2.0 PFLOP/s) and 128x256 tiles otherwise; a plain loop (128x128 tile, four waves of 64x64, the K
+// block's two panels and two scale vectors copied global -> LDS by `buffer_load ... lds`, double buffered, one barrier per K
+// block) runs what has few K blocks and few tiles.  K % 128 == 0 (the callers contract over a padded token count).
 #include "fp8_gemm_tile.h"
 
 namespace mdy {
@@ -122,19 +124,35 @@ __global__ __launch_bounds__(256) void fp8_gemm_rowscaled_kernel(
     }
 }
 
-// The scheduled tile body of fp8_gemm_tile.h in its row-scaled-weight form, 128x256 tiles (8 waves of 64x64, ring of three
-// K blocks): for problems that give every CU a tile.  Smaller problems run the plain kernel above, two workgroups per CU.
-template <typename OUT, int FMT>
+// The scheduled tile body of fp8_gemm_tile.h in its row-scaled-weight form; a grid smaller than the number of tiles walks them.
+template <int BM, int BN, int STAGES, typename OUT, int FMT>
 __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_tile_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, int bs_rs, int bs_cs, uint32_t bs_bytes,
     OUT* __restrict__ c, int M, int N, int K, int tiles_m, int tiles_n) {
-    __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<128, 256, 8, 3>::bytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<BM, BN, 8, STAGES>::bytes];
     const int ntiles = tiles_m * tiles_n;
-    int tm, tn;
-    const Duty duty = tile_of(xcd_contiguous(blockIdx.x, ntiles), tiles_m, tiles_n, tm, tn);
-    fp8_gemm_tile<128, 256, 2, 4, 3, OUT, 0, 0, 0, FMT, true>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, nullptr, tm * 128, M, M,
-                                                              tn * 256, N, K, N, duty, 0, K >> 7, pool, bs_rs, bs_cs, bs_bytes);
+    for (int pid = blockIdx.x; pid < ntiles; pid += gridDim.x) {
+        int tm, tn;
+        const Duty duty = tile_of(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
+        fp8_gemm_tile<BM, BN, 2, 4, STAGES, OUT, 0, 0, 0, FMT, true>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, nullptr, tm * BM, M, M,
+                                                                     tn * BN, N, K, N, duty, 0, K >> 7, pool, bs_rs, bs_cs, bs_bytes);
+        __syncthreads();
+    }
+}
+
+// Which kernel: 2 = 256x256 tiles, 1 = 128x256 tiles of the scheduled body, 0 = the plain loop.
+// A round of tiles takes, at K = 4096, 56.5 us with 256x256 tiles and 33.3 us with 128x256 ones whether the round is full or not
+// (2048x2048 56.3 / 33.4, 4096x4096 56.5 / 66.6, 6144x1536 57.4 / 71.9, 4096x7168 130 / 154, 18432x7168 561 / 662 us), so the
+// rounds decide.  Up to 4 K blocks the plain loop's two short workgroups per CU hide each other's ends as long as they
+// all fit at once (4096x1024x512 7.5 us against 8.2 and 11.6; but 4096x4096x512 16.3 against 18.3 and 16.1); from 8 on they
+// do not (3072x3072x1024 21.3 against 23.3 and 18.4, 2304x2304x2048 22.3 against 19.3, 1024x1024x8192 65.8 against 60.7 us).
+static int rowscaled_config(int64_t M, int64_t N, int64_t K) {
+    if (K > (1 << 16)) return 0;
+    const int64_t cus = cu_count(), rows256 = (M + 255) / 256, rows128 = (M + 127) / 128, cols256 = (N + 255) / 256;
+    if (K <= 512 && rows128 * ((N + 127) / 128) <= 2 * cus) return 0;
+    const int64_t big = (rows256 * cols256 + cus - 1) / cus, mid = (rows128 * cols256 + cus - 1) / cus;
+    return 17 * big <= 10 * mid ? 2 : 1;
 }
 
 // returns hipError_t, or -1 when the operands do not qualify (K % 128 != 0, misaligned, scale extents >= 2^31 bytes)
@@ -148,16 +166,21 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
         b_ext >= ((int64_t)1 << 31) || ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) != 0 ||
         128 * K >= ((int64_t)1 << 31))
         return -1;
-    // 128x256 tiles of the scheduled body once they fill the CUs (and K fits its weight-scale staging)
-    const int64_t big_m = (M + 127) / 128, big_n = (N + 255) / 256;
-    if (big_m * big_n >= 200 && K <= (1 << 16) && big_m * big_n <= 0x7FFFFFFF) {
-#define MDY_RST(OUT_T, FMT)                                                                                              \
-    hipLaunchKernelGGL((fp8_gemm_rowscaled_tile_kernel<OUT_T, FMT>), dim3((unsigned)(big_m * big_n)), dim3(512), 0, stream, \
+    const int cfg = rowscaled_config(M, N, K);
+    if (cfg != 0) {
+        const int bm = cfg == 2 ? 256 : 128;
+        const int64_t tm = (M + bm - 1) / bm, tn = (N + 255) / 256, cus = cu_count();
+        if (tm * tn > 0x7FFFFFFF) return kErrTooManyBlocks;
+        const dim3 grid((unsigned)(cfg == 2 && tm * tn > cus ? cus : tm * tn));      // 256x256: a workgroup per CU walks its tiles
+#define MDY_RST(BM, ST, OUT_T, FMT)                                                                                      \
+    hipLaunchKernelGGL((fp8_gemm_rowscaled_tile_kernel<BM, 256, ST, OUT_T, FMT>), grid, dim3(512), 0, stream,            \
                        static_cast<const uint8_t*>(a), a_s, (int)as_rs, (int)as_cs, (uint32_t)a_ext,                      \
                        static_cast<const uint8_t*>(b), b_s, (int)bs_rs, (int)bs_cs, (uint32_t)b_ext, static_cast<OUT_T*>(c), \
-                       (int)M, (int)N, (int)K, (int)big_m, (int)big_n)
-        if (out_dtype == 0) { if (fmt == 0) MDY_RST(uint16_t, 0); else MDY_RST(uint16_t, 1); }
-        else { if (fmt == 0) MDY_RST(float, 0); else MDY_RST(float, 1); }
+                       (int)M, (int)N, (int)K, (int)tm, (int)tn)
+#define MDY_RST_C(OUT_T, FMT) do { if (cfg == 2) MDY_RST(256, 2, OUT_T, FMT); else MDY_RST(128, 3, OUT_T, FMT); } while (0)
+        if (out_dtype == 0) { if (fmt == 0) MDY_RST_C(uint16_t, 0); else MDY_RST_C(uint16_t, 1); }
+        else { if (fmt == 0) MDY_RST_C(float, 0); else MDY_RST_C(float, 1); }
+#undef MDY_RST_C
 #undef MDY_RST
         return (int)hipGetLastError();
     }

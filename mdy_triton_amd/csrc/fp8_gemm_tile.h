@@ -391,7 +391,6 @@ __device__ __forceinline__ void fp8_gemm_tile(
         const uint8_t* lx_n = HOLD_A ? lds_b[nxt] : lds_a[nxt];
         const float* ls_n = lds_s[nxt];
         float sc_n[TI], sc_hi_n[STRADDLE ? TI : 1];
-        floatx4 sbv_n[BROW_ ? TJ : 1];
         floatx4 p[DEPTH + 1];
 #pragma unroll
         for (int t = 0; t < NT + DEPTH; ++t) {
@@ -416,10 +415,6 @@ __device__ __forceinline__ void fp8_gemm_tile(
                     if (!NO_LDS) {
                         fx[0] = read_frag(lx_n, x0, x1, 0);      // queue slot 0 was last used by streamed fragment NS-2
                         const float sb = BROW_ ? 1.0f : my_bs[min(kb + 1, KB - 1)], sb_hi = BROW_ ? 1.0f : my_bs_hi[min(kb + 1, KB - 1)];
-                        if (BROW_) {
-#pragma unroll
-                            for (int j = 0; j < TJ; ++j) sbv_n[j] = *reinterpret_cast<const floatx4*>(sbr_lane + nxt * BN + j * 16);
-                        }
 #pragma unroll
                         for (int i = 0; i < TI; ++i) {
                             const float sa = ls_n[s_rd + i * 16];
@@ -462,16 +457,18 @@ __device__ __forceinline__ void fp8_gemm_tile(
                 }
             }
             if (t == TOUCH && !NO_TOUCH) touch(me, kb + TD);
+            if (BROW_ && t == NT + DEPTH - 1) {
+                // the block's last fold is done: its weight-row scales make room for the next block's, which are first used
+                // DEPTH MFMAs from here (a second set of registers would not fit the 256x256 tile)
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) sbv[j] = *reinterpret_cast<const floatx4*>(sbr_lane + nxt * BN + j * 16);
+            }
             __builtin_amdgcn_sched_barrier(0);  // keep the MFMA / FMA / ds_read / copy interleaving as written
         }
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
             sc[i] = sc_n[i];
             if (STRADDLE) sc_hi[i] = sc_hi_n[i];
-        }
-        if (BROW_) {
-#pragma unroll
-            for (int j = 0; j < TJ; ++j) sbv[j] = sbv_n[j];
         }
         cur = nxt;
     }
