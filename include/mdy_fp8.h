@@ -170,6 +170,15 @@ int mdy_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, void*
 int mdy_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride,
                               const void* b, const float* b_s, int64_t bs_row_stride, int64_t bs_col_stride, void* c,
                               int64_t M, int64_t N, int64_t K, int fmt, int out_dtype, void* stream);
+/* The same with scratch memory: outputs with few tiles against a long K are cut along K (fp32 partial sums in the
+ * workspace, added in a fixed order).  mdy_fp8_gemm_rowscaled_workspace_bytes says how much a shape can use, 0 when it is
+ * not cut; NULL or a smaller workspace gives mdy_fp8_gemm_nt_rowscaled.  workspace 16-byte aligned, free again once the
+ * work on the stream is done. */
+int64_t mdy_fp8_gemm_rowscaled_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int mdy_fp8_gemm_nt_rowscaled_ws(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride,
+                                 const void* b, const float* b_s, int64_t bs_row_stride, int64_t bs_col_stride, void* c,
+                                 int64_t M, int64_t N, int64_t K, int fmt, int out_dtype, void* workspace,
+                                 int64_t workspace_bytes, void* stream);
 
 /* SwiGLU, alone or fused with the 1x128 activation quantizer that feeds the next GEMM.
  *   act[m, n] = bf16( silu(gate[m, n]) * up[m, n] ), silu(g) = g / (1 + exp(-g)) in fp32;

@@ -30,6 +30,8 @@ SIGNATURES = {
     "mdy_fp8_grouped_gemm_nt": [_p, _p, _i64, _i64, _p, _p, _p, _p, _p, _i64, _i64, _i64, _int, _p],
     "mdy_act_quant_transpose": [_p, _int, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p],
     "mdy_fp8_gemm_nt_rowscaled": [_p, _p, _i64, _i64, _p, _p, _i64, _i64, _p, _i64, _i64, _i64, _int, _int, _p],
+    "mdy_fp8_gemm_nt_rowscaled_ws": [_p, _p, _i64, _i64, _p, _p, _i64, _i64, _p, _i64, _i64, _i64, _int, _int, _p, _i64, _p],
+    "mdy_fp8_gemm_rowscaled_workspace_bytes": [_i64, _i64, _i64],
     "mdy_swiglu": [_p, _p, _p, _p, _i64, _i64, _i64, _int, _i64, _i64, _i64, _i64, _int, _p],
     "mdy_swiglu_bwd": [_p, _p, _p, _i64, _i64, _i64, _int, _p],
     "mdy_weight_dequant": [_p, _p, _p, _i64, _i64, _int, _p],
@@ -75,8 +77,7 @@ def load():
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = (ctypes.c_char_p if name == "mdy_fp8_last_error" else
-                          ctypes.c_int64 if name in ("mdy_fp8_gemm_workspace_bytes", "mdy_fp8_gemm_static_workspace_bytes")
-                          else ctypes.c_int)
+                          ctypes.c_int64 if name.endswith("workspace_bytes") else ctypes.c_int)
         got = lib.mdy_fp8_abi_version()
         if got != ABI_VERSION:
             raise MdyFp8Error("libmdyfp8.so ABI version %d, expected %d: rebuild" % (got, ABI_VERSION))

@@ -78,19 +78,27 @@ check = _lib.check
 _WS_BYTES = {}
 
 
-def gemm_workspace(device, M, N, K):
-    """Scratch tensor for mdy_fp8_gemm_nt_ws, or None when the shape is never split along K.  It comes
-    from torch's caching allocator on the current stream, so it may be dropped as soon as the launch
-    has been enqueued: the allocator hands the memory out again in stream order only."""
-    key = (M, N, K)
+def _workspace(device, key, query):
     nbytes = _WS_BYTES.get(key)
     if nbytes is None:                      # one library call per shape, not per GEMM
         if len(_WS_BYTES) > 4096:
             _WS_BYTES.clear()
-        nbytes = _WS_BYTES[key] = _lib.load().mdy_fp8_gemm_workspace_bytes(M, N, K)
+        nbytes = _WS_BYTES[key] = query(*key[1:])
     if nbytes <= 0:
         return None
     return torch.empty(nbytes, device=device, dtype=torch.uint8)
+
+
+def gemm_workspace(device, M, N, K):
+    """Scratch tensor for mdy_fp8_gemm_nt_ws, or None when the shape is never split along K.  It comes
+    from torch's caching allocator on the current stream, so it may be dropped as soon as the launch
+    has been enqueued: the allocator hands the memory out again in stream order only."""
+    return _workspace(device, (0, M, N, K), _lib.load().mdy_fp8_gemm_workspace_bytes)
+
+
+def rowscaled_workspace(device, M, N, K):
+    """The same for mdy_fp8_gemm_nt_rowscaled_ws."""
+    return _workspace(device, (1, M, N, K), _lib.load().mdy_fp8_gemm_rowscaled_workspace_bytes)
 
 
 _SLOW_WARNED = set()

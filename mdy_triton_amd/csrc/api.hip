@@ -164,9 +164,9 @@ int mdy_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, void*
                     "act_quant_transpose");
 }
 
-int mdy_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,
+int mdy_fp8_gemm_nt_rowscaled_ws(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,
                               const float* b_s, int64_t bs_row_stride, int64_t bs_col_stride, void* c, int64_t M, int64_t N,
-                              int64_t K, int fmt, int out_dtype, void* stream) {
+                              int64_t K, int fmt, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
     if (fmt != MDY_FMT_E4M3 && fmt != MDY_FMT_E5M2) return fail(MDY_E_DTYPE, "fp8_gemm_nt_rowscaled: unknown operand format %d", fmt);
     if (out_dtype != MDY_DT_BF16 && out_dtype != MDY_DT_F32) return fail(MDY_E_DTYPE, "fp8_gemm_nt_rowscaled: unknown out_dtype %d", out_dtype);
     if (M < 0 || N < 0 || K < 128 || K % 128 != 0 || M > kMaxDim || N > kMaxDim || K > (1 << 20))
@@ -176,11 +176,26 @@ int mdy_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_row_st
     if (!a || !a_s || !b || !b_s || !c) return fail(MDY_E_NULL, "fp8_gemm_nt_rowscaled: null pointer");
     if (!aligned(a, 16) || !aligned(b, 16) || !aligned(c, out_dtype == MDY_DT_BF16 ? 2 : 4) || !aligned(a_s, 4) || !aligned(b_s, 4))
         return fail(MDY_E_ALIGN, "fp8_gemm_nt_rowscaled: a and b must be 16-byte aligned, c and the scales aligned for their type");
+    if (workspace_bytes < 0) return fail(MDY_E_SHAPE, "fp8_gemm_nt_rowscaled: workspace_bytes < 0");
+    if (workspace && !aligned(workspace, 16)) return fail(MDY_E_ALIGN, "fp8_gemm_nt_rowscaled: workspace must be 16-byte aligned");
     if (int e = check_device()) return e;
     const int rc = mdy::launch_fp8_gemm_nt_rowscaled(a, a_s, as_row_stride, as_col_stride, b, b_s, bs_row_stride, bs_col_stride, c,
-                                                     M, N, K, fmt, out_dtype, static_cast<hipStream_t>(stream));
+                                                     M, N, K, fmt, out_dtype, workspace, workspace_bytes,
+                                                     static_cast<hipStream_t>(stream));
     if (rc == -1) return fail(MDY_E_SHAPE, "fp8_gemm_nt_rowscaled: scale strides must be non-negative and span less than 2^31 bytes");
     return launched(rc, "fp8_gemm_nt_rowscaled");
+}
+
+int mdy_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,
+                              const float* b_s, int64_t bs_row_stride, int64_t bs_col_stride, void* c, int64_t M, int64_t N,
+                              int64_t K, int fmt, int out_dtype, void* stream) {
+    return mdy_fp8_gemm_nt_rowscaled_ws(a, a_s, as_row_stride, as_col_stride, b, b_s, bs_row_stride, bs_col_stride, c, M, N, K, fmt,
+                                        out_dtype, nullptr, 0, stream);
+}
+
+int64_t mdy_fp8_gemm_rowscaled_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K < 128 || K % 128 != 0 || M > kMaxDim || N > kMaxDim || K > kMaxDim) return 0;
+    return mdy::fp8_gemm_rowscaled_workspace_bytes(M, N, K);
 }
 
 int mdy_swiglu(const void* x, void* act, void* y, float* s, int64_t M, int64_t N, int64_t x_row_stride, int gate_first,

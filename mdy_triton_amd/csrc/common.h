@@ -271,7 +271,8 @@ int launch_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, vo
                                int64_t x_row_stride, int64_t x_col_stride, int64_t PM, int64_t PK, int mode, hipStream_t stream);
 int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs, int64_t as_cs, const void* b,
                                  const float* b_s, int64_t bs_rs, int64_t bs_cs, void* c, int64_t M, int64_t N, int64_t K,
-                                 int fmt, int out_dtype, hipStream_t stream);
+                                 int fmt, int out_dtype, void* workspace, int64_t workspace_bytes, hipStream_t stream);
+int64_t fp8_gemm_rowscaled_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int launch_swiglu(const void* x, void* act, void* y, float* s, int64_t M, int64_t N, int64_t x_row_stride,
                   int gate_first, int64_t PM, int64_t PN, int64_t s_row_stride, int64_t s_col_stride, int mode,
                   hipStream_t stream);
@@ -286,6 +287,7 @@ int launch_fp8_gemm_nt_e5m2(const void* a, const float* a_s, int64_t as_row_stri
                             const void* b, const float* b_s, void* c, const void* bias, int64_t M, int64_t N,
                             int64_t K, int out_dtype, hipStream_t stream);
 int cu_count();      // compute units of the current device
+int launch_splitk_reduce(const float* ws, void* c, int out_dtype, const uint16_t* bias, int64_t M, int64_t N, int ksplit, hipStream_t stream);
 int64_t fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int launch_fp8_gemm_nt_ws(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride,
                           const void* b, const float* b_s, void* c, const void* bias, int64_t M, int64_t N,

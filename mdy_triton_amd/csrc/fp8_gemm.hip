@@ -121,6 +121,19 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     }
 }
 
+// slabs [ksplit][M][N] of partial sums -> c [M][N] of out_dtype (0 bf16, 1 fp32)
+int launch_splitk_reduce(const float* ws, void* c, int out_dtype, const uint16_t* bias, int64_t M, int64_t N, int ksplit, hipStream_t stream) {
+    const int64_t MN = M * N;
+    const bool vec = (N % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
+    const dim3 grid((unsigned)((MN / (vec ? 4 : 1) + 255) / 256));
+#define MDY_RED(OUT, VEC) \
+    hipLaunchKernelGGL((splitk_reduce_kernel<OUT, VEC>), grid, dim3(256), 0, stream, ws, static_cast<OUT*>(c), bias, MN, (int)N, ksplit)
+    if (out_dtype == 0) { if (vec) MDY_RED(uint16_t, true); else MDY_RED(uint16_t, false); }
+    else { if (vec) MDY_RED(float, true); else MDY_RED(float, false); }
+#undef MDY_RED
+    return (int)hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // Grouped (mixture-of-experts) GEMM: rows row_start[g] .. row_start[g+1] of a are multiplied with
 // expert g's weight b[g] ([N, K], scales b_s[g]); c has the rows of a.  The table travels as a kernel
@@ -1199,17 +1212,9 @@ static int launch_splitk(const uint8_t* a, const float* a_s, int64_t as_rs, int6
     else MDY_SPLIT(64, 64, 8)
 #undef MDY_SPLIT
 #undef MDY_SPLIT_WS
-    int rc = (int)hipGetLastError();
+    const int rc = (int)hipGetLastError();
     if (rc != 0) return rc;
-    const int64_t MN = (int64_t)M * N;
-    const bool vec = (N % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
-    if (vec)
-        hipLaunchKernelGGL((splitk_reduce_kernel<OUT, true>), dim3((unsigned)((MN / 4 + 255) / 256)), dim3(256), 0, stream,
-                           ws, c, bias, MN, N, p.ksplit);
-    else
-        hipLaunchKernelGGL((splitk_reduce_kernel<OUT, false>), dim3((unsigned)((MN + 255) / 256)), dim3(256), 0, stream, ws,
-                           c, bias, MN, N, p.ksplit);
-    return (int)hipGetLastError();
+    return launch_splitk_reduce(ws, c, sizeof(OUT) == 2 ? 0 : 1, bias, M, N, p.ksplit, stream);
 }
 
 int launch_fp8_gemm_nt_ws(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,

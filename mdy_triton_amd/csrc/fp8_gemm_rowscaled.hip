@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_rowscaled_kernel(
 
     if (sizeof(OUT) == 2 && N % 8 == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0) {
         __syncthreads();     // the operand panels are free: 8 KB of results per wave
-        store_rows<4, 4>(acc, &lds_a[0][0] + wave * 8192, reinterpret_cast<uint16_t*>(c), N, nullptr, m0 + wm * 64, n0 + wn * 64, M, N, lane);
+        store_rows<4, 4, OUT>(acc, &lds_a[0][0] + wave * 8192, c, N, nullptr, m0 + wm * 64, n0 + wn * 64, M, N, lane);
         return;
     }
     const bool vec_ok = (N % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
@@ -141,6 +141,54 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_tile_kernel(
     }
 }
 
+// The same cut along K: workgroup (slab, tile) writes the fp32 partial sums of K blocks slab * kb_per .. of its tile into a
+// workspace [slabs][M][N]; splitk_reduce_kernel adds the slabs in order.
+template <int FMT>
+__global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
+    const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
+    const uint8_t* __restrict__ b, const float* __restrict__ b_s, int bs_rs, int bs_cs, uint32_t bs_bytes,
+    float* __restrict__ ws, int M, int N, int K, int tiles_m, int tiles_n, int slabs, int kb_per) {
+    __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<128, 256, 8, 3>::bytes];
+    const int ntiles = tiles_m * tiles_n;
+    const int pid = xcd_contiguous(blockIdx.x, ntiles * slabs);
+    const int ks = __builtin_amdgcn_readfirstlane(pid / ntiles);
+    int tm, tn;
+    const Duty duty = tile_of(pid - ks * ntiles, tiles_m, tiles_n, tm, tn);
+    const int kb0 = ks * kb_per, kb1 = min(K >> 7, kb0 + kb_per);
+    fp8_gemm_tile<128, 256, 2, 4, 3, float, 0, 0, 0, FMT, true>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, nullptr,
+                                                                tm * 128, M, M, tn * 256, N, K, N, duty, kb0, kb1, pool, bs_rs, bs_cs,
+                                                                bs_bytes);
+}
+
+struct RowscaledSplit {
+    int slabs, kb_per;
+};
+// How many slabs: while the tiles leave half of the CUs idle, a K block takes a workgroup about 1.0 us on top of 3.5 us for the
+// launch and the ends of a tile, and the reduction 4 us plus its traffic (slabs written and read at about 6 TB/s).  The cheapest
+// count is taken if it promises 15 % (measured, one launch -> cut: 1024x1024x8192 60.6 -> 26.6 us with 8 slabs, 1536x1536x16384
+// 115 -> 62 us with 3, 1024x2048x4096 33.1 -> 26.4 us with 4, 512x512x4096 35 -> 15.5 us with 8; without that margin
+// 2048x2048x4096 would lose, 33.0 -> 38.7 us with 2, and 1024x1024x2048 18.3 -> 20.9 us).
+static RowscaledSplit plan_rowscaled_split(int64_t M, int64_t N, int64_t K) {
+    RowscaledSplit p{1, (int)(K / 128)};
+    const int64_t cus = cu_count(), tiles = ((M + 127) / 128) * ((N + 255) / 256), KB = K / 128;
+    if (K > (1 << 16) || 2 * tiles > cus) return p;
+    const double traffic = (double)M * (double)N * 8.0 / 6e6;      // us per slab
+    double best = ((double)KB + 3.5) / 1.15;
+    for (int64_t ks = 2; ks <= 16 && ks <= cus / tiles && ks <= KB / 4; ++ks) {
+        const double cost = (double)((KB + ks - 1) / ks) + 7.5 + (double)ks * traffic;
+        if (cost < best) {
+            best = cost;
+            p.kb_per = (int)((KB + ks - 1) / ks);
+            p.slabs = (int)((KB + p.kb_per - 1) / p.kb_per);
+        }
+    }
+    return p;
+}
+int64_t fp8_gemm_rowscaled_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    const RowscaledSplit p = plan_rowscaled_split(M, N, K);
+    return p.slabs > 1 ? (int64_t)p.slabs * M * N * 4 : 0;
+}
+
 // Which kernel: 2 = 256x256 tiles, 1 = 128x256 tiles of the scheduled body, 0 = the plain loop.
 // A round of tiles takes, at K = 4096, 56.5 us with 256x256 tiles and 33.3 us with 128x256 ones whether the round is full or not
 // (2048x2048 56.3 / 33.4, 4096x4096 56.5 / 66.6, 6144x1536 57.4 / 71.9, 4096x7168 130 / 154, 18432x7168 561 / 662 us), so the
@@ -158,7 +206,7 @@ static int rowscaled_config(int64_t M, int64_t N, int64_t K) {
 // returns hipError_t, or -1 when the operands do not qualify (K % 128 != 0, misaligned, scale extents >= 2^31 bytes)
 int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs, int64_t as_cs, const void* b,
                                  const float* b_s, int64_t bs_rs, int64_t bs_cs, void* c, int64_t M, int64_t N, int64_t K,
-                                 int fmt, int out_dtype, hipStream_t stream) {
+                                 int fmt, int out_dtype, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
     if (M == 0 || N == 0) return 0;
     const int64_t KB = K / 128;
     const int64_t a_ext = ((M - 1) * as_rs + (KB - 1) * as_cs + 1) * 4, b_ext = ((N - 1) * bs_rs + (KB - 1) * bs_cs + 1) * 4;
@@ -166,6 +214,19 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
         b_ext >= ((int64_t)1 << 31) || ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) != 0 ||
         128 * K >= ((int64_t)1 << 31))
         return -1;
+    const RowscaledSplit sp = plan_rowscaled_split(M, N, K);
+    if (sp.slabs > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && workspace_bytes >= (int64_t)sp.slabs * M * N * 4) {
+        const int tm = (int)((M + 127) / 128), tn = (int)((N + 255) / 256);
+        float* ws = static_cast<float*>(workspace);
+#define MDY_RSS(FMT)                                                                                                     \
+    hipLaunchKernelGGL((fp8_gemm_rowscaled_split_kernel<FMT>), dim3((unsigned)(tm * tn * sp.slabs)), dim3(512), 0, stream, \
+                       static_cast<const uint8_t*>(a), a_s, (int)as_rs, (int)as_cs, (uint32_t)a_ext, static_cast<const uint8_t*>(b), b_s, \
+                       (int)bs_rs, (int)bs_cs, (uint32_t)b_ext, ws, (int)M, (int)N, (int)K, tm, tn, sp.slabs, sp.kb_per)
+        if (fmt == 0) MDY_RSS(0); else MDY_RSS(1);
+#undef MDY_RSS
+        const int rc = (int)hipGetLastError();
+        return rc != 0 ? rc : launch_splitk_reduce(ws, c, out_dtype, nullptr, M, N, sp.slabs, stream);
+    }
     const int cfg = rowscaled_config(M, N, K);
     if (cfg != 0) {
         const int bm = cfg == 2 ? 256 : 128;

@@ -61,34 +61,46 @@ __device__ __forceinline__ void store4(OUT* c, int64_t ldc, int m, int n, int M,
 // 4096x18432x7168 473 -> 456 -> 451 us, 8192x4096x4096 126 -> 120 -> 117 us, 16384x4096x1024 100 -> 91 -> 84 us, 4096x7168x2048
 // 70 -> 63 -> 63 us, with row scales 4096x7168x512 45 -> 36 -> 35 us.  The 16-byte pieces of a row are XOR-swizzled by
 // the row (no bank conflict either way).  Needs N % 8 == 0 and 16-byte aligned rows of c (the caller checks).
-template <int TI, int TJ>
-__device__ __forceinline__ void store_rows(const floatx4 (&acc)[TI][TJ], uint8_t* buf, uint16_t* __restrict__ c, int64_t ldc,
+// fp32 results (the slabs of a K split, an fp32 output) go the same way with twice the row length where the pool holds them;
+// those stores stay cached: the reduction reads the slabs next.
+template <int TI, int TJ, typename OUT>
+__device__ __forceinline__ void store_rows(const floatx4 (&acc)[TI][TJ], uint8_t* buf, OUT* __restrict__ c, int64_t ldc,
                                            const uint16_t* __restrict__ bias, int m_base, int n_base, int M, int N, int lane) {
     static_assert(TJ % 2 == 0, "a row is a multiple of four 16-byte pieces");
-    constexpr int CH = TJ * 2, ROW = TJ * 32, MASK = CH % 8 == 0 ? 7 : 3;
+    constexpr bool HALF = sizeof(OUT) == 2;
+    constexpr int EPP = 16 / sizeof(OUT);      // elements per 16-byte piece
+    constexpr int CH = TJ * 16 / EPP, ROW = CH * 16, MASK = CH % 8 == 0 ? 7 : 3;
     asm volatile("" : "+v"(lane));      // the addresses below belong here and not in registers held across the K loop
     const int frow = lane & 15, fk = lane >> 4;
 #pragma unroll
     for (int j = 0; j < TJ; ++j) {
         float bv[4] = {0.f, 0.f, 0.f, 0.f};
         const int n = n_base + j * 16 + 4 * fk;
-        if (bias != nullptr && n < N) {      // N % 8 == 0: all four columns are in range
+        if (bias != nullptr && n < N) {      // N is a multiple of the piece: all four columns are in range
 #pragma unroll
             for (int e = 0; e < 4; ++e) bv[e] = bf16_one(bias[n + e]);
         }
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
             const floatx4 v = acc[i][j];
-            *reinterpret_cast<uint2*>(buf + (i * 16 + frow) * ROW + (((2 * j + (fk >> 1)) ^ (frow & MASK)) << 4) + (fk & 1) * 8) =
-                make_uint2(pack2_bf16(v[0] + bv[0], v[1] + bv[1]), pack2_bf16(v[2] + bv[2], v[3] + bv[3]));
+            uint8_t* row = buf + (i * 16 + frow) * ROW;
+            if (HALF)
+                *reinterpret_cast<uint2*>(row + (((2 * j + (fk >> 1)) ^ (frow & MASK)) << 4) + (fk & 1) * 8) =
+                    make_uint2(pack2_bf16(v[0] + bv[0], v[1] + bv[1]), pack2_bf16(v[2] + bv[2], v[3] + bv[3]));
+            else
+                *reinterpret_cast<float4*>(row + (((4 * j + fk) ^ (frow & MASK)) << 4)) =
+                    make_float4(v[0] + bv[0], v[1] + bv[1], v[2] + bv[2], v[3] + bv[3]);
         }
     }
 #pragma unroll
     for (int t = 0; t < TI * CH / 4; ++t) {
         const int q = t * 64 + lane, row = q / CH, ch = q % CH;
-        const int m = m_base + row, n = n_base + ch * 8;
+        const int m = m_base + row, n = n_base + ch * EPP;
         const uint4 v = *reinterpret_cast<const uint4*>(buf + row * ROW + ((ch ^ (row & MASK)) << 4));
-        if (m < M && n < N) store_nt16(c + (int64_t)m * ldc + n, v);
+        if (m < M && n < N) {
+            if (HALF) store_nt16(c + (int64_t)m * ldc + n, v);
+            else *reinterpret_cast<uint4*>(c + (int64_t)m * ldc + n) = v;
+        }
     }
 }
 
@@ -475,12 +487,10 @@ __device__ __forceinline__ void fp8_gemm_tile(
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing may still be writing LDS when the wave ends
 
     // ---- epilogue: lane holds c[m][n..n+3], m = .. + lane%16, n = .. + 4*(lane/16)
-    if (sizeof(OUT) == 2) {
-        static_assert(sizeof(OUT) != 2 || WAVES * WM * WN * 2 <= L::bytes, "the tile's results fit the pool");
+    if (WAVES * WM * WN * (int)sizeof(OUT) <= L::bytes) {
         __syncthreads();                               // every wave's copies have landed: the pool is free
-        if (((N | ldc) & 7) == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0) {
-            store_rows<TI, TJ>(acc, pool + wave * (WM * WN * 2), reinterpret_cast<uint16_t*>(c), ldc, bias, m0 + wm * WM, n0 + wn * WN, M, N,
-                               lane);
+        if (((N | ldc) & (16 / (int)sizeof(OUT) - 1)) == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0) {
+            store_rows<TI, TJ, OUT>(acc, pool + wave * (WM * WN * (int)sizeof(OUT)), c, ldc, bias, m0 + wm * WM, n0 + wn * WN, M, N, lane);
             return;
         }
     }
@@ -664,7 +674,7 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
             fs = fs + 1 == SS ? 0 : fs + 1;
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing may still be writing LDS when the wave ends
-        if (sizeof(OUT) == 2) __syncthreads();             // the consumers' epilogue goes through the pool
+        if (CW * WM * WN * (int)sizeof(OUT) <= L::bytes) __syncthreads();      // the consumers' epilogue goes through the pool
         return;
     }
 
@@ -766,16 +776,13 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
         if (kb < kb1) block(fh_a, fh_b, sc_a, sc_b, kb);     // odd number of K blocks
     }
 
-    if (sizeof(OUT) == 2) {
-        static_assert(sizeof(OUT) != 2 || CW * WM * WN * 2 <= L::bytes, "the tile's results fit the pool");
+    if (CW * WM * WN * (int)sizeof(OUT) <= L::bytes) {
         __syncthreads();                                 // the producers' copies have landed, every consumer has left the K loop
-        if (((N | ldc) & 7) == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0) {
-            store_rows<TI, TJ>(acc, pool + wave * (WM * WN * 2), reinterpret_cast<uint16_t*>(c), ldc, bias, m0 + wm * WM, n0 + wn * WN, M, N,
-                               lane);
+        if (((N | ldc) & (16 / (int)sizeof(OUT) - 1)) == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0) {
+            store_rows<TI, TJ, OUT>(acc, pool + wave * (WM * WN * (int)sizeof(OUT)), c, ldc, bias, m0 + wm * WM, n0 + wn * WN, M, N, lane);
             return;
         }
     }
-
     const bool vec_ok = (ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
 #pragma unroll
     for (int i = 0; i < TI; ++i) {

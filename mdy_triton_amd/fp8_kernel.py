@@ -15,7 +15,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from ._torch_glue import FP8, check, lib, on_device, ptr, require_gpu, stream_ptr, xt_code
+from ._torch_glue import FP8, check, lib, on_device, ptr, require_gpu, rowscaled_workspace, stream_ptr, xt_code
 
 _ORDERS = ("up-gate", "gate-up")
 
@@ -305,10 +305,16 @@ def _matmul_rowscaled(x2, sx, w, sw, M, N, K, dev, fmt=0):
     out = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
     if M * N == 0:
         return out
-    with on_device(dev):
-        check(lib().mdy_fp8_gemm_nt_rowscaled(ptr(a), ptr(sx), sx.stride(0), sx.stride(1), ptr(b), ptr(sw), sw.stride(0),
-                                              sw.stride(1), ptr(out), M, N, PK, fmt, 0, stream_ptr(dev)), "fp8_matmul")
+    _rowscaled_into(out, a, sx, b, sw, M, N, PK, fmt, dev, "fp8_matmul")
     return out
+
+
+def _rowscaled_into(out, a, sa, b, sb, M, N, K, fmt, dev, who):
+    with on_device(dev):
+        ws = rowscaled_workspace(dev, M, N, K)      # scratch for outputs that are cut along K, else None
+        check(lib().mdy_fp8_gemm_nt_rowscaled_ws(ptr(a), ptr(sa), sa.stride(0), sa.stride(1), ptr(b), ptr(sb), sb.stride(0), sb.stride(1),
+                                                 ptr(out), M, N, K, fmt, 0, ptr(ws), ws.numel() if ws is not None else 0,
+                                                 stream_ptr(dev)), who)
 
 
 def fp8_matmul_bwd(xt, w, dy, dyt, scale_xt, scale_w, scale_dy, scale_dyt):
@@ -338,10 +344,7 @@ def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8):
         if qdyt.size(1) == 0:
             dw.zero_()                                   # no tokens: an empty sum
         elif N * K > 0:
-            with on_device(dev):
-                check(lib().mdy_fp8_gemm_nt_rowscaled(ptr(qdyt), ptr(sdyt), sdyt.stride(0), sdyt.stride(1), ptr(qxt), ptr(sxt),
-                                                      sxt.stride(0), sxt.stride(1), ptr(dw), N, K, qdyt.size(1), fmt, 0,
-                                                      stream_ptr(dev)), "Fp8Linear.backward")
+            _rowscaled_into(dw, qdyt, sdyt, qxt, sxt, N, K, qdyt.size(1), fmt, dev, "Fp8Linear.backward")
     return dx, dw
 
 
