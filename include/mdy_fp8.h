@@ -265,6 +265,16 @@ int mdy_fp8_gemm_nt_ws(const void* a, const float* a_s, int64_t as_row_stride, i
                        const void* b, const float* b_s, void* c, const void* bias, int64_t M, int64_t N,
                        int64_t K, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same GEMM with every choice in the argument list: operand format fmt (MDY_FMT_E5M2: the conditions of
+ * mdy_fp8_gemm_nt_e5m2, MDY_E_SHAPE otherwise), a workspace as in mdy_fp8_gemm_nt_ws (NULL: none), and how the bias is added:
+ * MDY_BIAS_IN_SUM to the fp32 sum before it is rounded, MDY_BIAS_AFTER_ROUNDING (bf16 results only) to the sum rounded to bf16,
+ * the bits of mdy_add_bias on the product without a pass over it (fp8.py:310-311 calls the two one after the other). */
+#define MDY_BIAS_IN_SUM 0
+#define MDY_BIAS_AFTER_ROUNDING 1
+int mdy_fp8_gemm_nt_ex(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,
+                       const float* b_s, void* c, const void* bias, int bias_mode, int64_t M, int64_t N, int64_t K, int fmt,
+                       int out_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Which kernel family mdy_fp8_gemm_nt (with_workspace = 0) or mdy_fp8_gemm_nt_ws with a sufficient workspace
  * (with_workspace = 1) runs for these operands; launches nothing, needs no GPU.  No counterpart in the reference
  * (its Triton kernel has one code path); the Python wrappers use it to warn when a large shape would take the

@@ -38,6 +38,7 @@ SIGNATURES = {
     "mdy_weight_dequant_block": [_p, _p, _p, _i64, _i64, _int, _int, _p],
     "mdy_fp8_gemm_nt": [_p, _p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _i64, _int, _p],
     "mdy_fp8_gemm_nt_e5m2": [_p, _p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _i64, _int, _p],
+    "mdy_fp8_gemm_nt_ex": [_p, _p, _i64, _i64, _p, _p, _p, _p, _int, _i64, _i64, _i64, _int, _int, _p, _i64, _p],
     "mdy_fp8_gemm_nt_ws": [_p, _p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _i64, _int, _p, _i64, _p],
     "mdy_fp8_gemm_workspace_bytes": [_i64, _i64, _i64],
     "mdy_fp8_gemm_path": [_p, _p, _i64, _i64, _i64, _i64, _i64, _int],

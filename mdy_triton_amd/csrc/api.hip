@@ -46,6 +46,8 @@ int check_device() {
     return 0;
 }
 
+mdy::Bias bias_of(const void* bias, int after_rounding = 0) { return mdy::Bias{static_cast<const uint16_t*>(bias), bias ? after_rounding : 0}; }
+
 }  // namespace
 
 extern "C" {
@@ -260,8 +262,8 @@ int mdy_fp8_gemm_nt(const void* a, const float* a_s, int64_t as_row_stride, int6
     if (!aligned(c, out_dtype == MDY_DT_BF16 ? 2 : 4) || !aligned(a_s, 4) || !aligned(b_s, 4) || (bias && !aligned(bias, 2)))
         return fail(MDY_E_ALIGN, "fp8_gemm_nt: misaligned pointer");
     if (int e = check_device()) return e;
-    return launched(mdy::launch_fp8_gemm_nt(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias, M, N, K, out_dtype,
-                                            static_cast<hipStream_t>(stream)),
+    return launched(mdy::launch_fp8_gemm_nt(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias_of(bias), M, N, K, 0, out_dtype,
+                                            nullptr, 0, static_cast<hipStream_t>(stream)),
                     "fp8_gemm_nt");
 }
 
@@ -276,12 +278,34 @@ int mdy_fp8_gemm_nt_e5m2(const void* a, const float* a_s, int64_t as_row_stride,
     if (!aligned(c, out_dtype == MDY_DT_BF16 ? 2 : 4) || !aligned(a_s, 4) || !aligned(b_s, 4) || (bias && !aligned(bias, 2)))
         return fail(MDY_E_ALIGN, "fp8_gemm_nt_e5m2: misaligned pointer");
     if (int e = check_device()) return e;
-    const int rc = mdy::launch_fp8_gemm_nt_e5m2(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias, M, N, K, out_dtype,
-                                                static_cast<hipStream_t>(stream));
+    const int rc = mdy::launch_fp8_gemm_nt(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias_of(bias), M, N, K, 1, out_dtype, nullptr, 0,
+                                           static_cast<hipStream_t>(stream));
     if (rc == -1)
         return fail(MDY_E_SHAPE, "fp8_gemm_nt_e5m2: needs K a multiple of 128 up to 65536, 16-byte aligned a and b, activation scales within 2^31 bytes "
                     "(other e5m2 problems: mdy_fp8_gemm_nt_rowscaled with the weight scales expanded to one per row)");
     return launched(rc, "fp8_gemm_nt_e5m2");
+}
+
+int mdy_fp8_gemm_nt_ex(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b, const float* b_s,
+                       void* c, const void* bias, int bias_mode, int64_t M, int64_t N, int64_t K, int fmt, int out_dtype,
+                       void* workspace, int64_t workspace_bytes, void* stream) {
+    if (out_dtype != MDY_DT_BF16 && out_dtype != MDY_DT_F32) return fail(MDY_E_DTYPE, "fp8_gemm_nt_ex: unknown out_dtype %d", out_dtype);
+    if (fmt != MDY_FMT_E4M3 && fmt != MDY_FMT_E5M2) return fail(MDY_E_DTYPE, "fp8_gemm_nt_ex: unknown operand format %d", fmt);
+    if (bias_mode != MDY_BIAS_IN_SUM && (bias_mode != MDY_BIAS_AFTER_ROUNDING || out_dtype != MDY_DT_BF16))
+        return fail(MDY_E_DTYPE, "fp8_gemm_nt_ex: bias_mode %d with out_dtype %d", bias_mode, out_dtype);
+    if (M < 0 || N < 0 || K < 1 || M > kMaxDim || N > kMaxDim || K > kMaxDim)
+        return fail(MDY_E_SHAPE, "fp8_gemm_nt_ex: bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
+    if (workspace_bytes < 0) return fail(MDY_E_SHAPE, "fp8_gemm_nt_ex: workspace_bytes < 0");
+    if (M == 0 || N == 0) return 0;
+    if (!a || !a_s || !b || !b_s || !c) return fail(MDY_E_NULL, "fp8_gemm_nt_ex: null pointer");
+    if (!aligned(c, out_dtype == MDY_DT_BF16 ? 2 : 4) || !aligned(a_s, 4) || !aligned(b_s, 4) || (bias && !aligned(bias, 2)))
+        return fail(MDY_E_ALIGN, "fp8_gemm_nt_ex: misaligned pointer");
+    if (workspace && !aligned(workspace, 16)) return fail(MDY_E_ALIGN, "fp8_gemm_nt_ex: workspace must be 16-byte aligned");
+    if (int e = check_device()) return e;
+    const int rc = mdy::launch_fp8_gemm_nt(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias_of(bias, bias_mode), M, N, K, fmt,
+                                           out_dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+    if (rc == -1) return fail(MDY_E_SHAPE, "fp8_gemm_nt_ex: e5m2 operands need what mdy_fp8_gemm_nt_e5m2 needs");
+    return launched(rc, "fp8_gemm_nt_ex");
 }
 
 int64_t mdy_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -302,8 +326,8 @@ int mdy_fp8_gemm_nt_ws(const void* a, const float* a_s, int64_t as_row_stride, i
         return fail(MDY_E_ALIGN, "fp8_gemm_nt_ws: misaligned pointer");
     if (workspace && !aligned(workspace, 16)) return fail(MDY_E_ALIGN, "fp8_gemm_nt_ws: workspace must be 16-byte aligned");
     if (int e = check_device()) return e;
-    return launched(mdy::launch_fp8_gemm_nt_ws(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias, M, N, K, out_dtype,
-                                               workspace, workspace_bytes, static_cast<hipStream_t>(stream)),
+    return launched(mdy::launch_fp8_gemm_nt(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias_of(bias), M, N, K, 0, out_dtype,
+                                            workspace, workspace_bytes, static_cast<hipStream_t>(stream)),
                     "fp8_gemm_nt_ws");
 }
 
@@ -338,7 +362,7 @@ int mdy_fp8_gemm_nt_static_ws(const void* a, const float* a_s, int64_t as_row_st
                     "use mdy_fp8_gemm_nt_ws with a caller-owned workspace (or mdy_fp8_gemm_nt)",
                     (long long)M, (long long)N, (long long)K, (long long)need, (long long)mdy::kStaticScratchBytes);
     if (int e = check_device()) return e;
-    return launched(mdy::launch_fp8_gemm_nt_static(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias, M, N, K, out_dtype,
+    return launched(mdy::launch_fp8_gemm_nt_static(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias_of(bias), M, N, K, out_dtype,
                                                    static_cast<hipStream_t>(stream)),
                     "fp8_gemm_nt_static_ws");
 }
@@ -362,7 +386,7 @@ int mdy_fp8_grouped_gemm_nt(const void* a, const float* a_s, int64_t as_row_stri
     if (!aligned(c, out_dtype == MDY_DT_BF16 ? 2 : 4) || !aligned(a_s, 4) || !aligned(b_s, 4) || (bias && !aligned(bias, 2)))
         return fail(MDY_E_ALIGN, "fp8_grouped_gemm_nt: misaligned pointer");
     if (int e = check_device()) return e;
-    return launched(mdy::launch_fp8_grouped_gemm_nt(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias, m_splits, G, M, N, K,
+    return launched(mdy::launch_fp8_grouped_gemm_nt(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias_of(bias), m_splits, G, M, N, K,
                                                     out_dtype, static_cast<hipStream_t>(stream)),
                     "fp8_grouped_gemm_nt");
 }

@@ -238,6 +238,18 @@ __device__ __forceinline__ uint32_t pack2_bf16(float a, float b) {
     return __builtin_bit_cast(uint32_t, h);
 }
 
+// The bias of a GEMM, bf16 [N]; p == nullptr: none.  It is added to the fp32 sum, which is then rounded once; with
+// after_rounding the sum is rounded to bf16 first: the bits of add_bias on a bf16 product, without a pass over it.
+struct Bias {
+    const uint16_t* p = nullptr;
+    int after_rounding = 0;
+    __host__ __device__ Bias at(int64_t n) const { return Bias{p != nullptr ? p + n : nullptr, after_rounding}; }
+    __device__ __forceinline__ float add(float v, int n) const {
+        if (after_rounding) v = bf16_lo(pack2_bf16(v, 0.0f));
+        return v + bf16_one(p[n]);
+    }
+};
+
 // Blocks that tile a matrix, nx wide and ny high (x fastest): grid.y takes at most 65535 blocks and a token
 // dimension can need more, so the block rows beyond kGridRowChunk continue in grid.z.  The last z slice may
 // reach past ny: kernels drop block rows >= ny.  (A 1-D grid with a division per block measured 3-7 % slower
@@ -280,28 +292,22 @@ int launch_swiglu_bwd(const void* x, const void* dy, void* dx, int64_t M, int64_
                       int gate_first, hipStream_t stream);
 int launch_weight_dequant(const void* x, const float* s, void* y, int64_t N, int64_t K, int block_size, int out_dtype,
                           hipStream_t stream);
-int launch_fp8_gemm_nt(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride,
-                       const void* b, const float* b_s, void* c, const void* bias, int64_t M, int64_t N,
-                       int64_t K, int out_dtype, hipStream_t stream);
-int launch_fp8_gemm_nt_e5m2(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride,
-                            const void* b, const float* b_s, void* c, const void* bias, int64_t M, int64_t N,
-                            int64_t K, int out_dtype, hipStream_t stream);
+int launch_fp8_gemm_nt(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,
+                       const float* b_s, void* c, Bias bias, int64_t M, int64_t N, int64_t K, int fmt, int out_dtype,
+                       void* workspace, int64_t workspace_bytes, hipStream_t stream);
 int cu_count();      // compute units of the current device
-int launch_splitk_reduce(const float* ws, void* c, int out_dtype, const uint16_t* bias, int64_t M, int64_t N, int ksplit, hipStream_t stream);
+int launch_splitk_reduce(const float* ws, void* c, int out_dtype, Bias bias, int64_t M, int64_t N, int ksplit, hipStream_t stream);
 int64_t fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
-int launch_fp8_gemm_nt_ws(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride,
-                          const void* b, const float* b_s, void* c, const void* bias, int64_t M, int64_t N,
-                          int64_t K, int out_dtype, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 int fp8_gemm_path(const void* a, const void* b, int64_t as_rs, int64_t as_cs, int64_t M, int64_t N, int64_t K,
                   int with_workspace);
 // static device scratch of the no-allocation GEMM entry point (defined in fp8_gemm.hip)
 constexpr int64_t kStaticScratchBytes = (int64_t)32 << 20;
 int static_scratch_ptr(void** out);
 int launch_fp8_gemm_nt_static(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride,
-                              const void* b, const float* b_s, void* c, const void* bias, int64_t M, int64_t N,
+                              const void* b, const float* b_s, void* c, Bias bias, int64_t M, int64_t N,
                               int64_t K, int out_dtype, hipStream_t stream);
 int launch_fp8_grouped_gemm_nt(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride,
-                               const void* b, const float* b_s, void* c, const void* bias, const int64_t* m_splits,
+                               const void* b, const float* b_s, void* c, Bias bias, const int64_t* m_splits,
                                int64_t G, int64_t M, int64_t N, int64_t K, int out_dtype, hipStream_t stream);
 int launch_group_pad(const void* x, void* y, const int64_t* m_splits, int64_t G, int64_t row_bytes, int64_t multiple,
                      int unpad, hipStream_t stream);

@@ -48,7 +48,7 @@ namespace mdy {
 // into slab ks of a caller-provided workspace [ksplit][M][N]; splitk_reduce_kernel then adds the slabs in
 // slab order (so the result does not depend on scheduling), adds the bias and converts.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int WGM, int WGN, int STAGES>
+template <int BM, int BN, int WGM, int WGN, int STAGES, int FMT>
 __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_splitk_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, float* __restrict__ ws, int M, int N, int K,
@@ -61,14 +61,14 @@ __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_splitk_kernel(
     int tm, tn;
     const Duty duty = tile_of(pid - ks * ntiles, tiles_m, tiles_n, tm, tn);
     const int kb0 = ks * kb_per, kb1 = min(K >> 7, kb0 + kb_per);
-    fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, float>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, nullptr,
+    fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, float, 0, 0, 0, FMT>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, Bias{},
                                                    tm * BM, M, M, tn * BN, N, K, N, duty, kb0, kb1, pool);
 }
 
 // The same on the producer / consumer tile (128x128 and 128x64 tiles, 4 consumer + 4 producer waves): against the one-body
 // tile, after a cache flush / back to back, results identical: 512x4096x7168 42.6 -> 36.5 / 32.1 -> 29.4 us, 256x7168x18432
 // 89.9 -> 74.1 / 57.9 -> 53.2 us, 128x2112x7168 20.4 -> 19.2 / 15.6 -> 14.4 us, 96x4096x7168 25.3 -> 24.4 / 17.3 -> 15.4 us.
-template <int BM, int BN, int STAGES>
+template <int BM, int BN, int STAGES, int FMT>
 __global__ __launch_bounds__(512) void fp8_gemm_splitk_ws_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, float* __restrict__ ws, int M, int N, int K,
@@ -82,13 +82,13 @@ __global__ __launch_bounds__(512) void fp8_gemm_splitk_ws_kernel(
     int tm, tn;
     const Duty duty = tile_of(pid - ks * ntiles, tiles_m, tiles_n, tm, tn);
     const int kb0 = ks * kb_per, kb1 = min(K >> 7, kb0 + kb_per);
-    fp8_gemm_tile_ws<BM, BN, 2, 2, 4, STAGES, float>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, nullptr, tm * BM, M, M,
+    fp8_gemm_tile_ws<BM, BN, 2, 2, 4, STAGES, float, FMT>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, Bias{}, tm * BM, M, M,
                                                      tn * BN, N, K, N, duty, kb0, kb1, pool);
 }
 
 template <typename OUT, bool VEC>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, OUT* __restrict__ c,
-                                                            const uint16_t* __restrict__ bias, int64_t MN, int N,
+                                                            const Bias bias, int64_t MN, int N,
                                                             int ksplit) {
     const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * (VEC ? 4 : 1);
     if (i >= MN) return;
@@ -102,9 +102,9 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
             for (int kk = 0; kk < 4; ++kk)
                 if (k0 + kk < ksplit) { s.x += v[kk].x; s.y += v[kk].y; s.z += v[kk].z; s.w += v[kk].w; }
         }
-        if (bias != nullptr) {
+        if (bias.p != nullptr) {
             const int n = (int)(i % N);
-            s.x += bf16_one(bias[n]); s.y += bf16_one(bias[n + 1]); s.z += bf16_one(bias[n + 2]); s.w += bf16_one(bias[n + 3]);
+            s.x = bias.add(s.x, n); s.y = bias.add(s.y, n + 1); s.z = bias.add(s.z, n + 2); s.w = bias.add(s.w, n + 3);
         }
         if (sizeof(OUT) == 2)
             *reinterpret_cast<uint2*>(c + i) = make_uint2(pack2_bf16(s.x, s.y), pack2_bf16(s.z, s.w));
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     } else {
         float s = ws[i];
         for (int k = 1; k < ksplit; ++k) s += ws[(int64_t)k * MN + i];
-        if (bias != nullptr) s += bf16_one(bias[i % N]);
+        if (bias.p != nullptr) s = bias.add(s, (int)(i % N));
         if (sizeof(OUT) == 2)
             reinterpret_cast<uint16_t*>(c)[i] = (uint16_t)(pack2_bf16(s, 0.0f) & 0xFFFFu);
         else
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 }
 
 // slabs [ksplit][M][N] of partial sums -> c [M][N] of out_dtype (0 bf16, 1 fp32)
-int launch_splitk_reduce(const float* ws, void* c, int out_dtype, const uint16_t* bias, int64_t M, int64_t N, int ksplit, hipStream_t stream) {
+int launch_splitk_reduce(const float* ws, void* c, int out_dtype, const Bias bias, int64_t M, int64_t N, int ksplit, hipStream_t stream) {
     const int64_t MN = M * N;
     const bool vec = (N % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
     const dim3 grid((unsigned)((MN / (vec ? 4 : 1) + 255) / 256));
@@ -154,7 +154,7 @@ template <typename OUT>
 __global__ __launch_bounds__(512) void fp8_grouped_gemm_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
-    const uint16_t* __restrict__ bias, int N, int K, int tiles_n, const GroupTable tbl) {
+    const Bias bias, int N, int K, int tiles_n, const GroupTable tbl) {
     constexpr int kBig = TileLds<256, 256, 8, 2>::bytes, kSmall = TileLds<128, 256, 8, 3>::bytes;
     __shared__ __attribute__((aligned(1024))) uint8_t pool[kBig > kSmall ? kBig : kSmall];
     const int G = tbl.n_groups;
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(512) void fp8_grouped_gemm_kernel(
     const int n0 = __builtin_amdgcn_readfirstlane(tn * 256);
     const uint8_t* bg = b + (size_t)g * N * K;
     const float* bsg = b_s + (size_t)g * NB * KB;
-    const uint16_t* biasg = bias ? bias + (size_t)g * N : nullptr;
+    const Bias biasg = bias.at((size_t)g * N);
     if (r1 - m0 <= 128)
         fp8_gemm_tile<128, 256, 2, 4, 3, OUT>(a, a_s, as_rs, as_cs, as_bytes, bg, bsg, c, biasg, m0, r1, m_total, n0, N, K, N, duty, 0, KB, pool);
     else
@@ -207,7 +207,7 @@ constexpr int kSmWaves = 8;      // waves per workgroup of the small-M kernels
 template <int MT, int NC, int UF, typename OUT, int FMT, bool HALF = false, int WK = kSmWaves>
 __device__ __forceinline__ void smallm_lines_body(const uint8_t* __restrict__ a, const float* __restrict__ a_s, int64_t as_rs, int64_t as_cs,
                                                   const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
-                                                  const uint16_t* __restrict__ bias, int M, int N, int K, int kb_lo = 0,
+                                                  const Bias bias, int M, int N, int K, int kb_lo = 0,
                                                   int kb_hi = -1) {
     constexpr int SUB = NC * MT, TILES = NC + MT;      // (column group, row sub-tile) pairs; 16-row operand tiles per K block
     // WK waves share out the K blocks of one set of columns; with a short K (fewer blocks than waves) the 8 waves form
@@ -338,10 +338,10 @@ __device__ __forceinline__ void smallm_lines_body(const uint8_t* __restrict__ a,
             v[e] = t;
         }
         const int m = i * 16 + frow, n = n0 + 16 * j + 4 * fk;
-        if (bias != nullptr) {
+        if (bias.p != nullptr) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (n + e < N) v[e] += bf16_one(bias[n + e]);
+                if (n + e < N) v[e] = bias.add(v[e], n + e);
         }
         if (!HALF || fk < 2) store4<OUT>(c, N, m, n, M, N, v, vec_ok);      // HALF: columns 8 .. 15 of the tile belong to the next workgroup
     }
@@ -351,20 +351,20 @@ template <int MT, int NC, int UF, typename OUT, int FMT>
 __global__ __launch_bounds__(kSmWaves * 64) void fp8_gemm_smallm_lines_kernel(const uint8_t* __restrict__ a, const float* __restrict__ a_s,
                                                                                int64_t as_rs, int64_t as_cs, const uint8_t* __restrict__ b,
                                                                                const float* __restrict__ b_s, OUT* __restrict__ c,
-                                                                               const uint16_t* __restrict__ bias, int M, int N, int K) {
+                                                                               const Bias bias, int M, int N, int K) {
     smallm_lines_body<MT, NC, UF, OUT, FMT>(a, a_s, as_rs, as_cs, b, b_s, c, bias, M, N, K);
 }
 
 // 33..64 rows against a narrow weight and a long K: K is cut into slabs as well (grid row = slab), workgroup (32 columns, slab)
 // writes the fp32 partial sums of its K blocks into slab blockIdx.y of a workspace [slabs][M][N], and splitk_reduce_kernel adds
 // the slabs in slab order.
-template <int UF>
+template <int UF, int FMT>
 __global__ __launch_bounds__(kSmWaves * 64) void fp8_gemm_smallm_lines_slab_kernel(const uint8_t* __restrict__ a, const float* __restrict__ a_s,
                                                                                     int64_t as_rs, int64_t as_cs, const uint8_t* __restrict__ b,
                                                                                     const float* __restrict__ b_s, float* __restrict__ ws, int M,
                                                                                     int N, int K, int kb_per) {
     const int kb_lo = blockIdx.y * kb_per;
-    smallm_lines_body<4, 2, UF, float, 0>(a, a_s, as_rs, as_cs, b, b_s, ws + (size_t)blockIdx.y * M * N, nullptr, M, N, K, kb_lo,
+    smallm_lines_body<4, 2, UF, float, FMT>(a, a_s, as_rs, as_cs, b, b_s, ws + (size_t)blockIdx.y * M * N, Bias{}, M, N, K, kb_lo,
                                           min(K >> 7, kb_lo + kb_per));
 }
 
@@ -372,7 +372,7 @@ __global__ __launch_bounds__(kSmWaves * 64) void fp8_gemm_smallm_lines_slab_kern
 template <int UF, typename OUT, int FMT>
 __global__ __launch_bounds__(kSmWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void fp8_gemm_smallm_lines_occ2_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int64_t as_rs, int64_t as_cs, const uint8_t* __restrict__ b,
-    const float* __restrict__ b_s, OUT* __restrict__ c, const uint16_t* __restrict__ bias, int M, int N, int K) {
+    const float* __restrict__ b_s, OUT* __restrict__ c, const Bias bias, int M, int N, int K) {
     smallm_lines_body<1, 2, UF, OUT, FMT>(a, a_s, as_rs, as_cs, b, b_s, c, bias, M, N, K);
 }
 
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(kSmWaves * 64) void fp8_gemm_smallm_lines_shortk_ke
                                                                                       const float* __restrict__ a_s, int64_t as_rs,
                                                                                       int64_t as_cs, const uint8_t* __restrict__ b,
                                                                                       const float* __restrict__ b_s, OUT* __restrict__ c,
-                                                                                      const uint16_t* __restrict__ bias, int M, int N, int K) {
+                                                                                      const Bias bias, int M, int N, int K) {
     smallm_lines_body<1, NC, UF, OUT, FMT, false, WK>(a, a_s, as_rs, as_cs, b, b_s, c, bias, M, N, K);
 }
 
@@ -391,7 +391,7 @@ template <int UF, typename OUT, int FMT>
 __global__ __launch_bounds__(kSmWaves * 64) void fp8_gemm_smallm_lines_half_kernel(const uint8_t* __restrict__ a, const float* __restrict__ a_s,
                                                                                     int64_t as_rs, int64_t as_cs, const uint8_t* __restrict__ b,
                                                                                     const float* __restrict__ b_s, OUT* __restrict__ c,
-                                                                                    const uint16_t* __restrict__ bias, int M, int N, int K) {
+                                                                                    const Bias bias, int M, int N, int K) {
     smallm_lines_body<1, 1, UF, OUT, FMT, true>(a, a_s, as_rs, as_cs, b, b_s, c, bias, M, N, K);
 }
 
@@ -405,7 +405,7 @@ template <int MT, int NC, int UF, typename OUT>
 __global__ __launch_bounds__(kSmWaves * 64) void fp8_grouped_lines_kernel(const uint8_t* __restrict__ a, const float* __restrict__ a_s,
                                                                            int64_t as_rs, int64_t as_cs, const uint8_t* __restrict__ b,
                                                                            const float* __restrict__ b_s, OUT* __restrict__ c,
-                                                                           const uint16_t* __restrict__ bias, int N, int K,
+                                                                           const Bias bias, int N, int K,
                                                                            const GroupRows rows) {
     const int g = blockIdx.y;
     const int r0 = __builtin_amdgcn_readfirstlane(rows.row_start[g]);
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(kSmWaves * 64) void fp8_grouped_lines_kernel(const 
     if (M <= 0) return;      // uniform in the workgroup
     const int KB = K >> 7, NB = (N + 127) >> 7;
     smallm_lines_body<MT, NC, UF, OUT, 0>(a + (size_t)r0 * K, a_s + (int64_t)r0 * as_rs, as_rs, as_cs, b + (size_t)g * N * K,
-                                          b_s + (size_t)g * NB * KB, c + (size_t)r0 * N, bias ? bias + (size_t)g * N : nullptr, M, N, K);
+                                          b_s + (size_t)g * NB * KB, c + (size_t)r0 * N, bias.at((size_t)g * N), M, N, K);
 }
 
 // ---------------------------------------------------------------------------
@@ -447,7 +447,7 @@ __device__ __forceinline__ void fp8x4_to_f32(uint32_t w, float (&f)[4]) {
 template <int MR, int R, typename OUT, int FMT>
 __global__ __launch_bounds__(512) void fp8_gemv_kernel(const uint8_t* __restrict__ a, const float* __restrict__ a_s, int64_t as_rs,
                                                         int64_t as_cs, const uint8_t* __restrict__ b, const float* __restrict__ b_s,
-                                                        OUT* __restrict__ c, const uint16_t* __restrict__ bias, int N, int K) {
+                                                        OUT* __restrict__ c, const Bias bias, int N, int K) {
     __shared__ __attribute__((aligned(16))) uint8_t lds_x[MR * kGemvMaxK];
     __shared__ float lds_sa[MR * (kGemvMaxK / 128)];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(512) void fp8_gemv_kernel(const uint8_t* __restrict
             for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
             const int n = n0 + r;
             if (lane == 0 && n < N) {
-                if (bias != nullptr) v += bf16_one(bias[n]);
+                if (bias.p != nullptr) v = bias.add(v, n);
                 if (sizeof(OUT) == 2)
                     reinterpret_cast<uint16_t*>(c)[(int64_t)m * N + n] = (uint16_t)(pack2_bf16(v, 0.0f) & 0xFFFFu);
                 else
@@ -563,7 +563,7 @@ template <int MT, typename OUT, int FMT = 0, int KC_ = kStripKC>
 __global__ __launch_bounds__(512) void fp8_gemm_strip_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
-    const uint16_t* __restrict__ bias, int N, int K, const GroupTable tbl) {
+    const Bias bias, int N, int K, const GroupTable tbl) {
     constexpr int ROWS = MT * 16, KC = KC_;
     constexpr int CPW = KC * MT / 4;      // activation copy instructions (8 rows x one K block) per wave and step
     static_assert(CPW * 4 == KC * MT, "the step's copies divide evenly among the 8 waves");
@@ -685,15 +685,15 @@ __global__ __launch_bounds__(512) void fp8_gemm_strip_kernel(
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     const bool vec_ok = (N % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
-    const uint16_t* gbias = bias ? bias + (size_t)g * N : nullptr;
+    const Bias gbias = bias.at((size_t)g * N);
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const int m = r0 + i * 16 + frow, n = n0 + wave * 16 + 4 * fk;
         float v[4] = {acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
-        if (gbias != nullptr) {
+        if (gbias.p != nullptr) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (n + e < N) v[e] += bf16_one(gbias[n + e]);
+                if (n + e < N) v[e] = gbias.add(v[e], n + e);
         }
         store4<OUT>(c, N, m, n, r1, N, v, vec_ok);
     }
@@ -713,7 +713,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_scalar_kernel(const uint8_t* __r
                                                                const float* __restrict__ a_s, int64_t as_rs,
                                                                int64_t as_cs, const uint8_t* __restrict__ b,
                                                                const float* __restrict__ b_s, OUT* __restrict__ c,
-                                                               const uint16_t* __restrict__ bias, int M, int N, int K) {
+                                                               const Bias bias, int M, int N, int K) {
     const int n = blockIdx.x * 16 + (threadIdx.x & 15);
     const int m = block_row() * 16 + (threadIdx.x >> 4);
     if (m >= M || n >= N) return;
@@ -727,7 +727,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_scalar_kernel(const uint8_t* __r
         const float sc = a_s[(int64_t)m * as_rs + (int64_t)kb * as_cs] * b_s[(int64_t)(n >> 7) * KB + kb];
         acc = __builtin_fmaf(p, sc, acc);
     }
-    if (bias != nullptr) acc += bf16_one(bias[n]);
+    if (bias.p != nullptr) acc = bias.add(acc, n);
     if (sizeof(OUT) == 2)
         reinterpret_cast<uint16_t*>(c)[(int64_t)m * N + n] = (uint16_t)(pack2_bf16(acc, 0.0f) & 0xFFFFu);
     else
@@ -764,7 +764,7 @@ static bool pretouch_enabled() {
 
 template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int FMT = 0>
 static int launch_mfma(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t as_cs, uint32_t as_bytes,
-                       const uint8_t* b, const float* b_s, OUT* c, const uint16_t* bias, int M, int N, int K,
+                       const uint8_t* b, const float* b_s, OUT* c, const Bias bias, int M, int N, int K,
                        int ldc, hipStream_t stream) {
     const int cus = cu_count();
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
@@ -840,7 +840,7 @@ static int few_tiles_config(int M, int N, int K) {
 
 template <typename OUT, int FMT = 0>
 static int launch_strip(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t as_cs, uint32_t as_bytes,
-                        const uint8_t* b, const float* b_s, OUT* c, const uint16_t* bias, const int64_t* m_splits, int G,
+                        const uint8_t* b, const float* b_s, OUT* c, const Bias bias, const int64_t* m_splits, int G,
                         int max_rows, int N, int K, hipStream_t stream) {
     GroupTable tbl;
     tbl.n_groups = G;
@@ -890,7 +890,7 @@ static bool strip_pays(int64_t max_rows, int64_t strips) { return max_rows > 4 &
 // 32-bit addressing).  FMT: operand byte format, 0 e4m3fn, 1 e5m2.
 template <typename OUT, int FMT>
 static int dispatch_small(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t as_cs, int64_t as_extent, bool big_ok,
-                          const uint8_t* b, const float* b_s, OUT* c, const uint16_t* bias, int M, int N, int K, hipStream_t stream) {
+                          const uint8_t* b, const float* b_s, OUT* c, const Bias bias, int M, int N, int K, hipStream_t stream) {
     if (gemv_pays(M, K)) {
         dim3 grid((unsigned)((N + 7) / 8)), block(512);      // one weight row per wave
         hipLaunchKernelGGL((fp8_gemv_kernel<1, 1, OUT, FMT>), grid, block, 0, stream, a, a_s, as_rs, as_cs, b, b_s, c, bias, N, K);
@@ -1021,7 +1021,7 @@ static int dispatch_small(const uint8_t* a, const float* a_s, int64_t as_rs, int
 // checks).  FMT: operand byte format, 0 e4m3fn, 1 e5m2.
 template <typename OUT, int FMT>
 static int dispatch_tiles(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t as_cs, int64_t as_extent, const uint8_t* b,
-                          const float* b_s, OUT* c, const uint16_t* bias, int M, int N, int K, hipStream_t stream) {
+                          const float* b_s, OUT* c, const Bias bias, int M, int N, int K, hipStream_t stream) {
     const int KB = K / 128;
     if (big_tiles_pay(M, N)) {
         const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
@@ -1034,7 +1034,7 @@ static int dispatch_tiles(const uint8_t* a, const float* a_s, int64_t as_rs, int
         // call); n_main is a multiple of 256, so every pointer below keeps its alignment
         return launch_mfma<128, 256, 2, 4, 3, OUT, FMT>(a, a_s, as_rs, as_cs, (uint32_t)as_extent, b + (size_t)n_main * K,
                                                      b_s + (size_t)(n_main >> 7) * KB, c + n_main,
-                                                     bias ? bias + n_main : nullptr, M, N - n_main, K, N, stream);
+                                                     bias.at(n_main), M, N - n_main, K, N, stream);
     }
     // Fewer tiles than that: the workgroups no longer fill the CUs, every K block's copy latency shows, and
     // the time goes with K.  Use the LDS that the missing co-resident workgroups leave free for a deeper ring of
@@ -1062,15 +1062,17 @@ static int dispatch_tiles(const uint8_t* a, const float* a_s, int64_t as_rs, int
 #undef MDY_FEW
 }
 
-template <typename OUT>
+// FMT 1 (e5m2) has no scalar kernel: -1 when the operands do not qualify for the MFMA kernels.
+template <typename OUT, int FMT = 0>
 static int dispatch(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t as_cs, const uint8_t* b,
-                    const float* b_s, OUT* c, const uint16_t* bias, int M, int N, int K, hipStream_t stream) {
+                    const float* b_s, OUT* c, const Bias bias, int M, int N, int K, hipStream_t stream) {
     const int KB = (K + 127) / 128;
     // byte extent of the activation scales as the MFMA kernel addresses them
     const int64_t as_extent = ((int64_t)(M - 1) * as_rs + (int64_t)(KB - 1) * as_cs + 1) * 4;
     const bool mfma_ok = (K % 128 == 0) && ((reinterpret_cast<uintptr_t>(a) & 15) == 0) &&
                          ((reinterpret_cast<uintptr_t>(b) & 15) == 0);
     const bool big_ok = mfma_ok && K <= (1 << 16) && as_rs >= 0 && as_cs >= 0 && as_extent < ((int64_t)1 << 31);
+    if (FMT != 0 && !big_ok) return -1;
     if (!mfma_ok || (M > 64 && !big_ok)) {
         dim3 grid;
         if (!grid_rows((N + 15) / 16, (M + 15) / 16, grid)) return kErrTooManyBlocks;
@@ -1078,8 +1080,8 @@ static int dispatch(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t a
                            bias, M, N, K);
         return (int)hipGetLastError();
     }
-    if (M <= 64) return dispatch_small<OUT, 0>(a, a_s, as_rs, as_cs, as_extent, big_ok, b, b_s, c, bias, M, N, K, stream);
-    return dispatch_tiles<OUT, 0>(a, a_s, as_rs, as_cs, as_extent, b, b_s, c, bias, M, N, K, stream);
+    if (M <= 64) return dispatch_small<OUT, FMT>(a, a_s, as_rs, as_cs, as_extent, big_ok, b, b_s, c, bias, M, N, K, stream);
+    return dispatch_tiles<OUT, FMT>(a, a_s, as_rs, as_cs, as_extent, b, b_s, c, bias, M, N, K, stream);
 }
 
 // ---- split-K plan: which tile, how many K slices; ksplit == 1 means "do not split"
@@ -1172,9 +1174,9 @@ int64_t fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 }
 
 // returns -1 when the shape / pointers do not qualify (the caller then runs the plain path)
-template <typename OUT>
+template <typename OUT, int FMT>
 static int launch_splitk(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t as_cs, const uint8_t* b,
-                         const float* b_s, OUT* c, const uint16_t* bias, int M, int N, int K, float* ws,
+                         const float* b_s, OUT* c, const Bias bias, int M, int N, int K, float* ws,
                          int64_t ws_bytes, hipStream_t stream) {
     const SplitPlan p = plan_split(M, N, K);
     if (p.ksplit < 2 || ws == nullptr || ws_bytes < (int64_t)p.ksplit * M * N * 4) return -1;
@@ -1187,23 +1189,23 @@ static int launch_splitk(const uint8_t* a, const float* a_s, int64_t as_rs, int6
 #define MDY_SPLIT(BM_, BN_, ST_)                                                                                      \
     {                                                                                                                 \
         const int tiles_m = (M + BM_ - 1) / BM_, tiles_n = (N + BN_ - 1) / BN_;                                       \
-        hipLaunchKernelGGL((fp8_gemm_splitk_kernel<BM_, BN_, 2, 2, ST_>), dim3((unsigned)(tiles_m * tiles_n * p.ksplit)), \
+        hipLaunchKernelGGL((fp8_gemm_splitk_kernel<BM_, BN_, 2, 2, ST_, FMT>), dim3((unsigned)(tiles_m * tiles_n * p.ksplit)), \
                            dim3(256), 0, stream, a, a_s, (int)as_rs, (int)as_cs, (uint32_t)as_extent, b, b_s, ws, M, N, K, \
                            tiles_m, tiles_n, p.ksplit, p.kb_per);                                                     \
     }
     if (p.config == 4) {
         dim3 grid((unsigned)((N + 31) / 32), (unsigned)p.ksplit);
         if (p.kb_per <= kSmWaves)
-            hipLaunchKernelGGL((fp8_gemm_smallm_lines_slab_kernel<1>), grid, dim3(kSmWaves * 64), 0, stream, a, a_s, as_rs, as_cs, b, b_s, ws,
+            hipLaunchKernelGGL((fp8_gemm_smallm_lines_slab_kernel<1, FMT>), grid, dim3(kSmWaves * 64), 0, stream, a, a_s, as_rs, as_cs, b, b_s, ws,
                                M, N, K, p.kb_per);
         else
-            hipLaunchKernelGGL((fp8_gemm_smallm_lines_slab_kernel<2>), grid, dim3(kSmWaves * 64), 0, stream, a, a_s, as_rs, as_cs, b, b_s, ws,
+            hipLaunchKernelGGL((fp8_gemm_smallm_lines_slab_kernel<2, FMT>), grid, dim3(kSmWaves * 64), 0, stream, a, a_s, as_rs, as_cs, b, b_s, ws,
                                M, N, K, p.kb_per);
     }
 #define MDY_SPLIT_WS(BM_, BN_, ST_)                                                                                   \
     {                                                                                                                 \
         const int tiles_m = (M + BM_ - 1) / BM_, tiles_n = (N + BN_ - 1) / BN_;                                       \
-        hipLaunchKernelGGL((fp8_gemm_splitk_ws_kernel<BM_, BN_, ST_>), dim3((unsigned)(tiles_m * tiles_n * p.ksplit)), \
+        hipLaunchKernelGGL((fp8_gemm_splitk_ws_kernel<BM_, BN_, ST_, FMT>), dim3((unsigned)(tiles_m * tiles_n * p.ksplit)), \
                            dim3(512), 0, stream, a, a_s, (int)as_rs, (int)as_cs, (uint32_t)as_extent, b, b_s, ws, M, N, K, \
                            tiles_m, tiles_n, p.ksplit, p.kb_per);                                                     \
     }
@@ -1217,36 +1219,45 @@ static int launch_splitk(const uint8_t* a, const float* a_s, int64_t as_rs, int6
     return launch_splitk_reduce(ws, c, sizeof(OUT) == 2 ? 0 : 1, bias, M, N, p.ksplit, stream);
 }
 
-int launch_fp8_gemm_nt_ws(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,
-                          const float* b_s, void* c, const void* bias, int64_t M, int64_t N, int64_t K, int out_dtype,
-                          void* workspace, int64_t workspace_bytes, hipStream_t stream) {
-    if (M == 0 || N == 0) return 0;
-    int rc = -1;
-    if (out_dtype == 0)
-        rc = launch_splitk<uint16_t>(static_cast<const uint8_t*>(a), a_s, as_row_stride, as_col_stride,
-                                     static_cast<const uint8_t*>(b), b_s, static_cast<uint16_t*>(c),
-                                     static_cast<const uint16_t*>(bias), (int)M, (int)N, (int)K,
-                                     static_cast<float*>(workspace), workspace_bytes, stream);
-    else
-        rc = launch_splitk<float>(static_cast<const uint8_t*>(a), a_s, as_row_stride, as_col_stride,
-                                  static_cast<const uint8_t*>(b), b_s, static_cast<float*>(c),
-                                  static_cast<const uint16_t*>(bias), (int)M, (int)N, (int)K,
-                                  static_cast<float*>(workspace), workspace_bytes, stream);
+template <typename OUT, int FMT>
+static int launch_nt(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t as_cs, const uint8_t* b, const float* b_s, OUT* c, const Bias bias,
+                     int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+    if (workspace == nullptr) return dispatch<OUT, FMT>(a, a_s, as_rs, as_cs, b, b_s, c, bias, (int)M, (int)N, (int)K, stream);
+    int rc = launch_splitk<OUT, FMT>(a, a_s, as_rs, as_cs, b, b_s, c, bias, (int)M, (int)N, (int)K, static_cast<float*>(workspace),
+                                     workspace_bytes, stream);
     if (rc >= 0) return rc;
     // no K split: with row-major activation scales and room in the workspace, hand the tile kernels a
     // transposed copy (C3: 505 -> 491 us, C4: 487 -> 466 us for a 3 us copy kernel)
     const int64_t need = scale_scratch_bytes(M, N, K);
-    if (need > 0 && workspace != nullptr && workspace_bytes >= need && as_col_stride == 1 && as_row_stride >= K / 128 &&
-        as_row_stride > 1 && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
+    if (need > 0 && workspace_bytes >= need && as_cs == 1 && as_rs >= K / 128 && as_rs > 1 && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
         const int KB = (int)(K / 128);
         float* ts = static_cast<float*>(workspace);
         hipLaunchKernelGGL(transpose_scales_kernel, dim3((unsigned)((M + 31) / 32), (unsigned)((KB + 31) / 32)), dim3(256), 0,
-                           stream, a_s, ts, (int)M, KB, as_row_stride);
+                           stream, a_s, ts, (int)M, KB, as_rs);
         rc = (int)hipGetLastError();
         if (rc != 0) return rc;
-        return launch_fp8_gemm_nt(a, ts, 1, M, b, b_s, c, bias, M, N, K, out_dtype, stream);
+        a_s = ts;
+        as_rs = 1;
+        as_cs = M;
     }
-    return launch_fp8_gemm_nt(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias, M, N, K, out_dtype, stream);
+    return dispatch<OUT, FMT>(a, a_s, as_rs, as_cs, b, b_s, c, bias, (int)M, (int)N, (int)K, stream);
+}
+
+// fmt: byte format of both operands, 0 e4m3fn, 1 e5m2 (-1: its operands do not qualify); workspace may be NULL
+int launch_fp8_gemm_nt(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,
+                       const float* b_s, void* c, Bias bias, int64_t M, int64_t N, int64_t K, int fmt, int out_dtype,
+                       void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+    if (M == 0 || N == 0) return 0;
+#define MDY_NT(OUT, FMT)                                                                                                        \
+    return launch_nt<OUT, FMT>(static_cast<const uint8_t*>(a), a_s, as_row_stride, as_col_stride, static_cast<const uint8_t*>(b), b_s, \
+                               static_cast<OUT*>(c), bias, M, N, K, workspace, workspace_bytes, stream)
+    if (out_dtype == 0) {
+        if (fmt == 0) MDY_NT(uint16_t, 0);
+        MDY_NT(uint16_t, 1);
+    }
+    if (fmt == 0) MDY_NT(float, 0);
+    MDY_NT(float, 1);
+#undef MDY_NT
 }
 
 // Which kernel family a call would run (the same tests as dispatch() / launch_splitk(), no launch):
@@ -1302,61 +1313,18 @@ int static_scratch_ptr(void** out) {
 }
 
 int launch_fp8_gemm_nt_static(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,
-                              const float* b_s, void* c, const void* bias, int64_t M, int64_t N, int64_t K, int out_dtype,
+                              const float* b_s, void* c, Bias bias, int64_t M, int64_t N, int64_t K, int out_dtype,
                               hipStream_t stream) {
     void* ws = nullptr;
     const int rc = static_scratch_ptr(&ws);
     if (rc != 0) return rc;
-    return launch_fp8_gemm_nt_ws(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias, M, N, K, out_dtype, ws,
-                                 kStaticScratchBytes, stream);
-}
-
-// The MFMA kernels on e5m2 operands: the tile, weight-streaming and strip kernels (the K split and the grouped GEMM are
-// e4m3fn only).  Returns -1 when the operands do not qualify (K % 128 != 0, K > 65536, unaligned, scales beyond 2^31 bytes).
-int launch_fp8_gemm_nt_e5m2(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,
-                            const float* b_s, void* c, const void* bias, int64_t M, int64_t N, int64_t K, int out_dtype,
-                            hipStream_t stream) {
-    if (M == 0 || N == 0) return 0;
-    const int64_t KB = K / 128;
-    const int64_t as_extent = ((M - 1) * as_row_stride + (KB - 1) * as_col_stride + 1) * 4;
-    const bool ok = K % 128 == 0 && K <= (1 << 16) && as_row_stride >= 0 && as_col_stride >= 0 &&
-                    as_extent < ((int64_t)1 << 31) &&
-                    ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0;
-    if (!ok) return -1;
-    const uint8_t* ap = static_cast<const uint8_t*>(a);
-    const uint8_t* bp = static_cast<const uint8_t*>(b);
-    const uint16_t* biasp = static_cast<const uint16_t*>(bias);
-    if (M <= 64) {
-        if (out_dtype == 0)
-            return dispatch_small<uint16_t, 1>(ap, a_s, as_row_stride, as_col_stride, as_extent, true, bp, b_s, static_cast<uint16_t*>(c),
-                                               biasp, (int)M, (int)N, (int)K, stream);
-        return dispatch_small<float, 1>(ap, a_s, as_row_stride, as_col_stride, as_extent, true, bp, b_s, static_cast<float*>(c), biasp,
-                                        (int)M, (int)N, (int)K, stream);
-    }
-    if (out_dtype == 0)
-        return dispatch_tiles<uint16_t, 1>(ap, a_s, as_row_stride, as_col_stride, as_extent, bp, b_s, static_cast<uint16_t*>(c), biasp,
-                                           (int)M, (int)N, (int)K, stream);
-    return dispatch_tiles<float, 1>(ap, a_s, as_row_stride, as_col_stride, as_extent, bp, b_s, static_cast<float*>(c), biasp, (int)M,
-                                    (int)N, (int)K, stream);
-}
-
-int launch_fp8_gemm_nt(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,
-                       const float* b_s, void* c, const void* bias, int64_t M, int64_t N, int64_t K, int out_dtype,
-                       hipStream_t stream) {
-    if (M == 0 || N == 0) return 0;
-    const uint8_t* ap = static_cast<const uint8_t*>(a);
-    const uint8_t* bp = static_cast<const uint8_t*>(b);
-    const uint16_t* biasp = static_cast<const uint16_t*>(bias);
-    if (out_dtype == 0)
-        return dispatch<uint16_t>(ap, a_s, as_row_stride, as_col_stride, bp, b_s, static_cast<uint16_t*>(c), biasp,
-                                  (int)M, (int)N, (int)K, stream);
-    return dispatch<float>(ap, a_s, as_row_stride, as_col_stride, bp, b_s, static_cast<float*>(c), biasp, (int)M,
-                           (int)N, (int)K, stream);
+    return launch_fp8_gemm_nt(a, a_s, as_row_stride, as_col_stride, b, b_s, c, bias, M, N, K, 0, out_dtype, ws,
+                              kStaticScratchBytes, stream);
 }
 
 template <typename OUT>
 static int launch_grouped(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t as_cs, uint32_t as_bytes,
-                          const uint8_t* b, const float* b_s, OUT* c, const uint16_t* bias, const int64_t* m_splits,
+                          const uint8_t* b, const float* b_s, OUT* c, const Bias bias, const int64_t* m_splits,
                           int G, int N, int K, hipStream_t stream) {
     GroupTable tbl;
     tbl.n_groups = G;
@@ -1379,7 +1347,7 @@ static int launch_grouped(const uint8_t* a, const float* a_s, int64_t as_rs, int
 // Groups of at most 64 rows each on the whole-line small-M kernel, one grid row per group (32 weight columns per workgroup).
 template <typename OUT>
 static int launch_grouped_lines(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t as_cs, const uint8_t* b, const float* b_s,
-                                OUT* c, const uint16_t* bias, const int64_t* m_splits, int G, int max_rows, int N, int K,
+                                OUT* c, const Bias bias, const int64_t* m_splits, int G, int max_rows, int N, int K,
                                 hipStream_t stream) {
     GroupRows rows;
     int row = 0;
@@ -1418,7 +1386,7 @@ static int launch_grouped_lines(const uint8_t* a, const float* a_s, int64_t as_r
 
 template <typename OUT>
 static int dispatch_grouped(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t as_cs, const uint8_t* b,
-                            const float* b_s, OUT* c, const uint16_t* bias, const int64_t* m_splits, int G, int64_t M,
+                            const float* b_s, OUT* c, const Bias bias, const int64_t* m_splits, int G, int64_t M,
                             int N, int K, hipStream_t stream) {
     const int KB = (K + 127) / 128, NB = (N + 127) / 128;
     const int64_t as_extent = ((M - 1) * as_rs + (int64_t)(KB - 1) * as_cs + 1) * 4;
@@ -1447,7 +1415,7 @@ static int dispatch_grouped(const uint8_t* a, const float* a_s, int64_t as_rs, i
         const int64_t mg = m_splits[g];
         if (mg > 0) {
             int rc = dispatch<OUT>(a + row * K, a_s + row * as_rs, as_rs, as_cs, b + (size_t)g * N * K,
-                                   b_s + (size_t)g * NB * KB, c + row * N, bias ? bias + (size_t)g * N : nullptr, (int)mg, N, K,
+                                   b_s + (size_t)g * NB * KB, c + row * N, bias.at((size_t)g * N), (int)mg, N, K,
                                    stream);
             if (rc != 0) return rc;
         }
@@ -1457,16 +1425,15 @@ static int dispatch_grouped(const uint8_t* a, const float* a_s, int64_t as_rs, i
 }
 
 int launch_fp8_grouped_gemm_nt(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride,
-                               const void* b, const float* b_s, void* c, const void* bias, const int64_t* m_splits,
+                               const void* b, const float* b_s, void* c, Bias bias, const int64_t* m_splits,
                                int64_t G, int64_t M, int64_t N, int64_t K, int out_dtype, hipStream_t stream) {
     if (M == 0 || N == 0 || G == 0) return 0;
     const uint8_t* ap = static_cast<const uint8_t*>(a);
     const uint8_t* bp = static_cast<const uint8_t*>(b);
-    const uint16_t* biasp = static_cast<const uint16_t*>(bias);
     if (out_dtype == 0)
-        return dispatch_grouped<uint16_t>(ap, a_s, as_row_stride, as_col_stride, bp, b_s, static_cast<uint16_t*>(c), biasp,
+        return dispatch_grouped<uint16_t>(ap, a_s, as_row_stride, as_col_stride, bp, b_s, static_cast<uint16_t*>(c), bias,
                                           m_splits, (int)G, M, (int)N, (int)K, stream);
-    return dispatch_grouped<float>(ap, a_s, as_row_stride, as_col_stride, bp, b_s, static_cast<float*>(c), biasp, m_splits,
+    return dispatch_grouped<float>(ap, a_s, as_row_stride, as_col_stride, bp, b_s, static_cast<float*>(c), bias, m_splits,
                                    (int)G, M, (int)N, (int)K, stream);
 }
 

@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_rowscaled_kernel(
 
     if (sizeof(OUT) == 2 && N % 8 == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0) {
         __syncthreads();     // the operand panels are free: 8 KB of results per wave
-        store_rows<4, 4, OUT>(acc, &lds_a[0][0] + wave * 8192, c, N, nullptr, m0 + wm * 64, n0 + wn * 64, M, N, lane);
+        store_rows<4, 4, OUT>(acc, &lds_a[0][0] + wave * 8192, c, N, Bias{}, m0 + wm * 64, n0 + wn * 64, M, N, lane);
         return;
     }
     const bool vec_ok = (N % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_tile_kernel(
     for (int pid = blockIdx.x; pid < ntiles; pid += gridDim.x) {
         int tm, tn;
         const Duty duty = tile_of(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
-        fp8_gemm_tile<BM, BN, 2, 4, STAGES, OUT, 0, 0, 0, FMT, true>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, nullptr, tm * BM, M, M,
+        fp8_gemm_tile<BM, BN, 2, 4, STAGES, OUT, 0, 0, 0, FMT, true>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, Bias{}, tm * BM, M, M,
                                                                      tn * BN, N, K, N, duty, 0, K >> 7, pool, bs_rs, bs_cs, bs_bytes);
         __syncthreads();
     }
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
     int tm, tn;
     const Duty duty = tile_of(pid - ks * ntiles, tiles_m, tiles_n, tm, tn);
     const int kb0 = ks * kb_per, kb1 = min(K >> 7, kb0 + kb_per);
-    fp8_gemm_tile<128, 256, 2, 4, 3, float, 0, 0, 0, FMT, true>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, nullptr,
+    fp8_gemm_tile<128, 256, 2, 4, 3, float, 0, 0, 0, FMT, true>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, Bias{},
                                                                 tm * 128, M, M, tn * 256, N, K, N, duty, kb0, kb1, pool, bs_rs, bs_cs,
                                                                 bs_bytes);
 }
@@ -225,7 +225,7 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
         if (fmt == 0) MDY_RSS(0); else MDY_RSS(1);
 #undef MDY_RSS
         const int rc = (int)hipGetLastError();
-        return rc != 0 ? rc : launch_splitk_reduce(ws, c, out_dtype, nullptr, M, N, sp.slabs, stream);
+        return rc != 0 ? rc : launch_splitk_reduce(ws, c, out_dtype, Bias{}, M, N, sp.slabs, stream);
     }
     const int cfg = rowscaled_config(M, N, K);
     if (cfg != 0) {

@@ -65,7 +65,7 @@ __device__ __forceinline__ void store4(OUT* c, int64_t ldc, int m, int n, int M,
 // those stores stay cached: the reduction reads the slabs next.
 template <int TI, int TJ, typename OUT>
 __device__ __forceinline__ void store_rows(const floatx4 (&acc)[TI][TJ], uint8_t* buf, OUT* __restrict__ c, int64_t ldc,
-                                           const uint16_t* __restrict__ bias, int m_base, int n_base, int M, int N, int lane) {
+                                           const Bias bias, int m_base, int n_base, int M, int N, int lane) {
     static_assert(TJ % 2 == 0, "a row is a multiple of four 16-byte pieces");
     constexpr bool HALF = sizeof(OUT) == 2;
     constexpr int EPP = 16 / sizeof(OUT);      // elements per 16-byte piece
@@ -76,13 +76,17 @@ __device__ __forceinline__ void store_rows(const floatx4 (&acc)[TI][TJ], uint8_t
     for (int j = 0; j < TJ; ++j) {
         float bv[4] = {0.f, 0.f, 0.f, 0.f};
         const int n = n_base + j * 16 + 4 * fk;
-        if (bias != nullptr && n < N) {      // N is a multiple of the piece: all four columns are in range
+        if (bias.p != nullptr && n < N) {      // N is a multiple of the piece: all four columns are in range
 #pragma unroll
-            for (int e = 0; e < 4; ++e) bv[e] = bf16_one(bias[n + e]);
+            for (int e = 0; e < 4; ++e) bv[e] = bf16_one(bias.p[n + e]);
         }
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
-            const floatx4 v = acc[i][j];
+            floatx4 v = acc[i][j];
+            if (bias.after_rounding) {
+                const uint32_t lo = pack2_bf16(v[0], v[1]), hi = pack2_bf16(v[2], v[3]);
+                v = floatx4{bf16_lo(lo), bf16_hi(lo), bf16_lo(hi), bf16_hi(hi)};
+            }
             uint8_t* row = buf + (i * 16 + frow) * ROW;
             if (HALF)
                 *reinterpret_cast<uint2*>(row + (((2 * j + (fk >> 1)) ^ (frow & MASK)) << 4) + (fk & 1) * 8) =
@@ -203,7 +207,7 @@ template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ =
 __device__ __forceinline__ void fp8_gemm_tile(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
-    const uint16_t* __restrict__ bias, int m0, int m_end, int m_total, int n0, int N, int K, int ldc, const Duty duty,
+    const Bias bias, int m0, int m_end, int m_total, int n0, int N, int K, int ldc, const Duty duty,
     int kb0, int kb1, uint8_t* __restrict__ pool, int bs_rs = 0, int bs_cs = 0, uint32_t bs_bytes = 0) {
     // ABL_ switches parts of the K loop off for the timing probe (mdy_fp8_gemm_probe); the product uses 0.
     //   1: no global->LDS copies in the loop (the ring is filled once and replayed)   2: no LDS fragment / scale reads
@@ -502,10 +506,10 @@ __device__ __forceinline__ void fp8_gemm_tile(
         for (int j = 0; j < TJ; ++j) {
             const int n = n0 + wn * WN + j * 16 + 4 * fk;
             float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-            if (bias != nullptr) {
+            if (bias.p != nullptr) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (n + e < N) v[e] += bf16_one(bias[n + e]);
+                    if (n + e < N) v[e] = bias.add(v[e], n + e);
             }
             store4<OUT>(c, ldc, m, n, M, N, v, vec_ok);
         }
@@ -563,7 +567,7 @@ template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, in
 __device__ __forceinline__ void fp8_gemm_tile_ws(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
-    const uint16_t* __restrict__ bias, int m0, int m_end, int m_total, int n0, int N, int K, int ldc, const Duty duty,
+    const Bias bias, int m0, int m_end, int m_total, int n0, int N, int K, int ldc, const Duty duty,
     int kb0, int kb1, uint8_t* __restrict__ pool) {
     constexpr int CW = WGM * WGN;                       // consumer waves
     constexpr int WM = BM / WGM, WN = BN / WGN, TI = WM / 16, TJ = WN / 16;
@@ -791,10 +795,10 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
         for (int j = 0; j < TJ; ++j) {
             const int n = n0 + wn * WN + j * 16 + 4 * fk;
             float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-            if (bias != nullptr) {
+            if (bias.p != nullptr) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (n + e < N) v[e] += bf16_one(bias[n + e]);
+                    if (n + e < N) v[e] = bias.add(v[e], n + e);
             }
             store4<OUT>(c, ldc, m, n, M, N, v, vec_ok);
         }
@@ -806,7 +810,7 @@ template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, in
 __global__ __launch_bounds__((WGM * WGN + PW) * 64) void fp8_gemm_ws_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
-    const uint16_t* __restrict__ bias, int M, int N, int K, int ldc, int tiles_m, int tiles_n, int pretouch) {
+    const Bias bias, int M, int N, int K, int ldc, int tiles_m, int tiles_n, int pretouch) {
     constexpr bool HOLD_A = BM / WGM <= BN / WGN;
     __shared__ __attribute__((aligned(1024)))
     uint8_t pool[TileLdsWs<BM, BN, WGM * WGN + PW, HOLD_A ? STAGES - 1 : STAGES, HOLD_A ? STAGES : STAGES - 1, STAGES - 1>::bytes];
@@ -825,7 +829,7 @@ template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ =
 __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
-    const uint16_t* __restrict__ bias, int M, int N, int K, int ldc, int tiles_m, int tiles_n, int pretouch) {
+    const Bias bias, int M, int N, int K, int ldc, int tiles_m, int tiles_n, int pretouch) {
     // The grid may be smaller than the number of tiles (one workgroup per CU for the 256x256 tile): a workgroup
     // then walks tiles blockIdx.x, blockIdx.x + gridDim.x, ... itself, which saves the ~4.5 us that pass between
     // the end of a workgroup and the start of its successor on the same CU.  Workgroup ids keep their XCD

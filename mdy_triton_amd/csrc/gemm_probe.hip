@@ -15,7 +15,7 @@ static int probe_launch(const uint8_t* a, const float* a_s, int as_rs, int as_cs
     const int wgs = (BM * BN >= 256 * 256 && tiles_m * tiles_n > max_wgs) ? max_wgs : tiles_m * tiles_n;
     hipLaunchKernelGGL((fp8_gemm_mfma_kernel<BM, BN, WGM, WGN, STAGES, uint16_t, GAP, 0, ABL>), dim3((unsigned)wgs),
                        dim3(WGM * WGN * 64), 0, stream, a, a_s, as_rs, as_cs, as_bytes, b, b_s, c,
-                       static_cast<const uint16_t*>(nullptr), M, N, K, N, tiles_m, tiles_n, 1);
+                       Bias{}, M, N, K, N, tiles_m, tiles_n, 1);
     return (int)hipGetLastError();
 }
 
@@ -71,7 +71,7 @@ static int launch_fp8_gemm_order_probe(int gm, int pretouch, const void* a, cons
 #define MDY_ORDER(GM)                                                                                                   \
     hipLaunchKernelGGL((fp8_gemm_mfma_kernel<256, 256, 2, 4, 2, uint16_t, 0, 0, 0, 0, GM>), dim3((unsigned)wgs), dim3(512), 0, stream, \
                        static_cast<const uint8_t*>(a), a_s, (int)as_rs, (int)as_cs, (uint32_t)as_extent,                  \
-                       static_cast<const uint8_t*>(b), b_s, static_cast<uint16_t*>(c), static_cast<const uint16_t*>(nullptr), \
+                       static_cast<const uint8_t*>(b), b_s, static_cast<uint16_t*>(c), Bias{}, \
                        (int)M, (int)N, (int)K, (int)N, tiles_m, tiles_n, pretouch)
     if (gm == 2) MDY_ORDER(2);
     else if (gm == 4) MDY_ORDER(4);

@@ -131,6 +131,15 @@ def fp8_matmul(qa: torch.Tensor, sa: torch.Tensor, qb: torch.Tensor, sb: torch.T
     column-major tensor quant_input returns is used in place); sb [N/128, K/128]
     contiguous.  `bias` (bf16 [N]) is an extension folded into the epilogue.
     """
+    return _matmul(qa, sa, qb, sb, out, bias, BIAS_IN_SUM)
+
+
+BIAS_IN_SUM, BIAS_AFTER_ROUNDING = 0, 1      # MDY_BIAS_*
+
+
+def _matmul(qa, sa, qb, sb, out, bias, bias_mode):
+    """fp8_matmul with the choice of where the bias goes: into the fp32 sum, or onto the product rounded to bf16 (what a
+    following add_bias would give, without its pass over the output)."""
     if qa.dtype != FP8 or qb.dtype != FP8:
         raise TypeError("fp8_matmul expects float8_e4m3fn operands")
     if not qa.is_contiguous() or not qb.is_contiguous() or not sb.is_contiguous():
@@ -151,8 +160,8 @@ def fp8_matmul(qa: torch.Tensor, sa: torch.Tensor, qb: torch.Tensor, sb: torch.T
     with on_device(dev):
         warn_if_scalar_gemm(qa, qb, sa.stride(0), sa.stride(1), M, N, K, "fp8_matmul")
         ws = gemm_workspace(dev, M, N, K)      # scratch for shapes that are split along K, else None
-        check(lib().mdy_fp8_gemm_nt_ws(ptr(qa), ptr(sa), sa.stride(0), sa.stride(1), ptr(qb), ptr(sb), ptr(out),
-                                       ptr(bias), M, N, K, 0, ptr(ws), ws.numel() if ws is not None else 0,
+        check(lib().mdy_fp8_gemm_nt_ex(ptr(qa), ptr(sa), sa.stride(0), sa.stride(1), ptr(qb), ptr(sb), ptr(out),
+                                       ptr(bias), bias_mode, M, N, K, 0, 0, ptr(ws), ws.numel() if ws is not None else 0,
                                        stream_ptr(dev)), "fp8_matmul")
     return out
 
@@ -164,7 +173,8 @@ class _DeepLinear(torch.autograd.Function):
 
     The GEMMs run on the unpadded row counts (the quantizers pad rows to 4/128/256, the
     padding is never multiplied), so shapes that are not multiples of 256 work and no
-    result is sliced.  The bias add can be folded into the GEMM epilogue (`fuse_bias`).
+    result is sliced.  A bf16 bias is added in the GEMM epilogue: to the product rounded to bf16, the reference's two
+    steps, or into the fp32 sum (`fuse_bias`).
     """
 
     @staticmethod
@@ -188,10 +198,11 @@ class _DeepLinear(torch.autograd.Function):
             ctx.dims = (M, N, K)
             ctx.quantized = (q_inp_t, s_inp_t, q_weight_t, s_weight_t)
             ctx.has_bias = bias is not None
-        fuse_bias = bool(fuse_bias and bias is not None and bias.dtype == torch.bfloat16)    # the epilogue takes a bf16 bias
-        out = fp8_matmul(q_inp[:M], s_inp[:M], q_weight[:N], s_weight[:_cdiv(N, 128)],
-                         bias=bias if fuse_bias else None)
-        if bias is not None and not fuse_bias:
+        # the epilogue takes a bf16 bias: before the product's rounding (fuse_bias) or after it, as add_bias does
+        in_epilogue = bias is not None and bias.dtype == torch.bfloat16
+        out = _matmul(q_inp[:M], s_inp[:M], q_weight[:N], s_weight[:_cdiv(N, 128)], None, bias if in_epilogue else None,
+                      BIAS_IN_SUM if fuse_bias else BIAS_AFTER_ROUNDING)
+        if bias is not None and not in_epilogue:
             add_bias(out, bias)
         return out.view(*inp_shape[:-1], N)
 
@@ -235,7 +246,7 @@ class DeepLinear(torch.nn.Linear):
     `check_weight_cache = True` (or the environment variable MDY_FP8_CHECK_WEIGHT_CACHE=1)
     verifies every cache hit against a checksum of the weight taken when it was quantized and
     raises if they differ - a debugging aid (one reduction and one host synchronisation per call).
-    `fuse_bias = True` adds the bias inside the GEMM epilogue.
+    `fuse_bias = True` adds the bias to the fp32 sum, before the product is rounded to bf16 instead of after it.
     """
 
     cache_weight = False

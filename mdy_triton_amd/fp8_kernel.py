@@ -15,7 +15,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from ._torch_glue import FP8, check, lib, on_device, ptr, require_gpu, rowscaled_workspace, stream_ptr, xt_code
+from ._torch_glue import FP8, check, gemm_workspace, lib, on_device, ptr, require_gpu, rowscaled_workspace, stream_ptr, xt_code
 
 _ORDERS = ("up-gate", "gate-up")
 
@@ -261,14 +261,15 @@ def fp8_matmul(x: torch.Tensor, w: torch.Tensor, scale_x: torch.Tensor, scale_w:
             sxc, swc = sx2.contiguous(), scale_w.contiguous()
             scales_ok = M == 0 or ((M - 1) * sxc.stride(0) + K // 128) * 4 < (1 << 31)
             if K <= 65536 and scales_ok and x2c.data_ptr() % 16 == 0 and wc.data_ptr() % 16 == 0:
-                # e5m2 on the MFMA kernels (operand format bf8): tile kernels, or the weight-streaming / strip kernels
-                # for up to 64 rows
+                # e5m2 on the MFMA kernels (operand format bf8): tile kernels, split along K where e4m3fn is, or the
+                # weight-streaming / strip kernels for up to 64 rows
                 fused = bias is not None and bias.dtype == torch.bfloat16
                 y = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
                 with on_device(dev):
-                    check(lib().mdy_fp8_gemm_nt_e5m2(ptr(x2c), ptr(sxc), sxc.stride(0), 1, ptr(wc), ptr(swc), ptr(y),
-                                                     ptr(bias.contiguous()) if fused else None, M, N, K, 0, stream_ptr(dev)),
-                          "fp8_matmul")
+                    ws = gemm_workspace(dev, M, N, K)
+                    check(lib().mdy_fp8_gemm_nt_ex(ptr(x2c), ptr(sxc), sxc.stride(0), 1, ptr(wc), ptr(swc), ptr(y),
+                                                   ptr(bias.contiguous()) if fused else None, 0, M, N, K, fmt, 0, ptr(ws),
+                                                   ws.numel() if ws is not None else 0, stream_ptr(dev)), "fp8_matmul")
             else:
                 # K beyond 65536, unaligned operands or scales spanning 2^31 bytes: the GEMM with row scales on both
                 # operands, the weight's block scales expanded to one per row
