@@ -154,6 +154,15 @@ int mdy_quant_transpose_typed(const void* x, int x_dtype, void* y, float* s, voi
 int mdy_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K,
                             int64_t x_row_stride, int64_t x_col_stride, int64_t PM, int64_t PK, int mode, void* stream);
 
+/* The two training quantizers with a scale per column and 128 rows (mdy_quant_transpose with MDY_T_COLUMN for mode
+ * MDY_QUANT_DEEPLINEAR, mdy_act_quant_transpose for the official modes: their layouts, s_kb_stride only used by the former)
+ * on a bf16 output gradient, and in the same pass the gradient's column sums, i.e. the bias gradient (fp8.py:342 and
+ * fp8_kernel.py:279 take dy.sum(0)): added in fp32, rounded to bf16 once.
+ *   partial  fp32 scratch [PM/128, PK]      col_sum  bf16 [K] */
+int mdy_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K,
+                               int64_t x_row_stride, int64_t x_col_stride, int64_t PM, int64_t PK, int64_t s_kb_stride,
+                               int mode, float* partial, void* col_sum, void* stream);
+
 /* Block-scaled FP8 GEMM, NT layout, with 1x128 scales on both operands:
  *   c[m, n] = sum_kb (sum_{k in kb} a[m,k] * b[n,k]) * a_s[m, kb] * b_s[n, kb]
  * Replaces fp8_matmul(..., have_w=False) (triton_kernels/deepseekv3/fp8_kernel.py:214-252, kernel branch :190-205),

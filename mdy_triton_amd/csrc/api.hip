@@ -166,6 +166,25 @@ int mdy_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, void*
                     "act_quant_transpose");
 }
 
+int mdy_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K, int64_t x_row_stride,
+                               int64_t x_col_stride, int64_t PM, int64_t PK, int64_t s_kb_stride, int mode, float* partial,
+                               void* col_sum, void* stream) {
+    if (mode != MDY_QUANT_OFFICIAL && mode != MDY_QUANT_DEEPLINEAR && mode != MDY_QUANT_OFFICIAL_E5M2) return fail(MDY_E_DTYPE, "quant_transpose_colsum: unknown mode %d", mode);
+    if (M < 0 || K < 0 || PM < M || PK < K || PM > kMaxDim || PK > kMaxDim)
+        return fail(MDY_E_SHAPE, "quant_transpose_colsum: need 0 <= M <= PM, 0 <= K <= PK");
+    if (PM % 128 != 0 || PK % 128 != 0) return fail(MDY_E_SHAPE, "quant_transpose_colsum: PM=%lld, PK=%lld must be multiples of 128", (long long)PM, (long long)PK);
+    if (mode == MDY_QUANT_DEEPLINEAR && s_kb_stride < PM) return fail(MDY_E_SHAPE, "quant_transpose_colsum: s_kb_stride=%lld < PM=%lld", (long long)s_kb_stride, (long long)PM);
+    if ((y == nullptr) != (s == nullptr)) return fail(MDY_E_NULL, "quant_transpose_colsum: y and s must be given together");
+    if (PM == 0 || PK == 0) return 0;
+    if (!y_t || !s_t || !partial || !col_sum || (!x && M > 0 && K > 0)) return fail(MDY_E_NULL, "quant_transpose_colsum: null pointer");
+    if ((y && !aligned(y, 8)) || !aligned(y_t, 8)) return fail(MDY_E_ALIGN, "quant_transpose_colsum: y / y_t must be 8-byte aligned");
+    if (!aligned(x, 2) || !aligned(col_sum, 2) || (s && !aligned(s, 4)) || !aligned(s_t, 4) || !aligned(partial, 4)) return fail(MDY_E_ALIGN, "quant_transpose_colsum: misaligned pointer");
+    if (int e = check_device()) return e;
+    return launched(mdy::launch_quant_transpose_colsum(x, y, s, y_t, s_t, M, K, x_row_stride, x_col_stride, PM, PK, s_kb_stride, mode, partial,
+                                                       col_sum, static_cast<hipStream_t>(stream)),
+                    "quant_transpose_colsum");
+}
+
 int mdy_fp8_gemm_nt_rowscaled_ws(const void* a, const float* a_s, int64_t as_row_stride, int64_t as_col_stride, const void* b,
                               const float* b_s, int64_t bs_row_stride, int64_t bs_col_stride, void* c, int64_t M, int64_t N,
                               int64_t K, int fmt, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {

@@ -281,6 +281,9 @@ int launch_quant_transpose(const void* x, int x_dtype, void* y, float* s, void* 
                            int t_mode, hipStream_t stream);
 int launch_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K,
                                int64_t x_row_stride, int64_t x_col_stride, int64_t PM, int64_t PK, int mode, hipStream_t stream);
+int launch_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K, int64_t x_row_stride,
+                                  int64_t x_col_stride, int64_t PM, int64_t PK, int64_t s_kb_stride, int mode, float* part, void* col_sum,
+                                  hipStream_t stream);
 int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs, int64_t as_cs, const void* b,
                                  const float* b_s, int64_t bs_rs, int64_t bs_cs, void* c, int64_t M, int64_t N, int64_t K,
                                  int fmt, int out_dtype, void* workspace, int64_t workspace_bytes, hipStream_t stream);

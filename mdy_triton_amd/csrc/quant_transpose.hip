@@ -36,16 +36,20 @@ __device__ __forceinline__ float qt_quot(float x, float s, float r) {
 // column k, row group a at s_t[a * st_a_stride + k * st_k_stride] (TMODE 0) / block scale at s_t[kb * (PM/128) + a]
 // (TMODE 1).  y may be null (MODE 0 callers that only want the transposed copy): the row-wise outputs are skipped.
 // XT: input type (0 bf16, 1 fp16, 2 fp32); the reciprocal quotient is proven for bf16 inputs only, other types divide.
-template <int MODE, int TMODE, bool VEC, int RPT, int XT>
+// CSUM (with TMODE 0): also the fp32 sums of the tile's columns, to col_sum[row tile * PK + column]: an output gradient's column
+// sums are the bias gradient, and here they cost 8 adds per 16 bytes loaded instead of a pass over the matrix.
+template <int MODE, int TMODE, bool VEC, int RPT, int XT, bool CSUM = false>
 __global__ __launch_bounds__(2048 / RPT) void quant_transpose_kernel(const void* __restrict__ x, uint8_t* __restrict__ y,
                                                                float* __restrict__ s, uint8_t* __restrict__ y_t,
                                                                float* __restrict__ s_t, int M, int K,
                                                                int64_t x_row_stride, int64_t x_col_stride, int PM,
                                                                int PK, int64_t s_kb_stride, int64_t s_m_stride,
-                                                               int64_t st_a_stride, int64_t st_k_stride) {
+                                                               int64_t st_a_stride, int64_t st_k_stride,
+                                                               float* __restrict__ col_sum) {
     constexpr int NRG = 128 / RPT;        // row groups of RPT consecutive rows; 16 threads (8 columns each) per group
     constexpr int WAVES = NRG / 4;
     __shared__ float col_part[WAVES][128];  // per wave (4 row groups) partial column maxima
+    __shared__ float sum_part[CSUM ? WAVES : 1][128];       // the same for the column sums
     __shared__ __attribute__((aligned(16))) float col_amax[128];
     __shared__ __attribute__((aligned(16))) float col_sc[128];   // per column: scale of the transposed copy ...
     __shared__ __attribute__((aligned(16))) float col_rc[128];   // ... and its reciprocal, computed once per column
@@ -63,9 +67,13 @@ __global__ __launch_bounds__(2048 / RPT) void quant_transpose_kernel(const void*
 
     float f[RPT][8];
     float rmax[RPT];
-    float cmax[8];
+    float cmax[8], csum[CSUM ? 8 : 1];
 #pragma unroll
     for (int j = 0; j < 8; ++j) cmax[j] = 0.0f;
+    if (CSUM) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) csum[CSUM ? j : 0] = 0.0f;
+    }
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
         load_row8_f32<XT, VEC>(x, bm * 128 + rg * RPT + i, c0, M, K, x_row_stride, x_col_stride, f[i]);
@@ -75,6 +83,10 @@ __global__ __launch_bounds__(2048 / RPT) void quant_transpose_kernel(const void*
             m = fmaxf(fmaxf(fabsf(f[i][2 * j]), fabsf(f[i][2 * j + 1])), m);
             cmax[2 * j] = fmaxf(cmax[2 * j], fabsf(f[i][2 * j]));
             cmax[2 * j + 1] = fmaxf(cmax[2 * j + 1], fabsf(f[i][2 * j + 1]));
+        }
+        if (CSUM) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) csum[CSUM ? j : 0] += f[i][j];
         }
         rmax[i] = row16_max(m);
     }
@@ -107,6 +119,12 @@ __global__ __launch_bounds__(2048 / RPT) void quant_transpose_kernel(const void*
             float m = fmaxf(cmax[j], __shfl_xor(cmax[j], 16, 64));
             m = fmaxf(m, __shfl_xor(m, 32, 64));
             if (lane < 16) col_part[wave][cl + j] = m;
+            if (CSUM) {
+                float v = csum[CSUM ? j : 0];
+                v += __shfl_xor(v, 16, 64);
+                v += __shfl_xor(v, 32, 64);
+                if (lane < 16) sum_part[CSUM ? wave : 0][cl + j] = v;
+            }
         }
         __syncthreads();
         if (t < 128) {
@@ -119,6 +137,12 @@ __global__ __launch_bounds__(2048 / RPT) void quant_transpose_kernel(const void*
             col_rc[t] = 1.0f / sc;
             s_t[(int64_t)bm * st_a_stride + (int64_t)(bk * 128 + t) * st_k_stride] = sc;
             if (y != nullptr) s[(int64_t)bk * s_kb_stride + (int64_t)(bm * 128 + t) * s_m_stride] = row_sc[t];
+            if (CSUM) {
+                float v = 0.0f;
+#pragma unroll
+                for (int g = 0; g < WAVES; ++g) v += sum_part[CSUM ? g : 0][t];
+                col_sum[(int64_t)bm * PK + bk * 128 + t] = v;
+            }
         }
         __syncthreads();
 #pragma unroll
@@ -217,11 +241,11 @@ static int launch_qt(int mode, const void* x, int x_dtype, void* y, float* s, vo
         if (wide)                                                                                                         \
             hipLaunchKernelGGL((quant_transpose_kernel<MODE, TM, VEC, 4, XT>), grid, block, 0, stream, x, yp, s, ytp, s_t, \
                                (int)M, (int)K, x_row_stride, x_col_stride, (int)PM, (int)PK, s_kb_stride, s_m_stride,     \
-                               st_a_stride, st_k_stride);                                                                 \
+                               st_a_stride, st_k_stride, static_cast<float*>(nullptr));                                   \
         else                                                                                                              \
             hipLaunchKernelGGL((quant_transpose_kernel<MODE, TM, VEC, 8, XT>), grid, block, 0, stream, x, yp, s, ytp, s_t, \
                                (int)M, (int)K, x_row_stride, x_col_stride, (int)PM, (int)PK, s_kb_stride, s_m_stride,     \
-                               st_a_stride, st_k_stride);                                                                 \
+                               st_a_stride, st_k_stride, static_cast<float*>(nullptr));                                   \
     } while (0)
 #define MDY_QT_V(MODE, TM, XT) do { if (vec) MDY_QT(MODE, TM, true, XT); else MDY_QT(MODE, TM, false, XT); } while (0)
 #define MDY_QT_X(MODE, TM) do { if (x_dtype == 0) MDY_QT_V(MODE, TM, 0); else if (x_dtype == 1) MDY_QT_V(MODE, TM, 1); else MDY_QT_V(MODE, TM, 2); } while (0)
@@ -246,6 +270,49 @@ int launch_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, vo
                                int64_t x_row_stride, int64_t x_col_stride, int64_t PM, int64_t PK, int mode, hipStream_t stream) {
     // official layouts, both row-major: s [PM][PK/128], s_t [PK][PM/128]; mode 0 (e4m3fn) or 2 (e5m2)
     return launch_qt(mode == 2 ? 2 : 0, x, x_dtype, y, s, y_t, s_t, M, K, x_row_stride, x_col_stride, PM, PK, 1, PK / 128, 1, PM / 128, 0, stream);
+}
+
+// bf16(sum over the row tiles of part[a][k]): 32 columns x 8 interleaved shares of the row tiles per block
+__global__ __launch_bounds__(256) void col_sum_reduce_kernel(const float* __restrict__ part, uint16_t* __restrict__ out, int A, int K, int PK) {
+    __shared__ float share[8][32];
+    const int c = threadIdx.x & 31, g = threadIdx.x >> 5, k = blockIdx.x * 32 + c;      // k < PK: PK % 128 == 0
+    float v = 0.0f;
+    for (int a = g; a < A; a += 8) v += part[(int64_t)a * PK + k];
+    share[g][c] = v;
+    __syncthreads();
+    if (g == 0 && k < K) {
+#pragma unroll
+        for (int h = 1; h < 8; ++h) v += share[h][c];
+        out[k] = (uint16_t)(pack2_bf16(v, 0.0f) & 0xFFFFu);
+    }
+}
+
+int launch_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K, int64_t x_row_stride,
+                                  int64_t x_col_stride, int64_t PM, int64_t PK, int64_t s_kb_stride, int mode, float* part, void* col_sum,
+                                  hipStream_t stream) {
+    if (PM == 0 || PK == 0) return 0;
+    dim3 grid;
+    if (!grid_rows(PK / 128, PM / 128, grid)) return kErrTooManyBlocks;
+    const bool wide = (PK / 128) * (PM / 128) < 256 * 24;      // as in launch_qt
+    const bool vec = rows_vectorizable(x, K, x_row_stride, x_col_stride, 2);
+    const bool deep = mode == 1;
+    const int64_t s_kb = deep ? s_kb_stride : 1, s_m = deep ? 1 : PK / 128, st_a = deep ? PK : 1, st_k = deep ? 1 : PM / 128;
+#define MDY_QTC(MODE, VEC, RPT)                                                                                                   \
+    hipLaunchKernelGGL((quant_transpose_kernel<MODE, 0, VEC, RPT, 0, true>), grid, dim3(2048 / RPT), 0, stream, x, static_cast<uint8_t*>(y), s, \
+                       static_cast<uint8_t*>(y_t), s_t, (int)M, (int)K, x_row_stride, x_col_stride, (int)PM, (int)PK, s_kb, s_m, st_a, st_k, part)
+#define MDY_QTC_V(MODE)                                                                        \
+    do {                                                                                       \
+        if (wide) { if (vec) MDY_QTC(MODE, true, 4); else MDY_QTC(MODE, false, 4); }           \
+        else { if (vec) MDY_QTC(MODE, true, 8); else MDY_QTC(MODE, false, 8); }                \
+    } while (0)
+    if (mode == 0) MDY_QTC_V(0); else if (mode == 1) MDY_QTC_V(1); else MDY_QTC_V(2);
+#undef MDY_QTC_V
+#undef MDY_QTC
+    const int rc = (int)hipGetLastError();
+    if (rc != 0) return rc;
+    hipLaunchKernelGGL(col_sum_reduce_kernel, dim3((unsigned)((K + 31) / 32)), dim3(256), 0, stream, part, static_cast<uint16_t*>(col_sum),
+                       (int)(PM / 128), (int)K, (int)PK);
+    return (int)hipGetLastError();
 }
 
 }  // namespace mdy

@@ -17,8 +17,9 @@ def _cdiv(a: int, b: int) -> int:
     return (a + b - 1) // b
 
 
-def _quant_transpose(x: torch.Tensor, t_mode: int, who: str):
-    """Shared launcher of the two training-time quantizers (row-wise copy + quantized transpose)."""
+def _quant_transpose(x: torch.Tensor, t_mode: int, who: str, col_sum: Optional[torch.Tensor] = None):
+    """Shared launcher of the two training-time quantizers (row-wise copy + quantized transpose); col_sum (t_mode 0, bf16 x):
+    a bf16 [K] tensor that receives the sums of x's columns from the same pass."""
     if x.dim() != 2:
         raise ValueError("%s expects a 2-D tensor" % who)
     xt = xt_code(x, who)
@@ -31,6 +32,11 @@ def _quant_transpose(x: torch.Tensor, t_mode: int, who: str):
     y_t = torch.empty(PN, PM, device=dev, dtype=FP8)
     s_t = torch.empty((A, PN) if t_mode == 0 else (B, A), device=dev, dtype=torch.float32)
     with on_device(dev):
+        if col_sum is not None:
+            part = torch.empty(A, PN, device=dev, dtype=torch.float32)
+            check(lib().mdy_quant_transpose_colsum(ptr(x), ptr(y), ptr(s), ptr(y_t), ptr(s_t), M, K, x.stride(0), x.stride(1), PM, PN, PM,
+                                                   1, ptr(part), ptr(col_sum), stream_ptr(dev)), who)
+            return y, s.transpose(0, 1), y_t, s_t
         check(lib().mdy_quant_transpose_typed(ptr(x), xt, ptr(y), ptr(s), ptr(y_t), ptr(s_t), M, K, x.stride(0), x.stride(1),
                                         PM, PN, PM, t_mode, stream_ptr(dev)), who)
     return y, s.transpose(0, 1), y_t, s_t
@@ -213,15 +219,18 @@ class _DeepLinear(torch.autograd.Function):
         dy = grad_output.reshape(-1, N)
         if dy.dtype != torch.bfloat16:
             dy = dy.to(torch.bfloat16)
-        q_dy, s_dy, q_dy_t, s_dy_t = quant_grad_output(dy)
         dgrad = wgrad = grad_bias = None
+        if ctx.has_bias and ctx.needs_input_grad[2] and M > 0:
+            grad_bias = torch.empty(N, device=dy.device, dtype=torch.bfloat16)
+        q_dy, s_dy, q_dy_t, s_dy_t = _quant_transpose(dy, 0, "quant_grad_output", grad_bias)
+        s_dy_t = s_dy_t.transpose(0, 1)
         if ctx.needs_input_grad[0]:
             # [M, PN] . [K, PN]^T, contraction over the (zero-padded) output features
             dgrad = fp8_matmul(q_dy[:M], s_dy[:M], q_weight_t[:K], s_weight_t[:_cdiv(K, 128)]).view(*ctx.inp_shape)
         if ctx.needs_input_grad[1]:
             # [N, PM] . [K, PM]^T, contraction over the (zero-padded) tokens
             wgrad = fp8_matmul(q_dy_t[:N], s_dy_t[:N], q_inp_t[:K], s_inp_t[:_cdiv(K, 128)])
-        if ctx.has_bias and ctx.needs_input_grad[2]:
+        if ctx.has_bias and ctx.needs_input_grad[2] and grad_bias is None:
             grad_bias = dy.sum(0)
         return dgrad, wgrad, grad_bias, None, None, None
 

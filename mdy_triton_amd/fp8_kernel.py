@@ -178,9 +178,10 @@ def _weight_quant_both(w: torch.Tensor, rows: bool, transposed: bool, dtype: tor
     return y, s, y_t, s_t
 
 
-def _act_quant_transposed(x2: torch.Tensor, with_rows: bool, who: str, dtype: torch.dtype = FP8):
+def _act_quant_transposed(x2: torch.Tensor, with_rows: bool, who: str, dtype: torch.dtype = FP8, col_sum: Optional[torch.Tensor] = None):
     """x2 [M, N] (any strides) -> (y, s, y_t_padded, s_t): the official-dialect row-wise quantization (None, None
-    unless with_rows) and the quantized transpose y_t [N, PM] with s_t [N, PM/128], PM = cdiv(M, 128) * 128."""
+    unless with_rows) and the quantized transpose y_t [N, PM] with s_t [N, PM/128], PM = cdiv(M, 128) * 128.  col_sum (bf16
+    x2): a bf16 [N] tensor that receives the sums of x2's columns from the same pass."""
     mode, _ = _fp8_mode(dtype, who)
     xt = xt_code(x2, who)
     dev = require_gpu(x2)
@@ -192,6 +193,11 @@ def _act_quant_transposed(x2: torch.Tensor, with_rows: bool, who: str, dtype: to
     s_t = torch.empty(N, PM // 128, device=dev, dtype=torch.float32)
     if PM * N > 0:
         with on_device(dev):
+            if col_sum is not None:
+                part = torch.empty(PM // 128, N, device=dev, dtype=torch.float32)
+                check(lib().mdy_quant_transpose_colsum(ptr(x2), ptr(y), ptr(s), ptr(y_t), ptr(s_t), M, N, x2.stride(0), x2.stride(1), PM, N, 0,
+                                                       mode, ptr(part), ptr(col_sum), stream_ptr(dev)), who)
+                return y, s, y_t, s_t
             check(lib().mdy_act_quant_transpose(ptr(x2), xt, ptr(y), ptr(s), ptr(y_t), ptr(s_t), M, N, x2.stride(0), x2.stride(1),
                                                 PM, N, mode, stream_ptr(dev)), who)
     return y, s, y_t, s_t
@@ -325,17 +331,17 @@ def fp8_matmul_bwd(xt, w, dy, dyt, scale_xt, scale_w, scale_dy, scale_dyt):
     return dx, dw
 
 
-def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8):
+def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8, dbias=None):
     """Gradients of y = x . w^T in the official dialect (fp8_kernel.py:274-301): dx = dy . w on the row-wise copy of dy
     and the block-quantized w^T, dw = dy^T . x on the transposed copies of dy and x (row scales on both operands).
     w_t = (bytes, scales) of w^T, x_t = (bytes, scales) of the transposed x; either may be None when its gradient is not
-    needed.  One kernel pass over dy gives both of its copies; the transposed copies keep their zero padding to a multiple
+    needed.  One kernel pass over dy gives both of its copies and, in dbias (bf16 [N] or None), its column sums; the transposed copies keep their zero padding to a multiple
     of 128 tokens."""
     _, fmt = _fp8_mode(fp8_dtype, "Fp8Linear.backward")
     M, N = dy2.shape
     dev = dy2.device
     dx = dw = None
-    qdy, sdy, qdyt, sdyt = _act_quant_transposed(dy2, need_dx, "Fp8Linear.backward", fp8_dtype)
+    qdy, sdy, qdyt, sdyt = _act_quant_transposed(dy2, need_dx, "Fp8Linear.backward", fp8_dtype, dbias)
     if need_dx:
         dx = fp8_matmul(qdy[:M], w_t[0], sdy[:M], w_t[1], have_w=True)
     if need_dw:
@@ -383,11 +389,16 @@ class _Fp8LinearFunction(torch.autograd.Function):
         dy2 = dy.reshape(-1, dy.size(-1))
         if dy2.dtype != torch.bfloat16:
             dy2 = dy2.to(torch.bfloat16)
-        dbias = dy2.sum(0) if ctx.has_bias and ctx.needs_input_grad[2] else None
         qxt, sxt, qwt, swt = ctx.saved_tensors
-        dx = dw = None
+        dx = dw = dbias = None
+        need_dbias = ctx.has_bias and ctx.needs_input_grad[2]
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
-            dx, dw = _official_linear_backward(dy2, (qwt, swt), (qxt, sxt), ctx.needs_input_grad[0], ctx.needs_input_grad[1], ctx.fp8_dtype)
+            if need_dbias and dy2.numel() > 0:
+                dbias = torch.empty(dy2.size(1), device=dy2.device, dtype=torch.bfloat16)
+            dx, dw = _official_linear_backward(dy2, (qwt, swt), (qxt, sxt), ctx.needs_input_grad[0], ctx.needs_input_grad[1], ctx.fp8_dtype,
+                                               dbias)
+        if need_dbias and dbias is None:
+            dbias = dy2.sum(0)
         return (dx.view(ctx.input_shape) if dx is not None else None), dw, dbias, None, None
 
 
