@@ -23,13 +23,17 @@ struct PadTable {
     int64_t rows[kPadGroups];            // rows of group g that hold data (the smaller of its two slot sizes)
 };
 
-// grid.x: chunks of 64 lanes x 16 bytes of a row, grid.y/z: destination rows (block_row()), 4 rows per block
+// Pieces of a row that a lane moves: their loads are in flight together and share one search of the table (with one piece per
+// lane, 4000 rows of 14336 bytes to 5376: 28 us).
+constexpr int kPadPieces = 4;
+
+// grid.x: chunks of 64 lanes x kPadPieces pieces of a row, grid.y/z: destination rows (block_row()), 4 rows per block
 template <int VEC>
 __global__ __launch_bounds__(256) void group_pad_kernel(const uint8_t* __restrict__ x, uint8_t* __restrict__ y,
                                                          int64_t row_bytes, int64_t dst_rows, const PadTable tbl) {
-    const int64_t row = (int64_t)block_row() * 4 + (threadIdx.x >> 6);
-    const int64_t col = ((int64_t)blockIdx.x * 64 + (threadIdx.x & 63)) * VEC;
-    if (row >= dst_rows || col >= row_bytes) return;
+    const int64_t row = (int64_t)block_row() * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t col = ((int64_t)blockIdx.x * (64 * kPadPieces) + (threadIdx.x & 63)) * VEC;
+    if (row >= dst_rows) return;
     int lo = 0, hi = tbl.n_groups - 1;     // last group whose destination slot starts at or before this row
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
@@ -40,11 +44,24 @@ __global__ __launch_bounds__(256) void group_pad_kernel(const uint8_t* __restric
     const uint8_t* src = x + (tbl.src_start[lo] + r) * row_bytes + col;
     uint8_t* dst = y + row * row_bytes + col;
     if (VEC == 16) {
-        store_nt16(dst, data ? load_nt16(src) : make_uint4(0u, 0u, 0u, 0u));
-    } else if (VEC == 2) {
-        *reinterpret_cast<uint16_t*>(dst) = data ? *reinterpret_cast<const uint16_t*>(src) : (uint16_t)0;
-    } else {
-        *dst = data ? *src : (uint8_t)0;
+        uint4 v[kPadPieces];
+#pragma unroll
+        for (int p = 0; p < kPadPieces; ++p) {
+            v[p] = make_uint4(0u, 0u, 0u, 0u);
+            if (data && col + p * 64 * VEC < row_bytes) v[p] = load_nt16(src + p * 64 * VEC);
+        }
+#pragma unroll
+        for (int p = 0; p < kPadPieces; ++p)
+            if (col + p * 64 * VEC < row_bytes) store_nt16(dst + p * 64 * VEC, v[p]);
+        return;
+    }
+#pragma unroll
+    for (int p = 0; p < kPadPieces; ++p) {
+        if (col + p * 64 * VEC >= row_bytes) break;
+        if (VEC == 2)
+            *reinterpret_cast<uint16_t*>(dst + p * 64 * VEC) = data ? *reinterpret_cast<const uint16_t*>(src + p * 64 * VEC) : (uint16_t)0;
+        else
+            dst[p * 64 * VEC] = data ? src[p * 64 * VEC] : (uint8_t)0;
     }
 }
 
@@ -76,7 +93,7 @@ int launch_group_pad(const void* x, void* y, const int64_t* m_splits, int64_t G,
         const int64_t rows = dst_row - dst0;
         if (rows == 0 || row_bytes == 0) continue;
         dim3 grid;
-        if (!grid_rows((row_bytes + 64 * vec - 1) / (64 * vec), (rows + 3) / 4, grid)) return kErrTooManyBlocks;
+        if (!grid_rows((row_bytes + 64 * kPadPieces * vec - 1) / (64 * kPadPieces * vec), (rows + 3) / 4, grid)) return kErrTooManyBlocks;
         const uint8_t* xp = static_cast<const uint8_t*>(x) + src0 * row_bytes;
         uint8_t* yp = static_cast<uint8_t*>(y) + dst0 * row_bytes;
         if (vec == 16) hipLaunchKernelGGL(group_pad_kernel<16>, grid, dim3(256), 0, stream, xp, yp, row_bytes, rows, tbl);
