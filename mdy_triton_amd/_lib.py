@@ -29,6 +29,7 @@ SIGNATURES = {
     "mdy_quant_transpose_typed": [_p, _int, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p],
     "mdy_fp8_grouped_gemm_nt": [_p, _p, _i64, _i64, _p, _p, _p, _p, _p, _i64, _i64, _i64, _int, _p],
     "mdy_act_quant_transpose": [_p, _int, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p],
+    "mdy_quant_transpose_grouped": [_p, _int, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _p],
     "mdy_quant_transpose_colsum": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p, _p, _p],
     "mdy_fp8_gemm_nt_rowscaled": [_p, _p, _i64, _i64, _p, _p, _i64, _i64, _p, _i64, _i64, _i64, _int, _int, _p],
     "mdy_fp8_gemm_nt_rowscaled_ws": [_p, _p, _i64, _i64, _p, _p, _i64, _i64, _p, _i64, _i64, _i64, _int, _int, _p, _i64, _p],

@@ -166,6 +166,28 @@ int mdy_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, void*
                     "act_quant_transpose");
 }
 
+int mdy_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s, void* y_t, float* s_t, const int64_t* m_splits,
+                                int64_t G, int64_t K, int64_t x_row_stride, int64_t x_col_stride, void* stream) {
+    if (x_dtype != MDY_XT_BF16 && x_dtype != MDY_XT_F16 && x_dtype != MDY_XT_F32) return fail(MDY_E_DTYPE, "quant_transpose_grouped: unknown x_dtype %d", x_dtype);
+    if (G < 0 || G > 256 || K < 0 || K > kMaxDim || K % 128 != 0) return fail(MDY_E_SHAPE, "quant_transpose_grouped: G=%lld up to 256, K=%lld a multiple of 128", (long long)G, (long long)K);
+    if (G == 0 || K == 0) return 0;
+    if (!m_splits) return fail(MDY_E_NULL, "quant_transpose_grouped: null m_splits");
+    int64_t M = 0;
+    for (int64_t g = 0; g < G; ++g) {
+        if (m_splits[g] < 0 || m_splits[g] % 128 != 0 || m_splits[g] > kMaxDim) return fail(MDY_E_SHAPE, "quant_transpose_grouped: m_splits[%lld]=%lld is not a multiple of 128", (long long)g, (long long)m_splits[g]);
+        M += m_splits[g];
+    }
+    if (M > kMaxDim) return fail(MDY_E_SHAPE, "quant_transpose_grouped: too many rows (%lld)", (long long)M);
+    if (M == 0) return 0;
+    if (!x || !y || !s || !y_t || !s_t) return fail(MDY_E_NULL, "quant_transpose_grouped: null pointer");
+    if (!aligned(y, 8) || !aligned(y_t, 8) || !aligned(s, 4) || !aligned(s_t, 4) || !aligned(x, x_dtype == MDY_XT_F32 ? 4 : 2))
+        return fail(MDY_E_ALIGN, "quant_transpose_grouped: y / y_t must be 8-byte aligned, x and the scales aligned for their type");
+    if (int e = check_device()) return e;
+    return launched(mdy::launch_quant_transpose_grouped(x, x_dtype, y, s, y_t, s_t, m_splits, G, M, K, x_row_stride, x_col_stride,
+                                                        static_cast<hipStream_t>(stream)),
+                    "quant_transpose_grouped");
+}
+
 int mdy_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K, int64_t x_row_stride,
                                int64_t x_col_stride, int64_t PM, int64_t PK, int64_t s_kb_stride, int mode, float* partial,
                                void* col_sum, void* stream) {
