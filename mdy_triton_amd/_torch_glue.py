@@ -75,6 +75,32 @@ lib = _lib.load
 check = _lib.check
 
 
+class _NoHost:
+    """Stands in for the native host side where there is neither a GPU nor a build: every call goes the Python way, which
+    raises what it raises there."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+_host = None
+
+
+def host():
+    """The native host side of the serving operators (csrc/host.cpp): each function returns its result in the ordinary case and
+    None in every other, before it has done anything."""
+    global _host
+    if _host is None:
+        try:
+            from . import _host as module
+        except ImportError as e:
+            if torch.cuda.is_available():
+                raise _lib.MdyFp8Error("mdy_triton_amd/_host.so is not usable (%s): build it with `python -m mdy_triton_amd.csrc.build`" % e) from None
+            module = _NoHost()
+        _host = module
+    return _host
+
+
 _WS_BYTES = {}
 
 

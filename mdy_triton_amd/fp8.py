@@ -6,11 +6,12 @@ arguments, padding rules and returned layouts.  The GEMM that the reference
 delegates to deep_gemm.gemm_fp8_fp8_bf16_nt (fp8.py:310) is this package's own
 gfx950 kernel.
 """
+import os
 from typing import Optional, Tuple
 
 import torch
 
-from ._torch_glue import FP8, check, gemm_workspace, lib, on_device, ptr, require_gpu, stream_ptr, warn_if_scalar_gemm, xt_code
+from ._torch_glue import FP8, check, gemm_workspace, host, lib, on_device, ptr, require_gpu, stream_ptr, warn_if_scalar_gemm, xt_code
 
 
 def _cdiv(a: int, b: int) -> int:
@@ -67,6 +68,9 @@ def quant_input(x: torch.Tensor, only_forward: bool = True):
     """
     if not only_forward:
         return _quant_transpose(x, 1, "quant_input")
+    done = host().quant_input(x)
+    if done is not None:
+        return done[0], done[1], None, None
     if x.dim() != 2:
         raise ValueError("quant_input expects a 2-D tensor")
     xt = xt_code(x, "quant_input")
@@ -146,6 +150,10 @@ BIAS_IN_SUM, BIAS_AFTER_ROUNDING = 0, 1      # MDY_BIAS_*
 def _matmul(qa, sa, qb, sb, out, bias, bias_mode):
     """fp8_matmul with the choice of where the bias goes: into the fp32 sum, or onto the product rounded to bf16 (what a
     following add_bias would give, without its pass over the output)."""
+    if out is None:
+        done = host().matmul(qa, sa, qb, sb, bias, bias_mode, -1, -1)
+        if done is not None:
+            return done
     if qa.dtype != FP8 or qb.dtype != FP8:
         raise TypeError("fp8_matmul expects float8_e4m3fn operands")
     if not qa.is_contiguous() or not qb.is_contiguous() or not sb.is_contiguous():
@@ -278,9 +286,8 @@ class DeepLinear(torch.nn.Linear):
             self.invalidate_weight_cache()
 
     def _quantized_weight(self, with_transpose: bool):
-        import os
         w = self.weight
-        key = (w.data_ptr(), w._version, tuple(w.shape), w.device)
+        key = (w.data_ptr(), w._version, w.shape, w.device)
         checking = self.check_weight_cache or os.environ.get("MDY_FP8_CHECK_WEIGHT_CACHE", "0") not in ("", "0")
         cached = getattr(self, "_wq_cache", None)
         if cached is not None and cached[0] == key and (cached[1][2] is not None or not with_transpose):
@@ -295,5 +302,14 @@ class DeepLinear(torch.nn.Linear):
 
     def forward(self, input):
         grad = torch.is_grad_enabled()
+        bias = self.bias
+        if not grad and (bias is None or bias.dtype == torch.bfloat16):
+            # nothing to keep for a backward pass: both launches by one native call
+            weight = self._quantized_weight(False) if self.cache_weight else quant_weight(self.weight)
+            done = host().deep_linear(input, weight[0], weight[1], self.weight.size(0), bias,
+                                      BIAS_IN_SUM if self.fuse_bias else BIAS_AFTER_ROUNDING)
+            if done is not None:
+                return done
+            return _DeepLinear.apply(input, self.weight, bias, False, weight, self.fuse_bias)
         cache = self._quantized_weight(grad and input.requires_grad) if self.cache_weight else None
-        return _DeepLinear.apply(input, self.weight, self.bias, grad, cache, self.fuse_bias)
+        return _DeepLinear.apply(input, self.weight, bias, grad, cache, self.fuse_bias)

@@ -15,7 +15,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from ._torch_glue import FP8, check, gemm_workspace, lib, on_device, ptr, require_gpu, rowscaled_workspace, stream_ptr, xt_code
+from ._torch_glue import FP8, check, gemm_workspace, host, lib, on_device, ptr, require_gpu, rowscaled_workspace, stream_ptr, xt_code
 
 _ORDERS = ("up-gate", "gate-up")
 
@@ -103,6 +103,10 @@ def silu_act_quant(x: torch.Tensor, order: str = "up-gate", return_act: bool = F
     column-major scales).  With return_act=True the bf16 act comes back as a third value (the
     backward pass needs it); otherwise it is never written to memory.
     """
+    if not return_act and order in _ORDERS and dialect in ("official", "deeplinear"):
+        done = host().silu_act_quant(x, int(order == "gate-up"), int(dialect == "deeplinear"))
+        if done is not None:
+            return done
     x2, M, N = _flatten_up_gate(x, order, "silu_act_quant")
     dev = require_gpu(x)
     act = torch.empty(*x.shape[:-1], N, device=dev, dtype=x.dtype) if return_act else None
@@ -419,6 +423,27 @@ class Fp8Linear(torch.nn.Linear):
         return fp8_linear_with_quant_ops(x, self.weight, self.bias, self.fp8_dtype)
 
 
+def _deep_mlp(x, w_up_gate, w_down, order, up_gate_cache=None, down_cache=None):
+    """The MLP's forward pass on DeepLinear quantizers: up/gate projection, fused SwiGLU quantizer (the activation itself is
+    never written), down projection."""
+    from . import fp8 as L
+    shape = x.shape
+    N2, out_f = w_up_gate.size(0), w_down.size(0)
+    q_wu, s_wu = (up_gate_cache or L.quant_weight(w_up_gate, only_forward=True))[:2]
+    q_wd, s_wd = (down_cache or L.quant_weight(w_down, only_forward=True))[:2]
+    up_gate = host().deep_linear(x, q_wu, s_wu, N2, None, 0)
+    if up_gate is None:
+        x2 = x.reshape(-1, shape[-1])
+        q_x, s_x, _, _ = L.quant_input(x2, only_forward=True)
+        up_gate = L.fp8_matmul(q_x[:x2.size(0)], s_x[:x2.size(0)], q_wu[:N2], s_wu[:L._cdiv(N2, 128)])
+    M = up_gate.numel() // N2
+    q_act, s_act = silu_act_quant(up_gate, order, dialect="deeplinear")
+    y = host().matmul(q_act, s_act, q_wd, s_wd, None, 0, M, out_f)
+    if y is None:
+        y = L.fp8_matmul(q_act[:M], s_act[:M], q_wd[:out_f], s_wd[:L._cdiv(out_f, 128)])
+    return y if len(shape) == 2 else y.view(*shape[:-1], out_f)
+
+
 class _Fp8MlpCkptOps(torch.autograd.Function):
     """Memory-saving MLP step (fp8_kernel.py:436-494): the forward keeps only x and the two weights; the
     backward recomputes the up/gate projection and the activation, then runs the two weight-gradient and
@@ -426,21 +451,12 @@ class _Fp8MlpCkptOps(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w_up_gate, w_down, fp8_dtype=FP8, order="up-gate", up_gate_cache=None, down_cache=None):
-        from . import fp8 as L
         _require_e4m3(fp8_dtype, "fp8_ckpt_mlp")
-        shape = x.shape
-        x2 = x.reshape(-1, shape[-1])
-        M, H = x2.shape
-        N2, inter = w_up_gate.size(0), w_down.size(1)
-        q_x, s_x, _, _ = L.quant_input(x2, only_forward=True)
-        q_wu, s_wu = (up_gate_cache or L.quant_weight(w_up_gate, only_forward=True))[:2]
-        q_wd, s_wd = (down_cache or L.quant_weight(w_down, only_forward=True))[:2]
-        up_gate = L.fp8_matmul(q_x[:M], s_x[:M], q_wu[:N2], s_wu[:L._cdiv(N2, 128)])
-        q_act, s_act = silu_act_quant(up_gate, order, dialect="deeplinear")      # act itself is never written
-        y = L.fp8_matmul(q_act[:M], s_act[:M], q_wd[:w_down.size(0)], s_wd[:L._cdiv(w_down.size(0), 128)])
+        y = _deep_mlp(x, w_up_gate, w_down, order, up_gate_cache, down_cache)
+        x2 = x.reshape(-1, x.size(-1))
         ctx.save_for_backward(x2, w_up_gate, w_down)
-        ctx.order, ctx.shape, ctx.dims = order, shape, (M, H, N2, inter)
-        return y.view(*shape[:-1], w_down.size(0))
+        ctx.order, ctx.shape, ctx.dims = order, x.shape, (x2.size(0), x2.size(1), w_up_gate.size(0), w_down.size(1))
+        return y
 
     @staticmethod
     def backward(ctx, dy):
@@ -469,6 +485,21 @@ class _Fp8MlpCkptOps(torch.autograd.Function):
         return dx, dw_up_gate, dw_down, None, None, None, None
 
 
+def _official_mlp(x2, w_up_gate, w_down, fp8_dtype, order):
+    """The MLP's forward pass in the official dialect; in e4m3fn the activation is quantized by the fused SwiGLU kernel (the
+    bytes of silu_fwd + act_quant_block)."""
+    mode, _ = _fp8_mode(fp8_dtype, "fp8_ckpt_mlp")
+    qx, sx = act_quant_block(x2, dtype=fp8_dtype)
+    qwu, swu = weight_quant_block(w_up_gate, dtype=fp8_dtype)
+    qwd, swd = weight_quant_block(w_down, dtype=fp8_dtype)
+    up_gate = fp8_matmul(qx, qwu, sx, swu)
+    if mode == 0:
+        qact, sact = silu_act_quant(up_gate, order, dialect="official")       # one pass, e4m3fn
+    else:
+        qact, sact = act_quant_block(silu_fwd(up_gate, order), dtype=fp8_dtype)
+    return fp8_matmul(qact, qwd, sact, swd)
+
+
 class _Fp8MlpCkptOfficial(torch.autograd.Function):
     """The same memory-saving step in the official dialect, as the reference runs it (fp8_kernel.py:436-494):
     act_quant_block / weight_quant_block / fp8_matmul, the activation quantized by the fused SwiGLU kernel in the
@@ -476,18 +507,9 @@ class _Fp8MlpCkptOfficial(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w_up_gate, w_down, fp8_dtype=E5M2, order="up-gate"):
-        mode, _ = _fp8_mode(fp8_dtype, "fp8_ckpt_mlp")
         shape = x.shape
         x2 = x.reshape(-1, shape[-1])
-        qx, sx = act_quant_block(x2, dtype=fp8_dtype)
-        qwu, swu = weight_quant_block(w_up_gate, dtype=fp8_dtype)
-        qwd, swd = weight_quant_block(w_down, dtype=fp8_dtype)
-        up_gate = fp8_matmul(qx, qwu, sx, swu)
-        if mode == 0:
-            qact, sact = silu_act_quant(up_gate, order, dialect="official")       # one pass, e4m3fn
-        else:
-            qact, sact = act_quant_block(silu_fwd(up_gate, order), dtype=fp8_dtype)
-        y = fp8_matmul(qact, qwd, sact, swd)
+        y = _official_mlp(x2, w_up_gate, w_down, fp8_dtype, order)
         ctx.save_for_backward(x2, w_up_gate, w_down)
         ctx.order, ctx.shape, ctx.fp8_dtype = order, shape, fp8_dtype
         return y.view(*shape[:-1], w_down.size(0))
@@ -567,7 +589,14 @@ class Fp8MLP(torch.nn.Module):
         up, down = self.up_gate_proj, self.down_proj
         needs_grad = torch.is_grad_enabled() and (hidden_states.requires_grad or up.weight.requires_grad or
                                                   down.weight.requires_grad)
-        if not needs_grad or low_memory or self.low_memory:
+        if not needs_grad:
+            if self.dialect == "official":
+                y = _official_mlp(hidden_states.reshape(-1, hidden_states.size(-1)), up.weight, down.weight, self.fp8_dtype, self.order)
+                return y.view(*hidden_states.shape[:-1], down.weight.size(0))
+            return _deep_mlp(hidden_states, up.weight, down.weight, self.order,
+                             up._quantized_weight(False) if up.cache_weight else None,
+                             down._quantized_weight(False) if down.cache_weight else None)
+        if low_memory or self.low_memory:
             if self.dialect == "official":
                 return _Fp8MlpCkptOfficial.apply(hidden_states, up.weight, down.weight, self.fp8_dtype, self.order)
             # cached quantized weights (when the projections cache); the forward needs no transposed copies

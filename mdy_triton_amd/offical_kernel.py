@@ -8,7 +8,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from ._torch_glue import FP8, check, gemm_workspace, lib, on_device, out_code, ptr, require_gpu, stream_ptr, warn_if_scalar_gemm, xt_code
+from ._torch_glue import FP8, check, gemm_workspace, host, lib, on_device, out_code, ptr, require_gpu, stream_ptr, warn_if_scalar_gemm, xt_code
 
 
 def act_quant(x: torch.Tensor, block_size: int = 128) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -17,6 +17,9 @@ def act_quant(x: torch.Tensor, block_size: int = 128) -> Tuple[torch.Tensor, tor
     Mirrors act_quant at offical_kernel.py:21-28: x contiguous, last dim a multiple
     of block_size; returns (y like x in float8_e4m3fn, s fp32 [..., K/block_size]).
     """
+    done = host().act_quant(x, block_size)
+    if done is not None:
+        return done
     assert x.is_contiguous()
     assert x.size(-1) % block_size == 0
     if block_size < 8 or block_size > 512 or block_size & (block_size - 1):
@@ -66,6 +69,9 @@ def fp8_gemm(a: torch.Tensor, a_s: torch.Tensor, b: torch.Tensor, b_s: torch.Ten
     fp32, b [N, K] e4m3fn, b_s [ceil(N/128), ceil(K/128)] fp32, all contiguous; returns
     [..., N] in the default dtype.  `out_dtype` and a bf16 `bias` [N] are extensions.
     """
+    done = host().fp8_gemm(a, a_s, b, b_s, out_dtype, bias)
+    if done is not None:
+        return done
     assert a.is_contiguous() and b.is_contiguous()
     assert a_s.is_contiguous() and b_s.is_contiguous()
     if a.dtype != FP8 or b.dtype != FP8:
