@@ -109,6 +109,11 @@ int mdy_weight_quant(const void* w, void* y, float* s, void* y_t, float* s_t, in
  * kernels load with .to(tl.float32) (fp8.py:193), so an fp32 master weight is quantized from its exact values. */
 int mdy_weight_quant_typed(const void* w, int w_dtype, void* y, float* s, void* y_t, float* s_t, int64_t N, int64_t K,
                            int64_t w_row_stride, int64_t w_col_stride, int64_t PN, int64_t PK, int mode, void* stream);
+/* G weights of one shape and one pair of strides in one launch (per_block_cast_to_fp8 on a list of expert weights,
+ * megatron_patchs/fp8_matmul.py:334-392).  w: HOST array of G device pointers (read before the call returns); the outputs have
+ * a leading dimension G. */
+int mdy_weight_quant_group(const void* const* w, int64_t G, int w_dtype, void* y, float* s, void* y_t, float* s_t, int64_t N,
+                           int64_t K, int64_t w_row_stride, int64_t w_col_stride, int64_t PN, int64_t PK, int mode, void* stream);
 
 /* Training-time quantizer: row-wise 1x128 quantization of x AND the quantized transpose,
  * one read of x.  DeepLinear dialect only (clamp 1e4 + eps 1e-8, saturating cast).

@@ -25,6 +25,7 @@ SIGNATURES = {
     "mdy_act_quant_typed": [_p, _int, _int, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p],
     "mdy_weight_quant": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p],
     "mdy_weight_quant_typed": [_p, _int, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p],
+    "mdy_weight_quant_group": [_p, _i64, _int, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p],
     "mdy_quant_transpose": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p],
     "mdy_quant_transpose_typed": [_p, _int, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p],
     "mdy_fp8_grouped_gemm_nt": [_p, _p, _i64, _i64, _p, _p, _p, _p, _p, _i64, _i64, _i64, _int, _p],

@@ -99,22 +99,29 @@ int mdy_act_quant_typed(const void* x, int x_dtype, int block_size, void* y, flo
                     "act_quant_typed");
 }
 
-int mdy_weight_quant_typed(const void* w, int w_dtype, void* y, float* s, void* y_t, float* s_t, int64_t N, int64_t K,
+int mdy_weight_quant_group(const void* const* w, int64_t G, int w_dtype, void* y, float* s, void* y_t, float* s_t, int64_t N, int64_t K,
                            int64_t w_row_stride, int64_t w_col_stride, int64_t PN, int64_t PK, int mode, void* stream) {
     if (w_dtype != MDY_XT_BF16 && w_dtype != MDY_XT_F16 && w_dtype != MDY_XT_F32) return fail(MDY_E_DTYPE, "weight_quant: unknown w_dtype %d", w_dtype);
     if (mode != MDY_QUANT_OFFICIAL && mode != MDY_QUANT_DEEPLINEAR && mode != MDY_QUANT_OFFICIAL_E5M2) return fail(MDY_E_DTYPE, "weight_quant: unknown mode %d", mode);
-    if (N < 0 || K < 0 || PN < N || PK < K || PN > kMaxDim || PK > kMaxDim)
+    if (G < 0 || G > (1 << 20) || N < 0 || K < 0 || PN < N || PK < K || PN > kMaxDim || PK > kMaxDim)
         return fail(MDY_E_SHAPE, "weight_quant: need 0 <= N <= PN, 0 <= K <= PK");
     if (PN % 128 != 0 || PK % 128 != 0) return fail(MDY_E_SHAPE, "weight_quant: PN=%lld, PK=%lld must be multiples of 128", (long long)PN, (long long)PK);
     if ((y_t == nullptr) != (s_t == nullptr)) return fail(MDY_E_NULL, "weight_quant: y_t and s_t must be given together");
     if ((y == nullptr) != (s == nullptr)) return fail(MDY_E_NULL, "weight_quant: y and s must be given together");
-    if (PN == 0 || PK == 0) return 0;
-    if ((!y && !y_t) || (!w && N > 0 && K > 0)) return fail(MDY_E_NULL, "weight_quant: null pointer");
+    if (PN == 0 || PK == 0 || G == 0) return 0;
+    if (!w || (!y && !y_t)) return fail(MDY_E_NULL, "weight_quant: null pointer");
+    for (int64_t g = 0; g < G; ++g)
+        if (!w[g] && N > 0 && K > 0) return fail(MDY_E_NULL, "weight_quant: null pointer");
     if ((y && !aligned(y, 8)) || (y_t && !aligned(y_t, 8))) return fail(MDY_E_ALIGN, "weight_quant: y / y_t must be 8-byte aligned");
     if (int e = check_device()) return e;
-    return launched(mdy::launch_weight_quant(w, w_dtype, y, s, y_t, s_t, N, K, w_row_stride, w_col_stride, PN, PK, mode,
+    return launched(mdy::launch_weight_quant(w, G, w_dtype, y, s, y_t, s_t, N, K, w_row_stride, w_col_stride, PN, PK, mode,
                                              static_cast<hipStream_t>(stream)),
                     "weight_quant");
+}
+
+int mdy_weight_quant_typed(const void* w, int w_dtype, void* y, float* s, void* y_t, float* s_t, int64_t N, int64_t K,
+                           int64_t w_row_stride, int64_t w_col_stride, int64_t PN, int64_t PK, int mode, void* stream) {
+    return mdy_weight_quant_group(&w, 1, w_dtype, y, s, y_t, s_t, N, K, w_row_stride, w_col_stride, PN, PK, mode, stream);
 }
 
 int mdy_weight_quant(const void* w, void* y, float* s, void* y_t, float* s_t, int64_t N, int64_t K,

@@ -121,11 +121,17 @@ def per_block_cast_to_fp8(x, output_normal: bool = True, output_transpose: bool 
     s_t = torch.empty(G, B, A, device=dev, dtype=torch.float32) if output_transpose else None
     if PM * PN > 0:
         with on_device(dev):
-            for g, w in enumerate(xs):
-                check(lib().mdy_weight_quant_typed(ptr(w), xt, ptr(y[g]) if output_normal else None, ptr(s[g]) if output_normal else None,
-                                             ptr(y_t[g]) if output_transpose else None,
-                                             ptr(s_t[g]) if output_transpose else None, M, N, w.stride(0), w.stride(1), PM, PN, 1,
-                                             stream_ptr(dev)), "per_block_cast_to_fp8")
+            # one launch for all weights of the same strides
+            g = 0
+            while g < G:
+                n = 1
+                while g + n < G and xs[g + n].stride() == xs[g].stride():
+                    n += 1
+                w = (ctypes.c_void_p * n)(*[ptr(t) for t in xs[g:g + n]])
+                check(lib().mdy_weight_quant_group(w, n, xt, ptr(y[g]) if output_normal else None, ptr(s[g]) if output_normal else None,
+                                                   ptr(y_t[g]) if output_transpose else None, ptr(s_t[g]) if output_transpose else None, M, N,
+                                                   xs[g].stride(0), xs[g].stride(1), PM, PN, 1, stream_ptr(dev)), "per_block_cast_to_fp8")
+                g += n
     post = (lambda t: t.squeeze(0)) if G == 1 else (lambda t: t)
     out = ()
     if output_normal:

@@ -43,3 +43,14 @@ def test_padding_at_piece_edges(H, dtype):
         assert torch.equal(p[slot:slot + mg], x[row:row + mg]) and not p[slot + mg:slot + pm].any()
         row, slot = row + mg, slot + pm
     assert torch.equal(PG.unpad_groups(p, splits), x)
+
+
+@pytest.mark.parametrize("G,N,K", [(2, 128, 256), (65, 130, 200), (3, 300, 264)])      # 65: more than one launch holds
+@pytest.mark.parametrize("normal,transpose", [(True, False), (True, True), (False, True)])
+def test_weight_list(G, N, K, normal, transpose):
+    g = torch.Generator().manual_seed(G)
+    ws = [(torch.randn(N, K, generator=g) * (i + 1)).bfloat16() for i in range(G)]
+    wd = [w.cuda() if i != 1 else w.cuda().t().contiguous().t() for i, w in enumerate(ws)]      # one of other strides
+    for got, ref in zip(m.per_block_cast_to_fp8(wd, normal, transpose), O.per_block_cast_to_fp8(ws, normal, transpose)):
+        assert got.shape == ref.shape
+        assert np.array_equal(got.cpu().view(torch.uint8).numpy(), ref.view(torch.uint8).numpy())
