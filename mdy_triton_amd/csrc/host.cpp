@@ -1,6 +1,7 @@
-// Host side of the serving operators in native code: argument checks, output allocation, the current stream and the call
+// Host side of the operators in native code: argument checks, output allocation, the current stream and the call
 // into libmdyfp8.so, for the calls whose kernels take a few microseconds (one call of a Python wrapper cost 7.5 us of
-// host time against 2.3-4 us of kernel at one token).
+// host time against 2.3-4 us of kernel at one token; a small layer's training step made 110 us of them, one of 32 small
+// experts 1070 us).
 //
 // Every function takes the ordinary case - plain tensors on the current device, the layouts the operators document - and
 // returns None for anything else, before anything is allocated or launched: the Python wrapper then goes its own way, which
@@ -33,6 +34,19 @@ const Tensor* plain(PyObject* o, int& device) {
     if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.is_conj() || t.is_neg()) return nullptr;
     if (device < 0) device = (int)c10::hip::current_device();
     return t.get_device() == device ? &t : nullptr;
+}
+
+bool flag(PyObject* o) { return PyObject_IsTrue(o) == 1; }
+
+// Runs f without the interpreter lock: allocations and launches can wait (for memory, for room in the queue), and other threads
+// run meanwhile.
+template <typename F>
+auto unlocked(F f) {
+    struct Lock {
+        PyThreadState* state = PyEval_SaveThread();
+        ~Lock() { PyEval_RestoreThread(state); }
+    } lock;
+    return f();
 }
 
 void* stream_of(int device) { return (void*)c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream(); }
@@ -70,11 +84,11 @@ bool bias_arg(PyObject* o, int64_t N, int& device, const void*& p) {
 
 // c[M, N] = a . b^T with block scales; false when the library rejects the call
 bool gemm(const void* a, const float* a_s, int64_t rs, int64_t cs, const void* b, const float* b_s, void* c, const void* bias, int bias_mode,
-          int64_t M, int64_t N, int64_t K, int out_code, const at::Device& dev, void* stream) {
+          int64_t M, int64_t N, int64_t K, int fmt, int out_code, const at::Device& dev, void* stream) {
     const int64_t bytes = mdy_fp8_gemm_workspace_bytes(M, N, K);
     Tensor ws;      // handed back as soon as the launch is enqueued: the allocator reuses it in stream order only
     if (bytes > 0) ws = make({bytes}, ScalarType::Byte, dev);
-    return mdy_fp8_gemm_nt_ex(a, a_s, rs, cs, b, b_s, c, bias, bias_mode, M, N, K, MDY_FMT_E4M3, out_code, bytes > 0 ? ws.data_ptr() : nullptr,
+    return mdy_fp8_gemm_nt_ex(a, a_s, rs, cs, b, b_s, c, bias, bias_mode, M, N, K, fmt, out_code, bytes > 0 ? ws.data_ptr() : nullptr,
                               bytes > 0 ? bytes : 0, stream) == 0;
 }
 // What the MFMA kernels need of a GEMM (anything else may run the scalar kernel, about which the wrapper warns)
@@ -83,9 +97,13 @@ bool gemm_shape_ok(int64_t M, int64_t N, int64_t K, int64_t rs, int64_t cs) {
            ((M - 1) * rs + (K / 128 - 1) * cs + 1) * 4 < ((int64_t)1 << 31);
 }
 
-// act_quant(x, block_size) -> (y, s)
+ScalarType fmt_type(int fmt) { return fmt == MDY_FMT_E4M3 ? kE4m3 : ScalarType::Float8_e5m2; }
+int fmt_mode(int fmt) { return fmt == MDY_FMT_E4M3 ? MDY_QUANT_OFFICIAL : MDY_QUANT_OFFICIAL_E5M2; }
+
+// act_quant(x, block_size, fmt) -> (y, s)
 PyObject* act_quant(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    if (n != 2 || !PyLong_CheckExact(args[1])) Py_RETURN_NONE;
+    if (n != 3 || !PyLong_CheckExact(args[1]) || !PyLong_CheckExact(args[2])) Py_RETURN_NONE;
+    const int fmt = (int)PyLong_AsLong(args[2]);
     int device = -1;
     const Tensor* x = plain(args[0], device);
     const long bs = PyLong_AsLong(args[1]);
@@ -93,25 +111,29 @@ PyObject* act_quant(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int xt = xt_code(x->scalar_type());
     const int64_t K = x->size(-1), M = x->numel() / K;
     if (xt < 0 || K % bs != 0) Py_RETURN_NONE;
-    Tensor y = make(x->sizes(), kE4m3, x->device());
-    auto sizes = x->sizes().vec();
-    sizes.back() = K / bs;
-    Tensor s = make(sizes, ScalarType::Float, x->device());
-    if (mdy_act_quant_typed(x->data_ptr(), xt, (int)bs, y.data_ptr(), (float*)s.data_ptr(), M, K, K, M, K, K / bs, 1, MDY_QUANT_OFFICIAL, stream_of(device)) != 0)
-        Py_RETURN_NONE;
+    Tensor y, s;
+    const int rc = unlocked([&] {
+        y = make(x->sizes(), fmt_type(fmt), x->device());
+        auto sizes = x->sizes().vec();
+        sizes.back() = K / bs;
+        s = make(sizes, ScalarType::Float, x->device());
+        return mdy_act_quant_typed(x->data_ptr(), xt, (int)bs, y.data_ptr(), (float*)s.data_ptr(), M, K, K, M, K, K / bs, 1, fmt_mode(fmt), stream_of(device));
+    });
+    if (rc != 0) Py_RETURN_NONE;
     return tuple2(std::move(y), std::move(s));
 }
 
-// fp8_gemm(a, a_s, b, b_s, out_dtype or None, bias or None) -> c
+// fp8_gemm(a [.., K], a_s, b, b_s, out_dtype or None, bias or None, fmt) -> c [.., N]
 PyObject* fp8_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    if (n != 6) Py_RETURN_NONE;
+    if (n != 7 || !PyLong_CheckExact(args[6])) Py_RETURN_NONE;
+    const int fmt = (int)PyLong_AsLong(args[6]);
     int device = -1;
     const Tensor *a = plain(args[0], device), *as = plain(args[1], device), *b = plain(args[2], device), *bs = plain(args[3], device);
     if (a == nullptr || as == nullptr || b == nullptr || bs == nullptr) Py_RETURN_NONE;
     if (args[4] != Py_None && !THPDtype_Check(args[4])) Py_RETURN_NONE;
     const ScalarType out = args[4] == Py_None ? c10::get_default_dtype_as_scalartype() : reinterpret_cast<THPDtype*>(args[4])->scalar_type;
     const int code = out == ScalarType::BFloat16 ? MDY_DT_BF16 : out == ScalarType::Float ? MDY_DT_F32 : -1;
-    if (code < 0 || a->scalar_type() != kE4m3 || b->scalar_type() != kE4m3 || as->scalar_type() != ScalarType::Float ||
+    if (code < 0 || a->scalar_type() != fmt_type(fmt) || b->scalar_type() != fmt_type(fmt) || as->scalar_type() != ScalarType::Float ||
         bs->scalar_type() != ScalarType::Float || a->dim() < 1 || b->dim() != 2 || bs->dim() != 2 || a->numel() == 0 || !a->is_contiguous() ||
         !b->is_contiguous() || !as->is_contiguous() || !bs->is_contiguous())
         Py_RETURN_NONE;
@@ -120,13 +142,37 @@ PyObject* fp8_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (b->size(1) != K || !gemm_shape_ok(M, N, K, KB, 1) || as->numel() != M * KB || bs->size(0) != cdiv(N, 128) || bs->size(1) != KB ||
         !aligned16(*a) || !aligned16(*b) || !bias_arg(args[5], N, device, bias))
         Py_RETURN_NONE;
-    auto sizes = a->sizes().vec();
-    sizes.back() = N;
-    Tensor c = make(sizes, out, a->device());
-    if (!gemm(a->data_ptr(), (const float*)as->data_ptr(), KB, 1, b->data_ptr(), (const float*)bs->data_ptr(), c.data_ptr(), bias, MDY_BIAS_IN_SUM, M, N,
-              K, code, a->device(), stream_of(device)))
-        Py_RETURN_NONE;
+    Tensor c;
+    const bool ok = unlocked([&] {
+        auto sizes = a->sizes().vec();
+        sizes.back() = N;
+        c = make(sizes, out, a->device());
+        return gemm(a->data_ptr(), (const float*)as->data_ptr(), KB, 1, b->data_ptr(), (const float*)bs->data_ptr(), c.data_ptr(), bias, MDY_BIAS_IN_SUM,
+                    M, N, K, fmt, code, a->device(), stream_of(device));
+    });
+    if (!ok) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(c));
+}
+
+// weight_dequant(x [N, K], s, block_size, out_dtype or None) -> y
+PyObject* weight_dequant(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 4 || !PyLong_CheckExact(args[2]) || (args[3] != Py_None && !THPDtype_Check(args[3]))) Py_RETURN_NONE;
+    int device = -1;
+    const Tensor *x = plain(args[0], device), *s = plain(args[1], device);
+    const int64_t bs = PyLong_AsLongLong(args[2]);
+    const ScalarType out = args[3] == Py_None ? c10::get_default_dtype_as_scalartype() : reinterpret_cast<THPDtype*>(args[3])->scalar_type;
+    const int code = out == ScalarType::BFloat16 ? MDY_DT_BF16 : out == ScalarType::Float ? MDY_DT_F32 : -1;
+    if (x == nullptr || s == nullptr || code < 0 || bs < 8 || (bs & (bs - 1)) != 0 || x->scalar_type() != kE4m3 || s->scalar_type() != ScalarType::Float ||
+        x->dim() != 2 || s->dim() != 2 || x->numel() == 0 || !x->is_contiguous() || !s->is_contiguous() || s->size(0) != cdiv(x->size(0), bs) ||
+        s->size(1) != cdiv(x->size(1), bs) || bs > (1 << 20))
+        Py_RETURN_NONE;
+    Tensor y;
+    const int rc = unlocked([&] {
+        y = make(x->sizes(), out, x->device());
+        return mdy_weight_dequant_block(x->data_ptr(), (const float*)s->data_ptr(), y.data_ptr(), x->size(0), x->size(1), (int)bs, code, stream_of(device));
+    });
+    if (rc != 0) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(y));
 }
 
 // matmul(qa [>= M, K], sa logical [>= M, K/128], qb [>= N, K], sb, bias or None, bias_mode, M, N) -> bf16 [M, N]: the first M and N
@@ -146,10 +192,14 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (b->size(1) != K || !gemm_shape_ok(M, N, K, rs, cs) || M > a->size(0) || N > b->size(0) || as->size(1) != KB || bs->size(1) != KB ||
         (m < 0 ? as->size(0) != M : as->size(0) < M) || (nn < 0 ? bs->size(0) != cdiv(N, 128) : bs->size(0) < cdiv(N, 128)) || !aligned16(*a) || !aligned16(*b) || !bias_arg(args[4], N, device, bias))
         Py_RETURN_NONE;
-    Tensor c = make({M, N}, ScalarType::BFloat16, a->device());
-    if (!gemm(a->data_ptr(), (const float*)as->data_ptr(), rs, cs, b->data_ptr(), (const float*)bs->data_ptr(), c.data_ptr(), bias,
-              (int)PyLong_AsLong(args[5]), M, N, K, MDY_DT_BF16, a->device(), stream_of(device)))
-        Py_RETURN_NONE;
+    const int mode = (int)PyLong_AsLong(args[5]);
+    Tensor c;
+    const bool ok = unlocked([&] {
+        c = make({M, N}, ScalarType::BFloat16, a->device());
+        return gemm(a->data_ptr(), (const float*)as->data_ptr(), rs, cs, b->data_ptr(), (const float*)bs->data_ptr(), c.data_ptr(), bias, mode, M, N, K,
+                    MDY_FMT_E4M3, MDY_DT_BF16, a->device(), stream_of(device));
+    });
+    if (!ok) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(c));
 }
 
@@ -190,7 +240,7 @@ PyObject* quant_input(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Rows r;
     if (n != 1 || !rows_arg(args[0], device, r) || r.t->dim() != 2) Py_RETURN_NONE;
     Tensor y, s;
-    if (!quantize_rows(r, y, s, stream_of(device))) Py_RETURN_NONE;
+    if (!unlocked([&] { return quantize_rows(r, y, s, stream_of(device)); })) Py_RETURN_NONE;
     return tuple2(std::move(y), std::move(s));
 }
 
@@ -208,16 +258,483 @@ PyObject* deep_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
         !b->is_contiguous() || !bs->is_contiguous() || b->size(0) < N || b->size(1) != PK || bs->size(0) < cdiv(N, 128) || bs->size(1) != KB ||
         !gemm_shape_ok(r.M, N, PK, 1, PM) || !aligned16(*b) || !bias_arg(args[4], N, device, bias))
         Py_RETURN_NONE;
-    void* stream = stream_of(device);
-    Tensor y, s;
-    if (!quantize_rows(r, y, s, stream)) Py_RETURN_NONE;
-    auto sizes = r.t->sizes().vec();
-    sizes.back() = N;
-    Tensor c = make(sizes, ScalarType::BFloat16, r.t->device());
-    if (!gemm(y.data_ptr(), (const float*)s.data_ptr(), 1, PM, b->data_ptr(), (const float*)bs->data_ptr(), c.data_ptr(), bias,
-              (int)PyLong_AsLong(args[5]), r.M, N, PK, MDY_DT_BF16, r.t->device(), stream))
-        Py_RETURN_NONE;
+    const int mode = (int)PyLong_AsLong(args[5]);
+    Tensor c;
+    const bool ok = unlocked([&] {
+        void* stream = stream_of(device);
+        Tensor y, s;
+        if (!quantize_rows(r, y, s, stream)) return false;
+        auto sizes = r.t->sizes().vec();
+        sizes.back() = N;
+        c = make(sizes, ScalarType::BFloat16, r.t->device());
+        return gemm(y.data_ptr(), (const float*)s.data_ptr(), 1, PM, b->data_ptr(), (const float*)bs->data_ptr(), c.data_ptr(), bias, mode, r.M, N, PK,
+                    MDY_FMT_E4M3, MDY_DT_BF16, r.t->device(), stream);
+    });
+    if (!ok) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(c));
+}
+
+// ---------------------------------------------------------------------------------------------------------------------------
+// training
+// ---------------------------------------------------------------------------------------------------------------------------
+
+// Thrown when the library rejects a call in the middle of a composite one: the whole call returns None and is repeated by the
+// wrapper, whose own checks say what is wrong.  (Launches already made wrote outputs that nobody has seen.)
+struct Rejected {};
+void done(int rc) {
+    if (rc != 0) throw Rejected();
+}
+
+// a matrix: a 2-D tensor of any strides, or the flattened rows of a contiguous one
+struct Mat {
+    const Tensor* t = nullptr;
+    int64_t M = 0, K = 0, rs = 0, cs = 1;
+    int xt = -1;
+    const void* data() const { return t->data_ptr(); }
+    const at::Device dev() const { return t->device(); }
+};
+bool mat_arg(PyObject* o, int& device, Mat& m) {
+    m.t = plain(o, device);
+    if (m.t == nullptr || m.t->dim() < 1 || m.t->numel() == 0) return false;
+    m.xt = xt_code(m.t->scalar_type());
+    m.K = m.t->size(-1);
+    m.M = m.t->numel() / m.K;
+    if (m.t->dim() == 2) {
+        m.rs = m.t->stride(0);
+        m.cs = m.t->stride(1);
+    } else {
+        if (!m.t->is_contiguous()) return false;
+        m.rs = m.K;
+    }
+    return m.xt >= 0;
+}
+float* f32(const Tensor& t) { return t.defined() ? (float*)t.data_ptr() : nullptr; }
+void* raw(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+// row-wise copy y, s and transposed copy yt, st of one matrix (undefined: not asked for)
+struct Copies {
+    Tensor y, s, yt, st;
+};
+
+// DeepLinear dialect, padded to multiples of 256 (fp8.py:46-77, 122-161): s logical [PM, PK/128], strides (1, PM); t_mode 0: st
+// logical [PK, PM/128], strides (1, PK); t_mode 1: st [PK/128, PM/128].  col_sum (t_mode 0): bf16 [K], the columns' sums.
+Copies deep_copies(const Mat& x, int t_mode, const Tensor& col_sum, void* stream) {
+    const int64_t PM = cdiv(x.M, 256) * 256, PK = cdiv(x.K, 256) * 256;
+    Copies c;
+    c.y = make({PM, PK}, kE4m3, x.dev());
+    c.s = make_strided({PM, PK / 128}, {1, PM}, ScalarType::Float, x.dev());
+    c.yt = make({PK, PM}, kE4m3, x.dev());
+    c.st = t_mode == 0 ? make_strided({PK, PM / 128}, {1, PK}, ScalarType::Float, x.dev()) : make({PK / 128, PM / 128}, ScalarType::Float, x.dev());
+    if (col_sum.defined()) {
+        Tensor part = make({PM / 128, PK}, ScalarType::Float, x.dev());
+        done(mdy_quant_transpose_colsum(x.data(), raw(c.y), f32(c.s), raw(c.yt), f32(c.st), x.M, x.K, x.rs, x.cs, PM, PK, PM, MDY_QUANT_DEEPLINEAR,
+                                        f32(part), raw(col_sum), stream));
+    } else {
+        done(mdy_quant_transpose_typed(x.data(), x.xt, raw(c.y), f32(c.s), raw(c.yt), f32(c.st), x.M, x.K, x.rs, x.cs, PM, PK, PM, t_mode, stream));
+    }
+    return c;
+}
+
+// official dialect: y [PM, K], s [PM, K/128], yt [K, PM], st [K, PM/128], PM = M to a multiple of 128, K % 128 == 0
+Copies official_copies(const Mat& x, bool rows, int fmt, const Tensor& col_sum, void* stream) {
+    const int64_t PM = cdiv(x.M, 128) * 128;
+    Copies c;
+    if (rows) {
+        c.y = make({PM, x.K}, fmt_type(fmt), x.dev());
+        c.s = make({PM, x.K / 128}, ScalarType::Float, x.dev());
+    }
+    c.yt = make({x.K, PM}, fmt_type(fmt), x.dev());
+    c.st = make({x.K, PM / 128}, ScalarType::Float, x.dev());
+    if (col_sum.defined()) {
+        Tensor part = make({PM / 128, x.K}, ScalarType::Float, x.dev());
+        done(mdy_quant_transpose_colsum(x.data(), raw(c.y), f32(c.s), raw(c.yt), f32(c.st), x.M, x.K, x.rs, x.cs, PM, x.K, 0, fmt_mode(fmt), f32(part),
+                                        raw(col_sum), stream));
+    } else {
+        done(mdy_act_quant_transpose(x.data(), x.xt, raw(c.y), f32(c.s), raw(c.yt), f32(c.st), x.M, x.K, x.rs, x.cs, PM, x.K, fmt_mode(fmt), stream));
+    }
+    return c;
+}
+
+// 128x128 blocks of a weight, rows padded to PN and columns to PK
+Copies weight_copies(const Mat& w, bool rows, bool transposed, int64_t PN, int64_t PK, ScalarType type, int mode, void* stream) {
+    Copies c;
+    if (rows) {
+        c.y = make({PN, PK}, type, w.dev());
+        c.s = make({PN / 128, PK / 128}, ScalarType::Float, w.dev());
+    }
+    if (transposed) {
+        c.yt = make({PK, PN}, type, w.dev());
+        c.st = make({PK / 128, PN / 128}, ScalarType::Float, w.dev());
+    }
+    done(mdy_weight_quant_typed(w.data(), w.xt, raw(c.y), f32(c.s), raw(c.yt), f32(c.st), w.M, w.K, w.rs, w.cs, PN, PK, mode, stream));
+    return c;
+}
+
+// bf16 [sizes] = a . b^T, M rows of a (scales a_s[m * rs + kb * cs]) against N rows of b
+Tensor product(const Tensor& a, const Tensor& a_s, int64_t rs, int64_t cs, const Tensor& b, const Tensor& b_s, const void* bias, int bias_mode,
+               int64_t M, int64_t N, int64_t K, int fmt, at::IntArrayRef sizes, void* stream) {
+    if (!gemm_shape_ok(M, N, K, rs, cs)) throw Rejected();
+    Tensor c = make(sizes, ScalarType::BFloat16, a.device());
+    const int64_t bytes = mdy_fp8_gemm_workspace_bytes(M, N, K);
+    Tensor ws;
+    if (bytes > 0) ws = make({bytes}, ScalarType::Byte, a.device());
+    done(mdy_fp8_gemm_nt_ex(raw(a), f32(a_s), rs, cs, raw(b), f32(b_s), raw(c), bias, bias_mode, M, N, K, fmt, MDY_DT_BF16, raw(ws), bytes > 0 ? bytes : 0,
+                            stream));
+    return c;
+}
+
+// bf16 [M, N] = a . b^T with a scale per row and 128 columns on both sides
+Tensor row_scaled(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, int64_t M, int64_t N, int64_t K, int fmt, void* stream) {
+    Tensor c = make({M, N}, ScalarType::BFloat16, a.device());
+    const int64_t bytes = mdy_fp8_gemm_rowscaled_workspace_bytes(M, N, K);
+    Tensor ws;
+    if (bytes > 0) ws = make({bytes}, ScalarType::Byte, a.device());
+    done(mdy_fp8_gemm_nt_rowscaled_ws(raw(a), f32(a_s), a_s.stride(0), a_s.stride(1), raw(b), f32(b_s), b_s.stride(0), b_s.stride(1), raw(c), M, N, K, fmt,
+                                      MDY_DT_BF16, raw(ws), bytes > 0 ? bytes : 0, stream));
+    return c;
+}
+
+PyObject* wrap_or_none(const Tensor& t) {
+    if (!t.defined()) Py_RETURN_NONE;
+    return THPVariable_Wrap(t);
+}
+PyObject* tuple_of(std::initializer_list<Tensor> ts) {
+    PyObject* r = PyTuple_New((Py_ssize_t)ts.size());
+    if (r == nullptr) return nullptr;
+    Py_ssize_t i = 0;
+    for (const Tensor& t : ts) PyTuple_SET_ITEM(r, i++, wrap_or_none(t));
+    return r;
+}
+bool tensor_or_none(PyObject* o, int& device, Tensor& t) {
+    if (o == Py_None) return true;
+    const Tensor* p = plain(o, device);
+    if (p == nullptr) return false;
+    t = *p;
+    return true;
+}
+
+// deep_forward(x, weight, cached (y, s, yt, st) or None, bias or None, bias_mode, need_dx, need_dw) -> (out, xt, xt_s, wt, wt_s):
+// fp8.py:316-329; the transposed copies that the backward pass will need, else None
+PyObject* deep_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 7 || !PyLong_CheckExact(args[4])) Py_RETURN_NONE;
+    int device = -1;
+    Mat x, w;
+    if (!mat_arg(args[0], device, x) || !mat_arg(args[1], device, w) || w.t->dim() != 2 || w.K != x.K) Py_RETURN_NONE;
+    const bool need_dx = flag(args[5]), need_dw = flag(args[6]);
+    const int64_t N = w.M, PK = cdiv(x.K, 256) * 256, PN = cdiv(N, need_dx ? 256 : 128) * (need_dx ? 256 : 128);
+    Copies wc;
+    if (args[2] != Py_None) {
+        if (!PyTuple_CheckExact(args[2]) || PyTuple_GET_SIZE(args[2]) != 4 || !tensor_or_none(PyTuple_GET_ITEM(args[2], 0), device, wc.y) ||
+            !tensor_or_none(PyTuple_GET_ITEM(args[2], 1), device, wc.s) || !tensor_or_none(PyTuple_GET_ITEM(args[2], 2), device, wc.yt) ||
+            !tensor_or_none(PyTuple_GET_ITEM(args[2], 3), device, wc.st) || !wc.y.defined() || !wc.s.defined() || (need_dx && !wc.yt.defined()))
+            Py_RETURN_NONE;
+        if (wc.y.dim() != 2 || wc.y.size(0) < N || wc.y.size(1) != PK || !wc.y.is_contiguous() || wc.s.size(1) != PK / 128 || !wc.s.is_contiguous())
+            Py_RETURN_NONE;
+    }
+    const void* bias;
+    if (!bias_arg(args[3], N, device, bias)) Py_RETURN_NONE;
+    if (!need_dw && (x.cs != 1 || x.rs < x.K)) Py_RETURN_NONE;
+    const int mode = (int)PyLong_AsLong(args[4]);
+    Copies xc;
+    Tensor out = unlocked([&] {
+        void* stream = stream_of(device);
+        int64_t PM = cdiv(x.M, 4) * 4;
+        if (need_dw) {
+            xc = deep_copies(x, 1, Tensor(), stream);
+            PM = xc.y.size(0);
+        } else if (!quantize_rows(Rows{x.t, x.M, x.K, x.rs, x.xt}, xc.y, xc.s, stream)) {
+            throw Rejected();
+        }
+        if (!wc.y.defined()) wc = weight_copies(w, true, need_dx, PN, PK, kE4m3, MDY_QUANT_DEEPLINEAR, stream);
+        auto sizes = x.t->sizes().vec();
+        sizes.back() = N;
+        return product(xc.y, xc.s, 1, PM, wc.y, wc.s, bias, mode, x.M, N, PK, MDY_FMT_E4M3, sizes, stream);
+    });
+    return tuple_of({out, xc.yt, xc.st, wc.yt, wc.st});
+}
+
+// deep_backward(dy, xt, xt_s, wt, wt_s, K, need_dx, need_dw, need_db) -> (dx [M, K], dw [N, K], db [N]): fp8.py:330-343
+PyObject* deep_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 9 || !PyLong_CheckExact(args[5])) Py_RETURN_NONE;
+    int device = -1;
+    Mat dy;
+    Copies xc, wc;
+    if (!mat_arg(args[0], device, dy) || dy.xt != MDY_XT_BF16 || !tensor_or_none(args[1], device, xc.yt) || !tensor_or_none(args[2], device, xc.st) ||
+        !tensor_or_none(args[3], device, wc.yt) || !tensor_or_none(args[4], device, wc.st))
+        Py_RETURN_NONE;
+    const bool need_dx = flag(args[6]), need_dw = flag(args[7]), need_db = flag(args[8]);
+    const int64_t M = dy.M, N = dy.K, K = PyLong_AsLongLong(args[5]), PM = cdiv(M, 256) * 256, PN = cdiv(N, 256) * 256;
+    if ((need_dx && (!wc.yt.defined() || wc.yt.size(1) != PN || wc.yt.size(0) < K)) || (need_dw && (!xc.yt.defined() || xc.yt.size(1) != PM || xc.yt.size(0) < K)))
+        Py_RETURN_NONE;
+    Tensor db, dx, dw;
+    unlocked([&] {
+        void* stream = stream_of(device);
+        if (need_db) db = make({N}, ScalarType::BFloat16, dy.dev());
+        const Copies dc = deep_copies(dy, 0, db, stream);
+        if (need_dx) dx = product(dc.y, dc.s, 1, PM, wc.yt, wc.st, nullptr, 0, M, K, PN, MDY_FMT_E4M3, {M, K}, stream);
+        if (need_dw) dw = product(dc.yt, dc.st, 1, PN, xc.yt, xc.st, nullptr, 0, N, K, PM, MDY_FMT_E4M3, {N, K}, stream);
+    });
+    return tuple_of({dx, dw, db});
+}
+
+// official_forward(x, w, bias or None, fmt, need_dx, need_dw) -> (y, xt, xt_s, wt, wt_s): fp8_kernel.py:261-272
+PyObject* official_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 6 || !PyLong_CheckExact(args[3])) Py_RETURN_NONE;
+    int device = -1;
+    Mat x, w;
+    if (!mat_arg(args[0], device, x) || !mat_arg(args[1], device, w) || w.t->dim() != 2 || w.K != x.K || x.K % 128 != 0 || w.M % 128 != 0) Py_RETURN_NONE;
+    const int fmt = (int)PyLong_AsLong(args[3]);
+    const bool need_dx = flag(args[4]), need_dw = flag(args[5]);
+    const int64_t N = w.M, K = x.K;
+    const void* bias;
+    if (!bias_arg(args[2], N, device, bias)) Py_RETURN_NONE;
+    if (!need_dw && (x.cs != 1 || x.rs != K)) Py_RETURN_NONE;
+    Copies xc, wc;
+    Tensor y = unlocked([&] {
+        void* stream = stream_of(device);
+        if (need_dw) {
+            xc = official_copies(x, true, fmt, Tensor(), stream);
+        } else {
+            xc.y = make({x.M, K}, fmt_type(fmt), x.dev());
+            xc.s = make({x.M, K / 128}, ScalarType::Float, x.dev());
+            done(mdy_act_quant_typed(x.data(), x.xt, 128, raw(xc.y), f32(xc.s), x.M, K, K, x.M, K, K / 128, 1, fmt_mode(fmt), stream));
+        }
+        wc = weight_copies(w, true, need_dx, N, K, fmt_type(fmt), fmt_mode(fmt), stream);
+        auto sizes = x.t->sizes().vec();
+        sizes.back() = N;
+        return product(xc.y, xc.s, K / 128, 1, wc.y, wc.s, bias, MDY_BIAS_IN_SUM, x.M, N, K, fmt, sizes, stream);
+    });
+    return tuple_of({y, xc.yt, xc.st, wc.yt, wc.st});
+}
+
+// official_backward(dy, xt, xt_s, wt, wt_s, fmt, need_dx, need_dw, need_db) -> (dx, dw, db): fp8_kernel.py:274-301
+PyObject* official_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 9 || !PyLong_CheckExact(args[5])) Py_RETURN_NONE;
+    int device = -1;
+    Mat dy;
+    Copies xc, wc;
+    if (!mat_arg(args[0], device, dy) || dy.xt != MDY_XT_BF16 || dy.K % 128 != 0 || !tensor_or_none(args[1], device, xc.yt) ||
+        !tensor_or_none(args[2], device, xc.st) || !tensor_or_none(args[3], device, wc.yt) || !tensor_or_none(args[4], device, wc.st))
+        Py_RETURN_NONE;
+    const int fmt = (int)PyLong_AsLong(args[5]);
+    const bool need_dx = flag(args[6]), need_dw = flag(args[7]), need_db = flag(args[8]);
+    const int64_t M = dy.M, N = dy.K, PM = cdiv(M, 128) * 128;
+    if ((!need_dx && !need_dw) || (need_dx && (!wc.yt.defined() || wc.yt.size(1) != N)) || (need_dw && (!xc.yt.defined() || xc.yt.size(1) != PM)))
+        Py_RETURN_NONE;
+    Tensor db, dx, dw;
+    unlocked([&] {
+        void* stream = stream_of(device);
+        if (need_db) db = make({N}, ScalarType::BFloat16, dy.dev());
+        const Copies dc = official_copies(dy, need_dx, fmt, db, stream);
+        if (need_dx) dx = product(dc.y, dc.s, N / 128, 1, wc.yt, wc.st, nullptr, 0, M, wc.yt.size(0), N, fmt, {M, wc.yt.size(0)}, stream);
+        if (need_dw) dw = row_scaled(dc.yt, dc.st, xc.yt, xc.st, N, xc.yt.size(0), PM, fmt, stream);
+    });
+    return tuple_of({dx, dw, db});
+}
+
+// official_copies(x, rows, fmt) -> (y or None, s or None, yt, st), padded rows
+PyObject* act_copies(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 3 || !PyLong_CheckExact(args[2])) Py_RETURN_NONE;
+    int device = -1;
+    Mat x;
+    if (!mat_arg(args[0], device, x) || x.t->dim() != 2 || x.K % 128 != 0) Py_RETURN_NONE;
+    const bool rows = flag(args[1]);
+    const int fmt = (int)PyLong_AsLong(args[2]);
+    const Copies c = unlocked([&] { return official_copies(x, rows, fmt, Tensor(), stream_of(device)); });
+    return tuple_of({c.y, c.s, c.yt, c.st});
+}
+
+// block_copies(w, rows, transposed, fmt) -> (y, s, yt, st), None for what is not asked for
+PyObject* block_copies(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 4 || !PyLong_CheckExact(args[3])) Py_RETURN_NONE;
+    int device = -1;
+    Mat w;
+    const bool rows = flag(args[1]), transposed = flag(args[2]);
+    if (!mat_arg(args[0], device, w) || w.t->dim() != 2 || w.K % 128 != 0 || w.M % 128 != 0 || (!rows && !transposed)) Py_RETURN_NONE;
+    const int fmt = (int)PyLong_AsLong(args[3]);
+    const Copies c = unlocked([&] { return weight_copies(w, rows, transposed, w.M, w.K, fmt_type(fmt), fmt_mode(fmt), stream_of(device)); });
+    return tuple_of({c.y, c.s, c.yt, c.st});
+}
+
+// quant_weight(w, only_forward) -> (y, s, yt, st) of the DeepLinear dialect (fp8.py:206-247)
+PyObject* quant_weight(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    int device = -1;
+    Mat w;
+    if (n != 2 || !mat_arg(args[0], device, w) || w.t->dim() != 2) Py_RETURN_NONE;
+    const bool only_forward = flag(args[1]);
+    const int64_t b = only_forward ? 128 : 256;
+    const Copies c = unlocked([&] {
+        return weight_copies(w, true, !only_forward, cdiv(w.M, b) * b, cdiv(w.K, 256) * 256, kE4m3, MDY_QUANT_DEEPLINEAR, stream_of(device));
+    });
+    return tuple_of({c.y, c.s, c.yt, c.st});
+}
+
+// quant_transposed(x, t_mode) -> (y, s, yt, st) of the DeepLinear dialect's two training quantizers
+PyObject* quant_transposed(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    int device = -1;
+    Mat x;
+    if (n != 2 || !PyLong_CheckExact(args[1]) || !mat_arg(args[0], device, x) || x.t->dim() != 2) Py_RETURN_NONE;
+    const int t_mode = (int)PyLong_AsLong(args[1]);
+    const Copies c = unlocked([&] { return deep_copies(x, t_mode, Tensor(), stream_of(device)); });
+    return tuple_of({c.y, c.s, c.yt, c.st});
+}
+
+// row_scaled(x [M, K], w [N, K], sx, sw, fmt) -> bf16 [M, N]; K % 128 == 0, both scales one per row and 128 columns, any strides
+PyObject* row_scaled_product(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 5 || !PyLong_CheckExact(args[4])) Py_RETURN_NONE;
+    int device = -1;
+    const Tensor *a = plain(args[0], device), *b = plain(args[1], device), *as = plain(args[2], device), *bs = plain(args[3], device);
+    if (a == nullptr || b == nullptr || as == nullptr || bs == nullptr) Py_RETURN_NONE;
+    const int fmt = (int)PyLong_AsLong(args[4]);
+    if (a->scalar_type() != fmt_type(fmt) || b->scalar_type() != fmt_type(fmt) || as->scalar_type() != ScalarType::Float ||
+        bs->scalar_type() != ScalarType::Float || a->dim() != 2 || b->dim() != 2 || as->dim() != 2 || bs->dim() != 2 || a->numel() == 0 ||
+        b->numel() == 0 || !a->is_contiguous() || !b->is_contiguous() || !aligned16(*a) || !aligned16(*b))
+        Py_RETURN_NONE;
+    const int64_t M = a->size(0), K = a->size(1), N = b->size(0);
+    if (K % 128 != 0 || b->size(1) != K || as->size(0) != M || as->size(1) != K / 128 || bs->size(0) != N || bs->size(1) != K / 128) Py_RETURN_NONE;
+    return THPVariable_Wrap(unlocked([&] { return row_scaled(*a, *as, *b, *bs, M, N, K, fmt, stream_of(device)); }));
+}
+
+// silu_fwd(x [..., 2N], gate_first) -> bf16 [..., N];  silu_bwd(dy, x, gate_first) -> dx like x
+PyObject* silu_fwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    int device = -1;
+    if (n != 2 || !PyLong_CheckExact(args[1])) Py_RETURN_NONE;
+    const Tensor* x = plain(args[0], device);
+    if (x == nullptr || x->scalar_type() != ScalarType::BFloat16 || x->dim() < 1 || x->numel() == 0 || !x->is_contiguous() || x->size(-1) % 2 != 0)
+        Py_RETURN_NONE;
+    auto sizes = x->sizes().vec();
+    const int64_t N = sizes.back() / 2, M = x->numel() / (2 * N);
+    sizes.back() = N;
+    const int gate_first = flag(args[1]);
+    Tensor y = unlocked([&] {
+        Tensor t = make(sizes, ScalarType::BFloat16, x->device());
+        done(mdy_swiglu(x->data_ptr(), raw(t), nullptr, nullptr, M, N, 2 * N, gate_first, 0, 0, 0, 0, 0, stream_of(device)));
+        return t;
+    });
+    return THPVariable_Wrap(std::move(y));
+}
+PyObject* silu_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    int device = -1;
+    if (n != 3 || !PyLong_CheckExact(args[2])) Py_RETURN_NONE;
+    const Tensor *dy = plain(args[0], device), *x = plain(args[1], device);
+    if (x == nullptr || dy == nullptr || x->scalar_type() != ScalarType::BFloat16 || dy->scalar_type() != ScalarType::BFloat16 || x->dim() < 1 ||
+        x->numel() == 0 || !x->is_contiguous() || !dy->is_contiguous() || x->size(-1) % 2 != 0 || dy->numel() * 2 != x->numel())
+        Py_RETURN_NONE;
+    const int64_t N = x->size(-1) / 2, M = x->numel() / (2 * N);
+    const int gate_first = flag(args[2]);
+    Tensor dx = unlocked([&] {
+        Tensor t = make(x->sizes(), ScalarType::BFloat16, x->device());
+        done(mdy_swiglu_bwd(x->data_ptr(), dy->data_ptr(), raw(t), M, N, 2 * N, gate_first, stream_of(device)));
+        return t;
+    });
+    return THPVariable_Wrap(std::move(dx));
+}
+
+// ---------------------------------------------------------------------------------------------------------------------------
+// expert groups
+// ---------------------------------------------------------------------------------------------------------------------------
+bool ints_arg(PyObject* o, std::vector<int64_t>& v) {
+    const bool list = PyList_CheckExact(o);
+    if (!list && !PyTuple_CheckExact(o)) return false;
+    const Py_ssize_t n = list ? PyList_GET_SIZE(o) : PyTuple_GET_SIZE(o);
+    v.resize((size_t)n);
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        PyObject* e = list ? PyList_GET_ITEM(o, i) : PyTuple_GET_ITEM(o, i);
+        if (!PyLong_CheckExact(e)) return false;
+        const long long x = PyLong_AsLongLong(e);
+        if (x < 0) return false;      // also an overflow, cleared by the caller
+        v[(size_t)i] = x;
+    }
+    return true;
+}
+int64_t sum_of(const std::vector<int64_t>& v) {
+    int64_t t = 0;
+    for (int64_t x : v) t += x;
+    return t;
+}
+
+// group_cast(x [M, N], m_splits) -> (y, s, [yt], [st]): megatron_patchs/fp8_matmul.py:218-247
+PyObject* group_cast(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    int device = -1;
+    Mat x;
+    std::vector<int64_t> splits;
+    if (n != 2 || !mat_arg(args[0], device, x) || x.t->dim() != 2 || !ints_arg(args[1], splits) || splits.size() > 256 || sum_of(splits) != x.M ||
+        x.K % 256 != 0)
+        Py_RETURN_NONE;
+    for (int64_t m : splits)
+        if (m % 256 != 0) Py_RETURN_NONE;
+    Tensor y, s, yt, st;
+    unlocked([&] {
+        y = make({x.M, x.K}, kE4m3, x.dev());
+        s = make_strided({x.M, x.K / 128}, {1, x.M}, ScalarType::Float, x.dev());
+        yt = make({x.M * x.K}, kE4m3, x.dev());
+        st = make({x.M / 128 * x.K}, ScalarType::Float, x.dev());
+        done(mdy_quant_transpose_grouped(x.data(), x.xt, raw(y), f32(s), raw(yt), f32(st), splits.data(), (int64_t)splits.size(), x.K, x.rs, x.cs,
+                                         stream_of(device)));
+    });
+    PyObject* r = PyTuple_New(4);
+    PyObject *lt = PyList_New((Py_ssize_t)splits.size()), *ls = PyList_New((Py_ssize_t)splits.size());
+    if (r == nullptr || lt == nullptr || ls == nullptr) return nullptr;
+    int64_t row = 0;
+    for (size_t g = 0; g < splits.size(); ++g) {
+        const int64_t m = splits[g];
+        PyList_SET_ITEM(lt, (Py_ssize_t)g, THPVariable_Wrap(yt.as_strided({x.K, m}, {m > 0 ? m : 1, 1}, row * x.K)));
+        PyList_SET_ITEM(ls, (Py_ssize_t)g, THPVariable_Wrap(st.as_strided({x.K, m / 128}, {1, x.K}, row / 128 * x.K)));
+        row += m;
+    }
+    PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(std::move(y)));
+    PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(std::move(s)));
+    PyTuple_SET_ITEM(r, 2, lt);
+    PyTuple_SET_ITEM(r, 3, ls);
+    return r;
+}
+
+// grouped_matmul(qa [M, K], sa, qb [G, N, K], sb, m_splits, bias [G, N] or None) -> bf16 [M, N]
+PyObject* grouped_matmul(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 6) Py_RETURN_NONE;
+    int device = -1;
+    const Tensor *a = plain(args[0], device), *as = plain(args[1], device), *b = plain(args[2], device), *bs = plain(args[3], device);
+    std::vector<int64_t> splits;
+    if (a == nullptr || as == nullptr || b == nullptr || bs == nullptr || !ints_arg(args[4], splits)) Py_RETURN_NONE;
+    if (a->scalar_type() != kE4m3 || b->scalar_type() != kE4m3 || as->scalar_type() != ScalarType::Float || bs->scalar_type() != ScalarType::Float ||
+        a->dim() != 2 || b->dim() != 3 || as->dim() != 2 || bs->dim() != 3 || !a->is_contiguous() || !b->is_contiguous() || !bs->is_contiguous())
+        Py_RETURN_NONE;
+    const int64_t M = a->size(0), K = a->size(1), G = b->size(0), N = b->size(1), KB = K / 128;
+    const void* bias;
+    if (b->size(2) != K || !gemm_shape_ok(M, N, K, as->stride(0), as->stride(1)) || as->size(0) != M || as->size(1) != KB || bs->size(0) != G ||
+        bs->size(1) != cdiv(N, 128) || bs->size(2) != KB || (int64_t)splits.size() != G || sum_of(splits) != M || !bias_arg(args[5], G * N, device, bias))
+        Py_RETURN_NONE;
+    if (args[5] != Py_None && THPVariable_Unpack(args[5]).dim() != 2) Py_RETURN_NONE;
+    Tensor c = unlocked([&] {
+        Tensor t = make({M, N}, ScalarType::BFloat16, a->device());
+        done(mdy_fp8_grouped_gemm_nt(raw(*a), f32(*as), as->stride(0), as->stride(1), raw(*b), f32(*bs), raw(t), bias, splits.data(), G, N, K, MDY_DT_BF16,
+                                     stream_of(device)));
+        return t;
+    });
+    return THPVariable_Wrap(std::move(c));
+}
+
+// move_rows(x [rows, H] contiguous, m_splits, unpad, multiple) -> padded or unpadded rows
+PyObject* move_rows(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    int device = -1;
+    std::vector<int64_t> splits;
+    if (n != 4 || !PyLong_CheckExact(args[3])) Py_RETURN_NONE;
+    const Tensor* x = plain(args[0], device);
+    const int64_t multiple = PyLong_AsLongLong(args[3]);
+    if (x == nullptr || x->dim() != 2 || x->numel() == 0 || !x->is_contiguous() || multiple < 1 || !ints_arg(args[1], splits)) Py_RETURN_NONE;
+    const bool unpad = flag(args[2]);
+    int64_t padded = 0;
+    for (int64_t m : splits) padded += cdiv(m, multiple) * multiple;
+    const int64_t rows = sum_of(splits);
+    if (x->size(0) != (unpad ? padded : rows)) Py_RETURN_NONE;
+    if ((unpad ? rows : padded) == 0) Py_RETURN_NONE;
+    Tensor y = unlocked([&] {
+        Tensor t = make({unpad ? rows : padded, x->size(1)}, x->scalar_type(), x->device());
+        done(mdy_group_pad_rows(x->data_ptr(), raw(t), splits.data(), (int64_t)splits.size(), x->size(1) * (int64_t)x->element_size(), multiple,
+                                unpad ? 1 : 0, stream_of(device)));
+        return t;
+    });
+    return THPVariable_Wrap(std::move(y));
 }
 
 // silu_act_quant(x [..., 2N] bf16 contiguous, gate_first, deeplinear) -> (y, s) as the wrapper of that name returns them
@@ -231,28 +748,33 @@ PyObject* silu_act_quant(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int64_t N = x->size(-1) / 2, M = x->numel() / (2 * N);
     const int64_t PM = deep ? cdiv(M, 4) * 4 : M, PN = deep ? cdiv(N, 256) * 256 : N;
     if (PN % 128 != 0) Py_RETURN_NONE;
+    const int gate_first = flag(args[1]);
     Tensor y, s;
-    if (deep) {
-        y = make({PM, PN}, kE4m3, x->device());
-        s = make_strided({PM, PN / 128}, {1, PM}, ScalarType::Float, x->device());
-    } else {
-        auto sizes = x->sizes().vec();
-        sizes.back() = N;
-        y = make(sizes, kE4m3, x->device());
-        sizes.back() = N / 128;
-        s = make(sizes, ScalarType::Float, x->device());
-    }
-    if (mdy_swiglu(x->data_ptr(), nullptr, y.data_ptr(), (float*)s.data_ptr(), M, N, 2 * N, PyLong_AsLong(args[1]) != 0, PM, PN, deep ? 1 : N / 128,
-                   deep ? PM : 1, deep ? MDY_QUANT_DEEPLINEAR : MDY_QUANT_OFFICIAL, stream_of(device)) != 0)
-        Py_RETURN_NONE;
+    const int rc = unlocked([&] {
+        if (deep) {
+            y = make({PM, PN}, kE4m3, x->device());
+            s = make_strided({PM, PN / 128}, {1, PM}, ScalarType::Float, x->device());
+        } else {
+            auto sizes = x->sizes().vec();
+            sizes.back() = N;
+            y = make(sizes, kE4m3, x->device());
+            sizes.back() = N / 128;
+            s = make(sizes, ScalarType::Float, x->device());
+        }
+        return mdy_swiglu(x->data_ptr(), nullptr, y.data_ptr(), (float*)s.data_ptr(), M, N, 2 * N, gate_first, PM, PN, deep ? 1 : N / 128,
+                          deep ? PM : 1, deep ? MDY_QUANT_DEEPLINEAR : MDY_QUANT_OFFICIAL, stream_of(device));
+    });
+    if (rc != 0) Py_RETURN_NONE;
     return tuple2(std::move(y), std::move(s));
 }
 
-// A C++ exception (an allocation that fails) becomes None as well: the wrapper meets it again and reports it as torch does.
+// A C++ exception (a call that the library rejects, an allocation that fails) becomes None as well: the wrapper meets it again and reports it as torch does.
 template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
 PyObject* guarded(PyObject* self, PyObject* const* args, Py_ssize_t n) {
     try {
-        return F(self, args, n);
+        PyObject* r = F(self, args, n);
+        if (r == Py_None) PyErr_Clear();      // a number that did not fit: the wrapper meets it again
+        return r;
     } catch (...) {
         PyErr_Clear();
         Py_RETURN_NONE;
@@ -260,8 +782,12 @@ PyObject* guarded(PyObject* self, PyObject* const* args, Py_ssize_t n) {
 }
 
 #define MDY_METHOD(F) {#F, (PyCFunction)(void (*)(void))guarded<F>, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {MDY_METHOD(act_quant), MDY_METHOD(fp8_gemm), MDY_METHOD(matmul), MDY_METHOD(quant_input),
-                         MDY_METHOD(deep_linear), MDY_METHOD(silu_act_quant), {nullptr, nullptr, 0, nullptr}};
+PyMethodDef methods[] = {MDY_METHOD(act_quant), MDY_METHOD(fp8_gemm), MDY_METHOD(weight_dequant), MDY_METHOD(matmul), MDY_METHOD(quant_input),
+                         MDY_METHOD(deep_linear), MDY_METHOD(silu_act_quant), MDY_METHOD(deep_forward), MDY_METHOD(deep_backward),
+                         MDY_METHOD(official_forward), MDY_METHOD(official_backward), MDY_METHOD(act_copies), MDY_METHOD(block_copies),
+                         MDY_METHOD(quant_weight), MDY_METHOD(quant_transposed), MDY_METHOD(row_scaled_product), MDY_METHOD(silu_fwd),
+                         MDY_METHOD(silu_bwd), MDY_METHOD(group_cast), MDY_METHOD(grouped_matmul), MDY_METHOD(move_rows),
+                         {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

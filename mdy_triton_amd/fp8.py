@@ -20,7 +20,12 @@ def _cdiv(a: int, b: int) -> int:
 
 def _quant_transpose(x: torch.Tensor, t_mode: int, who: str, col_sum: Optional[torch.Tensor] = None):
     """Shared launcher of the two training-time quantizers (row-wise copy + quantized transpose); col_sum (t_mode 0, bf16 x):
-    a bf16 [K] tensor that receives the sums of x's columns from the same pass."""
+    a bf16 [K] tensor that receives the sums of x's columns from the same pass.  s and, for t_mode 0, s_t come back as the
+    logical [rows, groups] views."""
+    if col_sum is None:
+        done = host().quant_transposed(x, t_mode)
+        if done is not None:
+            return done
     if x.dim() != 2:
         raise ValueError("%s expects a 2-D tensor" % who)
     xt = xt_code(x, who)
@@ -37,10 +42,10 @@ def _quant_transpose(x: torch.Tensor, t_mode: int, who: str, col_sum: Optional[t
             part = torch.empty(A, PN, device=dev, dtype=torch.float32)
             check(lib().mdy_quant_transpose_colsum(ptr(x), ptr(y), ptr(s), ptr(y_t), ptr(s_t), M, K, x.stride(0), x.stride(1), PM, PN, PM,
                                                    1, ptr(part), ptr(col_sum), stream_ptr(dev)), who)
-            return y, s.transpose(0, 1), y_t, s_t
+            return y, s.transpose(0, 1), y_t, s_t.transpose(0, 1)
         check(lib().mdy_quant_transpose_typed(ptr(x), xt, ptr(y), ptr(s), ptr(y_t), ptr(s_t), M, K, x.stride(0), x.stride(1),
                                         PM, PN, PM, t_mode, stream_ptr(dev)), who)
-    return y, s.transpose(0, 1), y_t, s_t
+    return y, s.transpose(0, 1), y_t, s_t.transpose(0, 1) if t_mode == 0 else s_t
 
 
 def quant_grad_output(x: torch.Tensor):
@@ -51,8 +56,7 @@ def quant_grad_output(x: torch.Tensor):
     [PM, PN/128] with strides (1, PM); y_t [PN, PM] quantized along M in groups of
     128, s_t logical [PN, PM/128] with strides (1, PN).
     """
-    y, s, y_t, s_t = _quant_transpose(x, 0, "quant_grad_output")
-    return y, s, y_t, s_t.transpose(0, 1)
+    return _quant_transpose(x, 0, "quant_grad_output")
 
 
 def quant_input(x: torch.Tensor, only_forward: bool = True):
@@ -96,6 +100,9 @@ def quant_weight(x: torch.Tensor, only_forward: bool = True):
     padded to 128 (256 when only_forward=False) and columns to 256, s [PM/128, PN/128];
     with only_forward=False also the transposed copy y_t [PN, PM], s_t [PN/128, PM/128].
     """
+    done = host().quant_weight(x, only_forward)
+    if done is not None:
+        return done
     if x.dim() != 2:
         raise ValueError("quant_weight expects a 2-D tensor")
     xt = xt_code(x, "quant_weight")
@@ -194,11 +201,20 @@ class _DeepLinear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, input, weight, bias, is_grad_enable, weight_cache=None, fuse_bias=False):
         inp_shape = input.shape
+        need_dgrad = bool(is_grad_enable and input.requires_grad)
+        need_wgrad = bool(is_grad_enable and weight.requires_grad)
+        done = host().deep_forward(input, weight, weight_cache, bias, BIAS_IN_SUM if fuse_bias else BIAS_AFTER_ROUNDING, need_dgrad, need_wgrad)
+        if done is not None:
+            if is_grad_enable:
+                N, K = weight.shape
+                ctx.inp_shape = inp_shape
+                ctx.dims = (input.numel() // K, N, K)
+                ctx.quantized = done[1:]
+                ctx.has_bias = bias is not None
+            return done[0]
         x = input.reshape(-1, input.size(-1))
         M, K = x.shape
         N = weight.size(0)
-        need_dgrad = bool(is_grad_enable and input.requires_grad)
-        need_wgrad = bool(is_grad_enable and weight.requires_grad)
         # fp8.py:318: the transposed input copy is only needed for wgrad
         q_inp, s_inp, q_inp_t, s_inp_t = quant_input(x, only_forward=not need_wgrad)
         if weight_cache is not None:
@@ -224,6 +240,13 @@ class _DeepLinear(torch.autograd.Function):
     def backward(ctx, grad_output):
         q_inp_t, s_inp_t, q_weight_t, s_weight_t = ctx.quantized
         M, N, K = ctx.dims
+        need = ctx.needs_input_grad
+        done = host().deep_backward(grad_output, q_inp_t, s_inp_t, q_weight_t, s_weight_t, K, need[0], need[1], ctx.has_bias and need[2])
+        if done is not None:
+            dx = done[0]
+            if dx is not None and len(ctx.inp_shape) != 2:
+                dx = dx.view(ctx.inp_shape)
+            return dx, done[1], done[2], None, None, None
         dy = grad_output.reshape(-1, N)
         if dy.dtype != torch.bfloat16:
             dy = dy.to(torch.bfloat16)
@@ -231,7 +254,6 @@ class _DeepLinear(torch.autograd.Function):
         if ctx.has_bias and ctx.needs_input_grad[2] and M > 0:
             grad_bias = torch.empty(N, device=dy.device, dtype=torch.bfloat16)
         q_dy, s_dy, q_dy_t, s_dy_t = _quant_transpose(dy, 0, "quant_grad_output", grad_bias)
-        s_dy_t = s_dy_t.transpose(0, 1)
         if ctx.needs_input_grad[0]:
             # [M, PN] . [K, PN]^T, contraction over the (zero-padded) output features
             dgrad = fp8_matmul(q_dy[:M], s_dy[:M], q_weight_t[:K], s_weight_t[:_cdiv(K, 128)]).view(*ctx.inp_shape)

@@ -51,6 +51,10 @@ def _flatten_up_gate(x: torch.Tensor, order: str, who: str):
 
 def silu_fwd(x: torch.Tensor, order: str = "up-gate") -> torch.Tensor:
     """act = silu(gate) * up as bf16 [..., N] from x [..., 2N] (fp8_kernel.py:384-402)."""
+    if order in _ORDERS:
+        done = host().silu_fwd(x, int(order == "gate-up"))
+        if done is not None:
+            return done
     x2, M, N = _flatten_up_gate(x, order, "silu_fwd")
     dev = require_gpu(x)
     y = torch.empty(*x.shape[:-1], N, device=dev, dtype=x.dtype)
@@ -64,6 +68,10 @@ def silu_fwd(x: torch.Tensor, order: str = "up-gate") -> torch.Tensor:
 
 def silu_bwd(dy: torch.Tensor, x: torch.Tensor, order: str = "up-gate") -> torch.Tensor:
     """Gradient of silu_fwd with respect to x (fp8_kernel.py:404-421); dx has x's shape."""
+    if order in _ORDERS:
+        done = host().silu_bwd(dy, x, int(order == "gate-up"))
+        if done is not None:
+            return done
     x2, M, N = _flatten_up_gate(x, order, "silu_bwd")
     dev = require_gpu(x, dy)
     if dy.dtype != torch.bfloat16 or dy.numel() != M * N:
@@ -145,7 +153,10 @@ def weight_quant_block(x: torch.Tensor, BLOCK_M: int = 128, BLOCK_N: int = 128,
     assert x.size(-1) % BLOCK_N == 0
     if BLOCK_M != 128 or BLOCK_N != 128:
         raise ValueError("only 128x128 blocks are implemented (the reference default)")
-    mode, _ = _fp8_mode(dtype, "weight_quant_block")
+    mode, fmt = _fp8_mode(dtype, "weight_quant_block")
+    done = host().block_copies(x, True, False, fmt)
+    if done is not None:
+        return done[:2]
     if x.dim() != 2:
         raise TypeError("weight_quant_block expects a 2-D tensor")
     xt = xt_code(x, "weight_quant_block")
@@ -165,7 +176,10 @@ def _weight_quant_both(w: torch.Tensor, rows: bool, transposed: bool, dtype: tor
     """One pass over w [N, K] (multiples of 128, any strides): (y, s) as weight_quant_block(w) gives them and (y_t, s_t) as
     weight_quant_block(w.t()) gives them (a block's scale does not depend on its orientation); None for what is not asked for.
     Reading w once, in rows, instead of once in rows and once in columns: [4096, 4096] e5m2 14 + 40 -> 19 us."""
-    mode, _ = _fp8_mode(dtype, who)
+    mode, fmt = _fp8_mode(dtype, who)
+    done = host().block_copies(w, rows, transposed, fmt)
+    if done is not None:
+        return done
     xt = xt_code(w, who)
     dev = require_gpu(w)
     N, K = w.shape
@@ -186,7 +200,11 @@ def _act_quant_transposed(x2: torch.Tensor, with_rows: bool, who: str, dtype: to
     """x2 [M, N] (any strides) -> (y, s, y_t_padded, s_t): the official-dialect row-wise quantization (None, None
     unless with_rows) and the quantized transpose y_t [N, PM] with s_t [N, PM/128], PM = cdiv(M, 128) * 128.  col_sum (bf16
     x2): a bf16 [N] tensor that receives the sums of x2's columns from the same pass."""
-    mode, _ = _fp8_mode(dtype, who)
+    mode, fmt = _fp8_mode(dtype, who)
+    if col_sum is None:
+        done = host().act_copies(x2, with_rows, fmt)
+        if done is not None:
+            return done
     xt = xt_code(x2, who)
     dev = require_gpu(x2)
     M, N = x2.shape
@@ -219,8 +237,11 @@ def act_quant_block(x: torch.Tensor, transpose: bool = False, dtype: torch.dtype
     assert x.size(-1) % BLOCK_N == 0
     if BLOCK_N != 128:
         raise ValueError("only BLOCK_N=128 is implemented (the reference default)")
-    mode, _ = _fp8_mode(dtype, "act_quant_block")
+    mode, fmt = _fp8_mode(dtype, "act_quant_block")
     if not transpose:
+        done = host().act_quant(x, 128, fmt)
+        if done is not None:
+            return done
         xc = x if x.is_contiguous() else x.contiguous()
         if mode == 0:
             from .offical_kernel import act_quant
@@ -254,6 +275,9 @@ def fp8_matmul(x: torch.Tensor, w: torch.Tensor, scale_x: torch.Tensor, scale_w:
         raise TypeError("fp8_matmul expects operands of one fp8 dtype, got %s and %s" % (x.dtype, w.dtype))
     _, fmt = _fp8_mode(x.dtype, "fp8_matmul")
     if have_w:
+        done = host().fp8_gemm(x, scale_x, w, scale_w, torch.bfloat16, bias, fmt)
+        if done is not None:
+            return done
         assert x.size(-1) % 128 == 0, 'in forward x @ w.T'
         x2 = x.reshape(-1, x.size(-1))
         sx2 = scale_x.reshape(-1, scale_x.size(-1))
@@ -292,6 +316,9 @@ def fp8_matmul(x: torch.Tensor, w: torch.Tensor, scale_x: torch.Tensor, scale_w:
         return y.view(*x.shape[:-1], w.size(0))
     assert x.size(0) % 128 == 0, 'in backward dy.T @ x or dy @ w'
     assert bias is None
+    done = host().row_scaled_product(x, w, scale_x, scale_w, fmt)
+    if done is not None:
+        return done
     dev = require_gpu(x, w, scale_x, scale_w)
     x2 = x.reshape(-1, x.size(-1))
     M, K = x2.shape
@@ -335,16 +362,25 @@ def fp8_matmul_bwd(xt, w, dy, dyt, scale_xt, scale_w, scale_dy, scale_dyt):
     return dx, dw
 
 
-def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8, dbias=None):
+def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8, need_dbias=False):
     """Gradients of y = x . w^T in the official dialect (fp8_kernel.py:274-301): dx = dy . w on the row-wise copy of dy
     and the block-quantized w^T, dw = dy^T . x on the transposed copies of dy and x (row scales on both operands).
     w_t = (bytes, scales) of w^T, x_t = (bytes, scales) of the transposed x; either may be None when its gradient is not
-    needed.  One kernel pass over dy gives both of its copies and, in dbias (bf16 [N] or None), its column sums; the transposed copies keep their zero padding to a multiple
+    needed.  One kernel pass over dy gives both of its copies and, for the bias gradient, its column sums; the transposed copies keep their zero padding to a multiple
     of 128 tokens."""
     _, fmt = _fp8_mode(fp8_dtype, "Fp8Linear.backward")
+    done = host().official_backward(dy2, *x_t, *w_t, fmt, need_dx, need_dw, need_dbias)
+    if done is not None:
+        return done
+    dy2 = dy2.reshape(-1, dy2.size(-1))
+    if dy2.dtype != torch.bfloat16:
+        dy2 = dy2.to(torch.bfloat16)
     M, N = dy2.shape
     dev = dy2.device
     dx = dw = None
+    if not need_dx and not need_dw:
+        return None, None, dy2.sum(0) if need_dbias else None
+    dbias = torch.empty(N, device=dev, dtype=torch.bfloat16) if need_dbias and dy2.numel() > 0 else None
     qdy, sdy, qdyt, sdyt = _act_quant_transposed(dy2, need_dx, "Fp8Linear.backward", fp8_dtype, dbias)
     if need_dx:
         dx = fp8_matmul(qdy[:M], w_t[0], sdy[:M], w_t[1], have_w=True)
@@ -356,7 +392,9 @@ def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8, db
             dw.zero_()                                   # no tokens: an empty sum
         elif N * K > 0:
             _rowscaled_into(dw, qdyt, sdyt, qxt, sxt, N, K, qdyt.size(1), fmt, dev, "Fp8Linear.backward")
-    return dx, dw
+    if need_dbias and dbias is None:
+        dbias = dy2.sum(0)
+    return dx, dw, dbias
 
 
 class _Fp8LinearFunction(torch.autograd.Function):
@@ -369,10 +407,17 @@ class _Fp8LinearFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w, bias, fp8_dtype, grad_enabled=True):
-        _fp8_mode(fp8_dtype, "Fp8Linear")
+        _, fmt = _fp8_mode(fp8_dtype, "Fp8Linear")
         input_shape = x.shape
-        x2 = x.reshape(-1, input_shape[-1])
         need_dx, need_dw = [bool(grad_enabled and n) for n in ctx.needs_input_grad[:2]]
+        ctx.has_bias = bias is not None
+        ctx.fp8_dtype = fp8_dtype
+        ctx.input_shape = input_shape
+        done = host().official_forward(x, w, bias, fmt, need_dx, need_dw)
+        if done is not None:
+            ctx.save_for_backward(*done[1:])
+            return done[0]
+        x2 = x.reshape(-1, input_shape[-1])
         if need_dw:
             assert x2.size(-1) % 128 == 0
             qx, sx, qxt, sxt = _act_quant_transposed(x2, True, "Fp8Linear", fp8_dtype)
@@ -383,27 +428,16 @@ class _Fp8LinearFunction(torch.autograd.Function):
         qw, sw, qwt, swt = _weight_quant_both(w, True, need_dx, fp8_dtype, "Fp8Linear")
         y = fp8_matmul(qx, qw, sx, sw, bias, have_w=True)
         ctx.save_for_backward(qxt, sxt, qwt, swt)
-        ctx.has_bias = bias is not None
-        ctx.fp8_dtype = fp8_dtype
-        ctx.input_shape = input_shape
         return y.view(*input_shape[:-1], w.size(0))
 
     @staticmethod
     def backward(ctx, dy):
-        dy2 = dy.reshape(-1, dy.size(-1))
-        if dy2.dtype != torch.bfloat16:
-            dy2 = dy2.to(torch.bfloat16)
         qxt, sxt, qwt, swt = ctx.saved_tensors
-        dx = dw = dbias = None
-        need_dbias = ctx.has_bias and ctx.needs_input_grad[2]
-        if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
-            if need_dbias and dy2.numel() > 0:
-                dbias = torch.empty(dy2.size(1), device=dy2.device, dtype=torch.bfloat16)
-            dx, dw = _official_linear_backward(dy2, (qwt, swt), (qxt, sxt), ctx.needs_input_grad[0], ctx.needs_input_grad[1], ctx.fp8_dtype,
-                                               dbias)
-        if need_dbias and dbias is None:
-            dbias = dy2.sum(0)
-        return (dx.view(ctx.input_shape) if dx is not None else None), dw, dbias, None, None
+        need = ctx.needs_input_grad
+        dx, dw, dbias = _official_linear_backward(dy, (qwt, swt), (qxt, sxt), need[0], need[1], ctx.fp8_dtype, ctx.has_bias and need[2])
+        if dx is not None and len(ctx.input_shape) != 2:
+            dx = dx.view(ctx.input_shape)
+        return dx, dw, dbias, None, None
 
 
 def fp8_linear_with_quant_ops(x, w, bias, fp8_dtype):
@@ -529,9 +563,9 @@ class _Fp8MlpCkptOfficial(torch.autograd.Function):
         act = silu_fwd(up_gate, ctx.order)
         _, _, qwdt, swdt = _weight_quant_both(w_down, False, True, ctx.fp8_dtype, "fp8_ckpt_mlp")
         _, _, qactt, sactt = _act_quant_transposed(act, False, "fp8_ckpt_mlp", ctx.fp8_dtype)
-        dact, dw_down = _official_linear_backward(dy2, (qwdt, swdt), (qactt, sactt), True, True, ctx.fp8_dtype)
+        dact, dw_down, _ = _official_linear_backward(dy2, (qwdt, swdt), (qactt, sactt), True, True, ctx.fp8_dtype)
         dup_gate = silu_bwd(dact, up_gate, ctx.order)
-        dx, dw_up_gate = _official_linear_backward(dup_gate, (qwut, swut), (qxt, sxt), True, True, ctx.fp8_dtype)
+        dx, dw_up_gate, _ = _official_linear_backward(dup_gate, (qwut, swut), (qxt, sxt), True, True, ctx.fp8_dtype)
         return dx.view(ctx.shape), dw_up_gate, dw_down, None, None
 
 

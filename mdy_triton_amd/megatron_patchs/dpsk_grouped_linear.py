@@ -17,7 +17,7 @@ from typing import List, Sequence, Tuple
 
 import torch
 
-from .._torch_glue import check, lib, on_device, ptr, require_gpu, stream_ptr
+from .._torch_glue import check, host, lib, on_device, ptr, require_gpu, stream_ptr
 
 PAD_MULTIPLE = 256
 
@@ -27,6 +27,9 @@ def padded_splits(m_splits: Sequence[int], multiple: int = PAD_MULTIPLE) -> List
 
 
 def _move_rows(inp: torch.Tensor, m_splits: Sequence[int], unpad: bool, multiple: int) -> torch.Tensor:
+    done = host().move_rows(inp, m_splits, unpad, multiple)
+    if done is not None:
+        return done
     if any(int(m) < 0 for m in m_splits):
         raise ValueError("m_splits must be non-negative, got %s" % list(m_splits))
     dev = require_gpu(inp)

@@ -11,7 +11,7 @@ from typing import List, Optional, Sequence
 
 import torch
 
-from .._torch_glue import FP8, check, lib, on_device, ptr, require_gpu, stream_ptr, xt_code
+from .._torch_glue import FP8, check, host, lib, on_device, ptr, require_gpu, stream_ptr, xt_code
 from ..fp8 import _cdiv, fp8_matmul, quant_input  # noqa: F401  (fp8_matmul is re-exported under the reference's name)
 
 
@@ -54,6 +54,9 @@ def group_per_token_cast_to_fp8(x_all: torch.Tensor, m_splits: Sequence[int]):
     Returns (y_all [M, N], s_all logical [M, N/128] with strides (1, M), [y_t of group g: [N, m_g]],
     [s_t of group g: logical [N, m_g/128]]).
     """
+    done = host().group_cast(x_all, m_splits)
+    if done is not None:
+        return done
     xt = _check_2d(x_all, "group_per_token_cast_to_fp8")
     dev = require_gpu(x_all)
     Mtot, N = x_all.shape
@@ -149,6 +152,10 @@ def fp8_grouped_matmul(qa: torch.Tensor, sa: torch.Tensor, qb: torch.Tensor, sb:
     [G, N/128, K/128]; group sizes need no alignment.  `bias` (bf16 [G, N]) is an extension folded into
     the epilogue.
     """
+    if out is None:
+        done = host().grouped_matmul(qa, sa, qb, sb, m_splits, bias)
+        if done is not None:
+            return done
     if qa.dtype != FP8 or qb.dtype != FP8:
         raise TypeError("fp8_grouped_matmul expects float8_e4m3fn operands")
     if qb.dim() != 3 or not qa.is_contiguous() or not qb.is_contiguous() or not sb.is_contiguous():

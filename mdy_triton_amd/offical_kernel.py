@@ -17,7 +17,7 @@ def act_quant(x: torch.Tensor, block_size: int = 128) -> Tuple[torch.Tensor, tor
     Mirrors act_quant at offical_kernel.py:21-28: x contiguous, last dim a multiple
     of block_size; returns (y like x in float8_e4m3fn, s fp32 [..., K/block_size]).
     """
-    done = host().act_quant(x, block_size)
+    done = host().act_quant(x, block_size, 0)
     if done is not None:
         return done
     assert x.is_contiguous()
@@ -43,6 +43,9 @@ def weight_dequant(x: torch.Tensor, s: torch.Tensor, block_size: int = 128,
     Mirrors weight_dequant at offical_kernel.py:46-53 (2-D contiguous x and s; output
     dtype = torch.get_default_dtype() unless out_dtype is given).
     """
+    done = host().weight_dequant(x, s, block_size, out_dtype)
+    if done is not None:
+        return done
     assert x.is_contiguous() and s.is_contiguous()
     assert x.dim() == 2 and s.dim() == 2
     if block_size < 8 or block_size & (block_size - 1):
@@ -69,7 +72,7 @@ def fp8_gemm(a: torch.Tensor, a_s: torch.Tensor, b: torch.Tensor, b_s: torch.Ten
     fp32, b [N, K] e4m3fn, b_s [ceil(N/128), ceil(K/128)] fp32, all contiguous; returns
     [..., N] in the default dtype.  `out_dtype` and a bf16 `bias` [N] are extensions.
     """
-    done = host().fp8_gemm(a, a_s, b, b_s, out_dtype, bias)
+    done = host().fp8_gemm(a, a_s, b, b_s, out_dtype, bias, 0)
     if done is not None:
         return done
     assert a.is_contiguous() and b.is_contiguous()
