@@ -48,7 +48,7 @@ namespace mdy {
 // into slab ks of a caller-provided workspace [ksplit][M][N]; splitk_reduce_kernel then adds the slabs in
 // slab order (so the result does not depend on scheduling), adds the bias and converts.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int WGM, int WGN, int STAGES, int FMT>
+template <int BM, int BN, int WGM, int WGN, int STAGES, int FMT, int EPI>
 __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_splitk_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, float* __restrict__ ws, int M, int N, int K,
@@ -61,14 +61,14 @@ __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_splitk_kernel(
     int tm, tn;
     const Duty duty = tile_of(pid - ks * ntiles, tiles_m, tiles_n, tm, tn);
     const int kb0 = ks * kb_per, kb1 = min(K >> 7, kb0 + kb_per);
-    fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, float, 0, 0, 0, FMT>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, Bias{},
+    fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, float, 0, 0, 0, FMT, false, EPI>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, Bias{},
                                                    tm * BM, M, M, tn * BN, N, K, N, duty, kb0, kb1, pool);
 }
 
 // The same on the producer / consumer tile (128x128 and 128x64 tiles, 4 consumer + 4 producer waves): against the one-body
 // tile, after a cache flush / back to back, results identical: 512x4096x7168 42.6 -> 36.5 / 32.1 -> 29.4 us, 256x7168x18432
 // 89.9 -> 74.1 / 57.9 -> 53.2 us, 128x2112x7168 20.4 -> 19.2 / 15.6 -> 14.4 us, 96x4096x7168 25.3 -> 24.4 / 17.3 -> 15.4 us.
-template <int BM, int BN, int STAGES, int FMT>
+template <int BM, int BN, int STAGES, int FMT, int EPI>
 __global__ __launch_bounds__(512) void fp8_gemm_splitk_ws_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, float* __restrict__ ws, int M, int N, int K,
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_splitk_ws_kernel(
     int tm, tn;
     const Duty duty = tile_of(pid - ks * ntiles, tiles_m, tiles_n, tm, tn);
     const int kb0 = ks * kb_per, kb1 = min(K >> 7, kb0 + kb_per);
-    fp8_gemm_tile_ws<BM, BN, 2, 2, 4, STAGES, float, FMT>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, Bias{}, tm * BM, M, M,
+    fp8_gemm_tile_ws<BM, BN, 2, 2, 4, STAGES, float, FMT, EPI>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, Bias{}, tm * BM, M, M,
                                                      tn * BN, N, K, N, duty, kb0, kb1, pool);
 }
 
@@ -150,7 +150,7 @@ struct GroupTable {
 
 // Tile rows are 256 rows high; a group's last tile row, when it holds at most 128 rows, runs as a 128x256 tile
 // (ring of 3 K blocks in the LDS the 256x256 tile's ring of 2 would take).
-template <typename OUT>
+template <typename OUT, int EPI>
 __global__ __launch_bounds__(512) void fp8_grouped_gemm_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
@@ -183,9 +183,9 @@ __global__ __launch_bounds__(512) void fp8_grouped_gemm_kernel(
     const float* bsg = b_s + (size_t)g * NB * KB;
     const Bias biasg = bias.at((size_t)g * N);
     if (r1 - m0 <= 128)
-        fp8_gemm_tile<128, 256, 2, 4, 3, OUT>(a, a_s, as_rs, as_cs, as_bytes, bg, bsg, c, biasg, m0, r1, m_total, n0, N, K, N, duty, 0, KB, pool);
+        fp8_gemm_tile<128, 256, 2, 4, 3, OUT, 0, 0, 0, 0, false, EPI>(a, a_s, as_rs, as_cs, as_bytes, bg, bsg, c, biasg, m0, r1, m_total, n0, N, K, N, duty, 0, KB, pool);
     else
-        fp8_gemm_tile<256, 256, 2, 4, 2, OUT>(a, a_s, as_rs, as_cs, as_bytes, bg, bsg, c, biasg, m0, r1, m_total, n0, N, K, N, duty, 0, KB, pool);
+        fp8_gemm_tile<256, 256, 2, 4, 2, OUT, 0, 0, 0, 0, false, EPI>(a, a_s, as_rs, as_cs, as_bytes, bg, bsg, c, biasg, m0, r1, m_total, n0, N, K, N, duty, 0, KB, pool);
 }
 
 constexpr int kSmWaves = 8;      // waves per workgroup of the small-M kernels
@@ -771,11 +771,51 @@ static int launch_mfma(const uint8_t* a, const float* a_s, int64_t as_rs, int64_
     // the 256x256 tile fills a CU's LDS: one workgroup per CU that walks its tiles itself
     const int wgs = (BM * BN >= 256 * 256 && tiles_m * tiles_n > cus) ? cus : tiles_m * tiles_n;
     dim3 grid((unsigned)wgs), block(WGM * WGN * 64);
-    hipLaunchKernelGGL((fp8_gemm_mfma_kernel<BM, BN, WGM, WGN, STAGES, OUT, 0, 0, 0, FMT>), grid, block, 0, stream, a, a_s, (int)as_rs,
-                       (int)as_cs, as_bytes, b, b_s, c, bias, M, N, K, ldc, tiles_m, tiles_n, pretouch_enabled() ? 1 : 0);
+    constexpr bool FITS = BM * BN * (int)sizeof(OUT) <= TileLds<BM, BN, WGM * WGN, STAGES>::bytes, BIG = BM * BN >= 256 * 256;
+    const int epi = epilogue_kind(c, ldc, N, sizeof(OUT), BIG, FITS);
+#define MDY_MFMA(EPI)                                                                                                                   \
+    hipLaunchKernelGGL((fp8_gemm_mfma_kernel<BM, BN, WGM, WGN, STAGES, OUT, 0, 0, 0, FMT, 4, EPI>), grid, block, 0, stream, a, a_s, (int)as_rs, \
+                       (int)as_cs, as_bytes, b, b_s, c, bias, M, N, K, ldc, tiles_m, tiles_n, pretouch_enabled() ? 1 : 0)
+    if constexpr (FITS && sizeof(OUT) == 2) {
+        if (epi == kEpiLines) {
+            MDY_MFMA(kEpiLines);
+            return (int)hipGetLastError();
+        }
+    }
+    if constexpr (FITS && (BIG || sizeof(OUT) != 2)) {
+        if (epi == kEpiRows) {
+            MDY_MFMA(kEpiRows);
+            return (int)hipGetLastError();
+        }
+    }
+    MDY_MFMA(kEpiDirect);
+#undef MDY_MFMA
     return (int)hipGetLastError();
 }
 
+
+// The producer / consumer tile kernel, one workgroup per tile.
+template <int BM, int BN, int STAGES, typename OUT, int FMT>
+static int launch_ws(const uint8_t* a, const float* a_s, int64_t as_rs, int64_t as_cs, uint32_t as_bytes, const uint8_t* b, const float* b_s, OUT* c,
+                     const Bias bias, int M, int N, int K, hipStream_t stream) {
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    constexpr bool HOLD_A = BM / 2 <= BN / 2;
+    constexpr bool FITS = BM * BN * (int)sizeof(OUT) <= TileLdsWs<BM, BN, 8, HOLD_A ? STAGES - 1 : STAGES, HOLD_A ? STAGES : STAGES - 1, STAGES - 1>::bytes;
+    constexpr int ROWS = sizeof(OUT) == 2 ? kEpiLines : kEpiRows;
+    const int epi = epilogue_kind(c, N, N, sizeof(OUT), false, FITS);
+#define MDY_WS_K(EPI)                                                                                                                    \
+    hipLaunchKernelGGL((fp8_gemm_ws_kernel<BM, BN, 2, 2, 4, STAGES, OUT, FMT, EPI>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, stream, a, a_s, \
+                       (int)as_rs, (int)as_cs, as_bytes, b, b_s, c, bias, M, N, K, N, tiles_m, tiles_n, pretouch_enabled() ? 1 : 0)
+    if constexpr (FITS) {
+        if (epi == ROWS) {
+            MDY_WS_K(ROWS);
+            return (int)hipGetLastError();
+        }
+    }
+    MDY_WS_K(kEpiDirect);
+#undef MDY_WS_K
+    return (int)hipGetLastError();
+}
 
 // How many 256-wide tile columns the 256x256 kernel should take when the tile count is not a
 // multiple of the CU count: if the last, partly filled round holds at most half a round of
@@ -909,10 +949,7 @@ static int dispatch_small(const uint8_t* a, const float* a_s, int64_t as_rs, int
     // (128..199 tiles of 128x128, one per CU, on the producer / consumer body: against the one-body tile, back to back, M=64
     // N=18432 K=7168 36.1 -> 28.2 us, M=48 N=16384 K=2048 13.5 -> 10.7 us, M=64 N=24576 K=1536 12.6 -> 10.5 us; 2-3 % after a flush)
     if (!lines && M >= 32 && M <= 64 && big_ok && (N + 127) / 128 >= 128) {
-        const int tiles_n = (N + 127) / 128;
-        hipLaunchKernelGGL((fp8_gemm_ws_kernel<128, 128, 2, 2, 4, 4, OUT, FMT>), dim3((unsigned)tiles_n), dim3(512), 0, stream, a, a_s,
-                           (int)as_rs, (int)as_cs, (uint32_t)as_extent, b, b_s, c, bias, M, N, K, N, 1, tiles_n, pretouch_enabled() ? 1 : 0);
-        return (int)hipGetLastError();
+        return launch_ws<128, 128, 4, OUT, FMT>(a, a_s, as_rs, as_cs, (uint32_t)as_extent, b, b_s, c, bias, M, N, K, stream);
     }
     if (!lines && M >= 32 && M <= 64 && big_ok && (N + 63) / 64 >= 100)
         return launch_mfma<64, 64, 2, 2, 8, OUT, FMT>(a, a_s, as_rs, as_cs, (uint32_t)as_extent, b, b_s, c, bias, M, N, K, N, stream);
@@ -1042,18 +1079,9 @@ static int dispatch_tiles(const uint8_t* a, const float* a_s, int64_t as_rs, int
 #define MDY_FEW(BM_, BN_, WGM_, WGN_, ST_)                                                                            \
     return launch_mfma<BM_, BN_, WGM_, WGN_, ST_, OUT, FMT>(a, a_s, as_rs, as_cs, (uint32_t)as_extent, b, b_s, c, bias, M, N, K, N, stream)
     switch (few_tiles_config(M, N, K)) {
-#define MDY_WS(BM_, BN_, ST_)                                                                                          \
-    {                                                                                                                  \
-        const int tiles_m = (M + BM_ - 1) / BM_, tiles_n = (N + BN_ - 1) / BN_;                                        \
-        hipLaunchKernelGGL((fp8_gemm_ws_kernel<BM_, BN_, 2, 2, 4, ST_, OUT, FMT>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, \
-                           stream, a, a_s, (int)as_rs, (int)as_cs, (uint32_t)as_extent, b, b_s, c, bias, M, N, K, N, tiles_m, \
-                           tiles_n, pretouch_enabled() ? 1 : 0);                                                       \
-        return (int)hipGetLastError();                                                                                 \
-    }
-        case 1: MDY_WS(128, 128, 4)
-        case 2: MDY_WS(128, 64, 5)
-        case 6: MDY_WS(128, 192, 4)
-#undef MDY_WS
+        case 1: return launch_ws<128, 128, 4, OUT, FMT>(a, a_s, as_rs, as_cs, (uint32_t)as_extent, b, b_s, c, bias, M, N, K, stream);
+        case 2: return launch_ws<128, 64, 5, OUT, FMT>(a, a_s, as_rs, as_cs, (uint32_t)as_extent, b, b_s, c, bias, M, N, K, stream);
+        case 6: return launch_ws<128, 192, 4, OUT, FMT>(a, a_s, as_rs, as_cs, (uint32_t)as_extent, b, b_s, c, bias, M, N, K, stream);
         case 3: MDY_FEW(64, 64, 2, 2, 8);
         case 4: MDY_FEW(128, 256, 2, 4, 3);
         case 5: MDY_FEW(256, 128, 2, 4, 3);
@@ -1186,12 +1214,16 @@ static int launch_splitk(const uint8_t* a, const float* a_s, int64_t as_rs, int6
                     ((reinterpret_cast<uintptr_t>(ws) & 15) == 0) && as_rs >= 0 && as_cs >= 0 &&
                     as_extent < ((int64_t)1 << 31);
     if (!ok) return -1;
+    // the slabs are [M][N] fp32 like an fp32 result; a slab starts on 16 bytes when N % 4 == 0
+    const bool rows = epilogue_kind(ws, N, N, 4, false, true) == kEpiRows;
+#define MDY_SPLIT_E(KERNEL, BM_, BN_, THREADS)                                                                        \
+    hipLaunchKernelGGL(KERNEL, dim3((unsigned)(tiles_m * tiles_n * p.ksplit)), dim3(THREADS), 0, stream, a, a_s, (int)as_rs, (int)as_cs, \
+                       (uint32_t)as_extent, b, b_s, ws, M, N, K, tiles_m, tiles_n, p.ksplit, p.kb_per)
 #define MDY_SPLIT(BM_, BN_, ST_)                                                                                      \
     {                                                                                                                 \
         const int tiles_m = (M + BM_ - 1) / BM_, tiles_n = (N + BN_ - 1) / BN_;                                       \
-        hipLaunchKernelGGL((fp8_gemm_splitk_kernel<BM_, BN_, 2, 2, ST_, FMT>), dim3((unsigned)(tiles_m * tiles_n * p.ksplit)), \
-                           dim3(256), 0, stream, a, a_s, (int)as_rs, (int)as_cs, (uint32_t)as_extent, b, b_s, ws, M, N, K, \
-                           tiles_m, tiles_n, p.ksplit, p.kb_per);                                                     \
+        if (rows) MDY_SPLIT_E((fp8_gemm_splitk_kernel<BM_, BN_, 2, 2, ST_, FMT, kEpiRows>), BM_, BN_, 256);           \
+        else MDY_SPLIT_E((fp8_gemm_splitk_kernel<BM_, BN_, 2, 2, ST_, FMT, kEpiDirect>), BM_, BN_, 256);              \
     }
     if (p.config == 4) {
         dim3 grid((unsigned)((N + 31) / 32), (unsigned)p.ksplit);
@@ -1205,15 +1237,15 @@ static int launch_splitk(const uint8_t* a, const float* a_s, int64_t as_rs, int6
 #define MDY_SPLIT_WS(BM_, BN_, ST_)                                                                                   \
     {                                                                                                                 \
         const int tiles_m = (M + BM_ - 1) / BM_, tiles_n = (N + BN_ - 1) / BN_;                                       \
-        hipLaunchKernelGGL((fp8_gemm_splitk_ws_kernel<BM_, BN_, ST_, FMT>), dim3((unsigned)(tiles_m * tiles_n * p.ksplit)), \
-                           dim3(512), 0, stream, a, a_s, (int)as_rs, (int)as_cs, (uint32_t)as_extent, b, b_s, ws, M, N, K, \
-                           tiles_m, tiles_n, p.ksplit, p.kb_per);                                                     \
+        if (rows) MDY_SPLIT_E((fp8_gemm_splitk_ws_kernel<BM_, BN_, ST_, FMT, kEpiRows>), BM_, BN_, 512);              \
+        else MDY_SPLIT_E((fp8_gemm_splitk_ws_kernel<BM_, BN_, ST_, FMT, kEpiDirect>), BM_, BN_, 512);                 \
     }
     else if (p.config == 1) MDY_SPLIT_WS(128, 128, 4)
     else if (p.config == 2) MDY_SPLIT_WS(128, 64, 5)
     else MDY_SPLIT(64, 64, 8)
 #undef MDY_SPLIT
 #undef MDY_SPLIT_WS
+#undef MDY_SPLIT_E
     const int rc = (int)hipGetLastError();
     if (rc != 0) return rc;
     return launch_splitk_reduce(ws, c, sizeof(OUT) == 2 ? 0 : 1, bias, M, N, p.ksplit, stream);
@@ -1339,8 +1371,18 @@ static int launch_grouped(const uint8_t* a, const float* a_s, int64_t as_rs, int
     if (trow == 0) return 0;
     const int tiles_n = (N + 255) / 256;
     dim3 grid((unsigned)(trow * tiles_n)), block(512);
-    hipLaunchKernelGGL((fp8_grouped_gemm_kernel<OUT>), grid, block, 0, stream, a, a_s, (int)as_rs, (int)as_cs, as_bytes, b, b_s,
-                       c, bias, N, K, tiles_n, tbl);
+    const int epi = epilogue_kind(c, N, N, sizeof(OUT), true, sizeof(OUT) == 2);
+#define MDY_GRP(EPI)                                                                                                          \
+    hipLaunchKernelGGL((fp8_grouped_gemm_kernel<OUT, EPI>), grid, block, 0, stream, a, a_s, (int)as_rs, (int)as_cs, as_bytes, b, b_s, \
+                       c, bias, N, K, tiles_n, tbl)
+    if constexpr (sizeof(OUT) == 2) {
+        if (epi == kEpiLines) MDY_GRP(kEpiLines);
+        else if (epi == kEpiRows) MDY_GRP(kEpiRows);
+        else MDY_GRP(kEpiDirect);
+    } else {
+        MDY_GRP(kEpiDirect);
+    }
+#undef MDY_GRP
     return (int)hipGetLastError();
 }
 

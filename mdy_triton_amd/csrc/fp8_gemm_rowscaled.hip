@@ -18,7 +18,7 @@
 namespace mdy {
 
 // FMT: byte format of both operands, 0 e4m3fn, 1 e5m2 (the MFMA's cbsz / blgp operand-format fields).
-template <typename OUT, int FMT>
+template <typename OUT, int FMT, int EPI>
 __global__ __launch_bounds__(256) void fp8_gemm_rowscaled_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, int bs_rs, int bs_cs, uint32_t bs_bytes,
@@ -106,9 +106,10 @@ __global__ __launch_bounds__(256) void fp8_gemm_rowscaled_kernel(
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-    if (sizeof(OUT) == 2 && N % 8 == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0) {
+    if constexpr (EPI != kEpiDirect) {
+        static_assert(sizeof(OUT) == 2, "8 KB of LDS per wave");
         __syncthreads();     // the operand panels are free: 8 KB of results per wave
-        store_rows<4, 4, OUT>(acc, &lds_a[0][0] + wave * 8192, c, N, Bias{}, m0 + wm * 64, n0 + wn * 64, M, N, lane);
+        store_rows<4, 4, OUT, EPI == kEpiLines>(acc, &lds_a[0][0] + wave * 8192, c, N, Bias{}, m0 + wm * 64, n0 + wn * 64, M, N, lane);
         return;
     }
     const bool vec_ok = (N % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_rowscaled_kernel(
 }
 
 // The scheduled tile body of fp8_gemm_tile.h in its row-scaled-weight form; a grid smaller than the number of tiles walks them.
-template <int BM, int BN, int STAGES, typename OUT, int FMT>
+template <int BM, int BN, int STAGES, typename OUT, int FMT, int EPI>
 __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_tile_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, int bs_rs, int bs_cs, uint32_t bs_bytes,
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_tile_kernel(
     for (int pid = blockIdx.x; pid < ntiles; pid += gridDim.x) {
         int tm, tn;
         const Duty duty = tile_of(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
-        fp8_gemm_tile<BM, BN, 2, 4, STAGES, OUT, 0, 0, 0, FMT, true>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, Bias{}, tm * BM, M, M,
+        fp8_gemm_tile<BM, BN, 2, 4, STAGES, OUT, 0, 0, 0, FMT, true, EPI>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, Bias{}, tm * BM, M, M,
                                                                      tn * BN, N, K, N, duty, 0, K >> 7, pool, bs_rs, bs_cs, bs_bytes);
         __syncthreads();
     }
@@ -143,7 +144,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_tile_kernel(
 
 // The same cut along K: workgroup (slab, tile) writes the fp32 partial sums of K blocks slab * kb_per .. of its tile into a
 // workspace [slabs][M][N]; splitk_reduce_kernel adds the slabs in order.
-template <int FMT>
+template <int FMT, int EPI>
 __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, int bs_rs, int bs_cs, uint32_t bs_bytes,
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
     int tm, tn;
     const Duty duty = tile_of(pid - ks * ntiles, tiles_m, tiles_n, tm, tn);
     const int kb0 = ks * kb_per, kb1 = min(K >> 7, kb0 + kb_per);
-    fp8_gemm_tile<128, 256, 2, 4, 3, float, 0, 0, 0, FMT, true>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, Bias{},
+    fp8_gemm_tile<128, 256, 2, 4, 3, float, 0, 0, 0, FMT, true, EPI>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, Bias{},
                                                                 tm * 128, M, M, tn * 256, N, K, N, duty, kb0, kb1, pool, bs_rs, bs_cs,
                                                                 bs_bytes);
 }
@@ -218,11 +219,15 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
     if (sp.slabs > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && workspace_bytes >= (int64_t)sp.slabs * M * N * 4) {
         const int tm = (int)((M + 127) / 128), tn = (int)((N + 255) / 256);
         float* ws = static_cast<float*>(workspace);
-#define MDY_RSS(FMT)                                                                                                     \
-    hipLaunchKernelGGL((fp8_gemm_rowscaled_split_kernel<FMT>), dim3((unsigned)(tm * tn * sp.slabs)), dim3(512), 0, stream, \
+#define MDY_RSS(FMT, EPI)                                                                                                \
+    hipLaunchKernelGGL((fp8_gemm_rowscaled_split_kernel<FMT, EPI>), dim3((unsigned)(tm * tn * sp.slabs)), dim3(512), 0, stream, \
                        static_cast<const uint8_t*>(a), a_s, (int)as_rs, (int)as_cs, (uint32_t)a_ext, static_cast<const uint8_t*>(b), b_s, \
                        (int)bs_rs, (int)bs_cs, (uint32_t)b_ext, ws, (int)M, (int)N, (int)K, tm, tn, sp.slabs, sp.kb_per)
-        if (fmt == 0) MDY_RSS(0); else MDY_RSS(1);
+        if (epilogue_kind(ws, N, N, 4, false, true) == kEpiRows) {
+            if (fmt == 0) MDY_RSS(0, kEpiRows); else MDY_RSS(1, kEpiRows);
+        } else {
+            if (fmt == 0) MDY_RSS(0, kEpiDirect); else MDY_RSS(1, kEpiDirect);
+        }
 #undef MDY_RSS
         const int rc = (int)hipGetLastError();
         return rc != 0 ? rc : launch_splitk_reduce(ws, c, out_dtype, Bias{}, M, N, sp.slabs, stream);
@@ -233,14 +238,17 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
         const int64_t tm = (M + bm - 1) / bm, tn = (N + 255) / 256, cus = cu_count();
         if (tm * tn > 0x7FFFFFFF) return kErrTooManyBlocks;
         const dim3 grid((unsigned)(cfg == 2 && tm * tn > cus ? cus : tm * tn));      // 256x256: a workgroup per CU walks its tiles
-#define MDY_RST(BM, ST, OUT_T, FMT)                                                                                      \
-    hipLaunchKernelGGL((fp8_gemm_rowscaled_tile_kernel<BM, 256, ST, OUT_T, FMT>), grid, dim3(512), 0, stream,            \
+#define MDY_RST(BM, ST, OUT_T, FMT, EPI)                                                                                 \
+    hipLaunchKernelGGL((fp8_gemm_rowscaled_tile_kernel<BM, 256, ST, OUT_T, FMT, EPI>), grid, dim3(512), 0, stream,            \
                        static_cast<const uint8_t*>(a), a_s, (int)as_rs, (int)as_cs, (uint32_t)a_ext,                      \
                        static_cast<const uint8_t*>(b), b_s, (int)bs_rs, (int)bs_cs, (uint32_t)b_ext, static_cast<OUT_T*>(c), \
                        (int)M, (int)N, (int)K, (int)tm, (int)tn)
-#define MDY_RST_C(OUT_T, FMT) do { if (cfg == 2) MDY_RST(256, 2, OUT_T, FMT); else MDY_RST(128, 3, OUT_T, FMT); } while (0)
-        if (out_dtype == 0) { if (fmt == 0) MDY_RST_C(uint16_t, 0); else MDY_RST_C(uint16_t, 1); }
-        else { if (fmt == 0) MDY_RST_C(float, 0); else MDY_RST_C(float, 1); }
+#define MDY_RST_C(OUT_T, FMT, EPI) do { if (cfg == 2) MDY_RST(256, 2, OUT_T, FMT, EPI); else MDY_RST(128, 3, OUT_T, FMT, EPI); } while (0)
+        const int epi = epilogue_kind(c, N, N, out_dtype == 0 ? 2 : 4, cfg == 2, out_dtype == 0);
+        if (out_dtype != 0) { if (fmt == 0) MDY_RST_C(float, 0, kEpiDirect); else MDY_RST_C(float, 1, kEpiDirect); }
+        else if (epi == kEpiLines) { if (fmt == 0) MDY_RST_C(uint16_t, 0, kEpiLines); else MDY_RST_C(uint16_t, 1, kEpiLines); }
+        else if (epi == kEpiRows) { if (fmt == 0) MDY_RST(256, 2, uint16_t, 0, kEpiRows); else MDY_RST(256, 2, uint16_t, 1, kEpiRows); }
+        else { if (fmt == 0) MDY_RST_C(uint16_t, 0, kEpiDirect); else MDY_RST_C(uint16_t, 1, kEpiDirect); }
 #undef MDY_RST_C
 #undef MDY_RST
         return (int)hipGetLastError();
@@ -248,12 +256,14 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
     const int tiles_m = (int)((M + 127) / 128), tiles_n = (int)((N + 127) / 128);
     if ((int64_t)tiles_m * tiles_n > 0x7FFFFFFF) return kErrTooManyBlocks;
     dim3 grid((unsigned)(tiles_m * tiles_n)), block(256);
-#define MDY_RS(OUT_T, FMT)                                                                                                 \
-    hipLaunchKernelGGL((fp8_gemm_rowscaled_kernel<OUT_T, FMT>), grid, block, 0, stream, static_cast<const uint8_t*>(a), a_s, \
+#define MDY_RS(OUT_T, FMT, EPI)                                                                                            \
+    hipLaunchKernelGGL((fp8_gemm_rowscaled_kernel<OUT_T, FMT, EPI>), grid, block, 0, stream, static_cast<const uint8_t*>(a), a_s, \
                        (int)as_rs, (int)as_cs, (uint32_t)a_ext, static_cast<const uint8_t*>(b), b_s, (int)bs_rs, (int)bs_cs, \
                        (uint32_t)b_ext, static_cast<OUT_T*>(c), (int)M, (int)N, (int)K, tiles_n)
-    if (out_dtype == 0) { if (fmt == 0) MDY_RS(uint16_t, 0); else MDY_RS(uint16_t, 1); }
-    else { if (fmt == 0) MDY_RS(float, 0); else MDY_RS(float, 1); }
+    const int epi = epilogue_kind(c, N, N, out_dtype == 0 ? 2 : 4, false, out_dtype == 0);
+    if (out_dtype != 0) { if (fmt == 0) MDY_RS(float, 0, kEpiDirect); else MDY_RS(float, 1, kEpiDirect); }
+    else if (epi == kEpiLines) { if (fmt == 0) MDY_RS(uint16_t, 0, kEpiLines); else MDY_RS(uint16_t, 1, kEpiLines); }
+    else { if (fmt == 0) MDY_RS(uint16_t, 0, kEpiDirect); else MDY_RS(uint16_t, 1, kEpiDirect); }
 #undef MDY_RS
     return (int)hipGetLastError();
 }

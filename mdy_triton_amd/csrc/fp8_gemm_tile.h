@@ -53,17 +53,25 @@ __device__ __forceinline__ void store4(OUT* c, int64_t ldc, int m, int n, int M,
     }
 }
 
+// How a tile kernel writes its results: a template parameter, chosen by the host from N, ldc and the alignment of c (epilogue_kind).
+// With all three forms in one kernel the longer code costs every launch 0.15 us and 4096x1544x7168 1 us of 53.
+constexpr int kEpiDirect = 0;      // straight from registers, 8 (bf16) or 16 (fp32) bytes per lane, any N and alignment
+constexpr int kEpiLines = 1;       // bf16 through LDS in whole rows that start on 128-byte lines, non-temporal
+constexpr int kEpiRows = 2;        // through LDS in whole rows, cached: fp32, and bf16 rows that start inside lines
+
 // Epilogue of one wave's TI x TJ sub-tiles for bf16 results: through the wave's own part of LDS (TI * 16 rows of TJ * 32 bytes,
 // free once the K loop is over), so that a store instruction writes whole rows of the wave tile, 16 bytes per lane, instead of
 // 8-byte pieces of 16 different rows: a quarter of the cache lines per instruction and half the instructions.  All CUs end
 // a round of tiles together, so the stores of a tile are exposed; direct 8-byte stores -> rows through LDS -> the same with
 // non-temporal stores (whole lines, never read again by this kernel), operands rotating over three buffers:
 // 4096x18432x7168 473 -> 456 -> 451 us, 8192x4096x4096 126 -> 120 -> 117 us, 16384x4096x1024 100 -> 91 -> 84 us, 4096x7168x2048
-// 70 -> 63 -> 63 us, with row scales 4096x7168x512 45 -> 36 -> 35 us.  The 16-byte pieces of a row are XOR-swizzled by
+// 70 -> 63 -> 63 us, with row scales 4096x7168x512 45 -> 36 -> 35 us.  Where rows do not start on 128-byte lines a wave's rows
+// end inside lines that its neighbours complete, and the stores stay cached so that L2 joins the parts (3752x15224x768: 82 us direct, 86 through
+// LDS non-temporal, 80 through LDS cached).  The 16-byte pieces of a row are XOR-swizzled by
 // the row (no bank conflict either way).  Needs N % 8 == 0 and 16-byte aligned rows of c (the caller checks).
 // fp32 results (the slabs of a K split, an fp32 output) go the same way with twice the row length where the pool holds them;
 // those stores stay cached: the reduction reads the slabs next.
-template <int TI, int TJ, typename OUT>
+template <int TI, int TJ, typename OUT, bool NT>
 __device__ __forceinline__ void store_rows(const floatx4 (&acc)[TI][TJ], uint8_t* buf, OUT* __restrict__ c, int64_t ldc,
                                            const Bias bias, int m_base, int n_base, int M, int N, int lane) {
     static_assert(TJ % 2 == 0, "a row is a multiple of four 16-byte pieces");
@@ -102,10 +110,19 @@ __device__ __forceinline__ void store_rows(const floatx4 (&acc)[TI][TJ], uint8_t
         const int m = m_base + row, n = n_base + ch * EPP;
         const uint4 v = *reinterpret_cast<const uint4*>(buf + row * ROW + ((ch ^ (row & MASK)) << 4));
         if (m < M && n < N) {
-            if (HALF) store_nt16(c + (int64_t)m * ldc + n, v);
+            if (NT) store_nt16(c + (int64_t)m * ldc + n, v);
             else *reinterpret_cast<uint4*>(c + (int64_t)m * ldc + n) = v;
         }
     }
+}
+
+// The form of a launch.  Rows that do not start on whole lines go through LDS with 256x256 tiles only (3752x15224x768 83.0 us
+// direct -> 81.1; the narrower tiles tie or lose a little), fp32 results wherever the pool holds them (`fits`).
+inline int epilogue_kind(const void* c, int64_t ldc, int64_t N, int esz, bool big_tile, bool fits) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(c);
+    if (!fits || ((N | ldc) & (16 / esz - 1)) != 0 || (p & 15) != 0) return kEpiDirect;
+    if (esz != 2) return kEpiRows;
+    return ((ldc * esz) & 127) == 0 && (p & 127) == 0 ? kEpiLines : big_tile ? kEpiRows : kEpiDirect;
 }
 
 // raw buffer descriptor: base, byte range, no stride, no swizzle
@@ -203,7 +220,7 @@ struct TileLdsWs {
 // (copied by the waves behind the activation-scale waves), a lane keeps the four scales of its four columns of every
 // sub-tile, and the fold multiplies them in: 4 multiplies + 4 FMAs per MFMA instead of 4 FMAs.
 template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ = 0, int TD_ = 0, int ABL_ = 0, int FMT_ = 0,
-          bool BROW_ = false>
+          bool BROW_ = false, int EPI_ = kEpiDirect>
 __device__ __forceinline__ void fp8_gemm_tile(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
@@ -491,12 +508,12 @@ __device__ __forceinline__ void fp8_gemm_tile(
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing may still be writing LDS when the wave ends
 
     // ---- epilogue: lane holds c[m][n..n+3], m = .. + lane%16, n = .. + 4*(lane/16)
-    if (WAVES * WM * WN * (int)sizeof(OUT) <= L::bytes) {
+    if constexpr (EPI_ != kEpiDirect) {
+        static_assert(WAVES * WM * WN * (int)sizeof(OUT) <= L::bytes, "the tile's results fit the pool");
         __syncthreads();                               // every wave's copies have landed: the pool is free
-        if (((N | ldc) & (16 / (int)sizeof(OUT) - 1)) == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0) {
-            store_rows<TI, TJ, OUT>(acc, pool + wave * (WM * WN * (int)sizeof(OUT)), c, ldc, bias, m0 + wm * WM, n0 + wn * WN, M, N, lane);
-            return;
-        }
+        store_rows<TI, TJ, OUT, EPI_ == kEpiLines>(acc, pool + wave * (WM * WN * (int)sizeof(OUT)), c, ldc, bias, m0 + wm * WM, n0 + wn * WN, M, N,
+                                                   lane);
+        return;
     }
     const bool vec_ok = (ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
 #pragma unroll
@@ -563,7 +580,7 @@ __device__ __forceinline__ Duty tile_of(int local, int tiles_m, int tiles_n, int
 //   * on the 192-wide tile a wave's columns can straddle two 128-column blocks of weight scales: the combined scale is
 //     kept per row and 32-column group (multiplies once per block instead of a select per MFMA).
 // Swizzle, fragment layout, fold, epilogue and pre-touch shares are fp8_gemm_tile's.
-template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, int FMT_ = 0, int E_ = 2>
+template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, int FMT_ = 0, int EPI_ = kEpiDirect, int E_ = 2>
 __device__ __forceinline__ void fp8_gemm_tile_ws(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
@@ -608,6 +625,8 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
     const int M = m_end;
     const int KB = K >> 7;
 
+    constexpr bool through_lds = EPI_ != kEpiDirect;
+    static_assert(!through_lds || CW * WM * WN * (int)sizeof(OUT) <= L::bytes, "the tile's results fit the pool");
     if (wave >= CW) {
         // ------------------------------------------------------------------ producer
         const int pw = wave - CW;
@@ -678,7 +697,7 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
             fs = fs + 1 == SS ? 0 : fs + 1;
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing may still be writing LDS when the wave ends
-        if (CW * WM * WN * (int)sizeof(OUT) <= L::bytes) __syncthreads();      // the consumers' epilogue goes through the pool
+        if (through_lds) __syncthreads();                  // the consumers' epilogue goes through the pool
         return;
     }
 
@@ -780,12 +799,10 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
         if (kb < kb1) block(fh_a, fh_b, sc_a, sc_b, kb);     // odd number of K blocks
     }
 
-    if (CW * WM * WN * (int)sizeof(OUT) <= L::bytes) {
+    if constexpr (through_lds) {
         __syncthreads();                                 // the producers' copies have landed, every consumer has left the K loop
-        if (((N | ldc) & (16 / (int)sizeof(OUT) - 1)) == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0) {
-            store_rows<TI, TJ, OUT>(acc, pool + wave * (WM * WN * (int)sizeof(OUT)), c, ldc, bias, m0 + wm * WM, n0 + wn * WN, M, N, lane);
-            return;
-        }
+        store_rows<TI, TJ, OUT, EPI_ == kEpiLines>(acc, pool + wave * (WM * WN * (int)sizeof(OUT)), c, ldc, bias, m0 + wm * WM, n0 + wn * WN, M, N, lane);
+        return;
     }
     const bool vec_ok = (ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
 #pragma unroll
@@ -806,7 +823,7 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
 }
 
 // the wave-specialized tile as a kernel: one workgroup of WGM*WGN + PW waves per tile (or per several, walked in turn)
-template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, int FMT_ = 0, int E_ = 2>
+template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, int FMT_ = 0, int EPI_ = kEpiDirect, int E_ = 2>
 __global__ __launch_bounds__((WGM * WGN + PW) * 64) void fp8_gemm_ws_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
@@ -819,13 +836,14 @@ __global__ __launch_bounds__((WGM * WGN + PW) * 64) void fp8_gemm_ws_kernel(
         int tm, tn;
         Duty duty = tile_of(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
         if (!pretouch) duty.a_sh = duty.b_sh = 0;
-        fp8_gemm_tile_ws<BM, BN, WGM, WGN, PW, STAGES, OUT, FMT_, E_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M, M,
+        fp8_gemm_tile_ws<BM, BN, WGM, WGN, PW, STAGES, OUT, FMT_, EPI_, E_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M, M,
                                                                             tn * BN, N, K, ldc, duty, 0, K >> 7, pool);
         __syncthreads();
     }
 }
 
-template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ = 0, int TD_ = 0, int ABL_ = 0, int FMT_ = 0, int GM_ = 4>
+template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ = 0, int TD_ = 0, int ABL_ = 0, int FMT_ = 0, int GM_ = 4,
+          int EPI_ = kEpiDirect>
 __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
@@ -840,7 +858,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
         int tm, tn;
         Duty duty = tile_of<GM_>(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
         if (!pretouch) duty.a_sh = duty.b_sh = 0;
-        fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, OUT, GAP_, TD_, ABL_, FMT_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M,
+        fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, OUT, GAP_, TD_, ABL_, FMT_, false, EPI_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M,
                                                                             M, tn * BN, N, K, ldc, duty, 0, K >> 7, pool);
         __syncthreads();   // every wave has left the tile's LDS buffers before the next tile's copies land in them
     }
