@@ -149,16 +149,26 @@ struct GroupTable {
 };
 
 // Tile rows are 256 rows high; a group's last tile row, when it holds at most 128 rows, runs as a 128x256 tile
-// (ring of 3 K blocks in the LDS the 256x256 tile's ring of 2 would take).
+// (ring of 3 K blocks in the LDS the 256x256 tile's ring of 2 would take).  The first n_full tiles (whole rounds of the CUs)
+// run so; those of a last round that the CUs would not fill run in `parts` pieces each, 2 of 128x256 or 4 of 128x128
+// (producer / consumer body), which more CUs share: launch_grouped chooses.
 template <typename OUT, int EPI>
 __global__ __launch_bounds__(512) void fp8_grouped_gemm_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
-    const Bias bias, int N, int K, int tiles_n, const GroupTable tbl) {
-    constexpr int kBig = TileLds<256, 256, 8, 2>::bytes, kSmall = TileLds<128, 256, 8, 3>::bytes;
-    __shared__ __attribute__((aligned(1024))) uint8_t pool[kBig > kSmall ? kBig : kSmall];
+    const Bias bias, int N, int K, int tiles_n, int n_full, int parts, const GroupTable tbl) {
+    constexpr int kBig = TileLds<256, 256, 8, 2>::bytes, kSmall = TileLds<128, 256, 8, 3>::bytes, kQuarter = TileLdsWs<128, 128, 8, 3, 4, 3>::bytes;
+    __shared__ __attribute__((aligned(1024))) uint8_t pool[kBig > kSmall ? (kBig > kQuarter ? kBig : kQuarter) : (kSmall > kQuarter ? kSmall : kQuarter)];
     const int G = tbl.n_groups;
-    const int pid = xcd_contiguous(blockIdx.x, tbl.tile_start[G] * tiles_n);
+    int pid, part = -1;                           // tile, and which piece of it (-1: all of it)
+    if ((int)blockIdx.x < n_full) {
+        pid = xcd_contiguous(blockIdx.x, n_full);
+    } else {
+        const int q = xcd_contiguous(blockIdx.x - n_full, gridDim.x - n_full);
+        const int rest = q / parts;
+        pid = n_full + rest;
+        part = q - rest * parts;
+    }
     const int trow = pid / tiles_n;               // position in units of whole tile rows
     int lo = 0, hi = G - 1;                       // last g with tile_start[g] <= trow (empty groups skipped)
     while (lo < hi) {
@@ -174,18 +184,24 @@ __global__ __launch_bounds__(512) void fp8_grouped_gemm_kernel(
     duty.b_duty = __builtin_amdgcn_readfirstlane(duty.b_duty);
     duty.a_sh = __builtin_amdgcn_readfirstlane(duty.a_sh);
     duty.b_sh = __builtin_amdgcn_readfirstlane(duty.b_sh);
+    part = __builtin_amdgcn_readfirstlane(part);
     const int KB = K >> 7, NB = (N + 127) >> 7;
     const int r0 = __builtin_amdgcn_readfirstlane(tbl.row_start[g]), r1 = __builtin_amdgcn_readfirstlane(tbl.row_start[g + 1]);
-    const int m0 = __builtin_amdgcn_readfirstlane(r0 + tm * 256);
+    const int m0 = __builtin_amdgcn_readfirstlane(r0 + tm * 256 + (part > 0 ? (part & 1) * 128 : 0));
     const int m_total = __builtin_amdgcn_readfirstlane(tbl.row_start[G]);
-    const int n0 = __builtin_amdgcn_readfirstlane(tn * 256);
+    const int n0 = __builtin_amdgcn_readfirstlane(tn * 256 + (part > 1 ? 128 : 0));
+    if (m0 >= r1 || n0 >= N) return;              // a piece beyond the group's rows or the columns (the whole workgroup leaves)
     const uint8_t* bg = b + (size_t)g * N * K;
     const float* bsg = b_s + (size_t)g * NB * KB;
     const Bias biasg = bias.at((size_t)g * N);
-    if (r1 - m0 <= 128)
+    if (part >= 0 && parts == 4) {
+        duty.a_sh = duty.b_sh = 0;                // the pieces of a tile share no duties that tile_of could hand out
+        fp8_gemm_tile_ws<128, 128, 2, 2, 4, 4, OUT, 0, EPI>(a, a_s, as_rs, as_cs, as_bytes, bg, bsg, c, biasg, m0, r1, m_total, n0, N, K, N, duty, 0, KB, pool);
+    } else if (part >= 0 || r1 - m0 <= 128) {
         fp8_gemm_tile<128, 256, 2, 4, 3, OUT, 0, 0, 0, 0, false, EPI>(a, a_s, as_rs, as_cs, as_bytes, bg, bsg, c, biasg, m0, r1, m_total, n0, N, K, N, duty, 0, KB, pool);
-    else
+    } else {
         fp8_gemm_tile<256, 256, 2, 4, 2, OUT, 0, 0, 0, 0, false, EPI>(a, a_s, as_rs, as_cs, as_bytes, bg, bsg, c, biasg, m0, r1, m_total, n0, N, K, N, duty, 0, KB, pool);
+    }
 }
 
 constexpr int kSmWaves = 8;      // waves per workgroup of the small-M kernels
@@ -1369,12 +1385,19 @@ static int launch_grouped(const uint8_t* a, const float* a_s, int64_t as_rs, int
     }
     for (int g = G; g <= kMaxGroups; ++g) { tbl.row_start[g] = row; tbl.tile_start[g] = trow; }
     if (trow == 0) return 0;
-    const int tiles_n = (N + 255) / 256;
-    dim3 grid((unsigned)(trow * tiles_n)), block(512);
+    const int tiles_n = (N + 255) / 256, tiles = trow * tiles_n, cus = cu_count();
+    // Tiles of the last round: a tile takes its time whether the round is full or not, so up to half a round of them is cut
+    // into two pieces and up to a quarter into four (whole tiles -> pieces, 5376 rows in 8 groups: N=4096 K=7168, 256 + 80
+    // tiles, 194 -> 169 us; N=7168 K=4096, 512 + 76, 190 -> 162 us; 9 groups of 700 rows, N=4096 K=1536 76 -> 65 us; less than a round:
+    // 8 x 512 rows, N=2048 K=2048, 128 tiles, 31.5 -> 24.3 us; 2304 rows, N=1536 K=4096, 54 tiles, 60 -> 26 us; 1280 rows,
+    // N=1024 K=2048, 20 tiles, 26.5 -> 11.6 us).  Results are identical.
+    const int left = tiles % cus, parts = left == 0 || left * 2 > cus ? 1 : left * 4 > cus ? 2 : 4;
+    const int n_full = parts == 1 ? tiles : tiles - left;
+    dim3 grid((unsigned)(n_full + (tiles - n_full) * parts)), block(512);
     const int epi = epilogue_kind(c, N, N, sizeof(OUT), true, sizeof(OUT) == 2);
 #define MDY_GRP(EPI)                                                                                                          \
     hipLaunchKernelGGL((fp8_grouped_gemm_kernel<OUT, EPI>), grid, block, 0, stream, a, a_s, (int)as_rs, (int)as_cs, as_bytes, b, b_s, \
-                       c, bias, N, K, tiles_n, tbl)
+                       c, bias, N, K, tiles_n, n_full, parts, tbl)
     if constexpr (sizeof(OUT) == 2) {
         if (epi == kEpiLines) MDY_GRP(kEpiLines);
         else if (epi == kEpiRows) MDY_GRP(kEpiRows);

@@ -83,6 +83,38 @@ def test_grouped_gemm_exact_integer(m_splits, N, K):
     exact_grouped_case(m_splits, N, K, sum(m_splits) + N + K, call_f32)
 
 
+def call_bf16(qa, sa, qb, sb, m_splits):
+    return m.fp8_grouped_matmul(qa, sa, qb, sb, list(m_splits))
+
+
+@pytest.mark.parametrize("m_splits,N,K,pieces", [([256] * 17 + [130, 1, 257], 3848, 640, 2),     # 21 x 16 tiles: a round and 80 in halves
+                                                 ([256] * 16 + [130, 1, 257], 3848, 640, 4),     # 20 x 16: exactly a quarter of a round
+                                                 ([256] * 16 + [130, 0, 200], 3841, 384, 4),     # odd N: stores straight from registers
+                                                 ([256] * 18 + [300, 70, 128], 3904, 384, 2),    # 22 x 16: in halves, rows on whole lines
+                                                 ([256] * 21 + [300, 70, 128], 3904, 128, 1),    # 25 x 16: more than half a round left
+                                                 ([129, 70, 255, 256], 2300, 1152, 4),           # less than a round: 4 x 9 in quarters
+                                                 ([300, 256, 0, 520, 1000, 77], 2304, 512, 2)])  # 11 x 9 in halves
+def test_grouped_gemm_exact_integer_pieces_of_the_last_round(m_splits, N, K, pieces):
+    """Tiles of a last round that would leave CUs idle run in halves or quarters: edges of groups, columns and pieces."""
+    tiles, cus = sum(-(-v // 256) for v in m_splits) * -(-N // 256), torch.cuda.get_device_properties(0).multi_processor_count
+    if cus == 256:
+        left = tiles % cus
+        assert pieces == (1 if left == 0 or 2 * left > cus else 2 if 4 * left > cus else 4)
+    exact_grouped_case(m_splits, N, K, 7 * sum(m_splits) + N + K, call_f32)
+
+
+def test_grouped_gemm_pieces_bf16_results_through_lds():
+    for m_splits, N in (([256] * 16 + [130, 1, 257], 3904), ([256] * 18 + [300, 70, 128], 3848), ([256] * 18 + [300, 70, 128], 3904)):
+        g = torch.Generator().manual_seed(N)
+        G, M, K = len(m_splits), sum(m_splits), 512
+        qa = torch.randint(-4, 5, (M, K), generator=g).float().to(FP8).to(DEV)
+        qb = torch.randint(-4, 5, (G, N, K), generator=g).float().to(FP8).to(DEV)
+        sa = torch.exp2(torch.randint(-2, 3, (M, K // 128), generator=g).float()).to(DEV)
+        sb = torch.exp2(torch.randint(-2, 3, (G, -(-N // 128), K // 128), generator=g).float()).to(DEV)
+        # sums are exact in fp32: the bf16 results are the fp32 ones rounded
+        assert torch.equal(call_bf16(qa, sa, qb, sb, m_splits), call_f32(qa, sa, qb, sb, m_splits).bfloat16())
+
+
 @pytest.mark.parametrize("m_splits,N,K", [([1, 64, 0, 17, 33, 48, 16, 5], 3300, 896),    # ragged rows and columns, K tail step
                                           ([40] * 40, 640, 128),                          # one K block
                                           ([24] * 9, 3000, 2560),                         # 5 steps of 4 K blocks: odd number of steps
