@@ -13,10 +13,13 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DefaultDtype.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/variable.h>
 
 #include "../../include/mdy_fp8.h"
 
@@ -27,11 +30,22 @@ using at::Tensor;
 
 constexpr ScalarType kE4m3 = ScalarType::Float8_e4m3fn;
 
-// the tensor behind a Python object if it is a plain tensor on `device` (device < 0: on the current one, which is returned)
+// Tensors whose value is not simply what lies at their address: lazy ones, wrappers of the function transforms, subclasses.
+const c10::DispatchKeySet kWrapped({c10::DispatchKey::Conjugate, c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor, c10::DispatchKey::Python,
+                                    c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize,
+                                    c10::DispatchKey::NestedTensor});
+// Something watches the calls of this thread: a trace, a dispatch mode.
+bool watched() {
+    return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer) || c10::impl::TorchDispatchModeTLS::any_modes_set();
+}
+
+// the tensor behind a Python object if it is a plain tensor on `device` (device < 0: on the current one, which is returned), without
+// a forward-mode tangent and with nothing watching: what bypasses an autograd function must not bypass these
 const Tensor* plain(PyObject* o, int& device) {
     if (!THPVariable_CheckExact(o)) return nullptr;
     const Tensor& t = THPVariable_Unpack(o);
-    if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.is_conj() || t.is_neg()) return nullptr;
+    if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.key_set().has_any(kWrapped) || t._fw_grad(0).defined()) return nullptr;
+    if (device < 0 && watched()) return nullptr;      // every function looks at its first tensor with device < 0
     if (device < 0) device = (int)c10::hip::current_device();
     return t.get_device() == device ? &t : nullptr;
 }
@@ -413,6 +427,14 @@ bool tensor_or_none(PyObject* o, int& device, Tensor& t) {
     return true;
 }
 
+// ordinary(tensors...) -> True if every one is a plain tensor here: an autograd function may then be passed by
+PyObject* ordinary(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    int device = -1;
+    for (Py_ssize_t i = 0; i < n; ++i)
+        if (plain(args[i], device) == nullptr) Py_RETURN_NONE;
+    Py_RETURN_TRUE;
+}
+
 // deep_forward(x, weight, cached (y, s, yt, st) or None, bias or None, bias_mode, need_dx, need_dw) -> (out, xt, xt_s, wt, wt_s):
 // fp8.py:316-329; the transposed copies that the backward pass will need, else None
 PyObject* deep_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -428,7 +450,9 @@ PyObject* deep_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
             !tensor_or_none(PyTuple_GET_ITEM(args[2], 1), device, wc.s) || !tensor_or_none(PyTuple_GET_ITEM(args[2], 2), device, wc.yt) ||
             !tensor_or_none(PyTuple_GET_ITEM(args[2], 3), device, wc.st) || !wc.y.defined() || !wc.s.defined() || (need_dx && !wc.yt.defined()))
             Py_RETURN_NONE;
-        if (wc.y.dim() != 2 || wc.y.size(0) < N || wc.y.size(1) != PK || !wc.y.is_contiguous() || wc.s.size(1) != PK / 128 || !wc.s.is_contiguous())
+        if (wc.y.scalar_type() != kE4m3 || wc.s.scalar_type() != ScalarType::Float || wc.y.dim() != 2 || wc.s.dim() != 2 || wc.y.size(0) < N ||
+            wc.y.size(1) != PK || wc.s.size(0) < cdiv(N, 128) || wc.s.size(1) != PK / 128 || !wc.y.is_contiguous() || !wc.s.is_contiguous() ||
+            !aligned16(wc.y))
             Py_RETURN_NONE;
     }
     const void* bias;
@@ -477,7 +501,21 @@ PyObject* deep_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return tuple_of({dx, dw, db});
 }
 
-// official_forward(x, w, bias or None, fmt, need_dx, need_dw) -> (y, xt, xt_s, wt, wt_s): fp8_kernel.py:261-272
+// An empty tensor that shares t's version counter.  Saved for a backward pass in place of t it has autograd refuse the pass when t
+// was changed in place in between, and keeps none of t's memory.
+Tensor version_of(const Tensor& t) {
+    Tensor g = make({0}, t.scalar_type(), t.device());
+    torch::autograd::impl::set_version_counter(g, torch::autograd::impl::version_counter(t));
+    return g;
+}
+PyObject* version_guard(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 1 || !THPVariable_Check(args[0])) Py_RETURN_NONE;
+    const Tensor& t = THPVariable_Unpack(args[0]);
+    if (!t.defined() || t.is_inference()) Py_RETURN_NONE;
+    return THPVariable_Wrap(version_of(t));
+}
+
+// official_forward(x, w, bias or None, fmt, need_dx, need_dw) -> (y, xt, xt_s, wt, wt_s, version of x, version of w): fp8_kernel.py:261-272
 PyObject* official_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != 6 || !PyLong_CheckExact(args[3])) Py_RETURN_NONE;
     int device = -1;
@@ -489,6 +527,8 @@ PyObject* official_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const void* bias;
     if (!bias_arg(args[2], N, device, bias)) Py_RETURN_NONE;
     if (!need_dw && (x.cs != 1 || x.rs != K)) Py_RETURN_NONE;
+    const bool keeps = need_dx || need_dw;
+    if (keeps && (x.t->is_inference() || w.t->is_inference())) Py_RETURN_NONE;      // save_for_backward refuses them: the wrapper lets it
     Copies xc, wc;
     Tensor y = unlocked([&] {
         void* stream = stream_of(device);
@@ -504,7 +544,7 @@ PyObject* official_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
         sizes.back() = N;
         return product(xc.y, xc.s, K / 128, 1, wc.y, wc.s, bias, MDY_BIAS_IN_SUM, x.M, N, K, fmt, sizes, stream);
     });
-    return tuple_of({y, xc.yt, xc.st, wc.yt, wc.st});
+    return tuple_of({y, xc.yt, xc.st, wc.yt, wc.st, keeps ? version_of(*x.t) : Tensor(), keeps ? version_of(*w.t) : Tensor()});
 }
 
 // official_backward(dy, xt, xt_s, wt, wt_s, fmt, need_dx, need_dw, need_db) -> (dx, dw, db): fp8_kernel.py:274-301
@@ -637,12 +677,13 @@ bool ints_arg(PyObject* o, std::vector<int64_t>& v) {
     const bool list = PyList_CheckExact(o);
     if (!list && !PyTuple_CheckExact(o)) return false;
     const Py_ssize_t n = list ? PyList_GET_SIZE(o) : PyTuple_GET_SIZE(o);
+    if (n > (1 << 20)) return false;
     v.resize((size_t)n);
     for (Py_ssize_t i = 0; i < n; ++i) {
         PyObject* e = list ? PyList_GET_ITEM(o, i) : PyTuple_GET_ITEM(o, i);
         if (!PyLong_CheckExact(e)) return false;
         const long long x = PyLong_AsLongLong(e);
-        if (x < 0) return false;      // also an overflow, cleared by the caller
+        if (x < 0 || x > ((int64_t)1 << 40)) return false;      // also an overflow, cleared by the caller; sums of them fit 64 bits
         v[(size_t)i] = x;
     }
     return true;
@@ -721,7 +762,7 @@ PyObject* move_rows(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != 4 || !PyLong_CheckExact(args[3])) Py_RETURN_NONE;
     const Tensor* x = plain(args[0], device);
     const int64_t multiple = PyLong_AsLongLong(args[3]);
-    if (x == nullptr || x->dim() != 2 || x->numel() == 0 || !x->is_contiguous() || multiple < 1 || !ints_arg(args[1], splits)) Py_RETURN_NONE;
+    if (x == nullptr || x->dim() != 2 || x->numel() == 0 || !x->is_contiguous() || multiple < 1 || multiple > (1 << 20) || !ints_arg(args[1], splits)) Py_RETURN_NONE;
     const bool unpad = flag(args[2]);
     int64_t padded = 0;
     for (int64_t m : splits) padded += cdiv(m, multiple) * multiple;
@@ -784,7 +825,7 @@ PyObject* guarded(PyObject* self, PyObject* const* args, Py_ssize_t n) {
 #define MDY_METHOD(F) {#F, (PyCFunction)(void (*)(void))guarded<F>, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {MDY_METHOD(act_quant), MDY_METHOD(fp8_gemm), MDY_METHOD(weight_dequant), MDY_METHOD(matmul), MDY_METHOD(quant_input),
                          MDY_METHOD(deep_linear), MDY_METHOD(silu_act_quant), MDY_METHOD(deep_forward), MDY_METHOD(deep_backward),
-                         MDY_METHOD(official_forward), MDY_METHOD(official_backward), MDY_METHOD(act_copies), MDY_METHOD(block_copies),
+                         MDY_METHOD(official_forward), MDY_METHOD(ordinary), MDY_METHOD(version_guard), MDY_METHOD(official_backward), MDY_METHOD(act_copies), MDY_METHOD(block_copies),
                          MDY_METHOD(quant_weight), MDY_METHOD(quant_transposed), MDY_METHOD(row_scaled_product), MDY_METHOD(silu_fwd),
                          MDY_METHOD(silu_bwd), MDY_METHOD(group_cast), MDY_METHOD(grouped_matmul), MDY_METHOD(move_rows),
                          {nullptr, nullptr, 0, nullptr}};

@@ -332,6 +332,9 @@ class DeepLinear(torch.nn.Linear):
                                       BIAS_IN_SUM if self.fuse_bias else BIAS_AFTER_ROUNDING)
             if done is not None:
                 return done
+            # something else than a plain call: the function gets the arguments it always got where it is traced or transformed
+            if not self.cache_weight and not host().ordinary(self.weight):
+                weight = None
             return _DeepLinear.apply(input, self.weight, bias, False, weight, self.fuse_bias)
         cache = self._quantized_weight(grad and input.requires_grad) if self.cache_weight else None
         return _DeepLinear.apply(input, self.weight, bias, grad, cache, self.fuse_bias)

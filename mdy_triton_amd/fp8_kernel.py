@@ -397,13 +397,19 @@ def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8, ne
     return dx, dw, dbias
 
 
+def _versions(*tensors):
+    """What save_for_backward keeps of tensors that only their version is needed of; an inference tensor itself, which it refuses."""
+    return [t if t.is_inference() else host().version_guard(t) for t in tensors]
+
+
 class _Fp8LinearFunction(torch.autograd.Function):
     """fp8_kernel.py:259-301.  Forward: act_quant_block(x), weight_quant_block(w), GEMM with the bias in its epilogue.
     Backward: x and dy quantized along the tokens (transposed copies, one kernel pass over dy for both of its copies),
     w^T block-quantized; dx = dy . w through the tile kernels, dw = dy^T . x through the GEMM with row scales on both
     operands.  The transposed copies keep their zero padding to a multiple of 128 tokens, so any token count works.
     What the backward pass will need of x and w is quantized by the forward's own pass over them (x and w are read once per
-    step instead of twice) and kept in place of x: one byte per element instead of two."""
+    step instead of twice) and kept in place of x: one byte per element instead of two.  The version counters of x and w are
+    kept too, so that a backward pass after an in-place change of either is refused as for any saved tensor."""
 
     @staticmethod
     def forward(ctx, x, w, bias, fp8_dtype, grad_enabled=True):
@@ -427,12 +433,12 @@ class _Fp8LinearFunction(torch.autograd.Function):
             qxt = sxt = None
         qw, sw, qwt, swt = _weight_quant_both(w, True, need_dx, fp8_dtype, "Fp8Linear")
         y = fp8_matmul(qx, qw, sx, sw, bias, have_w=True)
-        ctx.save_for_backward(qxt, sxt, qwt, swt)
+        ctx.save_for_backward(qxt, sxt, qwt, swt, *(_versions(x2, w) if need_dx or need_dw else ()))
         return y.view(*input_shape[:-1], w.size(0))
 
     @staticmethod
     def backward(ctx, dy):
-        qxt, sxt, qwt, swt = ctx.saved_tensors
+        qxt, sxt, qwt, swt = ctx.saved_tensors[:4]
         need = ctx.needs_input_grad
         dx, dw, dbias = _official_linear_backward(dy, (qwt, swt), (qxt, sxt), need[0], need[1], ctx.fp8_dtype, ctx.has_bias and need[2])
         if dx is not None and len(ctx.input_shape) != 2:
@@ -623,14 +629,15 @@ class Fp8MLP(torch.nn.Module):
         up, down = self.up_gate_proj, self.down_proj
         needs_grad = torch.is_grad_enabled() and (hidden_states.requires_grad or up.weight.requires_grad or
                                                   down.weight.requires_grad)
-        if not needs_grad:
+        if not needs_grad and host().ordinary(hidden_states, up.weight, down.weight):
+            # nothing to differentiate and nothing that traces or transforms the call: no autograd function around it
             if self.dialect == "official":
                 y = _official_mlp(hidden_states.reshape(-1, hidden_states.size(-1)), up.weight, down.weight, self.fp8_dtype, self.order)
                 return y.view(*hidden_states.shape[:-1], down.weight.size(0))
             return _deep_mlp(hidden_states, up.weight, down.weight, self.order,
                              up._quantized_weight(False) if up.cache_weight else None,
                              down._quantized_weight(False) if down.cache_weight else None)
-        if low_memory or self.low_memory:
+        if not needs_grad or low_memory or self.low_memory:
             if self.dialect == "official":
                 return _Fp8MlpCkptOfficial.apply(hidden_states, up.weight, down.weight, self.fp8_dtype, self.order)
             # cached quantized weights (when the projections cache); the forward needs no transposed copies
