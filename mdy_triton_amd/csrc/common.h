@@ -157,6 +157,32 @@ __device__ __forceinline__ float row16_max(float v) {
     return __int_as_float(i);
 }
 
+// the value of lane L of every 16-lane DPP row, in all lanes of the row (row_newbcast)
+template <int L>
+__device__ __forceinline__ float row16_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + L, 0xF, 0xF, true));
+}
+
+// Eight values per lane, each to be combined over the four 16-lane rows of the wave, (row 0 . row 1) . (row 2 . row 3): every
+// swap combines two values at once, so the lane of DPP row r ends with the results of values b and b + 1, b = fold_base(r), and no
+// LDS permutation is needed.
+__device__ __forceinline__ int fold_base(int r) { return (r & 1) * 4 + (r & 2); }
+template <typename OP>
+__device__ __forceinline__ float2 fold_rows8(const float (&v)[8], OP op) {
+    float h[4], q[2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {      // rows 0 and 2 keep value j, rows 1 and 3 value j + 4
+        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[j]), __float_as_uint(v[j + 4]), false, false);
+        h[j] = op(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {      // rows 0 and 1 keep h[j], rows 2 and 3 h[j + 2]
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(h[j]), __float_as_uint(h[j + 2]), false, false);
+        q[j] = op(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    }
+    return make_float2(q[0], q[1]);
+}
+
 // Streaming (non-temporal) vector accesses: the quantizers and the dequantizer touch every
 // byte exactly once, so they bypass cache allocation; measured 1.25-1.5x over plain accesses.
 typedef unsigned uintx4_t __attribute__((ext_vector_type(4)));
@@ -179,54 +205,71 @@ __device__ __forceinline__ void store_nt8(void* p, const uint2& v) {
 }
 
 // 8 values of row `row`, columns c0 .. c0+7, of an [N, K] matrix of type XT (0 bf16, 1 fp16, 2 fp32; element (n, k) at
-// base[n * rs + k * cs]) as fp32, zeros outside the matrix.  VEC: cs == 1, all 8 columns in range, 16-byte aligned rows.
+// base[n * rs + k * cs]) as fp32, zeros outside the matrix.
 // The reference kernels load with .to(tl.float32): every input type is quantized from its exact fp32 value.
-template <int XT, bool VEC>
+template <int XT>
 __device__ __forceinline__ void load_row8_f32(const void* __restrict__ base, int row, int c0, int N, int K, int64_t rs, int64_t cs,
                                               float (&f)[8]) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) f[j] = 0.0f;
     if (row >= N || c0 >= K) return;
-    if (XT == 0) {
-        const uint16_t* p = static_cast<const uint16_t*>(base) + (int64_t)row * rs;
-        if (VEC) {
-            const uint4 v = load_nt16(p + c0);
-            f[0] = bf16_lo(v.x); f[1] = bf16_hi(v.x); f[2] = bf16_lo(v.y); f[3] = bf16_hi(v.y);
-            f[4] = bf16_lo(v.z); f[5] = bf16_hi(v.z); f[6] = bf16_lo(v.w); f[7] = bf16_hi(v.w);
-        } else {
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (c0 + j < K) f[j] = bf16_one(p[(int64_t)(c0 + j) * cs]);
-        }
-    } else if (XT == 1) {
-        const _Float16* p = static_cast<const _Float16*>(base) + (int64_t)row * rs;
-        if (VEC) {
-            const uint4 v = load_nt16(p + c0);
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    for (int j = 0; j < 8; ++j) {
+        if (c0 + j >= K) continue;
+        const int64_t at = (int64_t)row * rs + (int64_t)(c0 + j) * cs;
+        if (XT == 0) f[j] = bf16_one(static_cast<const uint16_t*>(base)[at]);
+        else if (XT == 1) f[j] = (float)static_cast<const _Float16*>(base)[at];
+        else f[j] = static_cast<const float*>(base)[at];
+    }
+}
+// The same for RPT consecutive rows from row0.  VEC (cs == 1, rows of whole 16-byte pieces, rows_vectorizable): 16-byte loads, all
+// rows asked for before the first is looked at.  (One guarded
+// load after the other had the compiler wait for each before the next: RPT memory latencies in a row.)  Rows and columns
+// outside the matrix load the last ones inside and become zeros.
+template <int XT, bool VEC, int RPT>
+__device__ __forceinline__ void load_rows8_f32(const void* __restrict__ base, int row0, int c0, int N, int K, int64_t rs, int64_t cs,
+                                               float (&f)[RPT][8]) {
+    if constexpr (!VEC) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                f[2 * j] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[j] & 0xFFFFu));
-                f[2 * j + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[j] >> 16));
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (c0 + j < K) f[j] = (float)p[(int64_t)(c0 + j) * cs];
-        }
+        for (int i = 0; i < RPT; ++i) load_row8_f32<XT>(base, row0 + i, c0, N, K, rs, cs, f[i]);
     } else {
-        const float* p = static_cast<const float*>(base) + (int64_t)row * rs;
-        if (VEC) {
-            const uint4 a = load_nt16(p + c0), b = load_nt16(p + c0 + 4);
-            f[0] = __uint_as_float(a.x); f[1] = __uint_as_float(a.y); f[2] = __uint_as_float(a.z); f[3] = __uint_as_float(a.w);
-            f[4] = __uint_as_float(b.x); f[5] = __uint_as_float(b.y); f[6] = __uint_as_float(b.z); f[7] = __uint_as_float(b.w);
-        } else {
+        constexpr int W = XT == 2 ? 2 : 1, ESZ = XT == 2 ? 4 : 2;      // 16-byte words and bytes per element of a piece
+        uint4 v[RPT][W];
+        if (N > 0 && K > 0) {                                          // uniform
+            const uint8_t* p = static_cast<const uint8_t*>(base) + (int64_t)min(c0, K - 8) * ESZ;
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (c0 + j < K) f[j] = p[(int64_t)(c0 + j) * cs];
+            for (int i = 0; i < RPT; ++i)
+#pragma unroll
+                for (int w = 0; w < W; ++w) v[i][w] = load_nt16(p + (int64_t)min(row0 + i, N - 1) * rs * ESZ + w * 16);
+        }
+        if (c0 >= K || row0 + RPT > N) {
+#pragma unroll
+            for (int i = 0; i < RPT; ++i)
+#pragma unroll
+                for (int w = 0; w < W; ++w)
+                    if (c0 >= K || row0 + i >= N) v[i][w] = make_uint4(0u, 0u, 0u, 0u);
+        }
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+            const uint4 a = v[i][0], b = v[i][W - 1];
+            if (XT == 0) {
+                f[i][0] = bf16_lo(a.x); f[i][1] = bf16_hi(a.x); f[i][2] = bf16_lo(a.y); f[i][3] = bf16_hi(a.y);
+                f[i][4] = bf16_lo(a.z); f[i][5] = bf16_hi(a.z); f[i][6] = bf16_lo(a.w); f[i][7] = bf16_hi(a.w);
+            } else if (XT == 1) {
+                const uint32_t h[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    f[i][2 * j] = (float)__builtin_bit_cast(_Float16, (uint16_t)(h[j] & 0xFFFFu));
+                    f[i][2 * j + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(h[j] >> 16));
+                }
+            } else {
+                f[i][0] = __uint_as_float(a.x); f[i][1] = __uint_as_float(a.y); f[i][2] = __uint_as_float(a.z); f[i][3] = __uint_as_float(a.w);
+                f[i][4] = __uint_as_float(b.x); f[i][5] = __uint_as_float(b.y); f[i][6] = __uint_as_float(b.z); f[i][7] = __uint_as_float(b.w);
+            }
         }
     }
 }
-// true when the vector form of load_row8_f32 applies to a matrix of element size esz
+// true when the vector form of load_rows8_f32 applies to a matrix of element size esz
 inline bool rows_vectorizable(const void* base, int64_t K, int64_t rs, int64_t cs, int esz) {
     return cs == 1 && K % 8 == 0 && (rs * esz) % 16 == 0 && (reinterpret_cast<uintptr_t>(base) & 15) == 0;
 }

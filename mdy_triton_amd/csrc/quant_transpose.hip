@@ -11,9 +11,13 @@
 // training branch of _quant_input_kernel (fp8.py:115-120; t_mode 1: one scale per 128x128 tile, the
 // max of the rows' clamped+eps maxima, stored ST[pid_n*num_programs(0) + pid_m]).
 //
-// One 256-thread block per 128x128 tile, the tile stays in registers (read once).  Thread t owns
-// columns (t%16)*8..+7 of the 8 consecutive rows (t/16)*8 + i: row maxima by DPP inside 16-lane rows, column maxima by
-// a per-thread max over its 8 rows followed by an LDS reduction over the 16 row groups.  Quotients
+// One block of 512 threads (256 where there are many tiles) per 128x128 tile, the tile stays in registers (read once).  Thread t
+// owns columns (t%16)*8..+7 of RPT = 4 (8) consecutive rows: row maxima by DPP inside 16-lane rows, column maxima by a per-thread
+// max over its rows, row swaps inside the wave and an LDS reduction over the waves.
+// What bounds it: memory at the asymptote (6.4 TB/s between 8192 and 16384 rows of 4096), and for the 2 to 8 tiles per CU of an
+// ordinary layer the length of one tile's chain, load - maxima - barrier - scales - barrier - quotients - store.  So the loads of
+// all rows are in flight together, a row's two divisions are done by one lane instead of 16, and no LDS permutation lies on
+// the way: 8192x4096 31.6 -> 27.4 us (4.9 TB/s), 4096x7168 26.6 -> 24.6 us, 4096x2048 11.4 -> 9.2 us, 700x1536 6.1 -> 5.1 us.  Quotients
 // use the reciprocal + 2-FMA form (bit-identical to IEEE division for every finite amax in this
 // dialect); groups whose amax exceeds the 1e4 clamp or is not finite divide plainly and clamp.
 // Because a thread's rows are consecutive, its 8 bytes of one column are 8 consecutive bytes of a row of the
@@ -22,6 +26,21 @@
 #include "common.h"
 
 namespace mdy {
+
+// v of lane i of every 16-lane row, for i = 0 .. RPT-1
+template <int RPT>
+__device__ __forceinline__ void bcast_rows(float v, float (&out)[RPT]) {
+    out[0] = row16_bcast<0>(v);
+    out[1] = row16_bcast<1>(v);
+    out[2] = row16_bcast<2>(v);
+    out[3] = row16_bcast<3>(v);
+    if constexpr (RPT == 8) {
+        out[4] = row16_bcast<4>(v);
+        out[5] = row16_bcast<5>(v);
+        out[6] = row16_bcast<6>(v);
+        out[7] = row16_bcast<7>(v);
+    }
+}
 
 // x / s.  FAST (the group's amax lies where the reciprocal form is proven bit-identical to IEEE division and,
 // in the DeepLinear dialect, amax <= 1e4, so |x/s| <= 448 needs no clamp) uses the reciprocal form; otherwise an
@@ -47,14 +66,16 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
                                                      int64_t st_k_stride, float* __restrict__ col_sum) {
     constexpr int NRG = 128 / RPT;        // row groups of RPT consecutive rows; 16 threads (8 columns each) per group
     constexpr int WAVES = NRG / 4;
-    __shared__ float col_part[WAVES][128];  // per wave (4 row groups) partial column maxima
-    __shared__ float sum_part[CSUM ? WAVES : 1][128];       // the same for the column sums
+    __shared__ __attribute__((aligned(8))) float col_part[WAVES][128];  // per wave (4 row groups) partial column maxima
+    __shared__ __attribute__((aligned(8))) float sum_part[CSUM ? WAVES : 1][128];       // the same for the column sums
     __shared__ __attribute__((aligned(16))) float col_amax[128];
     __shared__ __attribute__((aligned(16))) float col_sc[128];   // per column: scale of the transposed copy ...
     __shared__ __attribute__((aligned(16))) float col_rc[128];   // ... and its reciprocal, computed once per column
     __shared__ float row_sc[128];         // the tile's 128 row scales, written out as one contiguous run
     __shared__ float blk_part[WAVES];
-    __shared__ __attribute__((aligned(16))) uint8_t tile[128][128 + 8];   // [k][m], transposed
+    // [k][m], transposed; the 16-byte pieces of a row are exchanged by tile_at so that the 64 lanes of a write meet 64 banks
+    __shared__ __attribute__((aligned(16))) uint8_t tile[128][128 + 8];
+    const auto tile_at = [&](int k, int m) -> uint8_t* { return &tile[k][m ^ (((k >> 5) & 3) << 4)]; };
 
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;
@@ -64,16 +85,12 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
 
     float f[RPT][8];
     float rmax[RPT];
-    float cmax[8], csum[CSUM ? 8 : 1];
+    float cmax[8], csum[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) cmax[j] = 0.0f;
-    if (CSUM) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) csum[CSUM ? j : 0] = 0.0f;
-    }
+    for (int j = 0; j < 8; ++j) cmax[j] = csum[j] = 0.0f;
+    load_rows8_f32<XT, VEC, RPT>(x, bm * 128 + rg * RPT, c0, M, K, x_row_stride, x_col_stride, f);
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
-        load_row8_f32<XT, VEC>(x, bm * 128 + rg * RPT + i, c0, M, K, x_row_stride, x_col_stride, f[i]);
         float m = 0.0f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -83,46 +100,39 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
         }
         if (CSUM) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) csum[CSUM ? j : 0] += f[i][j];
+            for (int j = 0; j < 8; ++j) csum[j] += f[i][j];
         }
         rmax[i] = row16_max(m);
     }
 
-    // ---- (1) row-wise quantization straight from registers
+    // ---- (1) row-wise quantization straight from registers.  The 16 lanes of a row hold the same maximum: lane i of them computes
+    // the scale and the reciprocal of row i (two divisions per lane instead of two per row) and the others take them from it.
+    if (y != nullptr) {
+        float am = rmax[0];
 #pragma unroll
-    for (int i = 0; i < (y != nullptr ? RPT : 0); ++i) {
-        const int row = bm * 128 + rg * RPT + i;    // < PM
-        const float sc = group_scale<MODE>(rmax[i]);
-        const float r = 1.0f / sc;
-        float q[8];
-        if (XT == 0 && group_is_fast<MODE>(rmax[i])) {
+        for (int i = 1; i < RPT; ++i) am = (t & 15) == i ? rmax[i] : am;
+        const float lane_sc = group_scale<MODE>(am), lane_rc = 1.0f / lane_sc;
+        if ((t & 15) < RPT) row_sc[rg * RPT + (t & 15)] = lane_sc;
+        float rsc[RPT], rrc[RPT];
+        bcast_rows<RPT>(lane_sc, rsc);
+        bcast_rows<RPT>(lane_rc, rrc);
+        bool rfast = XT == 0;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) q[j] = qt_quot<MODE, true>(f[i][j], sc, r);
-        } else {
+        for (int i = 0; i < RPT; ++i) rfast = rfast && group_is_fast<MODE>(rmax[i]);
+        uint8_t* yp = y + (int64_t)(bm * 128 + rg * RPT) * PK + c0;      // rows < PM
 #pragma unroll
-            for (int j = 0; j < 8; ++j) q[j] = qt_quot<MODE, false>(f[i][j], sc, r);
-        }
-        store_nt8(y + (int64_t)row * PK + c0, make_uint2(pack4_fp8<MODE>(q[0], q[1], q[2], q[3]), pack4_fp8<MODE>(q[4], q[5], q[6], q[7])));
-        if ((t & 15) == 0) row_sc[rg * RPT + i] = sc;
+        for (int i = 0; i < RPT; ++i)
+            store_nt8(yp + (int64_t)i * PK, quantize8_scaled<MODE>(f[i], rsc[i], rrc[i], rfast));      // (slow rows divide, the same bytes)
     }
 
     // ---- (2) scales of the transposed copy
     float tamax[8];   // amax that scales this thread's 8 columns in the transposed copy
     float tsc[8], tr[8];
     if (TMODE == 0) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            // the 4 row groups of a wave hold the same columns in lanes 16 apart: fold them before going to LDS
-            float m = fmaxf(cmax[j], __shfl_xor(cmax[j], 16, 64));
-            m = fmaxf(m, __shfl_xor(m, 32, 64));
-            if (lane < 16) col_part[wave][cl + j] = m;
-            if (CSUM) {
-                float v = csum[CSUM ? j : 0];
-                v += __shfl_xor(v, 16, 64);
-                v += __shfl_xor(v, 32, 64);
-                if (lane < 16) sum_part[CSUM ? wave : 0][cl + j] = v;
-            }
-        }
+        // the 4 row groups of a wave hold the same columns in lanes 16 apart: fold them before going to LDS
+        const int fc = cl + fold_base(lane >> 4);
+        *reinterpret_cast<float2*>(&col_part[wave][fc]) = fold_rows8(cmax, [](float a, float b) { return fmaxf(a, b); });
+        if (CSUM) *reinterpret_cast<float2*>(&sum_part[CSUM ? wave : 0][fc]) = fold_rows8(csum, [](float a, float b) { return a + b; });
         __syncthreads();
         if (t < 128) {
             float m = 0.0f;
@@ -194,7 +204,7 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
         for (int i = 0; i < 8; ++i) { lo8[i] = qlo[i % RPT]; hi8[i] = qhi[i % RPT]; }
         transpose8x8_bytes(lo8, hi8, tb);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) *reinterpret_cast<uint2*>(&tile[cl + j][rg * 8]) = make_uint2(tb[j][0], tb[j][1]);
+        for (int j = 0; j < 8; ++j) *reinterpret_cast<uint2*>(tile_at(cl + j, rg * 8)) = make_uint2(tb[j][0], tb[j][1]);
     } else {
         const uint32_t rl[4] = {qlo[0], qlo[1 % RPT], qlo[2 % RPT], qlo[3 % RPT]};
         const uint32_t rh[4] = {qhi[0], qhi[1 % RPT], qhi[2 % RPT], qhi[3 % RPT]};
@@ -203,8 +213,8 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
         transpose4x4_bytes(rh, c_hi);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            *reinterpret_cast<uint32_t*>(&tile[cl + j][rg * 4]) = c_lo[j];
-            *reinterpret_cast<uint32_t*>(&tile[cl + 4 + j][rg * 4]) = c_hi[j];
+            *reinterpret_cast<uint32_t*>(tile_at(cl + j, rg * 4)) = c_lo[j];
+            *reinterpret_cast<uint32_t*>(tile_at(cl + 4 + j, rg * 4)) = c_hi[j];
         }
     }
     __syncthreads();
@@ -212,7 +222,7 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
         const int kk = rg + NRG * i;
-        const uint2 v = *reinterpret_cast<const uint2*>(&tile[kk][cl]);
+        const uint2 v = *reinterpret_cast<const uint2*>(tile_at(kk, cl));
         // plain (cached) store: the 128-byte pieces that neighbouring tiles write into the same rows of y_t are merged
         // in L2 before they go to memory (non-temporal stores measured 6-10 % slower here; y keeps them)
         *reinterpret_cast<uint2*>(y_t_tile + (int64_t)(bk * 128 + kk) * yt_stride + cl) = v;
@@ -220,7 +230,7 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
 }
 
 template <int MODE, int TMODE, bool VEC, int RPT, int XT, bool CSUM = false>
-__global__ __launch_bounds__(2048 / RPT) void quant_transpose_kernel(const void* __restrict__ x, uint8_t* __restrict__ y,
+__global__ __launch_bounds__(2048 / RPT, 32 / RPT) void quant_transpose_kernel(const void* __restrict__ x, uint8_t* __restrict__ y,
                                                                float* __restrict__ s, uint8_t* __restrict__ y_t,
                                                                float* __restrict__ s_t, int M, int K,
                                                                int64_t x_row_stride, int64_t x_col_stride, int PM,
@@ -235,14 +245,14 @@ __global__ __launch_bounds__(2048 / RPT) void quant_transpose_kernel(const void*
 
 // Expert groups of m_g rows (multiples of 128) one after the other: the row-wise copy and all scales lie as for one matrix, the
 // transposed copy of group g is an array [PK][m_g] of its own behind those of the groups before it.  One launch for all
-// groups: 8 ragged groups, 5376 rows x 7168 and x 4096, 16 launches of 8.8 us -> 2 launches, 141 -> 63 us.
+// groups: 8 ragged groups, 5376 rows x 7168 and x 4096, 16 launches of 8.8 us -> 2 launches, 141 -> 57 us.
 constexpr int kMaxQtGroups = 256;
 struct QtGroups {
     int n;
     int row_start[kMaxQtGroups + 1];
 };
 template <bool VEC, int RPT, int XT>
-__global__ __launch_bounds__(2048 / RPT) void quant_transpose_grouped_kernel(const void* __restrict__ x, uint8_t* __restrict__ y,
+__global__ __launch_bounds__(2048 / RPT, 32 / RPT) void quant_transpose_grouped_kernel(const void* __restrict__ x, uint8_t* __restrict__ y,
                                                                              float* __restrict__ s, uint8_t* __restrict__ y_t,
                                                                              float* __restrict__ s_t, int M, int K, int64_t x_row_stride,
                                                                              int64_t x_col_stride, const QtGroups groups) {

@@ -28,7 +28,9 @@ __device__ __forceinline__ void weight_quant_tile(int bn, int bk, const void* __
     constexpr int NRG = 128 / RPT;     // row groups of RPT consecutive rows, 16 threads (8 columns each) per group
     constexpr int WAVES = NRG / 4;
     __shared__ float wave_max[WAVES];
-    __shared__ __attribute__((aligned(16))) uint8_t tile[128][128 + 8];   // [k][n], transposed
+    // [k][n], transposed; pieces exchanged as in the activation quantizer's tile
+    __shared__ __attribute__((aligned(16))) uint8_t tile[128][128 + 8];
+    const auto tile_at = [&](int k, int n) -> uint8_t* { return &tile[k][n ^ (((k >> 5) & 3) << 4)]; };
 
     const int t = threadIdx.x;
     const int lane = t & 63;
@@ -38,9 +40,9 @@ __device__ __forceinline__ void weight_quant_tile(int bn, int bk, const void* __
 
     float f[RPT][8];
     float m = 0.0f;
+    load_rows8_f32<XT, VEC, RPT>(w, rbase, c0, N, K, w_row_stride, w_col_stride, f);
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
-        load_row8_f32<XT, VEC>(w, rbase + i, c0, N, K, w_row_stride, w_col_stride, f[i]);
 #pragma unroll
         for (int j = 0; j < 4; ++j) m = fmaxf(fmaxf(fabsf(f[i][2 * j]), fabsf(f[i][2 * j + 1])), m);
     }
@@ -77,8 +79,8 @@ __device__ __forceinline__ void weight_quant_tile(int bn, int bk, const void* __
         transpose4x4_bytes(qhi, c_hi);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            *reinterpret_cast<uint32_t*>(&tile[cl + j][rg * 4]) = c_lo[j];
-            *reinterpret_cast<uint32_t*>(&tile[cl + 4 + j][rg * 4]) = c_hi[j];
+            *reinterpret_cast<uint32_t*>(tile_at(cl + j, rg * 4)) = c_lo[j];
+            *reinterpret_cast<uint32_t*>(tile_at(cl + 4 + j, rg * 4)) = c_hi[j];
         }
         __syncthreads();
         // y_t[k][n]: thread owns output columns (t%16)*8..+7 (n) of output rows t/16 + NRG*i (k)
@@ -87,7 +89,7 @@ __device__ __forceinline__ void weight_quant_tile(int bn, int bk, const void* __
             const int kk = rg + NRG * i;
             // cached store: neighbouring tiles complete the rows of y_t in L2 (1-7 % faster than non-temporal here)
             *reinterpret_cast<uint2*>(y_t + (int64_t)(bk * 128 + kk) * PN + bn * 128 + cl) =
-                *reinterpret_cast<const uint2*>(&tile[kk][cl]);
+                *reinterpret_cast<const uint2*>(tile_at(kk, cl));
         }
     }
 }
