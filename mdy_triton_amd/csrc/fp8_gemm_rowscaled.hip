@@ -131,8 +131,19 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_tile_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, int bs_rs, int bs_cs, uint32_t bs_bytes,
     OUT* __restrict__ c, int M, int N, int K, int tiles_m, int tiles_n) {
-    __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<BM, BN, 8, STAGES>::bytes];
+    using L = TileLds<BM, BN, 8, STAGES>;
+    constexpr bool WALK = walks(BM, BN, STAGES, (int)sizeof(OUT), EPI);
+    __shared__ __attribute__((aligned(1024))) uint8_t pool[WALK ? L::walk_bytes : L::bytes];
     const int ntiles = tiles_m * tiles_n;
+    if constexpr (WALK) {
+        Walk<> walk{(int)blockIdx.x, ntiles, tiles_m, tiles_n, BM, BN, 1};
+        int m0, n0;
+        Duty duty;
+        if (!walk(m0, n0, duty)) return;
+        fp8_gemm_tile<BM, BN, 2, 4, STAGES, OUT, 0, 0, 0, FMT, true, EPI>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, Bias{}, m0, M, M, n0, N, K, N,
+                                                                          duty, 0, K >> 7, pool, bs_rs, bs_cs, bs_bytes, walk);
+        return;
+    }
     for (int pid = blockIdx.x; pid < ntiles; pid += gridDim.x) {
         int tm, tn;
         const Duty duty = tile_of(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);

@@ -3,6 +3,8 @@
 // K loop off); the description of the kernels is at the top of fp8_gemm.hip.  Two bodies: fp8_gemm_tile (every wave
 // does everything; the large tiles) and fp8_gemm_tile_ws (producer / consumer waves; 128x192 tiles).
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace mdy {
@@ -116,11 +118,69 @@ __device__ __forceinline__ void store_rows(const floatx4 (&acc)[TI][TJ], uint8_t
     }
 }
 
+// a byte offset beyond every descriptor of these kernels (their ranges stay below 2^31): such a lane accesses nothing
+constexpr int kOutOfRange = 0x7ffffff0;
+
+// store_rows for a wave of 64 bf16 columns through 2 KB of LDS, 16 rows at a time, in exactly TI * 2 store instructions: a bounded
+// descriptor drops what lies outside, no branch skips one, so a wait can count past them (NEXT of fp8_gemm_tile).
+template <int TI, bool NT>
+__device__ __forceinline__ void store_rows_beside(const floatx4 (&acc)[TI][4], uint8_t* buf, uint16_t* __restrict__ c, int ldc, const Bias bias,
+                                                  int m0, int m_wave, int n_base, int M, int rows, int N, int lane) {
+    asm volatile("" : "+v"(lane));      // as in store_rows
+    const int frow = lane & 15, fk = lane >> 4, ch = lane & 7;
+    float bv[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int n = n_base + j * 16 + 4 * fk;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bv[j][e] = 0.0f;
+        if (bias.p != nullptr && n < N) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bv[j][e] = bf16_one(bias.p[n + e]);
+        }
+    }
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(c + (size_t)m0 * ldc, 0, min(rows, M - m0) * ldc * 2, 0x00020000);
+    const int n = n_base + ch * 8;
+    const int off = n < N ? ((m_wave + (lane >> 3)) * ldc + n) * 2 : kOutOfRange;
+    const int row_step = n < N ? 16 * ldc : 0;      // bytes of 8 rows
+    const auto store = [&](auto round_first) __attribute__((always_inline)) {
+        uintx4_t v[2][2];      // rows on their way: those of step i - 1 are stored while the ones of step i come back from LDS
+#pragma unroll
+        for (int i = 0; i <= TI; ++i) {
+            if (i < TI) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    floatx4 r = acc[i][j];
+                    if (decltype(round_first)::value) {
+                        const uint32_t lo = pack2_bf16(r[0], r[1]), hi = pack2_bf16(r[2], r[3]);
+                        r = floatx4{bf16_lo(lo), bf16_hi(lo), bf16_lo(hi), bf16_hi(hi)};
+                    }
+                    *reinterpret_cast<uint2*>(buf + frow * 128 + (((2 * j + (fk >> 1)) ^ (frow & 7)) << 4) + (fk & 1) * 8) =
+                        make_uint2(pack2_bf16(r[0] + bv[j][0], r[1] + bv[j][1]), pack2_bf16(r[2] + bv[j][2], r[3] + bv[j][3]));
+                }
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {      // (a wave's LDS accesses are executed in order: the next 16 rows' writes come after these reads)
+                    const int row = t * 8 + (lane >> 3);
+                    v[i & 1][t] = *reinterpret_cast<const uintx4_t*>(buf + row * 128 + ((ch ^ (row & 7)) << 4));
+                }
+            }
+            if (i > 0) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+                    __builtin_amdgcn_raw_buffer_store_b128(v[(i - 1) & 1][t], rsrc, off + (2 * (i - 1) + t) * row_step, 0, NT ? 2 : 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    if (bias.after_rounding) store(std::true_type{});
+    else store(std::false_type{});
+}
+
 // The form of a launch.  Rows that do not start on whole lines go through LDS with 256x256 tiles only (3752x15224x768 83.0 us
 // direct -> 81.1; the narrower tiles tie or lose a little), fp32 results wherever the pool holds them (`fits`).
 inline int epilogue_kind(const void* c, int64_t ldc, int64_t N, int esz, bool big_tile, bool fits) {
     const uintptr_t p = reinterpret_cast<uintptr_t>(c);
-    if (!fits || ((N | ldc) & (16 / esz - 1)) != 0 || (p & 15) != 0) return kEpiDirect;
+    if (!fits || ((N | ldc) & (16 / esz - 1)) != 0 || (p & 15) != 0 || (big_tile && ldc >= (1 << 21))) return kEpiDirect;      // (256 rows within 2^31 bytes)
     if (esz != 2) return kEpiRows;
     return ((ldc * esz) & 127) == 0 && (p & 127) == 0 ? kEpiLines : big_tile ? kEpiRows : kEpiDirect;
 }
@@ -164,8 +224,6 @@ __device__ __forceinline__ void dma4(const intx4& rsrc, int voff, int soff, uint
 // The one-body kernel (hundreds of tiles, many workgroups on every panel) keeps single-line touches: bursts made
 // 4096x18432x7168 472 -> 491 us and 4096x7168x18432 455 -> 468 us back to back.
 constexpr int kTouchBurstLog = 2, kTouchBurst = 1 << kTouchBurstLog;
-// a byte offset beyond every descriptor of these kernels (their ranges stay below 2^31): such a lane accesses nothing
-constexpr int kOutOfRange = 0x7ffffff0;
 struct Duty {
     int a_duty, a_sh, b_duty, b_sh;
 };
@@ -181,6 +239,9 @@ struct TileLds {
     static constexpr int bs_off = s_off + (STAGES * BM * 4 + 255) / 256 * 256;
     static constexpr int dummy_off = bs_off + NBS * 512 * 4;
     static constexpr int bytes = dummy_off + WAVES * 512;
+    // a workgroup that walks its tiles: 16 rows of results of every wave on their way to memory, beside a ring that already
+    // receives the next tile
+    static constexpr int rows_off = bytes, walk_bytes = bytes + WAVES * 2048;
 };
 
 // LDS of a wave-specialized tile workgroup: separate ring depths for the a panels, the b panels and the activation scales.
@@ -195,6 +256,9 @@ struct TileLdsWs {
     static constexpr int dummy_off = bs_off + NBS * BSROW * 4;
     static constexpr int bytes = dummy_off + WAVES * 512;
 };
+
+// the `next` of a workgroup that computes one tile
+struct OneTile {};
 
 // One BM x BN tile of C: WGM x WGN waves, each wave (BM/WGM) x (BN/WGN).
 //   rows m0 .. min(m0+BM, m_end) of a (m_end = end of the matrix, or of the expert group the tile belongs to),
@@ -219,13 +283,21 @@ struct TileLdsWs {
 // one per 128x128 block: the scales of the tile's BN rows travel through LDS per K block like the activation scales
 // (copied by the waves behind the activation-scale waves), a lane keeps the four scales of its four columns of every
 // sub-tile, and the fold multiplies them in: 4 multiplies + 4 FMAs per MFMA instead of 4 FMAs.
+//
+// NEXT: a workgroup that walks its tiles passes next(m0, n0, duty) -> bool, which moves on to its next tile.  The copies of that
+// tile's first two K blocks are then issued BEFORE the results of this one are stored (through LDS beside the ring).  Loads
+// and stores complete in order, so with the stores first every wait for a copy was a wait for the stores as well: all CUs end
+// a tile together and stood still for the 33 MB of a round.  Now the first two K blocks of a tile run while the stores of the
+// last one drain: 4096x7168x512 with row scales 28.4 -> 24.9 us, 8192x8192x512 55 -> 50 us, 3752x15224x768 71 -> 64.5 us,
+// 16384x4096x1024 81 -> 76 us, 8192x4096x4096 117.5 -> 116 us; at the power limit of a long K it ties (4096x18432x7168).
 template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ = 0, int TD_ = 0, int ABL_ = 0, int FMT_ = 0,
-          bool BROW_ = false, int EPI_ = kEpiDirect>
+          bool BROW_ = false, int EPI_ = kEpiDirect, typename NEXT = OneTile>
 __device__ __forceinline__ void fp8_gemm_tile(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
-    const Bias bias, int m0, int m_end, int m_total, int n0, int N, int K, int ldc, const Duty duty,
-    int kb0, int kb1, uint8_t* __restrict__ pool, int bs_rs = 0, int bs_cs = 0, uint32_t bs_bytes = 0) {
+    const Bias bias, int m0, int m_end, int m_total, int n0, int N, int K, int ldc, Duty duty,
+    int kb0, int kb1, uint8_t* __restrict__ pool, int bs_rs = 0, int bs_cs = 0, uint32_t bs_bytes = 0, NEXT next = NEXT{}) {
+    constexpr bool WALK = !std::is_same<NEXT, OneTile>::value;
     // ABL_ switches parts of the K loop off for the timing probe (mdy_fp8_gemm_probe); the product uses 0.
     //   1: no global->LDS copies in the loop (the ring is filled once and replayed)   2: no LDS fragment / scale reads
     //   4: no FMA fold (the MFMAs accumulate in place, no block scales)                8: no pre-touches
@@ -325,7 +397,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
         t.n0 = tn0;
         return t;
     };
-    const TileAddr me = tile_addr(m0, n0, duty);
+    TileAddr me = tile_addr(m0, n0, duty);
 
     // copy i (0: scales, then the A passes, then the B passes) of K block kb into buffer buf.  Past the last K
     // block the offsets run beyond the descriptors: no memory access, zeros into a buffer nobody reads any more.
@@ -356,7 +428,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
             else touch(t, 1 << 20);      // same load count for the waits below: a copy of nothing
         }
 #pragma unroll
-        for (int i = 0; i < FIRST; ++i) issue(t, i, kb0 + STAGES - 1, STAGES - 1);
+        for (int i = 0; i < (WALK ? NDMA : FIRST); ++i) issue(t, i, kb0 + STAGES - 1, STAGES - 1);
         if (NO_COPY) {     // probe: the whole ring up front, nothing is copied later
 #pragma unroll
             for (int i = FIRST; i < NDMA; ++i) issue(t, i, kb0 + STAGES - 1, STAGES - 1);
@@ -378,10 +450,6 @@ __device__ __forceinline__ void fp8_gemm_tile(
     const int jsplit = STRADDLE ? min(TJ, (128 - (bs_col & 127)) >> 4) : TJ;   // sub-tiles j < jsplit lie in the first block
 
     floatx4 acc[TI][TJ];
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     auto read_frag = [&](const uint8_t* base, int rd0, int rd1, int idx) {
         const intx4 lo = *reinterpret_cast<const intx4*>(base + rd0 + idx * 2048);
@@ -389,9 +457,20 @@ __device__ __forceinline__ void fp8_gemm_tile(
         return intx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     };
 
-    // ---- prologue, wait for block 0, load the registers of step 0
+    constexpr int STORES = WALK ? TI * 2 : 0;        // store instructions of store_rows_beside
+    static_assert(!WALK || (STAGES == 2 && TJ == 4 && sizeof(OUT) == 2 && EPI_ != kEpiDirect && ABL_ == 0 && 2 + NDMA + STORES <= 63),
+                  "walking tiles: a ring of two, waves of 64 bf16 columns");
+    bool stores_pending = false;                     // WALK: the last tile's stores are younger than this tile's first copies
     prologue(me);
+    for (;;) {                                       // WALK: tile by tile; otherwise once
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // ---- wait for block 0, load the registers of step 0
     if (NO_COPY) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if (WALK && stores_pending) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(1 + NDMA + STORES) : "memory");
+    else if (WALK) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(1 + NDMA) : "memory");
     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * (NDMA + 1) + 1 + FIRST) : "memory");
     __syncthreads();
     intx8 fh[NH], fx[2];
@@ -416,14 +495,16 @@ __device__ __forceinline__ void fp8_gemm_tile(
     fx[0] = read_frag(HOLD_A ? lds_b[0] : lds_a[0], x0, x1, 0);
 
     int cur = 0;                                             // buffer of K block kb: kb % STAGES
-    for (int kb = kb0; kb < kb1; ++kb) {
+    // FRESH (WALK, a tile's first K block): the copies of block kb+1 are all under way
+    auto k_block = [&](int kb, auto fresh) __attribute__((always_inline)) {
+        constexpr bool FRESH = decltype(fresh)::value;
         const int nxt = cur + 1 == STAGES ? 0 : cur + 1;     // buffer of K block kb+1
         const int last = cur == 0 ? STAGES - 1 : cur - 1;    // buffer of K block kb+STAGES-1
         const uint8_t* lx = HOLD_A ? lds_b[cur] : lds_a[cur];            // streamed operand of this K block
         const uint8_t* lh_n = HOLD_A ? lds_a[nxt] : lds_b[nxt];          // operands and scales of the next one
         const uint8_t* lx_n = HOLD_A ? lds_b[nxt] : lds_a[nxt];
         const float* ls_n = lds_s[nxt];
-        float sc_n[TI], sc_hi_n[STRADDLE ? TI : 1];
+        float sa_n[TI], sb_n = 1.0f, sb_hi_n = 1.0f;         // scales of the next K block
         floatx4 p[DEPTH + 1];
 #pragma unroll
         for (int t = 0; t < NT + DEPTH; ++t) {
@@ -443,24 +524,18 @@ __device__ __forceinline__ void fp8_gemm_tile(
                 }
                 if (t == TB) {
                     // K block kb+1 has landed once only the younger loads are left in flight
-                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER) : "memory");
+                    if (FRESH && stores_pending) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER + STORES) : "memory");
+                    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER) : "memory");
                     __syncthreads();
                     if (!NO_LDS) {
                         fx[0] = read_frag(lx_n, x0, x1, 0);      // queue slot 0 was last used by streamed fragment NS-2
                         const float sb = BROW_ ? 1.0f : my_bs[min(kb + 1, KB - 1)], sb_hi = BROW_ ? 1.0f : my_bs_hi[min(kb + 1, KB - 1)];
 #pragma unroll
-                        for (int i = 0; i < TI; ++i) {
-                            const float sa = ls_n[s_rd + i * 16];
-                            sc_n[i] = sa * sb;
-                            if (STRADDLE) sc_hi_n[i] = sa * sb_hi;
-                        }
+                        for (int i = 0; i < TI; ++i) sa_n[i] = ls_n[s_rd + i * 16];      // combined at the end of the block: nothing waits here
+                        sb_n = sb;
+                        sb_hi_n = sb_hi;
                     } else {
                         asm volatile("" : "+v"(fx[0]));
-#pragma unroll
-                        for (int i = 0; i < TI; ++i) {
-                            sc_n[i] = sc[i];
-                            if (STRADDLE) sc_hi_n[i] = sc_hi[i];
-                        }
                     }
                 }
                 if (t >= TB) {
@@ -486,7 +561,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
                 for (int j = 0; j < NDMA; ++j) {
                     const int v = TB + 1 + GAP * j;
                     if (v < NSLOT && v == t) issue(me, j, kb + STAGES, cur);                    // behind the barrier: buffer cur is free
-                    if (v >= NSLOT && v - NSLOT == t) issue(me, j, kb + STAGES - 1, last);      // the rest of the block started in kb-1
+                    if (!FRESH && v >= NSLOT && v - NSLOT == t) issue(me, j, kb + STAGES - 1, last);      // the rest of the block started in kb-1
                 }
             }
             if (t == TOUCH && !NO_TOUCH) touch(me, kb + TD);
@@ -500,14 +575,31 @@ __device__ __forceinline__ void fp8_gemm_tile(
         }
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
-            sc[i] = sc_n[i];
-            if (STRADDLE) sc_hi[i] = sc_hi_n[i];
+            if (NO_LDS) continue;
+            sc[i] = BROW_ ? sa_n[i] : sa_n[i] * sb_n;
+            if (STRADDLE) sc_hi[i] = sa_n[i] * sb_hi_n;
         }
         cur = nxt;
-    }
+    };
+    int kb_first = kb0;
+    if constexpr (WALK) k_block(kb_first++, std::true_type{});
+    for (int kb = kb_first; kb < kb1; ++kb) k_block(kb, std::false_type{});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing may still be writing LDS when the wave ends
 
     // ---- epilogue: lane holds c[m][n..n+3], m = .. + lane%16, n = .. + 4*(lane/16)
+    if constexpr (WALK) {
+        __syncthreads();                               // every wave has left the ring
+        const int m_done = m0, n_done = n0;
+        const bool more = next(m0, n0, duty);
+        if (more) {
+            me = tile_addr(m0, n0, duty);
+            prologue(me);
+        }
+        store_rows_beside<TI, EPI_ == kEpiLines>(acc, pool + L::rows_off + wave * 2048, c, ldc, bias, m_done, wm * WM, n_done + wn * WN, M, BM, N, lane);
+        stores_pending = true;
+        if (!more) return;
+        continue;
+    }
     if constexpr (EPI_ != kEpiDirect) {
         static_assert(WAVES * WM * WN * (int)sizeof(OUT) <= L::bytes, "the tile's results fit the pool");
         __syncthreads();                               // every wave's copies have landed: the pool is free
@@ -530,6 +622,8 @@ __device__ __forceinline__ void fp8_gemm_tile(
             }
             store4<OUT>(c, ldc, m, n, M, N, v, vec_ok);
         }
+    }
+    break;
     }
 }
 
@@ -842,6 +936,25 @@ __global__ __launch_bounds__((WGM * WGN + PW) * 64) void fp8_gemm_ws_kernel(
     }
 }
 
+// Tiles blockIdx.x, blockIdx.x + gridDim.x, ... of a launch: the `next` of fp8_gemm_tile.
+template <int GM = 4>
+struct Walk {
+    int pid, ntiles, tiles_m, tiles_n, bm, bn, pretouch;
+    __device__ __forceinline__ bool operator()(int& m0, int& n0, Duty& duty) {
+        if (pid >= ntiles) return false;
+        int tm, tn;
+        duty = tile_of<GM>(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
+        if (!pretouch) duty.a_sh = duty.b_sh = 0;
+        m0 = tm * bm;
+        n0 = tn * bn;
+        pid += gridDim.x;
+        return true;
+    }
+};
+// Kernels whose workgroups walk their tiles with the next tile's copies in front of the results: 256x256 tiles of bf16 results in
+// whole rows.
+constexpr bool walks(int BM, int BN, int STAGES, int esz, int EPI) { return BM == 256 && BN == 256 && STAGES == 2 && esz == 2 && EPI != kEpiDirect; }
+
 template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ = 0, int TD_ = 0, int ABL_ = 0, int FMT_ = 0, int GM_ = 4,
           int EPI_ = kEpiDirect>
 __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
@@ -852,8 +965,19 @@ __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
     // then walks tiles blockIdx.x, blockIdx.x + gridDim.x, ... itself, which saves the ~4.5 us that pass between
     // the end of a workgroup and the start of its successor on the same CU.  Workgroup ids keep their XCD
     // (id % 8) from tile to tile when gridDim.x is a multiple of 8.
-    __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<BM, BN, WGM * WGN, STAGES>::bytes];
+    using L = TileLds<BM, BN, WGM * WGN, STAGES>;
+    constexpr bool WALK = walks(BM, BN, STAGES, (int)sizeof(OUT), EPI_) && ABL_ == 0;
+    __shared__ __attribute__((aligned(1024))) uint8_t pool[WALK ? L::walk_bytes : L::bytes];
     const int ntiles = tiles_m * tiles_n;
+    if constexpr (WALK) {
+        Walk<GM_> walk{(int)blockIdx.x, ntiles, tiles_m, tiles_n, BM, BN, pretouch};
+        int m0, n0;
+        Duty duty;
+        if (!walk(m0, n0, duty)) return;
+        fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, OUT, GAP_, TD_, ABL_, FMT_, false, EPI_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, m0, M, M, n0,
+                                                                                         N, K, ldc, duty, 0, K >> 7, pool, 0, 0, 0, walk);
+        return;
+    }
     for (int pid = blockIdx.x; pid < ntiles; pid += gridDim.x) {
         int tm, tn;
         Duty duty = tile_of<GM_>(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
