@@ -86,30 +86,50 @@ __global__ __launch_bounds__(512) void fp8_gemm_splitk_ws_kernel(
                                                      tn * BN, N, K, N, duty, kb0, kb1, pool);
 }
 
-template <typename OUT, bool VEC>
+// VEC columns per thread (N a multiple of it, aligned c), 1 otherwise.  KS: number of slabs, 0: `ksplit` of them, four at a time.  The
+// slabs lie in the caches and a launch lives for a few microseconds, so every load of a thread is in flight at once, nothing is loaded
+// twice (two slabs used to be read as four), and 8 columns share a thread where that still leaves a workgroup per CU (fewer waves lose:
+// 128x2112 13.4 -> 13.6 us).  GEMM and reduction: M=64 N=2048 K=7168 9.95 -> 9.5 us, M=48 9.4 -> 8.9, 777x2112x7168 29.3 -> 28.9.
+template <typename OUT, int VEC, int KS>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, OUT* __restrict__ c,
                                                             const Bias bias, int64_t MN, int N,
                                                             int ksplit) {
-    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * (VEC ? 4 : 1);
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VEC;
     if (i >= MN) return;
-    if (VEC) {   // N % 4 == 0: the 4 elements lie in one row
-        float4 s = *reinterpret_cast<const float4*>(ws + i);
-        for (int k0 = 1; k0 < ksplit; k0 += 4) {      // four slabs' loads in flight; added in slab order
-            float4 v[4];
+    if constexpr (VEC > 1) {   // the VEC elements lie in one row
+        constexpr int Q = VEC / 4, STEP = KS == 0 ? 4 : KS - 1;
+        float4 s[Q];
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) v[kk] = *reinterpret_cast<const float4*>(ws + (int64_t)min(k0 + kk, ksplit - 1) * MN + i);
+        for (int q = 0; q < Q; ++q) s[q] = *reinterpret_cast<const float4*>(ws + i + 4 * q);
+        for (int k0 = 1; k0 < (KS == 0 ? ksplit : KS); k0 += STEP) {      // added in slab order
+            float4 v[STEP][Q];
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk)
-                if (k0 + kk < ksplit) { s.x += v[kk].x; s.y += v[kk].y; s.z += v[kk].z; s.w += v[kk].w; }
+            for (int kk = 0; kk < STEP; ++kk)
+#pragma unroll
+                for (int q = 0; q < Q; ++q)
+                    v[kk][q] = *reinterpret_cast<const float4*>(ws + (int64_t)(KS == 0 ? min(k0 + kk, ksplit - 1) : k0 + kk) * MN + i + 4 * q);
+#pragma unroll
+            for (int kk = 0; kk < STEP; ++kk)
+#pragma unroll
+                for (int q = 0; q < Q; ++q)
+                    if (KS != 0 || k0 + kk < ksplit) { s[q].x += v[kk][q].x; s[q].y += v[kk][q].y; s[q].z += v[kk][q].z; s[q].w += v[kk][q].w; }
         }
         if (bias.p != nullptr) {
             const int n = (int)(i % N);
-            s.x = bias.add(s.x, n); s.y = bias.add(s.y, n + 1); s.z = bias.add(s.z, n + 2); s.w = bias.add(s.w, n + 3);
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                s[q].x = bias.add(s[q].x, n + 4 * q); s[q].y = bias.add(s[q].y, n + 4 * q + 1);
+                s[q].z = bias.add(s[q].z, n + 4 * q + 2); s[q].w = bias.add(s[q].w, n + 4 * q + 3);
+            }
         }
-        if (sizeof(OUT) == 2)
-            *reinterpret_cast<uint2*>(c + i) = make_uint2(pack2_bf16(s.x, s.y), pack2_bf16(s.z, s.w));
-        else
-            *reinterpret_cast<float4*>(c + i) = s;
+        if constexpr (sizeof(OUT) == 2 && Q == 1) {
+            *reinterpret_cast<uint2*>(c + i) = make_uint2(pack2_bf16(s[0].x, s[0].y), pack2_bf16(s[0].z, s[0].w));
+        } else if constexpr (sizeof(OUT) == 2) {
+            *reinterpret_cast<uint4*>(c + i) = make_uint4(pack2_bf16(s[0].x, s[0].y), pack2_bf16(s[0].z, s[0].w), pack2_bf16(s[1].x, s[1].y), pack2_bf16(s[1].z, s[1].w));
+        } else {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) *reinterpret_cast<float4*>(c + i + 4 * q) = s[q];
+        }
     } else {
         float s = ws[i];
         for (int k = 1; k < ksplit; ++k) s += ws[(int64_t)k * MN + i];
@@ -124,12 +144,20 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // slabs [ksplit][M][N] of partial sums -> c [M][N] of out_dtype (0 bf16, 1 fp32)
 int launch_splitk_reduce(const float* ws, void* c, int out_dtype, const Bias bias, int64_t M, int64_t N, int ksplit, hipStream_t stream) {
     const int64_t MN = M * N;
-    const bool vec = (N % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
-    const dim3 grid((unsigned)((MN / (vec ? 4 : 1) + 255) / 256));
-#define MDY_RED(OUT, VEC) \
-    hipLaunchKernelGGL((splitk_reduce_kernel<OUT, VEC>), grid, dim3(256), 0, stream, ws, static_cast<OUT*>(c), bias, MN, (int)N, ksplit)
-    if (out_dtype == 0) { if (vec) MDY_RED(uint16_t, true); else MDY_RED(uint16_t, false); }
-    else { if (vec) MDY_RED(float, true); else MDY_RED(float, false); }
+    const int per = (reinterpret_cast<uintptr_t>(c) & 15) != 0 ? 1 : out_dtype == 0 && N % 8 == 0 && MN >= (1 << 19) ? 8 : N % 4 == 0 ? 4 : 1;
+    const dim3 grid((unsigned)((MN / per + 255) / 256));
+#define MDY_RED(OUT, VEC, KS) \
+    hipLaunchKernelGGL((splitk_reduce_kernel<OUT, VEC, KS>), grid, dim3(256), 0, stream, ws, static_cast<OUT*>(c), bias, MN, (int)N, ksplit)
+#define MDY_RED_K(OUT, VEC)                                             \
+    do {                                                                \
+        if (ksplit == 2) MDY_RED(OUT, VEC, 2);                          \
+        else if (ksplit == 3) MDY_RED(OUT, VEC, 3);                     \
+        else if (ksplit == 4) MDY_RED(OUT, VEC, 4);                     \
+        else MDY_RED(OUT, VEC, 0);                                      \
+    } while (0)
+    if (out_dtype == 0) { if (per == 8) MDY_RED_K(uint16_t, 8); else if (per == 4) MDY_RED_K(uint16_t, 4); else MDY_RED(uint16_t, 1, 0); }
+    else { if (per == 4) MDY_RED_K(float, 4); else MDY_RED(float, 1, 0); }
+#undef MDY_RED_K
 #undef MDY_RED
     return (int)hipGetLastError();
 }
@@ -1020,10 +1048,11 @@ static int dispatch_small(const uint8_t* a, const float* a_s, int64_t as_rs, int
 #undef MDY_SK
             return (int)hipGetLastError();
         }
-        // a narrow weight (fewer than 100 groups of 16 columns): 8 columns per workgroup, twice the workgroups (per call in
-        // a replayed graph: M=16 N=1584 K=4096 4.6 -> 3.8 us, M=16 N=1024 K=8192 7.2 -> 6.3, M=4 N=1536 K=7168 5.3 -> 4.8,
-        // M=16 N=576 K=7168 6.0 -> 5.8; N=2048 and wider: no gain)
-        if (M <= 16 && (N + 15) / 16 < 100) {
+        // a narrow weight: 8 columns per workgroup as long as they all run at once, one per CU: what a CU can pull from beyond
+        // its L2 is the limit, and with 16 columns half of the CUs would pull nothing (16 -> 8 columns, weights in rotation out of
+        // the caches: M=16 N=2048 K=7168 7.0 -> 6.2 us, M=4 5.6 -> 5.0, M=16 N=1664 K=4096 5.2 -> 4.6, N=1792 K=18432 15.5 -> 11.9; the same weight
+        // again and again 4.9 -> 4.6, 4.7 -> 4.3, 4.3 -> 3.8, 13.8 -> 11.1; a second round loses: N=2560 K=5120 6.4 -> 7.8, N=3072 K=7168 7.2 -> 9.4)
+        if (M <= 16 && (N + 7) / 8 <= cu_count()) {
             grid = dim3((unsigned)((N + 7) / 8));
 #define MDY_HALF(UF)                                                                                                                \
     hipLaunchKernelGGL((fp8_gemm_smallm_lines_half_kernel<UF, OUT, FMT>), grid, dim3(kSmWaves * 64), 0, stream, a, a_s, as_rs, as_cs, b, \
