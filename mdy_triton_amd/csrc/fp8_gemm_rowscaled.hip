@@ -212,7 +212,10 @@ static int rowscaled_config(int64_t M, int64_t N, int64_t K) {
     const int64_t cus = cu_count(), rows256 = (M + 255) / 256, rows128 = (M + 127) / 128, cols256 = (N + 255) / 256;
     if (K <= 512 && rows128 * ((N + 127) / 128) <= 2 * cus) return 0;
     const int64_t big = (rows256 * cols256 + cus - 1) / cus, mid = (rows128 * cols256 + cus - 1) / cus;
-    return 17 * big <= 10 * mid ? 2 : 1;
+    // with few K blocks the ends of the tiles count, and a 256x256 workgroup copies its second tile's panels while the first one's
+    // results leave: two rounds of it against three of 128x256 (4096x4864x256 20.3 -> 17.9 us, 4096x6144x512 27.3 -> 24.2, 4096x6144x1024
+    // 42.2 -> 37.3, 4096x4864x1024 37.8 -> 37.2; but 4096x4864x4096 113.7 -> 126)
+    return (K <= 1024 ? 13 : 17) * big <= 10 * mid ? 2 : 1;
 }
 
 // returns hipError_t, or -1 when the operands do not qualify (K % 128 != 0, misaligned, scale extents >= 2^31 bytes)
