@@ -23,16 +23,18 @@ struct PadTable {
     int64_t rows[kPadGroups];            // rows of group g that hold data (the smaller of its two slot sizes)
 };
 
-// Pieces of a row that a lane moves: their loads are in flight together and share one search of the table (with one piece per
-// lane, 4000 rows of 14336 bytes to 5376: 28 us).
-constexpr int kPadPieces = 4;
+// Pieces of a row that a lane moves: their loads are in flight together and share one search of the table (with one piece per lane,
+// 4000 rows of 14336 bytes to 5376: 28 us).  Unpadding takes four; padding, which writes a third more rows than it reads, two: the
+// blocks of zeros are gone at once and leave their slots to the others (four -> two pieces: 25.2 -> 23.3 us there, 4000 rows of 8192 bytes
+// 16.1 -> 14.5, 12000 rows of 14336 66.4 -> 62.2; unpadding 22.3 = 22.3, 12.6 -> 13.5, 60.7 -> 58.7, 4000 rows of 4096 bytes 7.4 -> 8.1).
+constexpr int kPadPieces = 2, kUnpadPieces = 4;
 
-// grid.x: chunks of 64 lanes x kPadPieces pieces of a row, grid.y/z: destination rows (block_row()), 4 rows per block
-template <int VEC>
+// grid.x: chunks of 64 lanes x PIECES pieces of a row, grid.y/z: destination rows (block_row()), 4 rows per block
+template <int VEC, int PIECES>
 __global__ __launch_bounds__(256) void group_pad_kernel(const uint8_t* __restrict__ x, uint8_t* __restrict__ y,
                                                          int64_t row_bytes, int64_t dst_rows, const PadTable tbl) {
     const int64_t row = (int64_t)block_row() * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t col = ((int64_t)blockIdx.x * (64 * kPadPieces) + (threadIdx.x & 63)) * VEC;
+    const int64_t col = ((int64_t)blockIdx.x * (64 * PIECES) + (threadIdx.x & 63)) * VEC;
     if (row >= dst_rows) return;
     int lo = 0, hi = tbl.n_groups - 1;     // last group whose destination slot starts at or before this row
     while (lo < hi) {
@@ -44,19 +46,19 @@ __global__ __launch_bounds__(256) void group_pad_kernel(const uint8_t* __restric
     const uint8_t* src = x + (tbl.src_start[lo] + r) * row_bytes + col;
     uint8_t* dst = y + row * row_bytes + col;
     if (VEC == 16) {
-        uint4 v[kPadPieces];
+        uint4 v[PIECES];
 #pragma unroll
-        for (int p = 0; p < kPadPieces; ++p) {
+        for (int p = 0; p < PIECES; ++p) {
             v[p] = make_uint4(0u, 0u, 0u, 0u);
             if (data && col + p * 64 * VEC < row_bytes) v[p] = load_nt16(src + p * 64 * VEC);
         }
 #pragma unroll
-        for (int p = 0; p < kPadPieces; ++p)
+        for (int p = 0; p < PIECES; ++p)
             if (col + p * 64 * VEC < row_bytes) store_nt16(dst + p * 64 * VEC, v[p]);
         return;
     }
 #pragma unroll
-    for (int p = 0; p < kPadPieces; ++p) {
+    for (int p = 0; p < PIECES; ++p) {
         if (col + p * 64 * VEC >= row_bytes) break;
         if (VEC == 2)
             *reinterpret_cast<uint16_t*>(dst + p * 64 * VEC) = data ? *reinterpret_cast<const uint16_t*>(src + p * 64 * VEC) : (uint16_t)0;
@@ -70,7 +72,7 @@ int launch_group_pad(const void* x, void* y, const int64_t* m_splits, int64_t G,
                      int unpad, hipStream_t stream) {
     const bool a16 = row_bytes % 16 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
     const bool a2 = row_bytes % 2 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 1) == 0;
-    const int vec = a16 ? 16 : a2 ? 2 : 1;
+    const int vec = a16 ? 16 : a2 ? 2 : 1, pieces = unpad ? kUnpadPieces : kPadPieces;
     int64_t src_row = 0, dst_row = 0;
     for (int64_t g0 = 0; g0 < G; g0 += kPadGroups) {
         PadTable tbl;
@@ -93,12 +95,16 @@ int launch_group_pad(const void* x, void* y, const int64_t* m_splits, int64_t G,
         const int64_t rows = dst_row - dst0;
         if (rows == 0 || row_bytes == 0) continue;
         dim3 grid;
-        if (!grid_rows((row_bytes + 64 * kPadPieces * vec - 1) / (64 * kPadPieces * vec), (rows + 3) / 4, grid)) return kErrTooManyBlocks;
+        if (!grid_rows((row_bytes + 64 * pieces * vec - 1) / (64 * pieces * vec), (rows + 3) / 4, grid)) return kErrTooManyBlocks;
         const uint8_t* xp = static_cast<const uint8_t*>(x) + src0 * row_bytes;
         uint8_t* yp = static_cast<uint8_t*>(y) + dst0 * row_bytes;
-        if (vec == 16) hipLaunchKernelGGL(group_pad_kernel<16>, grid, dim3(256), 0, stream, xp, yp, row_bytes, rows, tbl);
-        else if (vec == 2) hipLaunchKernelGGL(group_pad_kernel<2>, grid, dim3(256), 0, stream, xp, yp, row_bytes, rows, tbl);
-        else hipLaunchKernelGGL(group_pad_kernel<1>, grid, dim3(256), 0, stream, xp, yp, row_bytes, rows, tbl);
+#define MDY_PAD(VEC, PIECES) hipLaunchKernelGGL((group_pad_kernel<VEC, PIECES>), grid, dim3(256), 0, stream, xp, yp, row_bytes, rows, tbl)
+#define MDY_PAD_P(VEC) do { if (unpad) MDY_PAD(VEC, kUnpadPieces); else MDY_PAD(VEC, kPadPieces); } while (0)
+        if (vec == 16) MDY_PAD_P(16);
+        else if (vec == 2) MDY_PAD_P(2);
+        else MDY_PAD_P(1);
+#undef MDY_PAD_P
+#undef MDY_PAD
         const int rc = (int)hipGetLastError();
         if (rc != 0) return rc;
     }
