@@ -128,23 +128,6 @@ __device__ __forceinline__ void transpose4x4_bytes(const uint32_t (&r)[4], uint3
     c[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
     c[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
 }
-// 8 rows x 8 columns of bytes: row i = (lo[i], hi[i]); column j comes back as tb[j][0] (rows 0..3), tb[j][1] (rows 4..7)
-__device__ __forceinline__ void transpose8x8_bytes(const uint32_t (&lo)[8], const uint32_t (&hi)[8], uint32_t (&tb)[8][2]) {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        const uint32_t rl[4] = {lo[4 * half], lo[4 * half + 1], lo[4 * half + 2], lo[4 * half + 3]};
-        const uint32_t rh[4] = {hi[4 * half], hi[4 * half + 1], hi[4 * half + 2], hi[4 * half + 3]};
-        uint32_t cl[4], ch[4];
-        transpose4x4_bytes(rl, cl);
-        transpose4x4_bytes(rh, ch);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            tb[j][half] = cl[j];
-            tb[4 + j][half] = ch[j];
-        }
-    }
-}
-
 // max over the 16 lanes of a DPP row (one 128-element quantization group: 16 lanes x 8 values)
 __device__ __forceinline__ float row16_max(float v) {
     // butterfly over the 16 lanes of a DPP row: xor 1, xor 2 (quad_perm), then

@@ -11,8 +11,8 @@
 // training branch of _quant_input_kernel (fp8.py:115-120; t_mode 1: one scale per 128x128 tile, the
 // max of the rows' clamped+eps maxima, stored ST[pid_n*num_programs(0) + pid_m]).
 //
-// One block of 512 threads (256 where there are many tiles) per 128x128 tile, the tile stays in registers (read once).  Thread t
-// owns columns (t%16)*8..+7 of RPT = 4 (8) consecutive rows: row maxima by DPP inside 16-lane rows, column maxima by a per-thread
+// One block of 512 threads per 128x128 tile, the tile stays in registers (read once).  Thread t
+// owns columns (t%16)*8..+7 of RPT = 4 consecutive rows: row maxima by DPP inside 16-lane rows, column maxima by a per-thread
 // max over its rows, row swaps inside the wave and an LDS reduction over the waves.
 // What bounds it: memory at the asymptote (6.4 TB/s between 8192 and 16384 rows of 4096), and for the 2 to 8 tiles per CU of an
 // ordinary layer the length of one tile's chain, load - maxima - barrier - scales - barrier - quotients - store.  So the loads of
@@ -20,26 +20,21 @@
 // the way: 8192x4096 31.6 -> 27.4 us (4.9 TB/s), 4096x7168 26.6 -> 24.6 us, 4096x2048 11.4 -> 9.2 us, 700x1536 6.1 -> 5.1 us.  Quotients
 // use the reciprocal + 2-FMA form (bit-identical to IEEE division for every finite amax in this
 // dialect); groups whose amax exceeds the 1e4 clamp or is not finite divide plainly and clamp.
-// Because a thread's rows are consecutive, its 8 bytes of one column are 8 consecutive bytes of a row of the
-// transposed tile: the transpose goes through a padded LDS tile with 8-byte writes and 8-byte reads, and both
+// Because a thread's rows are consecutive, its 4 bytes of one column are 4 consecutive bytes of a row of the
+// transposed tile: the transpose goes through a padded LDS tile with 4-byte writes and 8-byte reads, and both
 // outputs are written row-contiguously.
 #include "common.h"
 
 namespace mdy {
 
+constexpr int RPT = 4;      // consecutive rows per thread (8 rows and 256 threads per tile: 0.5-4 % slower from 4096x2048 to 16384x8192)
+
 // v of lane i of every 16-lane row, for i = 0 .. RPT-1
-template <int RPT>
 __device__ __forceinline__ void bcast_rows(float v, float (&out)[RPT]) {
     out[0] = row16_bcast<0>(v);
     out[1] = row16_bcast<1>(v);
     out[2] = row16_bcast<2>(v);
     out[3] = row16_bcast<3>(v);
-    if constexpr (RPT == 8) {
-        out[4] = row16_bcast<4>(v);
-        out[5] = row16_bcast<5>(v);
-        out[6] = row16_bcast<6>(v);
-        out[7] = row16_bcast<7>(v);
-    }
 }
 
 // x / s.  FAST (the group's amax lies where the reciprocal form is proven bit-identical to IEEE division and,
@@ -58,7 +53,7 @@ __device__ __forceinline__ float qt_quot(float x, float s, float r) {
 // CSUM (with TMODE 0): also the fp32 sums of the tile's columns, to col_sum[row tile * PK + column]: an output gradient's column
 // sums are the bias gradient, and here they cost 8 adds per 16 bytes loaded instead of a pass over the matrix.
 // y_t_tile: the transposed copy's element (column 0, first row of the tile), rows of yt_stride bytes.
-template <int MODE, int TMODE, bool VEC, int RPT, int XT, bool CSUM>
+template <int MODE, int TMODE, bool VEC, int XT, bool CSUM>
 __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void* __restrict__ x, uint8_t* __restrict__ y,
                                                      float* __restrict__ s, uint8_t* __restrict__ y_t_tile, int yt_stride,
                                                      float* __restrict__ s_t, int M, int K, int64_t x_row_stride, int64_t x_col_stride,
@@ -114,8 +109,8 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
         const float lane_sc = group_scale<MODE>(am), lane_rc = 1.0f / lane_sc;
         if ((t & 15) < RPT) row_sc[rg * RPT + (t & 15)] = lane_sc;
         float rsc[RPT], rrc[RPT];
-        bcast_rows<RPT>(lane_sc, rsc);
-        bcast_rows<RPT>(lane_rc, rrc);
+        bcast_rows(lane_sc, rsc);
+        bcast_rows(lane_rc, rrc);
         bool rfast = XT == 0;
 #pragma unroll
         for (int i = 0; i < RPT; ++i) rfast = rfast && group_is_fast<MODE>(rmax[i]);
@@ -197,25 +192,15 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
         qhi[i] = pack4_fp8<MODE>(q[4], q[5], q[6], q[7]);
     }
     // column j of the thread's RPT x 8 bytes = RPT consecutive bytes of row cl+j of the transposed tile
-    if (RPT == 8) {
-        uint32_t tb[8][2];   // [column j][rows 0..3 | 4..7]
-        uint32_t lo8[8], hi8[8];
+    const uint32_t rl[4] = {qlo[0], qlo[1], qlo[2], qlo[3]};
+    const uint32_t rh[4] = {qhi[0], qhi[1], qhi[2], qhi[3]};
+    uint32_t c_lo[4], c_hi[4];
+    transpose4x4_bytes(rl, c_lo);
+    transpose4x4_bytes(rh, c_hi);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) { lo8[i] = qlo[i % RPT]; hi8[i] = qhi[i % RPT]; }
-        transpose8x8_bytes(lo8, hi8, tb);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) *reinterpret_cast<uint2*>(tile_at(cl + j, rg * 8)) = make_uint2(tb[j][0], tb[j][1]);
-    } else {
-        const uint32_t rl[4] = {qlo[0], qlo[1 % RPT], qlo[2 % RPT], qlo[3 % RPT]};
-        const uint32_t rh[4] = {qhi[0], qhi[1 % RPT], qhi[2 % RPT], qhi[3 % RPT]};
-        uint32_t c_lo[4], c_hi[4];
-        transpose4x4_bytes(rl, c_lo);
-        transpose4x4_bytes(rh, c_hi);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            *reinterpret_cast<uint32_t*>(tile_at(cl + j, rg * 4)) = c_lo[j];
-            *reinterpret_cast<uint32_t*>(tile_at(cl + 4 + j, rg * 4)) = c_hi[j];
-        }
+    for (int j = 0; j < 4; ++j) {
+        *reinterpret_cast<uint32_t*>(tile_at(cl + j, rg * 4)) = c_lo[j];
+        *reinterpret_cast<uint32_t*>(tile_at(cl + 4 + j, rg * 4)) = c_hi[j];
     }
     __syncthreads();
     // y_t[k][m]: thread owns output columns (t%16)*8..+7 (m) of output rows t/16 + NRG*i (k)
@@ -229,7 +214,7 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
     }
 }
 
-template <int MODE, int TMODE, bool VEC, int RPT, int XT, bool CSUM = false>
+template <int MODE, int TMODE, bool VEC, int XT, bool CSUM = false>
 __global__ __launch_bounds__(2048 / RPT, 32 / RPT) void quant_transpose_kernel(const void* __restrict__ x, uint8_t* __restrict__ y,
                                                                float* __restrict__ s, uint8_t* __restrict__ y_t,
                                                                float* __restrict__ s_t, int M, int K,
@@ -239,7 +224,7 @@ __global__ __launch_bounds__(2048 / RPT, 32 / RPT) void quant_transpose_kernel(c
                                                                float* __restrict__ col_sum) {
     const int bm = block_row(), bk = blockIdx.x;
     if (bm >= (PM >> 7)) return;
-    quant_transpose_tile<MODE, TMODE, VEC, RPT, XT, CSUM>(bm, bk, x, y, s, y_t + (int64_t)bm * 128, PM, s_t, M, K, x_row_stride, x_col_stride,
+    quant_transpose_tile<MODE, TMODE, VEC, XT, CSUM>(bm, bk, x, y, s, y_t + (int64_t)bm * 128, PM, s_t, M, K, x_row_stride, x_col_stride,
                                                           PM, PK, s_kb_stride, s_m_stride, st_a_stride, st_k_stride, col_sum);
 }
 
@@ -251,7 +236,7 @@ struct QtGroups {
     int n;
     int row_start[kMaxQtGroups + 1];
 };
-template <bool VEC, int RPT, int XT>
+template <bool VEC, int XT>
 __global__ __launch_bounds__(2048 / RPT, 32 / RPT) void quant_transpose_grouped_kernel(const void* __restrict__ x, uint8_t* __restrict__ y,
                                                                              float* __restrict__ s, uint8_t* __restrict__ y_t,
                                                                              float* __restrict__ s_t, int M, int K, int64_t x_row_stride,
@@ -264,7 +249,7 @@ __global__ __launch_bounds__(2048 / RPT, 32 / RPT) void quant_transpose_grouped_
         if (groups.row_start[mid] <= bm * 128) lo = mid; else hi = mid - 1;
     }
     const int r0 = groups.row_start[lo];
-    quant_transpose_tile<1, 0, VEC, RPT, XT, false>(bm, bk, x, y, s, y_t + (int64_t)r0 * K + (bm * 128 - r0), groups.row_start[lo + 1] - r0,
+    quant_transpose_tile<1, 0, VEC, XT, false>(bm, bk, x, y, s, y_t + (int64_t)r0 * K + (bm * 128 - r0), groups.row_start[lo + 1] - r0,
                                                     s_t, M, K, x_row_stride, x_col_stride, M, K, M, 1, K, 1, nullptr);
 }
 
@@ -276,23 +261,14 @@ static int launch_qt(int mode, const void* x, int x_dtype, void* y, float* s, vo
     if (PM == 0 || PK == 0) return 0;
     dim3 grid;
     if (!grid_rows(PK / 128, PM / 128, grid)) return kErrTooManyBlocks;
-    // 512 threads (4 rows each) when there are few tiles per CU: more waves to hide the load and store latency
-    const bool wide = (PK / 128) * (PM / 128) < 256 * 24;
-    dim3 block(wide ? 512 : 256);
+    const dim3 block(2048 / RPT);
     const bool vec = rows_vectorizable(x, K, x_row_stride, x_col_stride, xt_size(x_dtype));
     uint8_t* yp = static_cast<uint8_t*>(y);
     uint8_t* ytp = static_cast<uint8_t*>(y_t);
-#define MDY_QT(MODE, TM, VEC, XT)                                                                                         \
-    do {                                                                                                                  \
-        if (wide)                                                                                                         \
-            hipLaunchKernelGGL((quant_transpose_kernel<MODE, TM, VEC, 4, XT>), grid, block, 0, stream, x, yp, s, ytp, s_t, \
-                               (int)M, (int)K, x_row_stride, x_col_stride, (int)PM, (int)PK, s_kb_stride, s_m_stride,     \
-                               st_a_stride, st_k_stride, static_cast<float*>(nullptr));                                   \
-        else                                                                                                              \
-            hipLaunchKernelGGL((quant_transpose_kernel<MODE, TM, VEC, 8, XT>), grid, block, 0, stream, x, yp, s, ytp, s_t, \
-                               (int)M, (int)K, x_row_stride, x_col_stride, (int)PM, (int)PK, s_kb_stride, s_m_stride,     \
-                               st_a_stride, st_k_stride, static_cast<float*>(nullptr));                                   \
-    } while (0)
+#define MDY_QT(MODE, TM, VEC, XT)                                                                                        \
+    hipLaunchKernelGGL((quant_transpose_kernel<MODE, TM, VEC, XT>), grid, block, 0, stream, x, yp, s, ytp, s_t,          \
+                       (int)M, (int)K, x_row_stride, x_col_stride, (int)PM, (int)PK, s_kb_stride, s_m_stride,           \
+                       st_a_stride, st_k_stride, static_cast<float*>(nullptr))
 #define MDY_QT_V(MODE, TM, XT) do { if (vec) MDY_QT(MODE, TM, true, XT); else MDY_QT(MODE, TM, false, XT); } while (0)
 #define MDY_QT_X(MODE, TM) do { if (x_dtype == 0) MDY_QT_V(MODE, TM, 0); else if (x_dtype == 1) MDY_QT_V(MODE, TM, 1); else MDY_QT_V(MODE, TM, 2); } while (0)
     if (mode == 0) MDY_QT_X(0, 0);
@@ -332,16 +308,11 @@ int launch_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s
     }
     dim3 grid;
     if (!grid_rows(K / 128, M / 128, grid)) return kErrTooManyBlocks;
-    const bool wide = (K / 128) * (M / 128) < 256 * 24;      // as in launch_qt
     const bool vec = rows_vectorizable(x, K, x_row_stride, x_col_stride, xt_size(x_dtype));
-#define MDY_QTG(VEC, RPT, XT)                                                                                                   \
-    hipLaunchKernelGGL((quant_transpose_grouped_kernel<VEC, RPT, XT>), grid, dim3(2048 / RPT), 0, stream, x, static_cast<uint8_t*>(y), s, \
+#define MDY_QTG(VEC, XT)                                                                                                        \
+    hipLaunchKernelGGL((quant_transpose_grouped_kernel<VEC, XT>), grid, dim3(2048 / RPT), 0, stream, x, static_cast<uint8_t*>(y), s, \
                        static_cast<uint8_t*>(y_t), s_t, (int)M, (int)K, x_row_stride, x_col_stride, groups)
-#define MDY_QTG_V(XT)                                                                          \
-    do {                                                                                       \
-        if (wide) { if (vec) MDY_QTG(true, 4, XT); else MDY_QTG(false, 4, XT); }               \
-        else { if (vec) MDY_QTG(true, 8, XT); else MDY_QTG(false, 8, XT); }                    \
-    } while (0)
+#define MDY_QTG_V(XT) do { if (vec) MDY_QTG(true, XT); else MDY_QTG(false, XT); } while (0)
     if (x_dtype == 0) MDY_QTG_V(0); else if (x_dtype == 1) MDY_QTG_V(1); else MDY_QTG_V(2);
 #undef MDY_QTG_V
 #undef MDY_QTG
@@ -369,18 +340,13 @@ int launch_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, f
     if (PM == 0 || PK == 0) return 0;
     dim3 grid;
     if (!grid_rows(PK / 128, PM / 128, grid)) return kErrTooManyBlocks;
-    const bool wide = (PK / 128) * (PM / 128) < 256 * 24;      // as in launch_qt
     const bool vec = rows_vectorizable(x, K, x_row_stride, x_col_stride, 2);
     const bool deep = mode == 1;
     const int64_t s_kb = deep ? s_kb_stride : 1, s_m = deep ? 1 : PK / 128, st_a = deep ? PK : 1, st_k = deep ? 1 : PM / 128;
-#define MDY_QTC(MODE, VEC, RPT)                                                                                                   \
-    hipLaunchKernelGGL((quant_transpose_kernel<MODE, 0, VEC, RPT, 0, true>), grid, dim3(2048 / RPT), 0, stream, x, static_cast<uint8_t*>(y), s, \
+#define MDY_QTC(MODE, VEC)                                                                                                        \
+    hipLaunchKernelGGL((quant_transpose_kernel<MODE, 0, VEC, 0, true>), grid, dim3(2048 / RPT), 0, stream, x, static_cast<uint8_t*>(y), s, \
                        static_cast<uint8_t*>(y_t), s_t, (int)M, (int)K, x_row_stride, x_col_stride, (int)PM, (int)PK, s_kb, s_m, st_a, st_k, part)
-#define MDY_QTC_V(MODE)                                                                        \
-    do {                                                                                       \
-        if (wide) { if (vec) MDY_QTC(MODE, true, 4); else MDY_QTC(MODE, false, 4); }           \
-        else { if (vec) MDY_QTC(MODE, true, 8); else MDY_QTC(MODE, false, 8); }                \
-    } while (0)
+#define MDY_QTC_V(MODE) do { if (vec) MDY_QTC(MODE, true); else MDY_QTC(MODE, false); } while (0)
     if (mode == 0) MDY_QTC_V(0); else if (mode == 1) MDY_QTC_V(1); else MDY_QTC_V(2);
 #undef MDY_QTC_V
 #undef MDY_QTC
