@@ -427,6 +427,13 @@ bool tensor_or_none(PyObject* o, int& device, Tensor& t) {
     return true;
 }
 
+// Are y [>= rows, cols] and s [>= s_rows, s_cols] a quantized copy and its fp32 scales as the kernels read them?  What comes back from
+// autograd's saved tensors has been through the user's hooks, and a cached copy through the caller's hands.
+bool copy_ok(const Tensor& y, const Tensor& s, ScalarType type, int64_t rows, int64_t cols, int64_t s_rows, int64_t s_cols) {
+    return y.defined() && s.defined() && y.scalar_type() == type && s.scalar_type() == ScalarType::Float && y.dim() == 2 && s.dim() == 2 &&
+           y.size(0) >= rows && y.size(1) == cols && s.size(0) >= s_rows && s.size(1) == s_cols && y.is_contiguous() && s.is_contiguous() && aligned16(y);
+}
+
 // ordinary(tensors...) -> True if every one is a plain tensor here: an autograd function may then be passed by
 PyObject* ordinary(PyObject*, PyObject* const* args, Py_ssize_t n) {
     int device = -1;
@@ -559,8 +566,9 @@ PyObject* official_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int fmt = (int)PyLong_AsLong(args[5]);
     const bool need_dx = flag(args[6]), need_dw = flag(args[7]), need_db = flag(args[8]);
     const int64_t M = dy.M, N = dy.K, PM = cdiv(M, 128) * 128;
-    if ((!need_dx && !need_dw) || (need_dx && (!wc.yt.defined() || wc.yt.size(1) != N)) || (need_dw && (!xc.yt.defined() || xc.yt.size(1) != PM)))
-        Py_RETURN_NONE;
+    if (!need_dx && !need_dw) Py_RETURN_NONE;
+    if (need_dx && (!wc.yt.defined() || wc.yt.dim() != 2 || !copy_ok(wc.yt, wc.st, fmt_type(fmt), 0, N, cdiv(wc.yt.size(0), 128), N / 128))) Py_RETURN_NONE;
+    if (need_dw && (!xc.yt.defined() || xc.yt.dim() != 2 || !copy_ok(xc.yt, xc.st, fmt_type(fmt), 0, PM, xc.yt.size(0), PM / 128))) Py_RETURN_NONE;
     Tensor db, dx, dw;
     unlocked([&] {
         void* stream = stream_of(device);

@@ -362,6 +362,21 @@ def fp8_matmul_bwd(xt, w, dy, dyt, scale_xt, scale_w, scale_dy, scale_dyt):
     return dx, dw
 
 
+def _saved_copy(copy, fp8_dtype, cols, scale_shape, dev, who):
+    """(bytes [rows, cols], scales) as the kernels read them, from what autograd's saved tensors gave back: a hook of the user's
+    may have moved them, changed their strides or returned something else."""
+    y, s = copy
+    require_gpu(y, s)
+    if y.device != dev or s.device != dev:
+        raise RuntimeError("%s: a saved copy came back on %s and %s, the gradient is on %s" % (who, y.device, s.device, dev))
+    if y.dtype != fp8_dtype or s.dtype != torch.float32:
+        raise TypeError("%s: a saved %s copy with float32 scales came back as %s and %s" % (who, fp8_dtype, y.dtype, s.dtype))
+    if y.dim() != 2 or y.size(1) != cols or tuple(s.shape) != scale_shape(y.size(0)):
+        raise ValueError("%s: a saved copy of %d columns came back as %s with scales %s" % (who, cols, tuple(y.shape), tuple(s.shape)))
+    y = y.contiguous()
+    return (y if y.data_ptr() % 16 == 0 else y.clone()), s.contiguous()
+
+
 def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8, need_dbias=False):
     """Gradients of y = x . w^T in the official dialect (fp8_kernel.py:274-301): dx = dy . w on the row-wise copy of dy
     and the block-quantized w^T, dw = dy^T . x on the transposed copies of dy and x (row scales on both operands).
@@ -383,9 +398,11 @@ def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8, ne
     dbias = torch.empty(N, device=dev, dtype=torch.bfloat16) if need_dbias and dy2.numel() > 0 else None
     qdy, sdy, qdyt, sdyt = _act_quant_transposed(dy2, need_dx, "Fp8Linear.backward", fp8_dtype, dbias)
     if need_dx:
-        dx = fp8_matmul(qdy[:M], w_t[0], sdy[:M], w_t[1], have_w=True)
+        qwt, swt = _saved_copy(w_t, fp8_dtype, N, lambda rows: ((rows + 127) // 128, N // 128), dev, "Fp8Linear.backward")
+        dx = fp8_matmul(qdy[:M], qwt, sdy[:M], swt, have_w=True)
     if need_dw:
-        qxt, sxt = x_t
+        PM = qdyt.size(1)
+        qxt, sxt = _saved_copy(x_t, fp8_dtype, PM, lambda rows: (rows, PM // 128), dev, "Fp8Linear.backward")
         K = qxt.size(0)
         dw = torch.empty(N, K, device=dev, dtype=torch.bfloat16)
         if qdyt.size(1) == 0:

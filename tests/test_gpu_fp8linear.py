@@ -499,3 +499,37 @@ def test_act_quant_block_e5m2_golden_codes_on_device():
     assert np.array_equal(u8(y_t), d["y_t"]) and np.array_equal(s_t.cpu().numpy(), d["s_t"])
     y, s = m.act_quant_block(x.t().contiguous())
     assert np.array_equal(u8(y), d["y_t"]) and np.array_equal(s.cpu().numpy(), d["s_t"])
+
+
+@pytest.mark.parametrize("dtype", [FP8, E5M2])
+def test_backward_takes_what_saved_tensor_hooks_give_back(dtype):
+    """Copies that come back with other strides, at an odd address or from the host give the same gradients; what is not the saved
+    copy any more is refused before a kernel sees it."""
+    g = torch.Generator().manual_seed(3)
+    lin = m.Fp8Linear(256, 384, bias=True, device=DEV, dtype=torch.bfloat16, fp8_dtype=dtype)
+    x0, dy = torch.randn(200, 256, generator=g).bfloat16().to(DEV), torch.randn(200, 384, generator=g).bfloat16().to(DEV)
+
+    def grads(pack, unpack):
+        lin.zero_grad()
+        x = x0.clone().requires_grad_(True)
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            y = lin(x)
+        y.backward(dy)
+        return x.grad, lin.weight.grad.clone(), lin.bias.grad.clone()
+
+    def shifted(t):
+        if t.dtype != dtype:
+            return t
+        raw = torch.empty(t.numel() + 1, dtype=torch.uint8, device=t.device)[1:].view(t.shape)
+        return raw.copy_(t.view(torch.uint8)).view(dtype)
+
+    same = lambda t: t
+    ref = grads(same, same)
+    for pack, unpack in ((same, lambda t: t.t().contiguous().t() if t.dim() == 2 else t), (same, shifted),
+                         (lambda t: t.cpu(), lambda t: t.to(DEV))):
+        for a, b in zip(grads(pack, unpack), ref):
+            assert torch.equal(a, b)
+    for error, unpack in ((RuntimeError, lambda t: t.cpu()), (TypeError, lambda t: t.to(torch.bfloat16) if t.dtype == dtype else t),
+                          (ValueError, lambda t: t.t().contiguous() if t.dtype == torch.float32 else t)):
+        with pytest.raises(error):
+            grads(same, unpack)
