@@ -495,7 +495,7 @@ PyObject* deep_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Py_RETURN_NONE;
     const bool need_dx = flag(args[6]), need_dw = flag(args[7]), need_db = flag(args[8]);
     const int64_t M = dy.M, N = dy.K, K = PyLong_AsLongLong(args[5]), PM = cdiv(M, 256) * 256, PN = cdiv(N, 256) * 256;
-    if ((need_dx && (!wc.yt.defined() || wc.yt.size(1) != PN || wc.yt.size(0) < K)) || (need_dw && (!xc.yt.defined() || xc.yt.size(1) != PM || xc.yt.size(0) < K)))
+    if ((need_dx && !copy_ok(wc.yt, wc.st, kE4m3, K, PN, cdiv(K, 128), PN / 128)) || (need_dw && !copy_ok(xc.yt, xc.st, kE4m3, K, PM, cdiv(K, 128), PM / 128)))
         Py_RETURN_NONE;
     Tensor db, dx, dw;
     unlocked([&] {

@@ -758,6 +758,24 @@ def test_deep_linear_backward_partial_requirements():
 
 
 # ------------------------------------------------------------------ non-finite values
+def test_deep_linear_backward_refuses_copies_that_are_no_operands():
+    """A caller's quantized weight whose transposed copy has another type, shape or layout than the kernels read is refused by the
+    backward pass (all of them hold enough bytes)."""
+    from mdy_triton_amd import fp8
+    g = torch.Generator().manual_seed(5)
+    x, w = torch.randn(64, 512, generator=g).bfloat16().to(DEV).requires_grad_(True), torch.randn(256, 512, generator=g).bfloat16().to(DEV)
+    y, s, yt, st = fp8.quant_weight(w, only_forward=False)
+
+    def dx(yt_, st_):
+        return torch.autograd.grad(fp8._DeepLinear.apply(x, w, None, True, (y, s, yt_, st_)).sum(), x)[0]
+
+    assert dx(yt, st).shape == x.shape
+    for error, args in ((TypeError, (yt.to(torch.bfloat16), st)), (ValueError, (yt, st.t().contiguous())),
+                        (ValueError, (yt, st.t().contiguous().t())), (ValueError, (yt.t().contiguous().t(), st))):
+        with pytest.raises(error):
+            dx(*args)
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 384, 512),       # MFMA tiles
                                    (8, 256, 512),         # weight-streaming kernel
                                    (130, 1100, 4224),     # split along K
