@@ -171,7 +171,7 @@ int mdy_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s, v
  * MDY_QUANT_DEEPLINEAR, mdy_act_quant_transpose for the official modes: their layouts, s_kb_stride only used by the former)
  * on a bf16 output gradient, and in the same pass the gradient's column sums, i.e. the bias gradient (fp8.py:342 and
  * fp8_kernel.py:279 take dy.sum(0)): added in fp32, rounded to bf16 once.
- *   partial  fp32 scratch [PM/128, PK]      col_sum  bf16 [K] */
+ *   partial  fp32 scratch [PM/128, PK]      col_sum  bf16 [K], zeros when M == 0 */
 int mdy_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K,
                                int64_t x_row_stride, int64_t x_col_stride, int64_t PM, int64_t PK, int64_t s_kb_stride,
                                int mode, float* partial, void* col_sum, void* stream);

@@ -204,8 +204,8 @@ int mdy_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, floa
     if (PM % 128 != 0 || PK % 128 != 0) return fail(MDY_E_SHAPE, "quant_transpose_colsum: PM=%lld, PK=%lld must be multiples of 128", (long long)PM, (long long)PK);
     if (mode == MDY_QUANT_DEEPLINEAR && s_kb_stride < PM) return fail(MDY_E_SHAPE, "quant_transpose_colsum: s_kb_stride=%lld < PM=%lld", (long long)s_kb_stride, (long long)PM);
     if ((y == nullptr) != (s == nullptr)) return fail(MDY_E_NULL, "quant_transpose_colsum: y and s must be given together");
-    if (PM == 0 || PK == 0) return 0;
-    if (!y_t || !s_t || !partial || !col_sum || (!x && M > 0 && K > 0)) return fail(MDY_E_NULL, "quant_transpose_colsum: null pointer");
+    if (PK == 0 || (PM == 0 && K == 0)) return 0;
+    if ((K > 0 && !col_sum) || (PM > 0 && (!y_t || !s_t || !partial)) || (!x && M > 0 && K > 0)) return fail(MDY_E_NULL, "quant_transpose_colsum: null pointer");
     if ((y && !aligned(y, 8)) || !aligned(y_t, 8)) return fail(MDY_E_ALIGN, "quant_transpose_colsum: y / y_t must be 8-byte aligned");
     if (!aligned(x, 2) || !aligned(col_sum, 2) || (s && !aligned(s, 4)) || !aligned(s_t, 4) || !aligned(partial, 4)) return fail(MDY_E_ALIGN, "quant_transpose_colsum: misaligned pointer");
     if (int e = check_device()) return e;

@@ -319,7 +319,7 @@ int launch_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s
     return (int)hipGetLastError();
 }
 
-// bf16(sum over the row tiles of part[a][k]): 32 columns x 8 interleaved shares of the row tiles per block
+// bf16(sum over the row tiles of part[a][k]; zeros without any): 32 columns x 8 interleaved shares of the row tiles per block
 __global__ __launch_bounds__(256) void col_sum_reduce_kernel(const float* __restrict__ part, uint16_t* __restrict__ out, int A, int K, int PK) {
     __shared__ float share[8][32];
     const int c = threadIdx.x & 31, g = threadIdx.x >> 5, k = blockIdx.x * 32 + c;      // k < PK: PK % 128 == 0
@@ -337,9 +337,9 @@ __global__ __launch_bounds__(256) void col_sum_reduce_kernel(const float* __rest
 int launch_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K, int64_t x_row_stride,
                                   int64_t x_col_stride, int64_t PM, int64_t PK, int64_t s_kb_stride, int mode, float* part, void* col_sum,
                                   hipStream_t stream) {
-    if (PM == 0 || PK == 0) return 0;
+    if (PK == 0) return 0;
     dim3 grid;
-    if (!grid_rows(PK / 128, PM / 128, grid)) return kErrTooManyBlocks;
+    if (PM > 0 && !grid_rows(PK / 128, PM / 128, grid)) return kErrTooManyBlocks;
     const bool vec = rows_vectorizable(x, K, x_row_stride, x_col_stride, 2);
     const bool deep = mode == 1;
     const int64_t s_kb = deep ? s_kb_stride : 1, s_m = deep ? 1 : PK / 128, st_a = deep ? PK : 1, st_k = deep ? 1 : PM / 128;
@@ -347,11 +347,13 @@ int launch_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, f
     hipLaunchKernelGGL((quant_transpose_kernel<MODE, 0, VEC, 0, true>), grid, dim3(2048 / RPT), 0, stream, x, static_cast<uint8_t*>(y), s, \
                        static_cast<uint8_t*>(y_t), s_t, (int)M, (int)K, x_row_stride, x_col_stride, (int)PM, (int)PK, s_kb, s_m, st_a, st_k, part)
 #define MDY_QTC_V(MODE) do { if (vec) MDY_QTC(MODE, true); else MDY_QTC(MODE, false); } while (0)
-    if (mode == 0) MDY_QTC_V(0); else if (mode == 1) MDY_QTC_V(1); else MDY_QTC_V(2);
+    if (PM > 0) {
+        if (mode == 0) MDY_QTC_V(0); else if (mode == 1) MDY_QTC_V(1); else MDY_QTC_V(2);
+    }
 #undef MDY_QTC_V
 #undef MDY_QTC
     const int rc = (int)hipGetLastError();
-    if (rc != 0) return rc;
+    if (rc != 0 || K == 0) return rc;
     hipLaunchKernelGGL(col_sum_reduce_kernel, dim3((unsigned)((K + 31) / 32)), dim3(256), 0, stream, part, static_cast<uint16_t*>(col_sum),
                        (int)(PM / 128), (int)K, (int)PK);
     return (int)hipGetLastError();

@@ -35,3 +35,16 @@ def test_ragged_columns():
     fp8._quant_transpose(x, 0, "t", out[:200])
     _check_sum(out[:200], x)
     assert torch.isnan(out[200])
+
+
+@pytest.mark.parametrize("M,K,PM,PK", [(0, 200, 0, 256), (0, 128, 128, 128), (0, 0, 128, 128), (5, 0, 128, 128), (0, 0, 0, 128), (0, 0, 0, 0)])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_empty_sums_are_zero(M, K, PM, PK, mode):
+    from mdy_triton_amd import _lib
+    x, y, yt = (torch.empty(128 * 256, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    s, st, part = (torch.empty(512, device="cuda") for _ in range(3))
+    out = torch.full((K + 1,), float("nan"), device="cuda", dtype=torch.bfloat16)
+    rc = _lib.load().mdy_quant_transpose_colsum(x.data_ptr(), y.data_ptr(), s.data_ptr(), yt.data_ptr(), st.data_ptr(), M, K, max(K, 1), 1, PM, PK,
+                                                PM, mode, part.data_ptr(), out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert not out[:K].any() and torch.isnan(out[K])
