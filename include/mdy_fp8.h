@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define MDY_FP8_ABI_VERSION 15
+#define MDY_FP8_ABI_VERSION 16
 
 /* error codes (negative = argument rejected before any launch) */
 #define MDY_OK 0

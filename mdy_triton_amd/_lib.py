@@ -10,7 +10,7 @@ import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libmdyfp8.so")
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 _lock = threading.Lock()
 _lib = None
@@ -77,14 +77,15 @@ def load():
                 "%s not found: build it with `python -m mdy_triton_amd.csrc.build` "
                 "(needs hipcc; cross-compiles for gfx950 without a GPU)" % LIB_PATH)
         lib = ctypes.CDLL(LIB_PATH)
+        # first of all: an older library lacks some of the names below
+        got = lib.mdy_fp8_abi_version()
+        if got != ABI_VERSION:
+            raise MdyFp8Error("libmdyfp8.so ABI version %d, expected %d: rebuild" % (got, ABI_VERSION))
         for name, argtypes in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = (ctypes.c_char_p if name == "mdy_fp8_last_error" else
                           ctypes.c_int64 if name.endswith("workspace_bytes") else ctypes.c_int)
-        got = lib.mdy_fp8_abi_version()
-        if got != ABI_VERSION:
-            raise MdyFp8Error("libmdyfp8.so ABI version %d, expected %d: rebuild" % (got, ABI_VERSION))
         _lib = lib
     return _lib
 

@@ -41,6 +41,19 @@ def test_abi_version(lib):
     assert lib.mdy_fp8_abi_version() == v
 
 
+def test_older_library_is_named_as_such(lib, tmp_path, monkeypatch):
+    """A library of another version is refused for its version, whatever else it lacks."""
+    import subprocess
+    from mdy_triton_amd import _lib
+    src, old = tmp_path / "old.c", tmp_path / "libmdyfp8.so"
+    src.write_text("int mdy_fp8_abi_version(void) { return %d; }\n" % (_lib.ABI_VERSION - 1))
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(old)], check=True)
+    monkeypatch.setattr(_lib, "LIB_PATH", str(old))
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(_lib.MdyFp8Error, match="rebuild"):
+        _lib.load()
+
+
 def test_argument_validation_without_device(lib):
     buf = ctypes.create_string_buffer(4096)
     p = ctypes.addressof(buf)
