@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define MDY_FP8_ABI_VERSION 16
+#define MDY_FP8_ABI_VERSION 17
 
 /* error codes (negative = argument rejected before any launch) */
 #define MDY_OK 0
@@ -159,13 +159,15 @@ int mdy_quant_transpose_typed(const void* x, int x_dtype, void* y, float* s, voi
 int mdy_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K,
                             int64_t x_row_stride, int64_t x_col_stride, int64_t PM, int64_t PK, int mode, void* stream);
 
-/* mdy_quant_transpose with MDY_T_COLUMN over G expert groups of m_splits[g] consecutive rows (multiples of 128, M in all) in one
- * launch.  Replaces the per-group launches of group_per_token_cast_to_fp8 (megatron_patchs/fp8_matmul.py:218-247).
+/* mdy_quant_transpose with MDY_T_COLUMN over G expert groups of m_splits[g] consecutive rows (multiples of 128, M in all), one
+ * launch for up to 128 groups.  Replaces the per-group launches of group_per_token_cast_to_fp8 (megatron_patchs/fp8_matmul.py:218-247).
  *   x    [M, K] of x_dtype         y    e4m3fn [M, K] row-major         s  fp32, row scale at s[(k/128) * M + m]
- *   y_t  e4m3fn, the arrays [K, m_g] of all groups one after the other   s_t fp32 [M/128, K]
- *   m_splits  HOST pointer to G row counts (read before the call returns), G <= 256;  K % 128 == 0 */
-int mdy_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s, void* y_t, float* s_t, const int64_t* m_splits,
-                                int64_t G, int64_t K, int64_t x_row_stride, int64_t x_col_stride, void* stream);
+ *   y_t  HOST array of G device pointers, group g: e4m3fn [K, m_g]      s_t  the same, group g: fp32 [m_g/128, K]
+ *   (the pointers of an empty group may be NULL)
+ *   m_splits  HOST pointer to G row counts;  all three are read before the call returns;  K % 128 == 0 */
+int mdy_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s, void* const* y_t, float* const* s_t,
+                                const int64_t* m_splits, int64_t G, int64_t K, int64_t x_row_stride, int64_t x_col_stride,
+                                void* stream);
 
 /* The two training quantizers with a scale per column and 128 rows (mdy_quant_transpose with MDY_T_COLUMN for mode
  * MDY_QUANT_DEEPLINEAR, mdy_act_quant_transpose for the official modes: their layouts, s_kb_stride only used by the former)

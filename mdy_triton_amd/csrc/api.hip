@@ -173,10 +173,10 @@ int mdy_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, void*
                     "act_quant_transpose");
 }
 
-int mdy_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s, void* y_t, float* s_t, const int64_t* m_splits,
+int mdy_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s, void* const* y_t, float* const* s_t, const int64_t* m_splits,
                                 int64_t G, int64_t K, int64_t x_row_stride, int64_t x_col_stride, void* stream) {
     if (x_dtype != MDY_XT_BF16 && x_dtype != MDY_XT_F16 && x_dtype != MDY_XT_F32) return fail(MDY_E_DTYPE, "quant_transpose_grouped: unknown x_dtype %d", x_dtype);
-    if (G < 0 || G > 256 || K < 0 || K > kMaxDim || K % 128 != 0) return fail(MDY_E_SHAPE, "quant_transpose_grouped: G=%lld up to 256, K=%lld a multiple of 128", (long long)G, (long long)K);
+    if (G < 0 || G > (1 << 20) || K < 0 || K > kMaxDim || K % 128 != 0) return fail(MDY_E_SHAPE, "quant_transpose_grouped: G=%lld up to 2^20, K=%lld a multiple of 128", (long long)G, (long long)K);
     if (G == 0 || K == 0) return 0;
     if (!m_splits) return fail(MDY_E_NULL, "quant_transpose_grouped: null m_splits");
     int64_t M = 0;
@@ -187,8 +187,13 @@ int mdy_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s, v
     if (M > kMaxDim) return fail(MDY_E_SHAPE, "quant_transpose_grouped: too many rows (%lld)", (long long)M);
     if (M == 0) return 0;
     if (!x || !y || !s || !y_t || !s_t) return fail(MDY_E_NULL, "quant_transpose_grouped: null pointer");
-    if (!aligned(y, 8) || !aligned(y_t, 8) || !aligned(s, 4) || !aligned(s_t, 4) || !aligned(x, x_dtype == MDY_XT_F32 ? 4 : 2))
-        return fail(MDY_E_ALIGN, "quant_transpose_grouped: y / y_t must be 8-byte aligned, x and the scales aligned for their type");
+    if (!aligned(y, 8) || !aligned(s, 4) || !aligned(x, x_dtype == MDY_XT_F32 ? 4 : 2))
+        return fail(MDY_E_ALIGN, "quant_transpose_grouped: y must be 8-byte aligned, x and s aligned for their type");
+    for (int64_t g = 0; g < G; ++g) {
+        if (m_splits[g] == 0) continue;
+        if (!y_t[g] || !s_t[g]) return fail(MDY_E_NULL, "quant_transpose_grouped: null pointer of group %lld", (long long)g);
+        if (!aligned(y_t[g], 8) || !aligned(s_t[g], 4)) return fail(MDY_E_ALIGN, "quant_transpose_grouped: y_t must be 8-byte aligned, s_t 4-byte aligned");
+    }
     if (int e = check_device()) return e;
     return launched(mdy::launch_quant_transpose_grouped(x, x_dtype, y, s, y_t, s_t, m_splits, G, M, K, x_row_stride, x_col_stride,
                                                         static_cast<hipStream_t>(stream)),

@@ -307,8 +307,8 @@ int launch_quant_transpose(const void* x, int x_dtype, void* y, float* s, void* 
                            int t_mode, hipStream_t stream);
 int launch_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K,
                                int64_t x_row_stride, int64_t x_col_stride, int64_t PM, int64_t PK, int mode, hipStream_t stream);
-int launch_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s, void* y_t, float* s_t, const int64_t* m_splits, int64_t G,
-                                   int64_t M, int64_t K, int64_t x_row_stride, int64_t x_col_stride, hipStream_t stream);
+int launch_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s, void* const* y_t, float* const* s_t, const int64_t* m_splits,
+                                   int64_t G, int64_t M, int64_t K, int64_t x_row_stride, int64_t x_col_stride, hipStream_t stream);
 int launch_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, float* s_t, int64_t M, int64_t K, int64_t x_row_stride,
                                   int64_t x_col_stride, int64_t PM, int64_t PK, int64_t s_kb_stride, int mode, float* part, void* col_sum,
                                   hipStream_t stream);

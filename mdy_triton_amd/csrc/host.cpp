@@ -702,34 +702,37 @@ int64_t sum_of(const std::vector<int64_t>& v) {
     return t;
 }
 
-// group_cast(x [M, N], m_splits) -> (y, s, [yt], [st]): megatron_patchs/fp8_matmul.py:218-247
+// group_cast(x [M, N], m_splits) -> (y, s, [yt], [st]): megatron_patchs/fp8_matmul.py:218-247.  Every group's copy is a tensor of its own.
 PyObject* group_cast(PyObject*, PyObject* const* args, Py_ssize_t n) {
     int device = -1;
     Mat x;
     std::vector<int64_t> splits;
-    if (n != 2 || !mat_arg(args[0], device, x) || x.t->dim() != 2 || !ints_arg(args[1], splits) || splits.size() > 256 || sum_of(splits) != x.M ||
-        x.K % 256 != 0)
-        Py_RETURN_NONE;
+    if (n != 2 || !mat_arg(args[0], device, x) || x.t->dim() != 2 || !ints_arg(args[1], splits) || sum_of(splits) != x.M || x.K % 256 != 0) Py_RETURN_NONE;
     for (int64_t m : splits)
         if (m % 256 != 0) Py_RETURN_NONE;
-    Tensor y, s, yt, st;
+    const size_t G = splits.size();
+    Tensor y, s;
+    std::vector<Tensor> yt(G), st(G);
     unlocked([&] {
         y = make({x.M, x.K}, kE4m3, x.dev());
         s = make_strided({x.M, x.K / 128}, {1, x.M}, ScalarType::Float, x.dev());
-        yt = make({x.M * x.K}, kE4m3, x.dev());
-        st = make({x.M / 128 * x.K}, ScalarType::Float, x.dev());
-        done(mdy_quant_transpose_grouped(x.data(), x.xt, raw(y), f32(s), raw(yt), f32(st), splits.data(), (int64_t)splits.size(), x.K, x.rs, x.cs,
+        std::vector<void*> ytp(G);
+        std::vector<float*> stp(G);
+        for (size_t g = 0; g < G; ++g) {
+            yt[g] = make({x.K, splits[g]}, kE4m3, x.dev());
+            st[g] = make_strided({x.K, splits[g] / 128}, {1, x.K}, ScalarType::Float, x.dev());
+            ytp[g] = raw(yt[g]);
+            stp[g] = f32(st[g]);
+        }
+        done(mdy_quant_transpose_grouped(x.data(), x.xt, raw(y), f32(s), ytp.data(), stp.data(), splits.data(), (int64_t)G, x.K, x.rs, x.cs,
                                          stream_of(device)));
     });
     PyObject* r = PyTuple_New(4);
-    PyObject *lt = PyList_New((Py_ssize_t)splits.size()), *ls = PyList_New((Py_ssize_t)splits.size());
+    PyObject *lt = PyList_New((Py_ssize_t)G), *ls = PyList_New((Py_ssize_t)G);
     if (r == nullptr || lt == nullptr || ls == nullptr) return nullptr;
-    int64_t row = 0;
-    for (size_t g = 0; g < splits.size(); ++g) {
-        const int64_t m = splits[g];
-        PyList_SET_ITEM(lt, (Py_ssize_t)g, THPVariable_Wrap(yt.as_strided({x.K, m}, {m > 0 ? m : 1, 1}, row * x.K)));
-        PyList_SET_ITEM(ls, (Py_ssize_t)g, THPVariable_Wrap(st.as_strided({x.K, m / 128}, {1, x.K}, row / 128 * x.K)));
-        row += m;
+    for (size_t g = 0; g < G; ++g) {
+        PyList_SET_ITEM(lt, (Py_ssize_t)g, THPVariable_Wrap(std::move(yt[g])));
+        PyList_SET_ITEM(ls, (Py_ssize_t)g, THPVariable_Wrap(std::move(st[g])));
     }
     PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(std::move(y)));
     PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(std::move(s)));

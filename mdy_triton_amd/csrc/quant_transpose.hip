@@ -52,13 +52,14 @@ __device__ __forceinline__ float qt_quot(float x, float s, float r) {
 // XT: input type (0 bf16, 1 fp16, 2 fp32); the reciprocal quotient is proven for bf16 inputs only, other types divide.
 // CSUM (with TMODE 0): also the fp32 sums of the tile's columns, to col_sum[row tile * PK + column]: an output gradient's column
 // sums are the bias gradient, and here they cost 8 adds per 16 bytes loaded instead of a pass over the matrix.
-// y_t_tile: the transposed copy's element (column 0, first row of the tile), rows of yt_stride bytes.
+// y_t_tile: the transposed copy's element (column 0, first row of the tile), rows of yt_stride bytes.  s_t_tile (TMODE 0): the scales of
+// the tile's row group, column k at s_t_tile[k * st_k_stride].
 template <int MODE, int TMODE, bool VEC, int XT, bool CSUM>
 __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void* __restrict__ x, uint8_t* __restrict__ y,
                                                      float* __restrict__ s, uint8_t* __restrict__ y_t_tile, int yt_stride,
-                                                     float* __restrict__ s_t, int M, int K, int64_t x_row_stride, int64_t x_col_stride,
-                                                     int PM, int PK, int64_t s_kb_stride, int64_t s_m_stride, int64_t st_a_stride,
-                                                     int64_t st_k_stride, float* __restrict__ col_sum) {
+                                                     float* __restrict__ s_t_tile, int M, int K, int64_t x_row_stride, int64_t x_col_stride,
+                                                     int PM, int PK, int64_t s_kb_stride, int64_t s_m_stride, int64_t st_k_stride,
+                                                     float* __restrict__ col_sum) {
     constexpr int NRG = 128 / RPT;        // row groups of RPT consecutive rows; 16 threads (8 columns each) per group
     constexpr int WAVES = NRG / 4;
     __shared__ __attribute__((aligned(8))) float col_part[WAVES][128];  // per wave (4 row groups) partial column maxima
@@ -137,7 +138,7 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
             col_amax[t] = m;
             col_sc[t] = sc;
             col_rc[t] = 1.0f / sc;
-            s_t[(int64_t)bm * st_a_stride + (int64_t)(bk * 128 + t) * st_k_stride] = sc;
+            s_t_tile[(int64_t)(bk * 128 + t) * st_k_stride] = sc;
             if (y != nullptr) s[(int64_t)bk * s_kb_stride + (int64_t)(bm * 128 + t) * s_m_stride] = row_sc[t];
             if (CSUM) {
                 float v = 0.0f;
@@ -164,7 +165,7 @@ __device__ __forceinline__ void quant_transpose_tile(int bm, int bk, const void*
         float bmax = blk_part[0];
 #pragma unroll
         for (int w = 1; w < WAVES; ++w) bmax = fmaxf(bmax, blk_part[w]);
-        if (t == 0) s_t[(int64_t)bk * (PM >> 7) + bm] = group_scale<MODE>(bmax);
+        if (t == 0) s_t_tile[(int64_t)bk * (PM >> 7) + bm] = group_scale<MODE>(bmax);
         if (t < 128 && y != nullptr) s[(int64_t)bk * s_kb_stride + (int64_t)(bm * 128 + t) * s_m_stride] = row_sc[t];
         const float bsc = group_scale<MODE>(bmax), brc = 1.0f / bsc;
 #pragma unroll
@@ -224,23 +225,24 @@ __global__ __launch_bounds__(2048 / RPT, 32 / RPT) void quant_transpose_kernel(c
                                                                float* __restrict__ col_sum) {
     const int bm = block_row(), bk = blockIdx.x;
     if (bm >= (PM >> 7)) return;
-    quant_transpose_tile<MODE, TMODE, VEC, XT, CSUM>(bm, bk, x, y, s, y_t + (int64_t)bm * 128, PM, s_t, M, K, x_row_stride, x_col_stride,
-                                                          PM, PK, s_kb_stride, s_m_stride, st_a_stride, st_k_stride, col_sum);
+    quant_transpose_tile<MODE, TMODE, VEC, XT, CSUM>(bm, bk, x, y, s, y_t + (int64_t)bm * 128, PM, TMODE == 0 ? s_t + bm * st_a_stride : s_t, M, K,
+                                                     x_row_stride, x_col_stride, PM, PK, s_kb_stride, s_m_stride, st_k_stride, col_sum);
 }
 
-// Expert groups of m_g rows (multiples of 128) one after the other: the row-wise copy and all scales lie as for one matrix, the
-// transposed copy of group g is an array [PK][m_g] of its own behind those of the groups before it.  One launch for all
-// groups: 8 ragged groups, 5376 rows x 7168 and x 4096, 16 launches of 8.8 us -> 2 launches, 141 -> 57 us.
-constexpr int kMaxQtGroups = 256;
+// Expert groups of m_g rows (multiples of 128) one after the other: the row-wise copy and its scales lie as for one matrix, the
+// transposed copy [PK][m_g] of every group and its scales are arrays of their own (a caller drops or changes one without the
+// others).  One launch for all groups: 8 ragged groups, 5376 rows x 7168 and x 4096, 16 launches of 8.8 us -> 2 launches, 141 -> 57 us.
+constexpr int kMaxQtGroups = 128;      // per launch: the table is a kernel argument of 2.5 KB
 struct QtGroups {
     int n;
     int row_start[kMaxQtGroups + 1];
+    uint8_t* y_t[kMaxQtGroups];
+    float* s_t[kMaxQtGroups];
 };
 template <bool VEC, int XT>
 __global__ __launch_bounds__(2048 / RPT, 32 / RPT) void quant_transpose_grouped_kernel(const void* __restrict__ x, uint8_t* __restrict__ y,
-                                                                             float* __restrict__ s, uint8_t* __restrict__ y_t,
-                                                                             float* __restrict__ s_t, int M, int K, int64_t x_row_stride,
-                                                                             int64_t x_col_stride, const QtGroups groups) {
+                                                                             float* __restrict__ s, int M, int K, int64_t x_row_stride,
+                                                                             int64_t x_col_stride, int64_t s_kb_stride, const QtGroups groups) {
     const int bm = block_row(), bk = blockIdx.x;
     if (bm >= (M >> 7)) return;
     int lo = 0, hi = groups.n - 1;                       // the last group that starts at or before the tile (empty ones skipped)
@@ -249,8 +251,9 @@ __global__ __launch_bounds__(2048 / RPT, 32 / RPT) void quant_transpose_grouped_
         if (groups.row_start[mid] <= bm * 128) lo = mid; else hi = mid - 1;
     }
     const int r0 = groups.row_start[lo];
-    quant_transpose_tile<1, 0, VEC, XT, false>(bm, bk, x, y, s, y_t + (int64_t)r0 * K + (bm * 128 - r0), groups.row_start[lo + 1] - r0,
-                                                    s_t, M, K, x_row_stride, x_col_stride, M, K, M, 1, K, 1, nullptr);
+    quant_transpose_tile<1, 0, VEC, XT, false>(bm, bk, x, y, s, groups.y_t[lo] + (bm * 128 - r0), groups.row_start[lo + 1] - r0,
+                                               groups.s_t[lo] + (int64_t)(bm - (r0 >> 7)) * K, M, K, x_row_stride, x_col_stride, M, K, s_kb_stride, 1, 1,
+                                               nullptr);
 }
 
 // Shared launcher.  mode: dialect (0 official, column groups only; 1 DeepLinear); t_mode: 0 per column group, 1 per
@@ -294,29 +297,41 @@ int launch_act_quant_transpose(const void* x, int x_dtype, void* y, float* s, vo
     return launch_qt(mode == 2 ? 2 : 0, x, x_dtype, y, s, y_t, s_t, M, K, x_row_stride, x_col_stride, PM, PK, 1, PK / 128, 1, PM / 128, 0, stream);
 }
 
-// M = sum of m_splits, every one a multiple of 128, K a multiple of 128; -1: more groups than the table holds.
-int launch_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s, void* y_t, float* s_t, const int64_t* m_splits, int64_t G,
-                                   int64_t M, int64_t K, int64_t x_row_stride, int64_t x_col_stride, hipStream_t stream) {
-    if (M == 0 || K == 0) return 0;
-    if (G > kMaxQtGroups) return -1;
-    QtGroups groups;
-    groups.n = (int)G;
-    int row = 0;
-    for (int g = 0; g <= kMaxQtGroups; ++g) {
-        groups.row_start[g] = row;
-        if (g < G) row += (int)m_splits[g];
-    }
-    dim3 grid;
-    if (!grid_rows(K / 128, M / 128, grid)) return kErrTooManyBlocks;
+// M = sum of m_splits, every one a multiple of 128, K a multiple of 128; y_t, s_t: host arrays of G device pointers
+int launch_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s, void* const* y_t, float* const* s_t, const int64_t* m_splits,
+                                   int64_t G, int64_t M, int64_t K, int64_t x_row_stride, int64_t x_col_stride, hipStream_t stream) {
+    if (K == 0) return 0;
     const bool vec = rows_vectorizable(x, K, x_row_stride, x_col_stride, xt_size(x_dtype));
+    int64_t row0 = 0;
+    for (int64_t g0 = 0; g0 < G; g0 += kMaxQtGroups) {
+        QtGroups groups = {};
+        groups.n = (int)(G - g0 < kMaxQtGroups ? G - g0 : kMaxQtGroups);
+        int rows = 0;
+        for (int g = 0; g < groups.n; ++g) {
+            groups.row_start[g] = rows;
+            groups.y_t[g] = static_cast<uint8_t*>(y_t[g0 + g]);
+            groups.s_t[g] = s_t[g0 + g];
+            rows += (int)m_splits[g0 + g];
+        }
+        groups.row_start[groups.n] = rows;
+        if (rows == 0) continue;
+        dim3 grid;
+        if (!grid_rows(K / 128, rows / 128, grid)) return kErrTooManyBlocks;
+        const void* xg = static_cast<const uint8_t*>(x) + row0 * x_row_stride * xt_size(x_dtype);
+        uint8_t* yg = static_cast<uint8_t*>(y) + row0 * K;
+        float* sg = s + row0;
 #define MDY_QTG(VEC, XT)                                                                                                        \
-    hipLaunchKernelGGL((quant_transpose_grouped_kernel<VEC, XT>), grid, dim3(2048 / RPT), 0, stream, x, static_cast<uint8_t*>(y), s, \
-                       static_cast<uint8_t*>(y_t), s_t, (int)M, (int)K, x_row_stride, x_col_stride, groups)
+    hipLaunchKernelGGL((quant_transpose_grouped_kernel<VEC, XT>), grid, dim3(2048 / RPT), 0, stream, xg, yg, sg, rows, (int)K, x_row_stride, \
+                       x_col_stride, M, groups)
 #define MDY_QTG_V(XT) do { if (vec) MDY_QTG(true, XT); else MDY_QTG(false, XT); } while (0)
-    if (x_dtype == 0) MDY_QTG_V(0); else if (x_dtype == 1) MDY_QTG_V(1); else MDY_QTG_V(2);
+        if (x_dtype == 0) MDY_QTG_V(0); else if (x_dtype == 1) MDY_QTG_V(1); else MDY_QTG_V(2);
 #undef MDY_QTG_V
 #undef MDY_QTG
-    return (int)hipGetLastError();
+        const int rc = (int)hipGetLastError();
+        if (rc != 0) return rc;
+        row0 += rows;
+    }
+    return 0;
 }
 
 // bf16(sum over the row tiles of part[a][k]; zeros without any): 32 columns x 8 interleaved shares of the row tiles per block

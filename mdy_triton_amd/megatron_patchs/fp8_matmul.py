@@ -65,37 +65,17 @@ def group_per_token_cast_to_fp8(x_all: torch.Tensor, m_splits: Sequence[int]):
     assert all(mg % 256 == 0 for mg in m_splits) and (N % 256 == 0 or not len(m_splits))
     y_all = torch.empty(Mtot, N, device=dev, dtype=FP8)
     s_all = torch.empty(N // 128, Mtot, device=dev, dtype=torch.float32)
-    # the transposed copies and their scales lie one after the other in two buffers; each group gets its piece
-    yt_buf = torch.empty(Mtot * N, device=dev, dtype=FP8)
-    st_buf = torch.empty(Mtot // 128, N, device=dev, dtype=torch.float32)
-    sizes = [int(mg) for mg in m_splits]
-    row = 0
-    with on_device(dev):
-        for g0 in range(0, len(sizes), 256):              # the kernel's group table holds 256
-            part = sizes[g0:g0 + 256]
-            rows = sum(part)
-            if rows == 0:
-                continue
-            if rows == Mtot:
-                check(lib().mdy_quant_transpose_grouped(ptr(x_all), xt, ptr(y_all), ptr(s_all), ptr(yt_buf), ptr(st_buf),
-                                                        (ctypes.c_int64 * len(part))(*part), len(part), N, x_all.stride(0),
-                                                        x_all.stride(1), stream_ptr(dev)), "group_per_token_cast_to_fp8")
-            else:
-                # row scales of all rows are one [N/128, Mtot] array: a part of the groups is launched group by group
-                for mg in part:
-                    if mg > 0:
-                        x = x_all[row:row + mg]
-                        check(lib().mdy_quant_transpose_typed(ptr(x), xt, ptr(y_all[row:]), s_all.data_ptr() + 4 * row,
-                                                              ptr(yt_buf[row * N:]), ptr(st_buf[row // 128:]), mg, N, x.stride(0), x.stride(1),
-                                                              mg, N, Mtot, 0, stream_ptr(dev)), "group_per_token_cast_to_fp8")
-                        row += mg
-    yt_all, st_all = [], []
-    row = 0
-    for mg in sizes:
-        yt_all.append(yt_buf[row * N:(row + mg) * N].view(N, mg))
-        st_all.append(st_buf[row // 128:(row + mg) // 128].transpose(0, 1))
-        row += mg
-    return y_all, s_all.transpose(0, 1), yt_all, st_all
+    # every group's transposed copy is a tensor of its own: one may be changed, saved or given up without the others
+    yt_all = [torch.empty(N, int(mg), device=dev, dtype=FP8) for mg in m_splits]
+    st_all = [torch.empty(int(mg) // 128, N, device=dev, dtype=torch.float32) for mg in m_splits]
+    G = len(yt_all)
+    if Mtot * N > 0:
+        pointers = ctypes.c_void_p * G
+        with on_device(dev):
+            check(lib().mdy_quant_transpose_grouped(ptr(x_all), xt, ptr(y_all), ptr(s_all), pointers(*[ptr(t) for t in yt_all]),
+                                                    pointers(*[ptr(t) for t in st_all]), (ctypes.c_int64 * G)(*[int(mg) for mg in m_splits]), G, N,
+                                                    x_all.stride(0), x_all.stride(1), stream_ptr(dev)), "group_per_token_cast_to_fp8")
+    return y_all, s_all.transpose(0, 1), yt_all, [t.transpose(0, 1) for t in st_all]
 
 
 def per_block_cast_to_fp8(x, output_normal: bool = True, output_transpose: bool = False):

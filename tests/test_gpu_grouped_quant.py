@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("splits,N,strided", [([256], 256, False), ([0, 256, 0, 0, 512, 0], 512, False), ([256, 0], 256, True),
                                               ([512, 256, 256], 7168, False), ([0, 0], 256, False), ([256] * 3 + [0] * 300, 256, False),
-                                              ([0] * 256 + [256], 256, False), ([256] + [0] * 270 + [256], 256, False)])
+                                              ([0] * 256 + [256], 256, False), ([256] + [0] * 270 + [256], 256, False),
+                                              ([0] * 127 + [512, 256], 256, True), ([256] * 130, 256, False)])
 def test_group_boundaries(splits, N, strided):
     x = torch.randn(sum(splits), N, generator=torch.Generator().manual_seed(len(splits))).bfloat16()
     xd = x.cuda()
@@ -29,6 +30,39 @@ def test_group_boundaries(splits, N, strided):
             for got, ref in ((y[row:row + mg], ry), (s[row:row + mg], rs), (a, ryt), (b, rst)):
                 assert np.array_equal(got.cpu().contiguous().view(torch.uint8).numpy(), ref.contiguous().view(torch.uint8).numpy())
         row += mg
+
+
+@pytest.mark.parametrize("wrapper", [False, True])       # the native call and the wrapper
+def test_every_group_is_a_tensor_of_its_own(wrapper):
+    """One group's copy changed or given up: the others can still be saved for a backward pass, and its memory is free."""
+    from mdy_triton_amd.megatron_patchs.manger import CustomManger
+
+    class Splits(tuple):      # what the native call leaves to the wrapper
+        pass
+
+    splits = (Splits if wrapper else list)([4096, 256, 512])
+    x = torch.randn(sum(splits), 2048, device="cuda").bfloat16()
+    _, _, yt, st = m.group_per_token_cast_to_fp8(x, splits)
+
+    class Keep(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, a, *saved):
+            ctx.save_for_backward(*saved)
+            return a * 2
+
+        @staticmethod
+        def backward(ctx, g):
+            assert len(ctx.saved_tensors) == 4
+            return (g * 2,) + (None,) * 4
+
+    a = torch.ones(1, requires_grad=True, device="cuda")
+    out = Keep.apply(a, yt[1], yt[2], st[1], st[2])
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    CustomManger.clear_tensor_data(yt[0], st[0])
+    assert before - torch.cuda.memory_allocated() >= 4096 * 2048
+    out.backward()
+    assert a.grad.item() == 2
 
 
 @pytest.mark.parametrize("H", [8, 504, 512, 520, 2040, 2048, 2056, 3, 255, 257])      # bf16: around 64 and 256 pieces of 16, 2 and 1 bytes
