@@ -61,6 +61,14 @@ constexpr int kEpiDirect = 0;      // straight from registers, 8 (bf16) or 16 (f
 constexpr int kEpiLines = 1;       // bf16 through LDS in whole rows that start on 128-byte lines, non-temporal
 constexpr int kEpiRows = 2;        // through LDS in whole rows, cached: fp32, and bf16 rows that start inside lines
 
+// Between LDS writes of some lanes of a wave and reads of them by others (or the other way round).  The hardware executes a wave's LDS
+// accesses in order; this keeps the compiler from moving one across.  No instruction.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Epilogue of one wave's TI x TJ sub-tiles for bf16 results: through the wave's own part of LDS (TI * 16 rows of TJ * 32 bytes,
 // free once the K loop is over), so that a store instruction writes whole rows of the wave tile, 16 bytes per lane, instead of
 // 8-byte pieces of 16 different rows: a quarter of the cache lines per instruction and half the instructions.  All CUs end
@@ -106,6 +114,7 @@ __device__ __forceinline__ void store_rows(const floatx4 (&acc)[TI][TJ], uint8_t
                     make_float4(v[0] + bv[0], v[1] + bv[1], v[2] + bv[2], v[3] + bv[3]);
         }
     }
+    wave_lds_fence();
 #pragma unroll
     for (int t = 0; t < TI * CH / 4; ++t) {
         const int q = t * 64 + lane, row = q / CH, ch = q % CH;
@@ -158,11 +167,13 @@ __device__ __forceinline__ void store_rows_beside(const floatx4 (&acc)[TI][4], u
                     *reinterpret_cast<uint2*>(buf + frow * 128 + (((2 * j + (fk >> 1)) ^ (frow & 7)) << 4) + (fk & 1) * 8) =
                         make_uint2(pack2_bf16(r[0] + bv[j][0], r[1] + bv[j][1]), pack2_bf16(r[2] + bv[j][2], r[3] + bv[j][3]));
                 }
+                wave_lds_fence();
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {      // (a wave's LDS accesses are executed in order: the next 16 rows' writes come after these reads)
+                for (int t = 0; t < 2; ++t) {
                     const int row = t * 8 + (lane >> 3);
                     v[i & 1][t] = *reinterpret_cast<const uintx4_t*>(buf + row * 128 + ((ch ^ (row & 7)) << 4));
                 }
+                wave_lds_fence();      // the next 16 rows are written to the same place
             }
             if (i > 0) {
 #pragma unroll
