@@ -522,36 +522,36 @@ PyObject* version_guard(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return THPVariable_Wrap(version_of(t));
 }
 
-// official_forward(x, w, bias or None, fmt, need_dx, need_dw) -> (y, xt, xt_s, wt, wt_s, version of x, version of w): fp8_kernel.py:261-272
+// official_forward(x, w, bias or None, fmt, keep_xt, keep_wt, versions) -> (y, xt, xt_s, wt, wt_s, version of x, version of w):
+// fp8_kernel.py:261-272; None for what is not asked for
 PyObject* official_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    if (n != 6 || !PyLong_CheckExact(args[3])) Py_RETURN_NONE;
+    if (n != 7 || !PyLong_CheckExact(args[3])) Py_RETURN_NONE;
     int device = -1;
     Mat x, w;
     if (!mat_arg(args[0], device, x) || !mat_arg(args[1], device, w) || w.t->dim() != 2 || w.K != x.K || x.K % 128 != 0 || w.M % 128 != 0) Py_RETURN_NONE;
     const int fmt = (int)PyLong_AsLong(args[3]);
-    const bool need_dx = flag(args[4]), need_dw = flag(args[5]);
+    const bool keep_xt = flag(args[4]), keep_wt = flag(args[5]), versions = flag(args[6]);
     const int64_t N = w.M, K = x.K;
     const void* bias;
     if (!bias_arg(args[2], N, device, bias)) Py_RETURN_NONE;
-    if (!need_dw && (x.cs != 1 || x.rs != K)) Py_RETURN_NONE;
-    const bool keeps = need_dx || need_dw;
-    if (keeps && (x.t->is_inference() || w.t->is_inference())) Py_RETURN_NONE;      // save_for_backward refuses them: the wrapper lets it
+    if (!keep_xt && (x.cs != 1 || x.rs != K)) Py_RETURN_NONE;
+    if (versions && (x.t->is_inference() || w.t->is_inference())) Py_RETURN_NONE;      // save_for_backward refuses them: the wrapper lets it
     Copies xc, wc;
     Tensor y = unlocked([&] {
         void* stream = stream_of(device);
-        if (need_dw) {
+        if (keep_xt) {
             xc = official_copies(x, true, fmt, Tensor(), stream);
         } else {
             xc.y = make({x.M, K}, fmt_type(fmt), x.dev());
             xc.s = make({x.M, K / 128}, ScalarType::Float, x.dev());
             done(mdy_act_quant_typed(x.data(), x.xt, 128, raw(xc.y), f32(xc.s), x.M, K, K, x.M, K, K / 128, 1, fmt_mode(fmt), stream));
         }
-        wc = weight_copies(w, true, need_dx, N, K, fmt_type(fmt), fmt_mode(fmt), stream);
+        wc = weight_copies(w, true, keep_wt, N, K, fmt_type(fmt), fmt_mode(fmt), stream);
         auto sizes = x.t->sizes().vec();
         sizes.back() = N;
         return product(xc.y, xc.s, K / 128, 1, wc.y, wc.s, bias, MDY_BIAS_IN_SUM, x.M, N, K, fmt, sizes, stream);
     });
-    return tuple_of({y, xc.yt, xc.st, wc.yt, wc.st, keeps ? version_of(*x.t) : Tensor(), keeps ? version_of(*w.t) : Tensor()});
+    return tuple_of({y, xc.yt, xc.st, wc.yt, wc.st, versions ? version_of(*x.t) : Tensor(), versions ? version_of(*w.t) : Tensor()});
 }
 
 // official_backward(dy, xt, xt_s, wt, wt_s, fmt, need_dx, need_dw, need_db) -> (dx, dw, db): fp8_kernel.py:274-301

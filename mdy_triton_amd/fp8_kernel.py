@@ -424,9 +424,12 @@ class _Fp8LinearFunction(torch.autograd.Function):
     Backward: x and dy quantized along the tokens (transposed copies, one kernel pass over dy for both of its copies),
     w^T block-quantized; dx = dy . w through the tile kernels, dw = dy^T . x through the GEMM with row scales on both
     operands.  The transposed copies keep their zero padding to a multiple of 128 tokens, so any token count works.
-    What the backward pass will need of x and w is quantized by the forward's own pass over them (x and w are read once per
-    step instead of twice) and kept in place of x: one byte per element instead of two.  The version counters of x and w are
-    kept too, so that a backward pass after an in-place change of either is refused as for any saved tensor."""
+    What the backward pass will need of x is quantized by the forward's own pass over it (x is read once per step instead of
+    twice) and kept in place of x: one byte per element of x, also where x stays alive for another reason.  The same is done with
+    w, one byte per element of it, as long as both copies take no more memory than x itself (N <= M for a bf16 x): every forward pass
+    whose backward pass is still to come holds its own.  Beyond that w is kept, which costs nothing, and quantized again
+    by the backward pass.  The version counters of x and w are kept too, so that a backward pass after an in-place change of either is
+    refused as for any saved tensor."""
 
     @staticmethod
     def forward(ctx, x, w, bias, fp8_dtype, grad_enabled=True):
@@ -436,9 +439,12 @@ class _Fp8LinearFunction(torch.autograd.Function):
         ctx.has_bias = bias is not None
         ctx.fp8_dtype = fp8_dtype
         ctx.input_shape = input_shape
-        done = host().official_forward(x, w, bias, fmt, need_dx, need_dw)
+        # both copies within x's memory (their scales, one 64th on top, apart).  Quantizing w again costs a pass over it: 256x8192x8192 170 -> 195 us
+        # a step, 1024x4096x4096 116 -> 121, 2048x7168x2048 148 -> 153 (351, 200 and 247 with x quantized again as well)
+        keep_wt = need_dx and w.numel() + (x.numel() if need_dw else 0) <= x.numel() * x.element_size()
+        done = host().official_forward(x, w, bias, fmt, need_dw, keep_wt, need_dx or need_dw)
         if done is not None:
-            ctx.save_for_backward(*done[1:])
+            ctx.save_for_backward(*(done[1:] if keep_wt or not need_dx else done[1:6] + (w,)))
             return done[0]
         x2 = x.reshape(-1, input_shape[-1])
         if need_dw:
@@ -448,15 +454,18 @@ class _Fp8LinearFunction(torch.autograd.Function):
         else:
             qx, sx = act_quant_block(x2, dtype=fp8_dtype)
             qxt = sxt = None
-        qw, sw, qwt, swt = _weight_quant_both(w, True, need_dx, fp8_dtype, "Fp8Linear")
+        qw, sw, qwt, swt = _weight_quant_both(w, True, keep_wt, fp8_dtype, "Fp8Linear")
         y = fp8_matmul(qx, qw, sx, sw, bias, have_w=True)
-        ctx.save_for_backward(qxt, sxt, qwt, swt, *(_versions(x2, w) if need_dx or need_dw else ()))
+        versions = _versions(x2, w) if need_dx or need_dw else (None, None)
+        ctx.save_for_backward(qxt, sxt, qwt, swt, versions[0], versions[1] if keep_wt or not need_dx else w)
         return y.view(*input_shape[:-1], w.size(0))
 
     @staticmethod
     def backward(ctx, dy):
-        qxt, sxt, qwt, swt = ctx.saved_tensors[:4]
+        qxt, sxt, qwt, swt, _, w = ctx.saved_tensors
         need = ctx.needs_input_grad
+        if need[0] and qwt is None:
+            _, _, qwt, swt = _weight_quant_both(w, False, True, ctx.fp8_dtype, "Fp8Linear.backward")
         dx, dw, dbias = _official_linear_backward(dy, (qwt, swt), (qxt, sxt), need[0], need[1], ctx.fp8_dtype, ctx.has_bias and need[2])
         if dx is not None and len(ctx.input_shape) != 2:
             dx = dx.view(ctx.input_shape)

@@ -533,3 +533,34 @@ def test_backward_takes_what_saved_tensor_hooks_give_back(dtype):
                           (ValueError, lambda t: t.t().contiguous() if t.dtype == torch.float32 else t)):
         with pytest.raises(error):
             grads(same, unpack)
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 4096, 512), (2048, 512, 512), (512, 512, 256), (3, 256, 1024)])
+@pytest.mark.parametrize("frozen", [False, True])      # of the weight: the input gradient alone
+@pytest.mark.parametrize("wrapper", [False, True])
+def test_a_pending_backward_pass_holds_no_more_than_its_input(M, N, K, frozen, wrapper):
+    """The copies kept between the passes take at most the bytes of x, also for few tokens against a large weight, and the
+    gradients are the ones of the quantized operands, whichever pass quantizes the weight."""
+    g = torch.Generator().manual_seed(M)
+    lin = m.Fp8Linear(K, N, bias=False, device=DEV, dtype=torch.bfloat16, fp8_dtype=FP8)
+    lin.weight.requires_grad_(not frozen)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    if wrapper:      # rows of 3 dimensions that are not contiguous go past the native call
+        x = x.view(M, 1, K).expand(M, 2, K)[:, :1]
+        x = torch.cat([x, x], 1)[:, :1]
+    x.requires_grad_(True)
+    lin(x.detach().clone().requires_grad_(True)).sum().backward()      # warm
+    lin.zero_grad()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    y = lin(x)
+    held = torch.cuda.memory_allocated() - before - y.numel() * 2
+    assert held <= max(M, 128) * K * 2 * 65 // 64 + 6 * 512, held      # tokens are padded to 128; scales
+    dy = torch.randn(M, N, generator=g).bfloat16().to(DEV)
+    y.backward(dy.view(y.shape))
+    qdy, sdy, qdyt, sdyt = FK._act_quant_transposed(dy, True, "t", FP8)
+    _, _, qwt, swt = FK._weight_quant_both(lin.weight.detach(), False, True, FP8, "t")
+    assert torch.equal(x.grad.reshape(M, K), FK.fp8_matmul(qdy[:M], qwt, sdy[:M], swt))
+    if not frozen:
+        _, _, qxt, sxt = FK._act_quant_transposed(x.detach().reshape(M, K), False, "t", FP8)
+        assert torch.equal(lin.weight.grad, FK.fp8_matmul(qdyt, qxt, sdyt, sxt, have_w=False))
