@@ -87,8 +87,8 @@ _host = None
 
 
 def host():
-    """The native host side of the serving operators (csrc/host.cpp): each function returns its result in the ordinary case and
-    None in every other, before it has done anything."""
+    """The native host side of the operators (csrc/host.cpp): each function returns its result in the ordinary case and
+    None in every other, which the wrapper that called it then handles or refuses."""
     global _host
     if _host is None:
         try:

@@ -1,4 +1,4 @@
-"""Build libmdyfp8.so (HIP kernels + C ABI) for gfx950 with hipcc, and _host.so (the native host side of the serving
+"""Build libmdyfp8.so (HIP kernels + C ABI) for gfx950 with hipcc, and _host.so (the native host side of the
 operators, against the installed torch) with g++, in-tree.
 
 Usage: python -m mdy_triton_amd.csrc.build   (or call build())

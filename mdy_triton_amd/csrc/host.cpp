@@ -3,9 +3,10 @@
 // host time against 2.3-4 us of kernel at one token; a small layer's training step made 110 us of them, one of 32 small
 // experts 1070 us).
 //
-// Every function takes the ordinary case - plain tensors on the current device, the layouts the operators document - and
-// returns None for anything else, before anything is allocated or launched: the Python wrapper then goes its own way, which
-// handles or rejects the rest with its own messages.  A call that the library rejects also returns None and is repeated there.
+// Every function takes the ordinary case - plain tensors on the current device, the layouts the operators document, sizes that
+// all of its products take - and returns None for anything else, before anything is allocated or launched: the Python wrapper
+// then goes its own way, which handles or rejects the rest with its own messages.  What only the library or the allocator can
+// refuse (a grid beyond the launch limits, memory that is not there) also returns None and is met again there.
 // Outputs come from torch's caching allocator on the current stream, as torch.empty gives them; nothing is kept between calls.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -107,8 +108,13 @@ bool gemm(const void* a, const float* a_s, int64_t rs, int64_t cs, const void* b
 }
 // What the MFMA kernels need of a GEMM (anything else may run the scalar kernel, about which the wrapper warns)
 bool gemm_shape_ok(int64_t M, int64_t N, int64_t K, int64_t rs, int64_t cs) {
-    return M > 0 && N > 0 && K > 0 && K % 128 == 0 && K <= 65536 && rs >= 0 && cs >= 0 &&
+    return M > 0 && N > 0 && K > 0 && M <= (1 << 30) && N <= (1 << 30) && K % 128 == 0 && K <= 65536 && rs >= 0 && cs >= 0 &&
            ((M - 1) * rs + (K / 128 - 1) * cs + 1) * 4 < ((int64_t)1 << 31);
+}
+// the same for the GEMM with row scales on both operands
+bool row_scaled_shape_ok(int64_t M, int64_t N, int64_t K, int64_t a_rs, int64_t a_cs, int64_t b_rs, int64_t b_cs) {
+    const auto extent_ok = [&](int64_t rows, int64_t rs, int64_t cs) { return rs >= 0 && cs >= 0 && ((rows - 1) * rs + (K / 128 - 1) * cs + 1) * 4 < ((int64_t)1 << 31); };
+    return M > 0 && N > 0 && K > 0 && M <= (1 << 30) && N <= (1 << 30) && K % 128 == 0 && K <= (1 << 20) && extent_ok(M, a_rs, a_cs) && extent_ok(N, b_rs, b_cs);
 }
 
 ScalarType fmt_type(int fmt) { return fmt == MDY_FMT_E4M3 ? kE4m3 : ScalarType::Float8_e5m2; }
@@ -292,8 +298,9 @@ PyObject* deep_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // training
 // ---------------------------------------------------------------------------------------------------------------------------
 
-// Thrown when the library rejects a call in the middle of a composite one: the whole call returns None and is repeated by the
-// wrapper, whose own checks say what is wrong.  (Launches already made wrote outputs that nobody has seen.)
+// Thrown when the library rejects a call in the middle of a composite one for what could not be told beforehand: the whole call
+// returns None and is repeated by the wrapper, whose own checks say what is wrong.  (Launches already made wrote outputs that
+// nobody has seen.)
 struct Rejected {};
 void done(int rc) {
     if (rc != 0) throw Rejected();
@@ -384,10 +391,9 @@ Copies weight_copies(const Mat& w, bool rows, bool transposed, int64_t PN, int64
     return c;
 }
 
-// bf16 [sizes] = a . b^T, M rows of a (scales a_s[m * rs + kb * cs]) against N rows of b
+// bf16 [sizes] = a . b^T, M rows of a (scales a_s[m * rs + kb * cs]) against N rows of b; the callers have asked gemm_shape_ok
 Tensor product(const Tensor& a, const Tensor& a_s, int64_t rs, int64_t cs, const Tensor& b, const Tensor& b_s, const void* bias, int bias_mode,
                int64_t M, int64_t N, int64_t K, int fmt, at::IntArrayRef sizes, void* stream) {
-    if (!gemm_shape_ok(M, N, K, rs, cs)) throw Rejected();
     Tensor c = make(sizes, ScalarType::BFloat16, a.device());
     const int64_t bytes = mdy_fp8_gemm_workspace_bytes(M, N, K);
     Tensor ws;
@@ -465,14 +471,14 @@ PyObject* deep_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const void* bias;
     if (!bias_arg(args[3], N, device, bias)) Py_RETURN_NONE;
     if (!need_dw && (x.cs != 1 || x.rs < x.K)) Py_RETURN_NONE;
+    const int64_t pad = need_dw ? 256 : 4, PM = cdiv(x.M, pad) * pad;
+    if (!gemm_shape_ok(x.M, N, PK, 1, PM)) Py_RETURN_NONE;
     const int mode = (int)PyLong_AsLong(args[4]);
     Copies xc;
     Tensor out = unlocked([&] {
         void* stream = stream_of(device);
-        int64_t PM = cdiv(x.M, 4) * 4;
         if (need_dw) {
             xc = deep_copies(x, 1, Tensor(), stream);
-            PM = xc.y.size(0);
         } else if (!quantize_rows(Rows{x.t, x.M, x.K, x.rs, x.xt}, xc.y, xc.s, stream)) {
             throw Rejected();
         }
@@ -497,6 +503,7 @@ PyObject* deep_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int64_t M = dy.M, N = dy.K, K = PyLong_AsLongLong(args[5]), PM = cdiv(M, 256) * 256, PN = cdiv(N, 256) * 256;
     if ((need_dx && !copy_ok(wc.yt, wc.st, kE4m3, K, PN, cdiv(K, 128), PN / 128)) || (need_dw && !copy_ok(xc.yt, xc.st, kE4m3, K, PM, cdiv(K, 128), PM / 128)))
         Py_RETURN_NONE;
+    if ((need_dx && !gemm_shape_ok(M, K, PN, 1, PM)) || (need_dw && !gemm_shape_ok(N, K, PM, 1, PN))) Py_RETURN_NONE;
     Tensor db, dx, dw;
     unlocked([&] {
         void* stream = stream_of(device);
@@ -534,7 +541,7 @@ PyObject* official_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int64_t N = w.M, K = x.K;
     const void* bias;
     if (!bias_arg(args[2], N, device, bias)) Py_RETURN_NONE;
-    if (!keep_xt && (x.cs != 1 || x.rs != K)) Py_RETURN_NONE;
+    if ((!keep_xt && (x.cs != 1 || x.rs != K)) || !gemm_shape_ok(x.M, N, K, K / 128, 1)) Py_RETURN_NONE;
     if (versions && (x.t->is_inference() || w.t->is_inference())) Py_RETURN_NONE;      // save_for_backward refuses them: the wrapper lets it
     Copies xc, wc;
     Tensor y = unlocked([&] {
@@ -569,6 +576,7 @@ PyObject* official_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!need_dx && !need_dw) Py_RETURN_NONE;
     if (need_dx && (!wc.yt.defined() || wc.yt.dim() != 2 || !copy_ok(wc.yt, wc.st, fmt_type(fmt), 0, N, cdiv(wc.yt.size(0), 128), N / 128))) Py_RETURN_NONE;
     if (need_dw && (!xc.yt.defined() || xc.yt.dim() != 2 || !copy_ok(xc.yt, xc.st, fmt_type(fmt), 0, PM, xc.yt.size(0), PM / 128))) Py_RETURN_NONE;
+    if ((need_dx && !gemm_shape_ok(M, wc.yt.size(0), N, N / 128, 1)) || (need_dw && !row_scaled_shape_ok(N, xc.yt.size(0), PM, PM / 128, 1, PM / 128, 1))) Py_RETURN_NONE;
     Tensor db, dx, dw;
     unlocked([&] {
         void* stream = stream_of(device);
@@ -639,7 +647,9 @@ PyObject* row_scaled_product(PyObject*, PyObject* const* args, Py_ssize_t n) {
         b->numel() == 0 || !a->is_contiguous() || !b->is_contiguous() || !aligned16(*a) || !aligned16(*b))
         Py_RETURN_NONE;
     const int64_t M = a->size(0), K = a->size(1), N = b->size(0);
-    if (K % 128 != 0 || b->size(1) != K || as->size(0) != M || as->size(1) != K / 128 || bs->size(0) != N || bs->size(1) != K / 128) Py_RETURN_NONE;
+    if (b->size(1) != K || as->size(0) != M || as->size(1) != K / 128 || bs->size(0) != N || bs->size(1) != K / 128 ||
+        !row_scaled_shape_ok(M, N, K, as->stride(0), as->stride(1), bs->stride(0), bs->stride(1)))
+        Py_RETURN_NONE;
     return THPVariable_Wrap(unlocked([&] { return row_scaled(*a, *as, *b, *bs, M, N, K, fmt, stream_of(device)); }));
 }
 

@@ -69,3 +69,31 @@ def test_inference_tensor_is_refused_in_training():
         assert lin(x).shape == (32, 256)
     with pytest.raises(RuntimeError, match="[Ii]nference"):
         lin(x)
+
+
+def _beyond(kind):
+    """A composite native call one of whose products is beyond the sizes the GEMMs take, as a function."""
+    from mdy_triton_amd._torch_glue import host
+    fp8 = lambda *s: torch.zeros(s, device="cuda", dtype=torch.uint8).view(torch.float8_e4m3fn)
+    f32, bf = lambda *s: torch.zeros(s, device="cuda"), lambda *s: torch.zeros(s, device="cuda", dtype=torch.bfloat16)
+    h = host()
+    if kind == "deep_backward":             # 65792 padded tokens: the weight gradient's contraction
+        args = (bf(65537, 256), fp8(256, 65792), f32(2, 514), fp8(256, 256), f32(2, 2), 256, True, True, True)
+        return lambda: h.deep_backward(*args)
+    if kind == "official_backward":         # more than 2^20 tokens
+        args = (bf(2 ** 20 + 1, 128), fp8(128, 2 ** 20 + 128), f32(128, 8193), fp8(128, 128), f32(1, 1), 0, True, True, True)
+        return lambda: h.official_backward(*args)
+    if kind == "deep_forward":              # more than 65536 input features
+        args = (bf(8, 65792), bf(128, 65792), None, None, 0, True, True)
+        return lambda: h.deep_forward(*args)
+    args = (bf(8, 65664), bf(128, 65664), None, 0, True, True, True)
+    return lambda: h.official_forward(*args)
+
+
+@pytest.mark.parametrize("kind", ["deep_backward", "official_backward", "deep_forward", "official_forward"])
+def test_native_call_that_is_left_to_the_wrapper_has_done_nothing(kind):
+    call = _beyond(kind)
+    count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    before = count()
+    assert call() is None
+    assert count() == before
