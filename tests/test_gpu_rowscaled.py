@@ -33,8 +33,10 @@ def test_exact_integer(M, N, K, fmt):
     exact_case(M, N, K, fmt, transposed_scales=bool(fmt))
 
 
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("transposed_scales", [False, True])      # row-major (what Fp8Linear passes) and column-major
 @pytest.mark.parametrize("M,N,K", [(512, 512, 4096), (1000, 1020, 4224), (130, 257, 9600), (1536, 1536, 5120)])
-def test_exact_integer_cut_along_k(M, N, K):
+def test_exact_integer_cut_along_k(M, N, K, transposed_scales, fmt):
     from mdy_triton_amd import _lib
     assert _lib.load().mdy_fp8_gemm_rowscaled_workspace_bytes(M, N, K) >= 2 * M * N * 4
-    exact_case(M, N, K, 0, transposed_scales=True)
+    exact_case(M, N, K, fmt, transposed_scales)
