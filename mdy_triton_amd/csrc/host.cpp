@@ -561,9 +561,10 @@ PyObject* official_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return tuple_of({y, xc.yt, xc.st, wc.yt, wc.st, versions ? version_of(*x.t) : Tensor(), versions ? version_of(*w.t) : Tensor()});
 }
 
-// official_backward(dy, xt, xt_s, wt, wt_s, fmt, need_dx, need_dw, need_db) -> (dx, dw, db): fp8_kernel.py:274-301
+// official_backward(dy, xt, xt_s, wt, wt_s, fmt, need_dx, need_dw, need_db, w or None) -> (dx, dw, db): fp8_kernel.py:274-301; wt, wt_s
+// None: from w
 PyObject* official_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    if (n != 9 || !PyLong_CheckExact(args[5])) Py_RETURN_NONE;
+    if (n != 10 || !PyLong_CheckExact(args[5])) Py_RETURN_NONE;
     int device = -1;
     Mat dy;
     Copies xc, wc;
@@ -574,15 +575,22 @@ PyObject* official_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const bool need_dx = flag(args[6]), need_dw = flag(args[7]), need_db = flag(args[8]);
     const int64_t M = dy.M, N = dy.K, PM = cdiv(M, 128) * 128;
     if (!need_dx && !need_dw) Py_RETURN_NONE;
-    if (need_dx && (!wc.yt.defined() || wc.yt.dim() != 2 || !copy_ok(wc.yt, wc.st, fmt_type(fmt), 0, N, cdiv(wc.yt.size(0), 128), N / 128))) Py_RETURN_NONE;
+    Mat w;      // to be quantized here
+    if (need_dx && !wc.yt.defined()) {
+        if (!mat_arg(args[9], device, w) || w.t->dim() != 2 || w.M != N || w.K % 128 != 0) Py_RETURN_NONE;
+    } else if (need_dx && (wc.yt.dim() != 2 || !copy_ok(wc.yt, wc.st, fmt_type(fmt), 0, N, cdiv(wc.yt.size(0), 128), N / 128))) {
+        Py_RETURN_NONE;
+    }
     if (need_dw && (!xc.yt.defined() || xc.yt.dim() != 2 || !copy_ok(xc.yt, xc.st, fmt_type(fmt), 0, PM, xc.yt.size(0), PM / 128))) Py_RETURN_NONE;
-    if ((need_dx && !gemm_shape_ok(M, wc.yt.size(0), N, N / 128, 1)) || (need_dw && !row_scaled_shape_ok(N, xc.yt.size(0), PM, PM / 128, 1, PM / 128, 1))) Py_RETURN_NONE;
+    const int64_t K = w.t != nullptr ? w.K : need_dx ? wc.yt.size(0) : 0;
+    if ((need_dx && !gemm_shape_ok(M, K, N, N / 128, 1)) || (need_dw && !row_scaled_shape_ok(N, xc.yt.size(0), PM, PM / 128, 1, PM / 128, 1))) Py_RETURN_NONE;
     Tensor db, dx, dw;
     unlocked([&] {
         void* stream = stream_of(device);
         if (need_db) db = make({N}, ScalarType::BFloat16, dy.dev());
         const Copies dc = official_copies(dy, need_dx, fmt, db, stream);
-        if (need_dx) dx = product(dc.y, dc.s, N / 128, 1, wc.yt, wc.st, nullptr, 0, M, wc.yt.size(0), N, fmt, {M, wc.yt.size(0)}, stream);
+        if (w.t != nullptr) wc = weight_copies(w, false, true, N, K, fmt_type(fmt), fmt_mode(fmt), stream);
+        if (need_dx) dx = product(dc.y, dc.s, N / 128, 1, wc.yt, wc.st, nullptr, 0, M, K, N, fmt, {M, K}, stream);
         if (need_dw) dw = row_scaled(dc.yt, dc.st, xc.yt, xc.st, N, xc.yt.size(0), PM, fmt, stream);
     });
     return tuple_of({dx, dw, db});

@@ -7,9 +7,9 @@ pair of the FP8 MLP (fp8_kernel.py:447-450, 500-515) into one pass over the up/g
 that file's own linear layer in the official dialect (s = amax / finfo.max, no clamp, no eps):
 act_quant_block (:62-87), fp8_matmul (:214-252), fp8_matmul_bwd (:254-257), Fp8Linear (:259-313).
 Both float8_e4m3fn and float8_e5m2 (the reference's default dtype, fp8_kernel.py:62, 124, 303) are implemented for the
-official-dialect functions; e4m3fn runs the tuned kernels, e5m2 the general quantizer kernels and the GEMM with row scales
-on both operands (a weight's 128x128 block scales are expanded to one per row for it).  The DeepLinear dialect and the
-fused silu_act_quant are e4m3fn only.
+official-dialect functions, on the same kernels with the byte format as a template parameter (an e5m2 product beyond what
+those take, K > 65536, unaligned operands or scales spanning 2^31 bytes, runs the GEMM with row scales on both operands, the
+weight's 128x128 block scales expanded to one per row).  The DeepLinear dialect and the fused silu_act_quant are e4m3fn only.
 """
 from typing import Optional, Tuple
 
@@ -377,14 +377,14 @@ def _saved_copy(copy, fp8_dtype, cols, scale_shape, dev, who):
     return (y if y.data_ptr() % 16 == 0 else y.clone()), s.contiguous()
 
 
-def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8, need_dbias=False):
+def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8, need_dbias=False, w=None):
     """Gradients of y = x . w^T in the official dialect (fp8_kernel.py:274-301): dx = dy . w on the row-wise copy of dy
     and the block-quantized w^T, dw = dy^T . x on the transposed copies of dy and x (row scales on both operands).
-    w_t = (bytes, scales) of w^T, x_t = (bytes, scales) of the transposed x; either may be None when its gradient is not
-    needed.  One kernel pass over dy gives both of its copies and, for the bias gradient, its column sums; the transposed copies keep their zero padding to a multiple
-    of 128 tokens."""
+    w_t = (bytes, scales) of w^T, or (None, None) for them to be taken from w; x_t = (bytes, scales) of the transposed x; either
+    may be None when its gradient is not needed.  One kernel pass over dy gives both of its copies and, for the bias gradient, its
+    column sums; the transposed copies keep their zero padding to a multiple of 128 tokens."""
     _, fmt = _fp8_mode(fp8_dtype, "Fp8Linear.backward")
-    done = host().official_backward(dy2, *x_t, *w_t, fmt, need_dx, need_dw, need_dbias)
+    done = host().official_backward(dy2, *x_t, *w_t, fmt, need_dx, need_dw, need_dbias, w)
     if done is not None:
         return done
     dy2 = dy2.reshape(-1, dy2.size(-1))
@@ -398,6 +398,8 @@ def _official_linear_backward(dy2, w_t, x_t, need_dx, need_dw, fp8_dtype=FP8, ne
     dbias = torch.empty(N, device=dev, dtype=torch.bfloat16) if need_dbias and dy2.numel() > 0 else None
     qdy, sdy, qdyt, sdyt = _act_quant_transposed(dy2, need_dx, "Fp8Linear.backward", fp8_dtype, dbias)
     if need_dx:
+        if w_t[0] is None:
+            w_t = _weight_quant_both(w, False, True, fp8_dtype, "Fp8Linear.backward")[2:]
         qwt, swt = _saved_copy(w_t, fp8_dtype, N, lambda rows: ((rows + 127) // 128, N // 128), dev, "Fp8Linear.backward")
         dx = fp8_matmul(qdy[:M], qwt, sdy[:M], swt, have_w=True)
     if need_dw:
@@ -464,9 +466,8 @@ class _Fp8LinearFunction(torch.autograd.Function):
     def backward(ctx, dy):
         qxt, sxt, qwt, swt, _, w = ctx.saved_tensors
         need = ctx.needs_input_grad
-        if need[0] and qwt is None:
-            _, _, qwt, swt = _weight_quant_both(w, False, True, ctx.fp8_dtype, "Fp8Linear.backward")
-        dx, dw, dbias = _official_linear_backward(dy, (qwt, swt), (qxt, sxt), need[0], need[1], ctx.fp8_dtype, ctx.has_bias and need[2])
+        dx, dw, dbias = _official_linear_backward(dy, (qwt, swt), (qxt, sxt), need[0], need[1], ctx.fp8_dtype, ctx.has_bias and need[2],
+                                                  w)
         if dx is not None and len(ctx.input_shape) != 2:
             dx = dx.view(ctx.input_shape)
         return dx, dw, dbias, None, None

@@ -501,13 +501,14 @@ def test_act_quant_block_e5m2_golden_codes_on_device():
     assert np.array_equal(u8(y), d["y_t"]) and np.array_equal(s.cpu().numpy(), d["s_t"])
 
 
+@pytest.mark.parametrize("tokens", [200, 512])      # the weight itself is saved, its transposed copy is
 @pytest.mark.parametrize("dtype", [FP8, E5M2])
-def test_backward_takes_what_saved_tensor_hooks_give_back(dtype):
+def test_backward_takes_what_saved_tensor_hooks_give_back(dtype, tokens):
     """Copies that come back with other strides, at an odd address or from the host give the same gradients; what is not the saved
     copy any more is refused before a kernel sees it."""
     g = torch.Generator().manual_seed(3)
     lin = m.Fp8Linear(256, 384, bias=True, device=DEV, dtype=torch.bfloat16, fp8_dtype=dtype)
-    x0, dy = torch.randn(200, 256, generator=g).bfloat16().to(DEV), torch.randn(200, 384, generator=g).bfloat16().to(DEV)
+    x0, dy = torch.randn(tokens, 256, generator=g).bfloat16().to(DEV), torch.randn(tokens, 384, generator=g).bfloat16().to(DEV)
 
     def grads(pack, unpack):
         lin.zero_grad()

@@ -81,7 +81,7 @@ def _beyond(kind):
         args = (bf(65537, 256), fp8(256, 65792), f32(2, 514), fp8(256, 256), f32(2, 2), 256, True, True, True)
         return lambda: h.deep_backward(*args)
     if kind == "official_backward":         # more than 2^20 tokens
-        args = (bf(2 ** 20 + 1, 128), fp8(128, 2 ** 20 + 128), f32(128, 8193), fp8(128, 128), f32(1, 1), 0, True, True, True)
+        args = (bf(2 ** 20 + 1, 128), fp8(128, 2 ** 20 + 128), f32(128, 8193), fp8(128, 128), f32(1, 1), 0, True, True, True, None)
         return lambda: h.official_backward(*args)
     if kind == "deep_forward":              # more than 65536 input features
         args = (bf(8, 65792), bf(128, 65792), None, None, 0, True, True)
