@@ -86,9 +86,9 @@ __global__ __launch_bounds__(512) void fp8_gemm_splitk_ws_kernel(
                                                      tn * BN, N, K, N, duty, kb0, kb1, pool);
 }
 
-// VEC columns per thread (N a multiple of it, aligned c), 1 otherwise.  KS: number of slabs, 0: `ksplit` of them, four at a time.  The
-// slabs lie in the caches and a launch lives for a few microseconds, so every load of a thread is in flight at once, nothing is loaded
-// twice (two slabs used to be read as four), and 8 columns share a thread where that still leaves a workgroup per CU (fewer waves lose:
+// VEC columns per thread (N a multiple of it, aligned c), 1 otherwise.  KS: number of slabs, 0: `ksplit` of them, four at a time (the
+// last step's loads beyond them repeat the last slab).  The slabs lie in the caches and a launch lives for a few microseconds, so with
+// 2 to 4 slabs every load of a thread is in flight at once and none is made twice (two slabs used to be read as four), and 8 columns share a thread where that still leaves a workgroup per CU (fewer waves lose:
 // 128x2112 13.4 -> 13.6 us).  GEMM and reduction: M=64 N=2048 K=7168 9.95 -> 9.5 us, M=48 9.4 -> 8.9, 777x2112x7168 29.3 -> 28.9.
 template <typename OUT, int VEC, int KS>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, OUT* __restrict__ c,

@@ -215,6 +215,9 @@ static int rowscaled_config(int64_t M, int64_t N, int64_t K) {
     // with few K blocks the ends of the tiles count, and a 256x256 workgroup copies its second tile's panels while the first one's
     // results leave: two rounds of it against three of 128x256 (4096x4864x256 20.3 -> 17.9 us, 4096x6144x512 27.3 -> 24.2, 4096x6144x1024
     // 42.2 -> 37.3, 4096x4864x1024 37.8 -> 37.2; but 4096x4864x4096 113.7 -> 126)
+    // and between (128x256 / 256x256): 4096x6144x1536 53.5 / 52.8, x2048 66.4 / 68.0, x3072 94.1 / 98.5; 4096x4864x1536 49.5 / 51.4.  Three
+    // rounds against five tie or win by 1 to 8 % at every K (8192x4352x2048 107 / 101, x4096 195 / 190, 6144x6144x4096 196.4 / 195.0), four
+    // against seven by 7 to 19 %: the line at K > 1024 takes the latter only
     return (K <= 1024 ? 13 : 17) * big <= 10 * mid ? 2 : 1;
 }
 

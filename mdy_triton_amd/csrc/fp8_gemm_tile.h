@@ -78,7 +78,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 // 70 -> 63 -> 63 us, with row scales 4096x7168x512 45 -> 36 -> 35 us.  Where rows do not start on 128-byte lines a wave's rows
 // end inside lines that its neighbours complete, and the stores stay cached so that L2 joins the parts (3752x15224x768: 82 us direct, 86 through
 // LDS non-temporal, 80 through LDS cached).  The 16-byte pieces of a row are XOR-swizzled by
-// the row (no bank conflict either way).  Needs N % 8 == 0 and 16-byte aligned rows of c (the caller checks).
+// the row: no bank conflict of the reads; of the writes rows r and r + 8 meet in pairs, 4 cycles a write.  Needs N % 8 == 0 and 16-byte aligned rows of c (the caller checks).
 // fp32 results (the slabs of a K split, an fp32 output) go the same way with twice the row length where the pool holds them;
 // those stores stay cached: the reduction reads the slabs next.
 template <int TI, int TJ, typename OUT, bool NT>
@@ -301,6 +301,8 @@ struct OneTile {};
 // a tile together and stood still for the 33 MB of a round.  Now the first two K blocks of a tile run while the stores of the
 // last one drain: 4096x7168x512 with row scales 28.4 -> 24.9 us, 8192x8192x512 55 -> 50 us, 3752x15224x768 71 -> 64.5 us,
 // 16384x4096x1024 81 -> 76 us, 8192x4096x4096 117.5 -> 116 us; at the power limit of a long K it ties (4096x18432x7168).
+// (Those without a bias.  With one its loads complete behind the copies that went out in front of them, and the stores wait for
+// both: 0 to 4 us more, 3752x15224x768 64.5 -> 68.6 us, 16384x4096x1024 78.1 -> 79.4, none from K = 4096 on.)
 template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ = 0, int TD_ = 0, int ABL_ = 0, int FMT_ = 0,
           bool BROW_ = false, int EPI_ = kEpiDirect, typename NEXT = OneTile>
 __device__ __forceinline__ void fp8_gemm_tile(
