@@ -431,7 +431,8 @@ class _Fp8LinearFunction(torch.autograd.Function):
     w, one byte per element of it, as long as both copies take no more memory than x itself (N <= M for a bf16 x): every forward pass
     whose backward pass is still to come holds its own.  Beyond that w is kept, which costs nothing, and quantized again
     by the backward pass.  The version counters of x and w are kept too, so that a backward pass after an in-place change of either is
-    refused as for any saved tensor."""
+    refused as for any saved tensor.  (A change through `.data` bumps none: a backward pass behind it takes w as the forward pass
+    saw it where the copy was kept, and as it is then where w was.)"""
 
     @staticmethod
     def forward(ctx, x, w, bias, fp8_dtype, grad_enabled=True):
