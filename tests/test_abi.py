@@ -152,3 +152,16 @@ def test_gemm_path_query_needs_no_gpu(lib):
     assert q(None, None, 32, 1, 128, 1536, 4096, 1) == 4            # split along K with a workspace ...
     assert q(None, None, 32, 1, 128, 1536, 4096, 0) == 3            # ... plain tiles without
     assert q(None, None, 56, 1, 0, 5, 128, 0) == -2
+
+
+def test_workspace_query_is_what_the_chosen_kernel_uses(lib):
+    """Room for slabs of K only where the call is cut along K; otherwise that of a transposed copy of the scales, or none."""
+    import random
+    r, cut = random.Random(7), 0
+    shapes = [(256, 4096, 4096)] + [(r.randrange(1, 1600), r.randrange(1, 9000), 128 * r.randrange(1, 130)) for _ in range(4000)]
+    for M, N, K in shapes:
+        need, path = lib.mdy_fp8_gemm_workspace_bytes(M, N, K), lib.mdy_fp8_gemm_path(None, None, K // 128, 1, M, N, K, 1)
+        scales = (M * (K // 128) * 4 + 255) // 256 * 256
+        cut += path == 4
+        assert need % (4 * M * N) == 0 and need >= 8 * M * N if path == 4 else need in (0, scales), (M, N, K)
+    assert cut > 100

@@ -44,7 +44,7 @@ def _bits(t):
 
 # (first call, second smaller call): split along K with 128x128 / 128x64 tiles and, for (40, 300, 8192), the whole-line kernel over
 # slabs of K; then a shape that needs no scratch
-CASES = [((256, 4096, 4096), (128, 1536, 4096)),
+CASES = [((256, 2304, 4096), (128, 1536, 4096)),
          ((130, 1100, 5120), (40, 300, 8192)),
          ((128, 2112, 7168), (16, 2048, 7168)),
          ((64, 2048, 7168), (33, 130, 4096))]
@@ -62,6 +62,7 @@ def test_static_workspace_matches_caller_workspace(first, second, dtype):
         need = lib.mdy_fp8_gemm_workspace_bytes(M, N, K)
         if i == 0:
             assert need > 0, "the first call of every case is meant to use the scratch memory"
+            assert lib.mdy_fp8_gemm_path(None, None, K // 128, 1, M, N, K, 1) == 4, "and to be cut along K"
         ws = torch.empty(max(need, 16), dtype=torch.uint8, device=DEV)
         rc_ws, want = _call("ws", a, a_s, b, b_s, dtype, bias, ws)
         rc_st, got = _call("static", a, a_s, b, b_s, dtype, bias)
