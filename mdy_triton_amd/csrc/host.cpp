@@ -875,14 +875,14 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return THPVariable_Wrap(unlocked([&] {
         const at::Device dev = r.t->device();
         void* stream = stream_of(device);
-        const Tensor y = make({PM, K}, kE4m3, dev), s = make({PM * (K / 128)}, ScalarType::Float, dev);
+        Tensor y = make({PM, K}, kE4m3, dev), s = make({PM * (K / 128)}, ScalarType::Float, dev);
         done(mdy_act_quant_typed(r.t->data_ptr(), r.xt, 128, raw(y), f32(s), M, r.K, r.stride, PM, K, rs, cs, mode, stream));
         const Tensor act = make({PM, PI}, kE4m3, dev), act_s = make({PM, PI / 128}, ScalarType::Float, dev);      // written [PI / 128, PM] with deep
         const int64_t bytes = mdy_fp8_gemm_swiglu_workspace_bytes(M, N2, K);
         Tensor ws = make({bytes}, ScalarType::Byte, dev);
         done(mdy_fp8_gemm_swiglu(raw(y), f32(s), rs, cs, raw(*qwu), f32(*swu), M, N2, K, gate_first, raw(act), f32(act_s), PM, PI, act_rs, cs, mode, raw(ws),
                                  bytes, stream));
-        ws.reset();
+        y.reset(), s.reset(), ws.reset();      // the down projection finds room where these were
         return product(act, act_s, act_rs, cs, *qwd, *swd, nullptr, 0, M, N, PI, MDY_FMT_E4M3, sizes, stream);
     }));
 }

@@ -165,3 +165,12 @@ def test_workspace_query_is_what_the_chosen_kernel_uses(lib):
         cut += path == 4
         assert need % (4 * M * N) == 0 and need >= 8 * M * N if path == 4 else need in (0, scales), (M, N, K)
     assert cut > 100
+
+
+def test_swiglu_workspace_holds_slabs_or_a_product(lib):
+    """The slabs alone where they go to the activation quantizer, else the product behind what its GEMM needs."""
+    q, gemm = lib.mdy_fp8_gemm_swiglu_workspace_bytes, lib.mdy_fp8_gemm_workspace_bytes
+    for M, N, K in ((200, 4096, 7168), (197, 2048, 7168), (61, 1536, 7168)):
+        assert q(M, N, K) == gemm(M, N, K) > 4 * M * N
+    assert q(250, 1034, 4096) == -(-gemm(250, 1034, 4096) // 256) * 256 + 2 * 250 * 1034 and gemm(250, 1034, 4096) > 0      # halves of odd columns
+    assert q(5, 1536, 2048) == 2 * 5 * 1536

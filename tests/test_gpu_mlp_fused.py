@@ -51,6 +51,45 @@ def test_slabs_are_what_these_shapes_take():
     assert q(200, 4096, 7168) == 4 * 200 * 4096 * 4 and q(197, 2048, 7168) > 0 and q(61, 1536, 7168) > 0 and q(5, 1536, 2048) == 0
 
 
+# split along K, and not: the quantized input, the projection and the down projection's result are not all held at once
+@pytest.mark.parametrize("M,H,I", [(500, 16384, 2048), (2048, 8192, 512)])
+def test_forward_peak_memory(M, H, I):
+    g = torch.Generator(device="cuda").manual_seed(I)
+    x = torch.randn(M, H, generator=g, device="cuda").bfloat16()
+    (qu, su), (qd, sd) = (L.quant_weight((torch.randn(*s, generator=g, device="cuda") * 0.02).bfloat16())[:2] for s in ((2 * I, H), (H, I)))
+    scales = lambda k: M * k // 128 * 4
+    up = lib().mdy_fp8_gemm_swiglu_workspace_bytes(M, 2 * I, H)
+    act = M * I + scales(I)
+    bound = act + max(M * H + scales(H) + up, 2 * M * H + lib().mdy_fp8_gemm_workspace_bytes(M, H, I))
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    y = host().mlp(x, qu, su, 2 * I, qd, sd, H, 0, 1)
+    assert y is not None and torch.cuda.max_memory_allocated() - before <= bound + (2 << 20)      # what the allocator rounds up
+
+
+def test_operands_that_the_slabs_do_not_take():
+    """A weight on 8 bytes runs the scalar kernel: the product lies where the slabs would."""
+    M, I, K = 70, 256, 4096
+    g = torch.Generator(device="cuda").manual_seed(3)
+    qa, sa = FK.act_quant_block(torch.randn(M, K, generator=g, device="cuda").bfloat16(), dtype=E4M3)
+    qb, sb = FK.weight_quant_block((torch.randn(2 * I, K, generator=g, device="cuda") * 0.05).bfloat16(), dtype=E4M3)
+    odd = torch.empty(qb.numel() + 8, dtype=torch.uint8, device="cuda")[8:]
+    odd.copy_(qb.view(torch.uint8).flatten())
+    C, need = lib(), lib().mdy_fp8_gemm_swiglu_workspace_bytes(M, 2 * I, K)
+    assert C.mdy_fp8_gemm_path(None, None, K // 128, 1, M, 2 * I, K, 1) == 4 and C.mdy_fp8_gemm_path(None, 8, K // 128, 1, M, 2 * I, K, 1) == 0
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda")
+    y, s = torch.empty(M, I, dtype=E4M3, device="cuda"), torch.empty(M, I // 128, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    assert C.mdy_fp8_gemm_swiglu(qa.data_ptr(), sa.data_ptr(), K // 128, 1, odd.data_ptr(), sb.data_ptr(), M, 2 * I, K, 0, y.data_ptr(), s.data_ptr(), M, I,
+                                 I // 128, 1, 0, ws.data_ptr(), need, stream) == 0
+    c = torch.empty(M, 2 * I, dtype=torch.bfloat16, device="cuda")
+    assert C.mdy_fp8_gemm_nt(qa.data_ptr(), sa.data_ptr(), K // 128, 1, odd.data_ptr(), sb.data_ptr(), c.data_ptr(), None, M, 2 * I, K, 0, stream) == 0
+    ry, rs = FK.silu_act_quant(c, "up-gate")
+    assert torch.equal(y.view(torch.uint8), ry.view(torch.uint8)) and torch.equal(s, rs)
+
+
 class _Without:
     """The native host side with one function that takes no call."""
 
