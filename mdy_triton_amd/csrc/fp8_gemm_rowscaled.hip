@@ -179,7 +179,10 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
     float* __restrict__ ws, int M, int N, int K, int tiles_m, int tiles_n, int slabs, int kb_per) {
     __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<128, 256, 8, 3>::bytes];
     const int ntiles = tiles_m * tiles_n;
-    const int pid = xcd_contiguous(blockIdx.x, ntiles * slabs);
+    // runs per XCD from 13 K blocks per slab on, against K > 8192 from 10 (runs against plain order, warm / cold: 768x512x11648, slabs of 7,
+    // 21.9 -> 23.5 / 23.7 -> 26.2 us, 512x1152x10368 (9) 24.0 -> 24.8 / 26.0 -> 27.1, 2304x512x3712 (10) 22.0 -> 23.5 / 24.8 -> 27.0; 640x768x15232
+    // (10) 1.08 / 1.06 times as fast, 1408x768x13440 (15) 1.08 / 1.10)
+    const int pid = slab_order(blockIdx.x, ntiles * slabs, kb_per >= 13 || (kb_per >= 10 && K > 8192));
     const int ks = __builtin_amdgcn_readfirstlane(pid / ntiles);
     int tm, tn;
     const Duty duty = tile_of(pid - ks * ntiles, tiles_m, tiles_n, tm, tn);

@@ -648,6 +648,9 @@ __device__ __forceinline__ int xcd_contiguous(int pid, int ntiles) {
     const int x = pid & 7, rest = ntiles & 7;
     return x * (ntiles >> 3) + min(x, rest) + (pid >> 3);
 }
+// The same for (slab, tile) pairs of a call cut along K, where a count that 8 does not divide stays in plain order with short slabs: in
+// runs, all workgroups of an XCD start on the same few panels, and a slab of few K blocks ends before their sharing pays.
+__device__ __forceinline__ int slab_order(int pid, int n, bool runs) { return (n & 7) != 0 && !runs ? pid : xcd_contiguous(pid, n); }
 // GM: tile rows per group; the 32 workgroups that an XCD runs at a time then cover a GM x (32 / GM) block of tiles
 // (4 x 8 in the product; the probe library also builds 2 x 16 and 8 x 4 to measure their fabric traffic and energy).
 template <int GM = 4>

@@ -35,7 +35,8 @@ def test_exact_integer(M, N, K, fmt):
 
 @pytest.mark.parametrize("fmt", [0, 1])
 @pytest.mark.parametrize("transposed_scales", [False, True])      # row-major (what Fp8Linear passes) and column-major
-@pytest.mark.parametrize("M,N,K", [(512, 512, 4096), (1000, 1020, 4224), (130, 257, 9600), (1536, 1536, 5120)])
+@pytest.mark.parametrize("M,N,K", [(512, 512, 4096), (1000, 1020, 4224), (130, 257, 9600), (1536, 1536, 5120),
+                                   (1530, 640, 4736), (2176, 638, 8576)])      # counts that 8 does not divide, short and long slabs
 def test_exact_integer_cut_along_k(M, N, K, transposed_scales, fmt):
     from mdy_triton_amd import _lib
     assert _lib.load().mdy_fp8_gemm_rowscaled_workspace_bytes(M, N, K) >= 2 * M * N * 4
