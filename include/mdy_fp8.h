@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define MDY_FP8_ABI_VERSION 19
+#define MDY_FP8_ABI_VERSION 20
 
 /* error codes (negative = argument rejected before any launch) */
 #define MDY_OK 0
@@ -334,6 +334,39 @@ int mdy_fp8_gemm_swiglu(const void* a, const float* a_s, int64_t as_row_stride, 
 #define MDY_PATH_TILES_SPLIT_K 4 /* K cut into slabs of the workspace: MFMA tiles, or the small-M kernel for up to 64 rows */
 int mdy_fp8_gemm_path(const void* a, const void* b, int64_t as_row_stride, int64_t as_col_stride, int64_t M,
                       int64_t N, int64_t K, int with_workspace);
+
+/* Which kernel within the family, so that a test can say what it runs: for operands and scales that every kernel takes, on the current
+ * device (256 CUs without one); launches nothing.  No counterpart in the reference.  The value's low 8 bits are one of MDY_FORM_..., the
+ * bits above are the number of slabs that K is cut into (0: one launch).
+ *   mdy_fp8_gemm_form            mdy_fp8_gemm_nt / _ws (with_workspace)
+ *   mdy_fp8_gemm_rowscaled_form  mdy_fp8_gemm_nt_rowscaled / _ws; the plain loop, 128x128 (one or two per CU), 128x256, 256x256
+ *   mdy_fp8_grouped_gemm_form    mdy_fp8_grouped_gemm_nt; REST_...: whole rounds of 256x256 tiles and, of what is left over, pieces; PIECES_...:
+ *                                pieces of 128 rows alone
+ */
+#define MDY_FORM_SCALAR 0
+#define MDY_FORM_WHOLE_LINES 1
+#define MDY_FORM_STRIP 2
+#define MDY_FORM_ROW_VECTOR 3
+#define MDY_FORM_64X64 4
+#define MDY_FORM_64X128 5
+#define MDY_FORM_128X64 6
+#define MDY_FORM_128X128 7
+#define MDY_FORM_128X128_TWO 8 /* two workgroups per CU */
+#define MDY_FORM_128X192 9
+#define MDY_FORM_128X256 10
+#define MDY_FORM_256X128 11
+#define MDY_FORM_256X256 12
+#define MDY_FORM_256X256_REST 13 /* and the last columns in 128x256 */
+#define MDY_FORM_PLAIN_LOOP 14
+#define MDY_FORM_PER_GROUP 15 /* a dense call per group */
+#define MDY_FORM_REST_128X128 16
+#define MDY_FORM_REST_128X192 17
+#define MDY_FORM_REST_128X256 18
+#define MDY_FORM_PIECES_128 19
+#define MDY_FORM_PIECES_192 20
+int mdy_fp8_gemm_form(int64_t M, int64_t N, int64_t K, int with_workspace);
+int mdy_fp8_gemm_rowscaled_form(int64_t M, int64_t N, int64_t K, int with_workspace);
+int mdy_fp8_grouped_gemm_form(const int64_t* m_splits, int64_t G, int64_t N, int64_t K);
 
 /* mdy_fp8_gemm_nt_ws for callers that cannot allocate device memory and so cannot bring a workspace: code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the reference.

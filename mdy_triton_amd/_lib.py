@@ -10,7 +10,7 @@ import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libmdyfp8.so")
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 _lock = threading.Lock()
 _lib = None
@@ -48,6 +48,9 @@ SIGNATURES = {
     "mdy_fp8_gemm_swiglu": [_p, _p, _i64, _i64, _p, _p, _i64, _i64, _i64, _int, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _i64, _p],
     "mdy_fp8_gemm_swiglu_workspace_bytes": [_i64, _i64, _i64],
     "mdy_fp8_gemm_path": [_p, _p, _i64, _i64, _i64, _i64, _i64, _int],
+    "mdy_fp8_gemm_form": [_i64, _i64, _i64, _int],
+    "mdy_fp8_gemm_rowscaled_form": [_i64, _i64, _i64, _int],
+    "mdy_fp8_grouped_gemm_form": [_p, _i64, _i64, _i64],
     "mdy_fp8_gemm_nt_static_ws": [_p, _p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _i64, _int, _p],
     "mdy_fp8_gemm_static_workspace_bytes": [],
     "mdy_fp8_gemm_static_workspace_init": [],

@@ -430,6 +430,30 @@ int mdy_fp8_gemm_path(const void* a, const void* b, int64_t as_row_stride, int64
     return mdy::fp8_gemm_path(a, b, as_row_stride, as_col_stride, M, N, K, with_workspace);
 }
 
+int mdy_fp8_gemm_form(int64_t M, int64_t N, int64_t K, int with_workspace) {
+    if (M < 1 || N < 1 || K < 1 || M > kMaxDim || N > kMaxDim || K > kMaxDim)
+        return fail(MDY_E_SHAPE, "fp8_gemm_form: bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
+    return mdy::fp8_gemm_form(M, N, K, with_workspace);
+}
+
+int mdy_fp8_gemm_rowscaled_form(int64_t M, int64_t N, int64_t K, int with_workspace) {
+    if (M < 1 || N < 1 || K < 1 || M > kMaxDim || N > kMaxDim || K > kMaxDim || K % 128 != 0)
+        return fail(MDY_E_SHAPE, "fp8_gemm_rowscaled_form: bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
+    return mdy::fp8_gemm_rowscaled_form(M, N, K, with_workspace);
+}
+
+int mdy_fp8_grouped_gemm_form(const int64_t* m_splits, int64_t G, int64_t N, int64_t K) {
+    if (!m_splits) return fail(MDY_E_NULL, "fp8_grouped_gemm_form: null m_splits");
+    int64_t M = 0;
+    for (int64_t g = 0; g < G && g < (1 << 20); ++g) {
+        if (m_splits[g] < 0 || m_splits[g] > kMaxDim) return fail(MDY_E_SHAPE, "fp8_grouped_gemm_form: m_splits[%lld]=%lld", (long long)g, (long long)m_splits[g]);
+        M += m_splits[g];
+    }
+    if (G < 1 || G > (1 << 20) || M < 1 || M > kMaxDim || N < 1 || K < 1 || N > kMaxDim || K > kMaxDim)
+        return fail(MDY_E_SHAPE, "fp8_grouped_gemm_form: bad shape G=%lld M=%lld N=%lld K=%lld", (long long)G, (long long)M, (long long)N, (long long)K);
+    return mdy::fp8_grouped_gemm_form(m_splits, G, N, K);
+}
+
 int64_t mdy_fp8_gemm_static_workspace_bytes(void) { return mdy::kStaticScratchBytes; }
 
 int mdy_fp8_gemm_static_workspace_init(void) {

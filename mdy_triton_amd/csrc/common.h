@@ -316,6 +316,9 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
                                  const float* b_s, int64_t bs_rs, int64_t bs_cs, void* c, int64_t M, int64_t N, int64_t K,
                                  int fmt, int out_dtype, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 int64_t fp8_gemm_rowscaled_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int fp8_gemm_rowscaled_form(int64_t M, int64_t N, int64_t K, int with_workspace);
+int fp8_gemm_form(int64_t M, int64_t N, int64_t K, int with_workspace);
+int fp8_grouped_gemm_form(const int64_t* m_splits, int64_t G, int64_t N, int64_t K);
 int launch_swiglu(const void* x, void* act, void* y, float* s, int64_t M, int64_t N, int64_t x_row_stride,
                   int gate_first, int64_t PM, int64_t PN, int64_t s_row_stride, int64_t s_col_stride, int mode,
                   hipStream_t stream);

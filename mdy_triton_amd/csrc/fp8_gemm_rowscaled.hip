@@ -14,6 +14,7 @@
 // loop (128x128 tile, four waves of 64x64, the K block's two panels and two scale vectors copied global -> LDS by `buffer_load
 // ... lds`, double buffered, one barrier per K block: short ends, but 0.93 us per K block against 0.72) runs what has few K blocks.
 // K % 128 == 0 (the callers contract over a padded token count).
+#include "../../include/mdy_fp8.h"
 #include "fp8_gemm_tile.h"
 
 namespace mdy {
@@ -232,6 +233,13 @@ static RowscaledPlan plan_rowscaled(int64_t M, int64_t N, int64_t K, bool slabs)
 int64_t fp8_gemm_rowscaled_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     const RowscaledPlan p = plan_rowscaled(M, N, K, true);
     return p.slabs > 1 ? (int64_t)p.slabs * M * N * 4 : 0;
+}
+
+// the form of a call whose operands qualify, and its slabs of K in the bits above
+int fp8_gemm_rowscaled_form(int64_t M, int64_t N, int64_t K, int with_workspace) {
+    constexpr int kForm[5] = {MDY_FORM_PLAIN_LOOP, MDY_FORM_128X256, MDY_FORM_256X256, MDY_FORM_128X128, MDY_FORM_128X128_TWO};
+    const RowscaledPlan p = plan_rowscaled(M, N, K, with_workspace != 0);
+    return kForm[p.config] | (p.slabs > 1 ? p.slabs << 8 : 0);
 }
 
 // returns hipError_t, or -1 when the operands do not qualify (K % 128 != 0, misaligned, scale extents >= 2^31 bytes)

@@ -174,3 +174,23 @@ def test_swiglu_workspace_holds_slabs_or_a_product(lib):
         assert q(M, N, K) == gemm(M, N, K) > 4 * M * N
     assert q(250, 1034, 4096) == -(-gemm(250, 1034, 4096) // 256) * 256 + 2 * 250 * 1034 and gemm(250, 1034, 4096) > 0      # halves of odd columns
     assert q(5, 1536, 2048) == 2 * 5 * 1536
+
+
+def test_form_queries(lib):
+    """The kernel that a call runs: within the family that the path query names, with the slabs that the workspace query makes room for."""
+    import random
+    r = random.Random(11)
+    path_of = {0: 0, 1: 1, 2: 2, 3: 1}
+    for _ in range(3000):
+        M, N, K, ws = r.choice([r.randrange(1, 65), r.randrange(65, 6000)]), r.randrange(1, 30000), 128 * r.randrange(1, 600), r.randrange(2)
+        v = lib.mdy_fp8_gemm_form(M, N, K, ws)
+        form, slabs = v & 255, v >> 8
+        assert lib.mdy_fp8_gemm_path(None, None, K // 128, 1, M, N, K, ws) == (4 if slabs else path_of.get(form, 3)), (M, N, K)
+        assert slabs == 0 or (ws == 1 and lib.mdy_fp8_gemm_workspace_bytes(M, N, K) == 4 * slabs * M * N), (M, N, K)
+        slabs = lib.mdy_fp8_gemm_rowscaled_form(M, N, K, 1) >> 8
+        assert lib.mdy_fp8_gemm_rowscaled_workspace_bytes(M, N, K) == 4 * slabs * M * N and lib.mdy_fp8_gemm_rowscaled_form(M, N, K, 0) >> 8 == 0
+    assert lib.mdy_fp8_gemm_form(4, 4, 100, 1) == 0 and lib.mdy_fp8_gemm_form(0, 4, 128, 1) == -2
+    assert lib.mdy_fp8_gemm_rowscaled_form(4, 4, 100, 1) == -2
+    form = lambda rows, N, K: lib.mdy_fp8_grouped_gemm_form((ctypes.c_int64 * len(rows))(*rows), len(rows), N, K)
+    assert form([1, 0, 7], 512, 1024) == 1 and form([24] * 9, 3000, 2560) == 2 and form([4, 4], 512, 100) == 15 and form([2] * 300, 48, 128) == 15
+    assert form([0, 0], 512, 128) == -2 and form([-1, 4], 512, 128) == -2 and lib.mdy_fp8_grouped_gemm_form(None, 2, 512, 128) == -1
