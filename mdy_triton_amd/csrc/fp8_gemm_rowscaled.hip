@@ -199,8 +199,11 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
 //   form writes the output, M x N.
 // Fits to 150 shapes of 512..8192 rows and columns and 1 to 128 K blocks, rms error 3-6 % (slabs 9 %).  Against lines between sizes: 5.5 %
 // less time in the mean, up to 1.41 times as fast (7296x2176x1792), the worst 4 % behind (5120x640x7424 46.3 -> 48.5); 4096x7168 and
-// 4096x4096 at any K stay on 256x256 tiles.  Up to 2 K blocks, and up to 4 where 128x128 tiles need two workgroups per
-// CU, the plain loop's shorter ends win (640x7680x256 5.8 us against 7.1, 1792x3072x384 7.4 / 8.4, 2816x768x256 5.0 / 5.3).
+// 4096x4096 from 2 K blocks on stay on 256x256 tiles.  Up to 2 K blocks, and up to 4 where 128x128 tiles need two workgroups per
+// CU, the plain loop's shorter ends win (640x7680x256 5.8 us against 7.1, 1792x3072x384 7.4 / 8.4, 2816x768x256 5.0 / 5.3).  With one K
+// block they do so for any number of tiles (against 256x256: 6400x8064 23.9 us / 28.6, 4224x4096 11.6 / 14.5, 5504x2048 8.2 / 8.9; two
+// 128x128 per CU are never ahead, 6656x3456 12.7 / 14.3), but where its rounds of two workgroups per CU are twice as many as those of
+// 256x256 tiles and the last is hardly begun (5504x4736 15.3 / 14.8, 5248x4992 15.2 / 14.7, 5504x5504 16.0 / 16.9).
 enum { kPlainLoop = 0, kTiles128x256 = 1, kTiles256x256 = 2, kTiles128Ring3 = 3, kTiles128Two = 4 };
 struct RowscaledPlan {
     int config, slabs, kb_per;
@@ -210,6 +213,10 @@ static RowscaledPlan plan_rowscaled(int64_t M, int64_t N, int64_t K, bool slabs)
                   big = ((M + 255) / 256) * ((N + 255) / 256);
     RowscaledPlan p{kPlainLoop, 1, (int)KB};
     if (K > (1 << 16) || (small <= 2 * cus && (KB <= 2 || (KB <= 4 && small > cus)))) return p;
+    if (KB == 1) {
+        if (2 * ((big + cus - 1) / cus) <= (small + 2 * cus - 1) / (2 * cus) && (small - 1) % (2 * cus) < cus * 3 / 4) p.config = kTiles256x256;
+        return p;
+    }
     const double kb = (double)KB, out = (double)M * (double)N * 1e-6;
     const int64_t per_cu = (small + cus - 1) / cus;
     double best = 2.96 + kb * (double)(per_cu / 2) * 1.284 + kb * (double)(per_cu % 2) * 0.82 + 0.283 * out;

@@ -63,7 +63,7 @@ def test_act_quant_block_leading_dims_and_asserts():
 
 
 @pytest.mark.parametrize("M,N,K", [(128, 128, 128), (256, 384, 512), (130, 200, 384), (1000, 260, 1024), (64, 64, 2304),
-                                   (2048, 3328, 256), (1990, 3300, 384)])        # the last two: 128x256 tiles of the scheduled body
+                                   (2048, 3328, 256), (1990, 3300, 384)])        # the last two: the plain loop, most of a round and more
 def test_rowscaled_gemm_exact_integer(M, N, K):
     """Integer operands and power-of-two scales on both sides: every product and sum is exact, so the bf16 result must
     equal the float64 computation rounded once (catches swapped scale roles, K-block order, tile edges)."""

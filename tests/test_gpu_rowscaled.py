@@ -3,6 +3,7 @@ product and partial sum exact in fp32, so any order of summation gives the float
 import pytest
 import torch
 
+from mdy_triton_amd import _lib
 from mdy_triton_amd import fp8_kernel as FK
 
 pytestmark = pytest.mark.gpu
@@ -24,12 +25,27 @@ def exact_case(M, N, K, fmt, transposed_scales):
     assert torch.equal(got, ref.float().bfloat16())
 
 
+# MDY_FORM_...: 128x128 tiles alone on a CU and two per CU, 128x256, 256x256, the plain loop
+RING3, TWO, T128X256, T256X256, PLAIN = 7, 8, 10, 12, 14
+
+
+def runs(M, N, K, form, workspace=1):
+    """The kernel that a case means, so that a later rule cannot send it elsewhere unnoticed; (form, slabs of K)."""
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        got = _lib.load().mdy_fp8_gemm_rowscaled_form(M, N, K, workspace)
+        assert got & 255 == form, (M, N, K, got)
+        return got >> 8
+
+
 @pytest.mark.parametrize("fmt", [0, 1])
-@pytest.mark.parametrize("M,N,K", [(4090, 3336, 384),      # 256x256 tiles, one round, ragged rows and columns
-                                   (4352, 4360, 128),      # 256x256 tiles, more than one per CU, one K block
-                                   (130, 1032, 640),       # 128x256 tiles
-                                   (250, 1036, 512)])      # the plain loop
-def test_exact_integer(M, N, K, fmt):
+@pytest.mark.parametrize("M,N,K,form", [(4090, 3336, 384, T256X256),      # one round, ragged rows and columns
+                                        (4358, 5519, 256, T256X256),      # more than one per CU: LDS handed from tile to tile; odd N
+                                        (644, 5433, 640, T128X256), (3074, 4879, 640, T128X256),      # less than a round, more than one
+                                        (250, 1036, 256, PLAIN), (1990, 3300, 384, PLAIN),
+                                        (4352, 4360, 128, PLAIN), (5504, 4735, 128, T256X256),       # one K block, several rounds
+                                        (130, 1032, 640, TWO), (250, 1036, 512, TWO)])
+def test_exact_integer(M, N, K, form, fmt):
+    assert not runs(M, N, K, form)
     exact_case(M, N, K, fmt, transposed_scales=bool(fmt))
 
 
@@ -38,22 +54,24 @@ def test_exact_integer(M, N, K, fmt):
 @pytest.mark.parametrize("M,N,K", [(512, 512, 4096), (1000, 1020, 4224), (130, 257, 9600), (1536, 1536, 5120),
                                    (1530, 640, 4736), (2176, 638, 8576)])      # counts that 8 does not divide, short and long slabs
 def test_exact_integer_cut_along_k(M, N, K, transposed_scales, fmt):
-    from mdy_triton_amd import _lib
-    assert _lib.load().mdy_fp8_gemm_rowscaled_workspace_bytes(M, N, K) >= 2 * M * N * 4
+    slabs = runs(M, N, K, T128X256)
+    assert slabs is None or slabs >= 2
     exact_case(M, N, K, fmt, transposed_scales)
 
 
 @pytest.mark.parametrize("fmt", [0, 1])
-@pytest.mark.parametrize("M,N,K", [(890, 3712, 3072), (250, 1036, 1664), (1000, 2301, 896),      # 128x128 tiles, ring of 3: one tile per CU at most
-                                   (2550, 3190, 1024), (7290, 2170, 640), (770, 260, 384), (512, 640, 512)])      # two workgroups per CU
-def test_exact_integer_128x128_tiles(M, N, K, fmt):
+@pytest.mark.parametrize("M,N,K,form", [(890, 3712, 3072, RING3), (250, 1036, 1664, RING3), (1000, 2301, 896, RING3),
+                                        (2550, 3190, 1024, TWO), (7290, 2170, 640, TWO), (770, 260, 384, TWO), (512, 640, 512, TWO)])
+def test_exact_integer_128x128_tiles(M, N, K, form, fmt):
+    assert not runs(M, N, K, form)
     exact_case(M, N, K, fmt, transposed_scales=bool(fmt))
 
 
-@pytest.mark.parametrize("M,N,K", [(890, 1028, 3072), (300, 700, 512), (2550, 3190, 1024)])
-def test_exact_integer_128x128_tiles_fp32(M, N, K):
-    from mdy_triton_amd import _lib
+@pytest.mark.parametrize("M,N,K,form", [(890, 1028, 3072, RING3), (300, 700, 512, TWO), (2550, 3190, 1024, TWO),
+                                        (644, 5433, 640, T128X256), (4090, 3336, 384, T256X256), (250, 1036, 256, PLAIN)])
+def test_exact_integer_fp32(M, N, K, form):
     lib = _lib.load()
+    runs(M, N, K, form, workspace=0)
     g = torch.Generator().manual_seed(M + N)
     ai, bi = (torch.randint(-2, 3, (r, K), generator=g) for r in (M, N))
     a, b = (v.float().to(torch.float8_e4m3fn).to(DEV) for v in (ai, bi))
