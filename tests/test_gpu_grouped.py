@@ -74,12 +74,26 @@ def call_f32(qa, sa, qb, sb, m_splits):
     return out
 
 
-@pytest.mark.parametrize("m_splits,N,K", [([256, 512, 0, 256], 520, 384),          # all multiples of 256: 256x256 tiles
-                                          ([100, 0, 1, 300, 129, 128], 776, 256),  # ragged groups: 128x256 last tiles, tails everywhere
-                                          ([384, 640, 129, 257, 0, 900, 128, 1], 776, 640),   # 256-row tiles + a 128-row last tile
-                                          ([16] * 32, 2048, 512),                  # decode-like: many tiny groups
-                                          ([3, 5], 40, 128)])
-def test_grouped_gemm_exact_integer(m_splits, N, K):
+# MDY_FORM_...: the small-row kernels, whole tiles of 256x256, what is left of a round in pieces, pieces alone
+LINES, STRIP, TILES, REST128, REST192, REST256, PIECES128, PIECES192 = 1, 2, 12, 16, 17, 18, 19, 20
+
+
+def runs(m_splits, N, K, form):
+    """The kernel that a case means, so that a later rule cannot send it elsewhere unnoticed."""
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        import ctypes
+        arr = (ctypes.c_int64 * len(m_splits))(*m_splits)
+        got = _lib.load().mdy_fp8_grouped_gemm_form(ctypes.cast(arr, ctypes.c_void_p), len(m_splits), N, K)
+        assert got == form, (m_splits, N, K, got)
+
+
+@pytest.mark.parametrize("m_splits,N,K,form", [([256, 512, 0, 256], 520, 384, REST128),          # all multiples of 256
+                                               ([100, 0, 1, 300, 129, 128], 776, 256, REST128),  # ragged groups, tails everywhere
+                                               ([384, 640, 129, 257, 0, 900, 128, 1], 776, 640, REST128),
+                                               ([16] * 32, 2048, 512, LINES),                    # decode-like: many tiny groups
+                                               ([3, 5], 40, 128, LINES)])
+def test_grouped_gemm_exact_integer(m_splits, N, K, form):
+    runs(m_splits, N, K, form)
     exact_grouped_case(m_splits, N, K, sum(m_splits) + N + K, call_f32)
 
 
@@ -87,26 +101,33 @@ def call_bf16(qa, sa, qb, sb, m_splits):
     return m.fp8_grouped_matmul(qa, sa, qb, sb, list(m_splits))
 
 
-@pytest.mark.parametrize("m_splits,N,K,pieces", [([256] * 17 + [130, 1, 257], 3848, 640, 2),     # 21 x 16 tiles: a round and 80 in halves
-                                                 ([256] * 16 + [130, 1, 257], 3848, 640, 4),     # 20 x 16: exactly a quarter of a round
-                                                 ([256] * 16 + [130, 0, 200], 3841, 384, 4),     # odd N: stores straight from registers
-                                                 ([256] * 18 + [300, 70, 128], 3904, 384, 2),    # 22 x 16: in halves, rows on whole lines
-                                                 ([256] * 21 + [300, 70, 128], 3904, 128, 1),    # 25 x 16: more than half a round left
-                                                 ([129, 70, 255, 256], 2300, 1152, 4),           # less than a round: 4 x 9 in quarters
-                                                 ([300, 256, 0, 520, 1000, 77], 2304, 512, 2)])  # 11 x 9 in halves
-def test_grouped_gemm_exact_integer_pieces_of_the_last_round(m_splits, N, K, pieces):
-    """Tiles of a last round that would leave CUs idle run in halves or quarters: edges of groups, columns and pieces."""
-    tiles, cus = sum(-(-v // 256) for v in m_splits) * -(-N // 256), torch.cuda.get_device_properties(0).multi_processor_count
-    if cus == 256:
-        left = tiles % cus
-        assert pieces == (1 if left == 0 or 2 * left > cus else 2 if 4 * left > cus else 4)
+@pytest.mark.parametrize("m_splits,N,K,form", [([256] * 17 + [130, 1, 257], 3848, 640, REST192),     # 21 x 16 tiles: a round and 80
+                                               ([256] * 16 + [130, 1, 257], 3848, 640, REST128),     # 20 x 16: a round and a quarter
+                                               ([256] * 16 + [130, 0, 200], 3841, 384, REST128),     # odd N: stores straight from registers
+                                               ([256] * 18 + [300, 70, 128], 3904, 384, REST192),    # 22 x 16, rows on whole lines
+                                               ([256] * 21 + [300, 70, 128], 3904, 128, TILES),      # 25 x 16: more than half a round left
+                                               ([257, 0, 385, 90] * 3, 2305, 640, TILES),            # 15 x 10, last tile rows of 1, 129 and 90 rows
+                                               ([129, 70, 255, 256], 2300, 1152, REST128),           # less than a round: 4 x 9
+                                               ([300, 256, 0, 520, 1000, 77], 2304, 512, PIECES192),
+                                               # 24 x 16: half a round in halves of a tile, too many for 192 columns; second halves that
+                                               # are empty (300, 70) or short (200); rows on whole lines, inside lines, odd N
+                                               ([256] * 20 + [300, 200, 70], 3904, 640, REST256),
+                                               ([256] * 20 + [300, 200, 70], 3848, 384, REST256),
+                                               ([256] * 20 + [300, 200, 70], 3841, 256, REST256),
+                                               ([300, 256, 0, 200] * 5, 1400, 384, REST256)])        # less than a round: 20 x 6
+def test_grouped_gemm_exact_integer_pieces_of_the_last_round(m_splits, N, K, form):
+    """Tiles of a last round that would leave CUs idle run in pieces: edges of groups, columns and pieces."""
+    runs(m_splits, N, K, form)
     exact_grouped_case(m_splits, N, K, 7 * sum(m_splits) + N + K, call_f32)
 
 
 def test_grouped_gemm_pieces_bf16_results_through_lds():
-    for m_splits, N in (([256] * 16 + [130, 1, 257], 3904), ([256] * 18 + [300, 70, 128], 3848), ([256] * 18 + [300, 70, 128], 3904)):
+    for m_splits, N, form in (([256] * 16 + [130, 1, 257], 3904, REST128), ([256] * 18 + [300, 70, 128], 3848, REST192),
+                              ([256] * 18 + [300, 70, 128], 3904, REST192), ([256] * 20 + [300, 200, 70], 3904, REST256),
+                              ([256] * 20 + [300, 200, 70], 3848, REST256), ([256] * 20 + [300, 200, 70], 3841, REST256)):
         g = torch.Generator().manual_seed(N)
         G, M, K = len(m_splits), sum(m_splits), 512
+        runs(m_splits, N, K, form)
         qa = torch.randint(-4, 5, (M, K), generator=g).float().to(FP8).to(DEV)
         qb = torch.randint(-4, 5, (G, N, K), generator=g).float().to(FP8).to(DEV)
         sa = torch.exp2(torch.randint(-2, 3, (M, K // 128), generator=g).float()).to(DEV)
@@ -122,12 +143,12 @@ def test_grouped_gemm_pieces_bf16_results_through_lds():
                                           ([56] * 25, 1024, 128), ([50, 64] * 13, 1000, 256),     # the same with one K block / one step
                                           ([49] * 30, 900, 640)])
 def test_grouped_gemm_exact_integer_strip_kernel(m_splits, N, K):
-    """17..64 rows in the largest group and >= 200 strips of 128 columns: the weight-streaming strip kernel runs."""
-    assert 16 < max(m_splits) <= 64 and len(m_splits) * ((N + 127) // 128) >= 200
+    """17..64 rows in the largest group and at least 144 strips of 128 columns: the weight-streaming strip kernel runs."""
+    runs(m_splits, N, K, STRIP)
     exact_grouped_case(m_splits, N, K, 3 * sum(m_splits) + N + K, call_f32)
 
 
-@pytest.mark.parametrize("m_splits,N,K", [([1, 16, 0, 7, 3, 24, 9, 2], 3001, 896),        # one or two row tiles, ragged N, 7 K blocks
+@pytest.mark.parametrize("m_splits,N,K", [([1, 16, 0, 7, 3, 24, 9, 2], 2505, 896),        # one or two row tiles, ragged N, 7 K blocks
                                           ([16] * 40, 640, 128),                          # one K block: 7 of 8 waves idle
                                           ([2] * 64, 1030, 7168),                         # routed experts at decode, 7 K blocks per wave
                                           ([33, 64, 0, 40], 2050, 1152),                  # up to 64 rows, too few strips for the strip kernel
@@ -135,24 +156,24 @@ def test_grouped_gemm_exact_integer_strip_kernel(m_splits, N, K):
                                           ([5, 0, 0, 11], 290, 9344),                     # several passes over K
                                           ([12] * 3, 515, 3072), ([20, 4], 777, 5120)])   # 3 and 5 K blocks per wave
 def test_grouped_gemm_exact_integer_whole_line_kernel(m_splits, N, K):
-    """At most 16 rows in the largest group, or at most 64 with fewer than 144 strips: every group is a small-M GEMM of
-    the whole-line kernel (one grid row per group, empty groups return at once)."""
-    strips = len(m_splits) * ((N + 127) // 128)
-    assert max(m_splits) <= 16 or (max(m_splits) <= 64 and strips < 200)
+    """At most 16 rows in the largest group, or at most 64 with fewer than 144 strips and outside of the range of pieces: every group is
+    a small-M GEMM of the whole-line kernel (one grid row per group, empty groups return at once)."""
+    runs(m_splits, N, K, LINES)
     exact_grouped_case(m_splits, N, K, 5 * sum(m_splits) + N + K, call_f32)
 
 
-@pytest.mark.parametrize("m_splits,N,K", [([9, 0, 16, 1], 515, 2304), ([3] * 9, 300, 3072),    # 3 K blocks per wave: 18 and all 24
-                                          ([16, 5], 700, 4736), ([2, 0, 13], 260, 5888),       # 5 (37 of 40) and 6 (46 of 48)
-                                          ([7, 1], 130, 9216),                                 # 9 as 2 passes of 5
-                                          ([17, 32, 3], 515, 2304), ([20, 4], 391, 4224),      # up to 32 rows: 3; 5 as 2 passes of 3
-                                          ([31, 0, 18], 140, 6144), ([19, 2], 100, 7168),      # 6 as 2 of 3; 7 as 2 of 4
-                                          ([32] * 9, 2044, 640), ([17, 33, 64, 20] * 4, 1152, 640),     # 144 strips: the strip kernel
-                                          # pieces of 128 rows: two rounds of strips, 80 strips, 144 strips
-                                          ([20, 64, 0, 33] * 8, 1500, 1152), ([17, 32] * 9, 1920, 1664), ([40, 0, 64] * 4, 1250, 1024),
-                                          ([64] * 8, 2304, 2048)])
-def test_grouped_gemm_exact_integer_pass_depths_and_first_strips(m_splits, N, K):
+@pytest.mark.parametrize("m_splits,N,K,form", [([9, 0, 16, 1], 515, 2304, LINES), ([3] * 9, 300, 3072, LINES),    # 3 K blocks per wave: 18 and all 24
+                                               ([16, 5], 700, 4736, LINES), ([2, 0, 13], 260, 5888, LINES),      # 5 (37 of 40) and 6 (46 of 48)
+                                               ([7, 1], 130, 9216, LINES),                                       # 9 as 2 passes of 5
+                                               ([17, 32, 3], 515, 2304, LINES), ([20, 4], 391, 4224, LINES),     # up to 32 rows: 3; 5 as 2 passes of 3
+                                               ([31, 0, 18], 140, 6144, LINES), ([19, 2], 100, 7168, LINES),     # 6 as 2 of 3; 7 as 2 of 4
+                                               ([32] * 9, 2044, 640, STRIP), ([17, 33, 64, 20] * 4, 1152, 640, STRIP),     # 144 strips
+                                               # pieces of 128 rows: two rounds of strips, 80 strips, 144 strips
+                                               ([20, 64, 0, 33] * 8, 1500, 1152, PIECES192), ([17, 32] * 9, 1920, 1664, PIECES192),
+                                               ([40, 0, 64] * 4, 1250, 1024, REST128), ([64] * 8, 2304, 2048, PIECES128)])
+def test_grouped_gemm_exact_integer_pass_depths_and_first_strips(m_splits, N, K, form):
     """Depths of a pass of the whole-line kernel that fill up the last one or not, and the fewest strips of the strip kernel."""
+    runs(m_splits, N, K, form)
     exact_grouped_case(m_splits, N, K, 7 * sum(m_splits) + N + K, call_f32)
 
 

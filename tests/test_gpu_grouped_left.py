@@ -7,24 +7,28 @@ import torch
 
 import mdy_triton_amd as m
 from mdy_triton_amd import _lib
+from tests.test_gpu_grouped import PIECES128, PIECES192, REST128, REST192, REST256, TILES, runs
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-# rows per group, N, K: pieces of 128 columns (less than a quarter round), of 192 (up to 3/8), behind a whole round, ragged rows and
-# columns, empty groups, a group that ends within the first half of a tile row, rows that start inside lines
-CASES = [([256, 300, 0, 1], 520, 384), ([100, 70, 513], 1032, 640), ([129] * 7, 264, 256),
-         ([700, 1, 0, 900, 411], 1536, 384), ([256] * 11, 1800, 256), ([2000, 130, 640], 1544, 128), ([300] * 9, 1100, 384),
-         ([640] * 7, 4096, 256), ([1000, 3000, 129, 1], 4104, 384), ([512, 700] * 4, 3848, 128), ([2500, 2500, 388], 4100, 256),
+# rows per group, N, K, kernel: pieces of 128 columns (less than a quarter round), of 192 (up to 3/8), behind a whole round, ragged rows
+# and columns, empty groups, a group that ends within the first half of a tile row, rows that start inside lines
+CASES = [([256, 300, 0, 1], 520, 384, REST128), ([100, 70, 513], 1032, 640, REST128), ([129] * 7, 264, 256, REST128),
+         ([700, 1, 0, 900, 411], 1536, 384, REST128), ([256] * 11, 1800, 256, REST192), ([2000, 130, 640], 1544, 128, REST192),
+         ([640] * 7, 4096, 256, REST192), ([1000, 3000, 129, 1], 4104, 384, REST128), ([512, 700] * 4, 3848, 128, REST128),
+         ([2500, 2500, 388], 4100, 256, REST256),      # too many pieces for 192 columns: halves of tiles
          # counted by pieces of 128 rows, of 128 columns and of 192: groups of one piece, two and three, empty and of one row
-         ([70, 128, 1, 0, 129, 300, 90, 65] * 2, 2050, 256), ([100] * 16, 2044, 384), ([66] * 32, 900, 640), ([128, 70] * 8, 3070, 256),
-         ([257, 0, 385, 90] * 3, 2305, 128)]
+         ([300] * 9, 1100, 384, PIECES128), ([70, 128, 1, 0, 129, 300, 90, 65] * 2, 2050, 256, PIECES192), ([100] * 16, 2044, 384, PIECES128),
+         ([66] * 32, 900, 640, PIECES128), ([128, 70] * 8, 3070, 256, PIECES192), ([257, 0, 385, 90] * 3, 1905, 128, PIECES192),
+         ([257, 0, 385, 90] * 3, 2305, 128, TILES)]
 
 
-@pytest.mark.parametrize("rows,N,K", CASES)
+@pytest.mark.parametrize("rows,N,K,form", CASES)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-def test_exact_integer(rows, N, K, dtype):
+def test_exact_integer(rows, N, K, form, dtype):
+    runs(rows, N, K, form)
     g = torch.Generator(device=DEV).manual_seed(sum(rows) + N + K)
     M, G, KB, NB = sum(rows), len(rows), K // 128, (N + 127) // 128
     ai, bi = torch.randint(-3, 4, (M, K), generator=g, device=DEV), torch.randint(-3, 4, (G, N, K), generator=g, device=DEV)
