@@ -194,3 +194,11 @@ def test_form_queries(lib):
     form = lambda rows, N, K: lib.mdy_fp8_grouped_gemm_form((ctypes.c_int64 * len(rows))(*rows), len(rows), N, K)
     assert form([1, 0, 7], 512, 1024) == 1 and form([24] * 9, 3000, 2560) == 2 and form([4, 4], 512, 100) == 15 and form([2] * 300, 48, 128) == 15
     assert form([0, 0], 512, 128) == -2 and form([-1, 4], 512, 128) == -2 and lib.mdy_fp8_grouped_gemm_form(None, 2, 512, 128) == -1
+
+
+@pytest.mark.parametrize("M,N,K,tiles", [(59, 6464, 2176, False), (47, 6837, 2432, False), (22, 10112, 1280, False), (28, 8704, 640, False),
+                                         (48, 4352, 640, False), (30, 15552, 2176, True), (25, 15040, 4608, True), (33, 8256, 2688, True),
+                                         (42, 6144, 1152, True)])
+def test_small_rows_leave_the_whole_line_kernel_where_its_rounds_cost(lib, M, N, K, tiles):
+    """17 to 64 rows: tiles in one launch only where the whole-line kernel needs another round or pass (256 CUs)."""
+    assert (lib.mdy_fp8_gemm_form(M, N, K, 1) == 1) != tiles
