@@ -13,8 +13,8 @@ pytestmark = pytest.mark.gpu
                                    (777, 7168, 1024), (1100, 6000, 1024),                        # 128x256
                                    (4097, 4400, 128), (3752, 15224, 256), (5000, 5000, 128),     # 256x256, walked
                                    (777, 2112, 4096), (200, 1100, 4096), (100, 1000, 7168),      # cut along K
-                                   # (slab, tile) counts that 8 does not divide: slabs of 9 and 10 K blocks, of 12 against a long K, of 16
-                                   (771, 896, 5632), (631, 760, 7808), (219, 704, 13568), (314, 1150, 13824), (130, 2624, 12160)])
+                                   # (slab, tile) counts that 8 does not divide: slabs of 9 and 10 K blocks, of 12 against a long K, of 16, of 9 against a long K
+                                   (771, 896, 5632), (631, 760, 7808), (219, 704, 13568), (314, 1150, 13824), (130, 2624, 12160), (164, 1280, 11264)])
 def test_exact_integer(M, N, K):
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     KB, NB = K // 128, -(-N // 128)
