@@ -202,3 +202,13 @@ def test_form_queries(lib):
 def test_small_rows_leave_the_whole_line_kernel_where_its_rounds_cost(lib, M, N, K, tiles):
     """17 to 64 rows: tiles in one launch only where the whole-line kernel needs another round or pass (256 CUs)."""
     assert (lib.mdy_fp8_gemm_form(M, N, K, 1) == 1) != tiles
+
+
+def grouped_form(lib, rows, N, K):
+    return lib.mdy_fp8_grouped_gemm_form((ctypes.c_int64 * len(rows))(*rows), len(rows), N, K)
+
+
+def test_grouped_form_of_33_to_64_rows(lib):
+    """Fewer than 144 strips: the whole-line kernel, which reads weights from HBM faster than pieces of 128 rows do."""
+    assert grouped_form(lib, [45] * 8, 1344, 1792) == grouped_form(lib, [58] * 4, 2880, 2048) == grouped_form(lib, [40] * 4, 2688, 1024) == 1
+    assert grouped_form(lib, [33] * 8, 2752, 1408) == 19 and grouped_form(lib, [64] * 8, 2304, 2048) == 19 and grouped_form(lib, [33] * 8, 2752, 2304) == 2

@@ -168,9 +168,9 @@ def test_grouped_gemm_exact_integer_whole_line_kernel(m_splits, N, K):
                                                ([17, 32, 3], 515, 2304, LINES), ([20, 4], 391, 4224, LINES),     # up to 32 rows: 3; 5 as 2 passes of 3
                                                ([31, 0, 18], 140, 6144, LINES), ([19, 2], 100, 7168, LINES),     # 6 as 2 of 3; 7 as 2 of 4
                                                ([32] * 9, 2044, 640, STRIP), ([17, 33, 64, 20] * 4, 1152, 640, STRIP),     # 144 strips
-                                               # pieces of 128 rows: two rounds of strips, 80 strips, 144 strips
+                                               # pieces of 128 rows: two rounds of strips, 144 strips; fewer strips: lines
                                                ([20, 64, 0, 33] * 8, 1500, 1152, PIECES192), ([17, 32] * 9, 1920, 1664, PIECES192),
-                                               ([40, 0, 64] * 4, 1250, 1024, REST128), ([64] * 8, 2304, 2048, PIECES128)])
+                                               ([40, 0, 64] * 4, 1250, 1024, LINES), ([64] * 8, 2304, 2048, PIECES128)])
 def test_grouped_gemm_exact_integer_pass_depths_and_first_strips(m_splits, N, K, form):
     """Depths of a pass of the whole-line kernel that fill up the last one or not, and the fewest strips of the strip kernel."""
     runs(m_splits, N, K, form)
