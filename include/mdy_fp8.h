@@ -364,6 +364,7 @@ int mdy_fp8_gemm_path(const void* a, const void* b, int64_t as_row_stride, int64
 #define MDY_FORM_REST_128X256 18
 #define MDY_FORM_PIECES_128 19
 #define MDY_FORM_PIECES_192 20
+#define MDY_FORM_REST_QUARTERS 21 /* whole tiles in four pieces of 128x128 */
 int mdy_fp8_gemm_form(int64_t M, int64_t N, int64_t K, int with_workspace);
 int mdy_fp8_gemm_rowscaled_form(int64_t M, int64_t N, int64_t K, int with_workspace);
 int mdy_fp8_grouped_gemm_form(const int64_t* m_splits, int64_t G, int64_t N, int64_t K);

@@ -212,3 +212,9 @@ def test_grouped_form_of_33_to_64_rows(lib):
     """Fewer than 144 strips: the whole-line kernel, which reads weights from HBM faster than pieces of 128 rows do."""
     assert grouped_form(lib, [45] * 8, 1344, 1792) == grouped_form(lib, [58] * 4, 2880, 2048) == grouped_form(lib, [40] * 4, 2688, 1024) == 1
     assert grouped_form(lib, [33] * 8, 2752, 1408) == 19 and grouped_form(lib, [64] * 8, 2304, 2048) == 19 and grouped_form(lib, [33] * 8, 2752, 2304) == 2
+
+
+def test_grouped_form_of_a_quarter_round(lib):
+    """Up to a quarter of a round behind whole ones, in whole tile rows more than a round of 128-column pieces: quarters of tiles."""
+    assert grouped_form(lib, [104] * 32, 4608, 896) == grouped_form(lib, [256] * 12 + [300, 70, 200], 5056, 256) == 21
+    assert grouped_form(lib, [256] * 16 + [130, 1, 257], 3848, 640) == 16 and grouped_form(lib, [256] * 17 + [130, 1, 257], 3848, 640) == 17

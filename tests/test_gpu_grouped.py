@@ -75,7 +75,7 @@ def call_f32(qa, sa, qb, sb, m_splits):
 
 
 # MDY_FORM_...: the small-row kernels, whole tiles of 256x256, what is left of a round in pieces, pieces alone
-LINES, STRIP, TILES, REST128, REST192, REST256, PIECES128, PIECES192 = 1, 2, 12, 16, 17, 18, 19, 20
+LINES, STRIP, TILES, REST128, REST192, REST256, PIECES128, PIECES192, QUARTERS = 1, 2, 12, 16, 17, 18, 19, 20, 21
 
 
 def runs(m_splits, N, K, form):

@@ -7,7 +7,7 @@ import torch
 
 import mdy_triton_amd as m
 from mdy_triton_amd import _lib
-from tests.test_gpu_grouped import PIECES128, PIECES192, REST128, REST192, REST256, TILES, runs
+from tests.test_gpu_grouped import PIECES128, PIECES192, QUARTERS, REST128, REST192, REST256, TILES, runs
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -19,6 +19,12 @@ CASES = [([256, 300, 0, 1], 520, 384, REST128), ([100, 70, 513], 1032, 640, REST
          ([700, 1, 0, 900, 411], 1536, 384, REST128), ([256] * 11, 1800, 256, REST192), ([2000, 130, 640], 1544, 128, REST192),
          ([640] * 7, 4096, 256, REST192), ([1000, 3000, 129, 1], 4104, 384, REST128), ([512, 700] * 4, 3848, 128, REST128),
          ([2500, 2500, 388], 4100, 256, REST256),      # too many pieces for 192 columns: halves of tiles
+         # a round and a quarter whose left tile rows are more than a round of 128-column pieces: quarters of tiles, on whole lines, with
+         # an empty column piece, odd N; empty, short and full second rows; 33 K blocks
+         ([256] * 12 + [300, 70, 200], 5056, 256, QUARTERS), ([256] * 13 + [0, 450, 129], 4900, 128, QUARTERS),
+         ([256] * 12 + [300, 70, 256], 5111, 384, QUARTERS), ([256] * 15 + [200], 5000, 4224, QUARTERS),
+         # 128-column pieces from 32 K blocks on, of full tile rows and of half empty ones
+         ([256, 100, 300], 1300, 4224, REST128),
          # counted by pieces of 128 rows, of 128 columns and of 192: groups of one piece, two and three, empty and of one row
          ([300] * 9, 1100, 384, PIECES128), ([70, 128, 1, 0, 129, 300, 90, 65] * 2, 2050, 256, PIECES192), ([100] * 16, 2044, 384, PIECES128),
          ([66] * 32, 900, 640, PIECES128), ([128, 70] * 8, 3070, 256, PIECES192), ([257, 0, 385, 90] * 3, 1905, 128, PIECES192),
