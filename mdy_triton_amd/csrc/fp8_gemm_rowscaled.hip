@@ -15,6 +15,8 @@
 // ... lds`, double buffered, one barrier per K block: short ends, but 0.93 us per K block against 0.72) runs what has few K blocks.
 // K % 128 == 0 (the callers contract over a padded token count).
 #include "../../include/mdy_fp8.h"
+#include <algorithm>
+
 #include "fp8_gemm_tile.h"
 
 namespace mdy {
@@ -197,9 +199,9 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
 //   128x128 tiles, ring of 3, one per CU; two per CU, a tile alone on its CU or a pair of them per K block; 128x256 and 256x256 tiles
 //   in rounds of the CUs (a round takes its time whether it is full or not); slabs of 128x256 tiles and their reduction.  Every
 //   form writes the output, M x N.
-// Fits to 150 shapes of 512..8192 rows and columns and 1 to 128 K blocks, rms error 3-6 % (slabs 9 %).  Against lines between sizes: 5.5 %
-// less time in the mean, up to 1.41 times as fast (7296x2176x1792), the worst 4 % behind (5120x640x7424 46.3 -> 48.5); 4096x7168 and
-// 4096x4096 from 2 K blocks on stay on 256x256 tiles.  Up to 2 K blocks, and up to 4 where 128x128 tiles need two workgroups per
+// Fits to 150 shapes of 512..8192 rows and columns and 1 to 128 K blocks, rms error 3-6 % (slabs 9 %).  Against lines between sizes, 250 other
+// shapes: 6 % less time in the mean, up to 1.41 times as fast (7296x2176x1792), two of them more than 5 % behind out of the
+// caches (3328x512x3456 25.2 -> 27.7 us); 4096x7168 and 4096x4096 from 2 K blocks on stay on 256x256 tiles.  Up to 2 K blocks, and up to 4 where 128x128 tiles need two workgroups per
 // CU, the plain loop's shorter ends win (640x7680x256 5.8 us against 7.1, 1792x3072x384 7.4 / 8.4, 2816x768x256 5.0 / 5.3).  With one K
 // block they do so for any number of tiles (against 256x256: 6400x8064 23.9 us / 28.6, 4224x4096 11.6 / 14.5, 5504x2048 8.2 / 8.9; two
 // 128x128 per CU are never ahead, 6656x3456 12.7 / 14.3), but where its rounds of two workgroups per CU are twice as many as those of
@@ -231,11 +233,21 @@ static RowscaledPlan plan_rowscaled(int64_t M, int64_t N, int64_t K, bool slabs)
     consider(kTiles128x256, 1, KB, 1.66 + (double)((wide + cus - 1) / cus) * (1.015 * kb + 2.09) + 0.262 * out);
     consider(kTiles256x256, 1, KB, 1.46 + (double)((big + cus - 1) / cus) * (1.703 * kb + 2.16) + 0.227 * out);
     best *= 1.05;      // ties go to slabs
+    // how many slabs: a K block takes a workgroup 1.0 us, a slab's traffic 1.333 us per million results.  The counts of the estimate that says
+    // whether to cut promise up to 5 % less, which is within its error: over 65 shapes that it cut into fewer slabs 1.1 % less time with operands
+    // in the caches, 1.1 % more without, up to 17 % (768x640x8192 22.7 us with 11, 26.5 with 8)
+    double slabs_us = best, least = 1e30;
+    RowscaledPlan cut = p;
     for (int64_t want = 2; slabs && want <= 16 && wide * want <= cus && KB / want >= 4; ++want) {
         const int64_t per = (KB + want - 1) / want, n = (KB + per - 1) / per;
-        consider(kTiles128x256, n, per, 8.22 + (double)per * (0.98 - 0.187 * (double)(wide * n) / (double)cus) + 1.857 * (double)n * out);
+        slabs_us = std::min(slabs_us, 8.22 + (double)per * (0.98 - 0.187 * (double)(wide * n) / (double)cus) + 1.857 * (double)n * out);
+        const double cost = (double)per + 1.333 * (double)want * out;
+        if (cost < least) {
+            least = cost;
+            cut = RowscaledPlan{kTiles128x256, (int)n, (int)per};
+        }
     }
-    return p;
+    return slabs_us < best ? cut : p;
 }
 int64_t fp8_gemm_rowscaled_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     const RowscaledPlan p = plan_rowscaled(M, N, K, true);

@@ -218,3 +218,9 @@ def test_grouped_form_of_a_quarter_round(lib):
     """Up to a quarter of a round behind whole ones, in whole tile rows more than a round of 128-column pieces: quarters of tiles."""
     assert grouped_form(lib, [104] * 32, 4608, 896) == grouped_form(lib, [256] * 12 + [300, 70, 200], 5056, 256) == 21
     assert grouped_form(lib, [256] * 16 + [130, 1, 257], 3848, 640) == 16 and grouped_form(lib, [256] * 17 + [130, 1, 257], 3848, 640) == 17
+
+
+def test_rowscaled_slab_counts(lib):
+    """Slabs of K of the row-scaled GEMM (kernel 10, 128x256 tiles): the counts in use before its times were estimated."""
+    for shape, slabs in (((768, 640, 8192), 11), ((1536, 768, 4480), 5), ((512, 1152, 5248), 7), ((1152, 640, 7680), 9), ((1024, 1024, 8192), 8)):
+        assert lib.mdy_fp8_gemm_rowscaled_form(*shape, 1) == 10 | slabs << 8, shape
