@@ -224,3 +224,11 @@ def test_rowscaled_slab_counts(lib):
     """Slabs of K of the row-scaled GEMM (kernel 10, 128x256 tiles): the counts in use before its times were estimated."""
     for shape, slabs in (((768, 640, 8192), 11), ((1536, 768, 4480), 5), ((512, 1152, 5248), 7), ((1152, 640, 7680), 9), ((1024, 1024, 8192), 8)):
         assert lib.mdy_fp8_gemm_rowscaled_form(*shape, 1) == 10 | slabs << 8, shape
+
+
+def test_short_calls_are_not_cut_by_an_estimate(lib):
+    """What one launch finishes in less than the host takes for a second one stays in one launch (256 CUs)."""
+    for shape in ((19, 576, 7424), (30, 576, 7552), (68, 384, 2048), (163, 384, 2176)):
+        assert lib.mdy_fp8_gemm_form(*shape, 1) >> 8 == 0, shape
+    for shape in ((20, 768, 10112), (109, 1280, 2560), (64, 832, 4096)):
+        assert lib.mdy_fp8_gemm_form(*shape, 1) >> 8 > 1, shape

@@ -11,12 +11,14 @@ from test_gpu_gemm import test_gemm_exact_integer_cases_all_kernels as exact_int
 WHOLE_LINES, T64X64, T64X128 = 1, 4, 5      # MDY_FORM_...
 # (M, N, K), form, slabs of K (0: one launch)
 FORMS = [((17, 5001, 512), WHOLE_LINES, 0), ((64, 7168, 2048), WHOLE_LINES, 0), ((17, 2050, 7168), WHOLE_LINES, 0),
-         ((17, 12802, 256), T64X64, 0), ((64, 16384, 128), T64X64, 0), ((33, 10945, 1280), T64X64, 0), ((64, 18181, 2816), T64X128, 0),
+         ((17, 14802, 256), T64X64, 0), ((64, 16384, 128), T64X64, 0), ((33, 10945, 1280), T64X64, 0), ((64, 18181, 2816), T64X128, 0),
          ((63, 18180, 640), T64X128, 0), ((63, 3001, 6528), T64X64, 5), ((64, 8900, 7168), T64X128, 3), ((17, 1537, 16384), T64X64, 8),
          ((40, 1025, 9088), WHOLE_LINES, 7), ((18, 9665, 6912), T64X128, 3), ((64, 9000, 7168), T64X128, 3), ((20, 4998, 11520), T64X128, 6),
          # where the lines between sizes and an estimate disagree by less than the estimate's error: the lines' form
          ((34, 4096, 8192), T64X64, 4), ((50, 512, 4992), WHOLE_LINES, 4), ((60, 1792, 6272), WHOLE_LINES, 4),
-         ((34, 832, 4864), WHOLE_LINES, 4), ((64, 1536, 4096), WHOLE_LINES, 4), ((64, 1536, 3968), WHOLE_LINES, 0)]
+         ((34, 832, 4864), WHOLE_LINES, 4), ((64, 1536, 4096), WHOLE_LINES, 4), ((64, 1536, 3968), WHOLE_LINES, 0),
+         # what one launch finishes before the host has enqueued a second
+         ((19, 576, 7424), WHOLE_LINES, 0), ((20, 768, 10112), WHOLE_LINES, 5)]
 
 
 @pytest.mark.parametrize("shape,form,slabs", FORMS)
@@ -45,7 +47,7 @@ def test_exact_integer(shape):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(33, 10944, 1280), (64, 9000, 7168), (17, 12801, 256)])
+@pytest.mark.parametrize("M,N,K", [(33, 10944, 1280), (64, 9000, 7168), (17, 14801, 256)])
 def test_e5m2_and_bias(M, N, K):
     """The same routes with e5m2 bytes and a bias (in the epilogue of one launch, in the reduction of slabs)."""
     g = torch.Generator().manual_seed(M + N)
