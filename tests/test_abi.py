@@ -198,7 +198,7 @@ def test_form_queries(lib):
 
 @pytest.mark.parametrize("M,N,K,tiles", [(59, 6464, 2176, False), (47, 6837, 2432, False), (22, 10112, 1280, False), (28, 8704, 640, False),
                                          (48, 4352, 640, False), (30, 15552, 2176, True), (25, 15040, 4608, True), (33, 8256, 2688, True),
-                                         (42, 6144, 1152, True)])
+                                         (64, 4928, 1792, False), (62, 6208, 3200, True)])
 def test_small_rows_leave_the_whole_line_kernel_where_its_rounds_cost(lib, M, N, K, tiles):
     """17 to 64 rows: tiles in one launch only where the whole-line kernel needs another round or pass (256 CUs)."""
     assert (lib.mdy_fp8_gemm_form(M, N, K, 1) == 1) != tiles
@@ -232,3 +232,10 @@ def test_short_calls_are_not_cut_by_an_estimate(lib):
         assert lib.mdy_fp8_gemm_form(*shape, 1) >> 8 == 0, shape
     for shape in ((20, 768, 10112), (109, 1280, 2560), (64, 832, 4096)):
         assert lib.mdy_fp8_gemm_form(*shape, 1) >> 8 > 1, shape
+
+
+def test_large_tiles_that_just_miss_a_round(lib):
+    """128x256 tiles in place of 256x256: at any K where they need no more rounds, from 16 K blocks on where they need one more (256 CUs)."""
+    assert lib.mdy_fp8_gemm_form(2383, 6656, 2176, 0) == lib.mdy_fp8_gemm_form(2841, 5632, 128, 0) == 10
+    assert lib.mdy_fp8_gemm_form(7172, 3264, 128, 0) == lib.mdy_fp8_gemm_form(1854, 12480, 1920, 0) != 10
+    assert lib.mdy_fp8_gemm_form(1854, 12480, 2048, 0) == 10
