@@ -159,8 +159,8 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_tile_kernel(
 
 // 128x128 tiles of the same body, four waves of 64x64, one tile per workgroup: for outputs that leave CUs idle with larger tiles, on a
 // ring of 3 K blocks (one workgroup per CU) or of 2 (two per CU).  It took these from the plain loop and from 128x256 tiles that ran one
-// to a CU and left others empty: 896x3712x3072 28.1 -> 20.7 us, 1536x1024x2304 20.4 -> 16.1, 2304x1280x640 9.9 -> 8.2, two per CU
-// 2560x3200x1024 17.9 -> 14.1, 7296x2176x1792 55.7 -> 39.4.
+// to a CU and left others empty: 896x3712x3072 33.2 -> 22.9 us, 1536x1024x2304 20.5 -> 16.5, two per CU 2304x1280x640
+// 10.2 -> 8.2, 2560x3200x1024 20.1 -> 15.3, 7296x2176x1792 56.7 -> 44.1.
 template <int STAGES, typename OUT, int FMT, int EPI>
 __global__ __launch_bounds__(256) void fp8_gemm_rowscaled_small_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
@@ -200,8 +200,8 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
 //   in rounds of the CUs (a round takes its time whether it is full or not); slabs of 128x256 tiles and their reduction.  Every
 //   form writes the output, M x N.
 // Fits to 150 shapes of 512..8192 rows and columns and 1 to 128 K blocks, rms error 3-6 % (slabs 9 %).  Against lines between sizes, 250 other
-// shapes: 6 % less time in the mean, up to 1.41 times as fast (7296x2176x1792), two of them more than 5 % behind out of the
-// caches (3328x512x3456 25.2 -> 27.7 us); 4096x7168 and 4096x4096 from 2 K blocks on stay on 256x256 tiles.  Up to 2 K blocks, and up to 4 where 128x128 tiles need two workgroups per
+// shapes: 6 % less time in the mean, up to 1.38 times as fast, one of them more than 5 % behind, out of the
+// caches alone (3328x512x3456 23.7 -> 23.7 / 25.3 -> 28.1 us); 4096x7168 and 4096x4096 from 2 K blocks on stay on 256x256 tiles.  Up to 2 K blocks, and up to 4 where 128x128 tiles need two workgroups per
 // CU, the plain loop's shorter ends win (640x7680x256 5.8 us against 7.1, 1792x3072x384 7.4 / 8.4, 2816x768x256 5.0 / 5.3).  With one K
 // block they do so for any number of tiles (against 256x256: 6400x8064 23.9 us / 28.6, 4224x4096 11.6 / 14.5, 5504x2048 8.2 / 8.9; two
 // 128x128 per CU are never ahead, 6656x3456 12.7 / 14.3), but where its rounds of two workgroups per CU are twice as many as those of

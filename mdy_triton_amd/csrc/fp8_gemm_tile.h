@@ -1,7 +1,7 @@
 // The MFMA tile body of the block-scaled FP8 GEMM and the kernel that walks tiles with it (gfx950 only).
 // Shared by fp8_gemm.hip (the product kernels) and gemm_probe.hip (the timing probe that switches parts of the
 // K loop off); the description of the kernels is at the top of fp8_gemm.hip.  Two bodies: fp8_gemm_tile (every wave
-// does everything; the large tiles) and fp8_gemm_tile_ws (producer / consumer waves; 128x192 tiles).
+// does everything; the large tiles) and fp8_gemm_tile_ws (producer / consumer waves; 64x128, 128x64, 128x128 and 128x192 tiles).
 #pragma once
 #include <type_traits>
 
@@ -643,7 +643,8 @@ __device__ __forceinline__ void fp8_gemm_tile(
 // Tile order shared by the kernels below: consecutive workgroup ids land on different XCDs (8 of
 // them); give each XCD a contiguous run of tiles, walked in groups of 4 tile rows.  With a tile count that 8 does not divide the
 // first XCDs get one tile more (such counts used to run in plain order, every panel pulled into every XCD's L2): 777x2112x7168
-// 29.9 -> 28.3 us, 777x7168x7168 62 -> 57, 250x9000x2048 13.4 -> 12.4, 3752x15224x768 68.8 -> 62.2, no shape of twenty slower.
+// 29.9 -> 28.3 us, 777x7168x7168 62.5 -> 57.2, 250x9000x2048 14.7 -> 13.3, 3752x15224x768 68.8 -> 65.6 (out of the caches 73.2 -> 76.4).  Up to 3
+// K blocks it is even (tiles in one launch: 0.94 to 1.07 of the time).
 __device__ __forceinline__ int xcd_contiguous(int pid, int ntiles) {
     const int x = pid & 7, rest = ntiles & 7;
     return x * (ntiles >> 3) + min(x, rest) + (pid >> 3);

@@ -137,17 +137,17 @@ def test_gemm_exact_integer_random_mid_shapes(M, N, K):
 
 SPLIT_SHAPES = [(128, 1536, 4096), (100, 777, 4224), (256, 2304, 4096), (130, 1100, 5120),
                 (130, 520, 6528), (300, 1536, 4480), (1000, 640, 8192),             # slabs of 9 / 12 and 11 / 11 K blocks, 3 and 8 tile rows
-                (64, 2304, 4352), (48, 4096, 7168),                                 # 33..64 rows on 64x64 tiles
-                # 33..64 rows against at most 2048 columns: the whole-line kernel over slabs of K (one or two K blocks per
-                # wave and pass, several passes, ragged N with the scalar reduction, a slab count that does not divide K)
-                (64, 2048, 4352), (40, 300, 8192), (33, 130, 4096), (50, 1536, 7168), (37, 2042, 8192), (64, 1024, 16384),
+                (64, 2304, 4352), (48, 4096, 7168), (64, 2048, 4352),               # 33..64 rows on 64x64 tiles
+                # the whole-line kernel over slabs of K (one or two K blocks per wave and pass, several passes, ragged N with the
+                # scalar reduction, a slab count that does not divide K)
+                (40, 300, 8192), (33, 130, 4096), (50, 1536, 7168), (37, 2042, 8192), (64, 1024, 16384),
                 (48, 256, 32768)]
 
 
 @pytest.mark.parametrize("M,N,K", SPLIT_SHAPES)
 def test_gemm_exact_integer_split_k(M, N, K):
     """Few rows against a long K: fp8_gemm hands the library a workspace and the shape runs split along K
-    (64x64 tiles, 128x64 and 128x128 tiles on the producer / consumer kernel, or the whole-line kernel for up to 64 rows against a narrow weight; N % 4 != 0 takes
+    (64x64 tiles, 128x64 and 128x128 tiles on the producer / consumer kernel, or the whole-line kernel for up to 64 rows; N % 4 != 0 takes
     the scalar reduction).  Exact operands stay exact."""
     lib = _lib.load()
     assert lib.mdy_fp8_gemm_path(None, None, K // 128, 1, M, N, K, 1) == 4 and lib.mdy_fp8_gemm_workspace_bytes(M, N, K) >= 2 * M * N * 4

@@ -42,7 +42,7 @@ def _bits(t):
     return t.cpu().view(torch.int16 if t.dtype == torch.bfloat16 else torch.int32).numpy()
 
 
-# (first call, second smaller call): split along K with 128x128 / 128x64 tiles and, for (40, 300, 8192), the whole-line kernel over
+# (first call, second smaller call): split along K with 128x64 and 64x64 tiles and, up to 64 rows, the whole-line kernel over
 # slabs of K; then a shape that needs no scratch
 CASES = [((256, 2304, 4096), (128, 1536, 4096)),
          ((130, 1100, 5120), (40, 300, 8192)),
