@@ -6,11 +6,11 @@
 // reference's Fp8Linear uses for its weight gradient dw = dy^T . x with both operands quantized along the token
 // dimension (fp8_matmul_bwd, :254-257).
 //
-// The combined scale differs for each of a lane's four results of an MFMA (four consecutive n of one m), so the
-// fold is 4 multiplies + 4 FMAs per MFMA instead of 4 FMAs: the VALU is as busy as the matrix cores, and what is left to
-// save is everything else a wave issues.  So the scheduled tile body of fp8_gemm_tile.h in its row-scaled-weight form takes
-// 256x256 tiles where their rounds come out ahead (a quarter fewer LDS reads and a third fewer copies per MFMA than 128x256:
-// 4096x7168x4096 154 -> 130 us = 1.85 PFLOP/s, 4096x4096x8192 159 -> 136 us = 2.0 PFLOP/s), 128x256 and 128x128 tiles otherwise; a plain
+// The combined scale differs for each of a lane's four results of an MFMA (four consecutive n of one m).  Multiplied on the VALU the
+// fold would be 4 multiplies + 4 FMAs per MFMA instead of 4 FMAs, as much work as the matrix cores have; the scheduled tile body of fp8_gemm_tile.h
+// forms the products on the matrix cores instead (scale_products there).  It takes 256x256 tiles where their rounds come out ahead (a
+// quarter fewer LDS reads and a third fewer copies per MFMA than 128x256: 4096x7168x4096 154 -> 130 us, 4096x4096x8192 159 -> 136 us; with the
+// products on the matrix cores 120.6 -> 115.0 and 129.1 -> 122.9 us = 2.09 and 2.24 PFLOP/s), 128x256 and 128x128 tiles otherwise; a plain
 // loop (128x128 tile, four waves of 64x64, the K block's two panels and two scale vectors copied global -> LDS by `buffer_load
 // ... lds`, double buffered, one barrier per K block: short ends, but 0.93 us per K block against 0.72) runs what has few K blocks.
 // K % 128 == 0 (the callers contract over a padded token count).
@@ -201,7 +201,8 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
 //   form writes the output, M x N.
 // Fits to 150 shapes of 512..8192 rows and columns and 1 to 128 K blocks, rms error 3-6 % (slabs 9 %).  Against lines between sizes, 250 other
 // shapes: 6 % less time in the mean, up to 1.38 times as fast, one of them more than 5 % behind, out of the
-// caches alone (3328x512x3456 23.7 -> 23.7 / 25.3 -> 28.1 us); 4096x7168 and 4096x4096 from 2 K blocks on stay on 256x256 tiles.  Up to 2 K blocks, and up to 4 where 128x128 tiles need two workgroups per
+// caches alone (3328x512x3456 23.7 -> 23.7 / 25.3 -> 28.1 us).  They were made with the scale products on the VALU; since then every form takes 7
+// to 13 % less (200 shapes, 180 others for the forms), too evenly to choose by: refitted constants move one call in fifteen, 0.3 % in the mean.  4096x7168 and 4096x4096 from 2 K blocks on stay on 256x256 tiles.  Up to 2 K blocks, and up to 4 where 128x128 tiles need two workgroups per
 // CU, the plain loop's shorter ends win (640x7680x256 5.8 us against 7.1, 1792x3072x384 7.4 / 8.4, 2816x768x256 5.0 / 5.3).  With one K
 // block they do so for any number of tiles (against 256x256: 6400x8064 23.9 us / 28.6, 4224x4096 11.6 / 14.5, 5504x2048 8.2 / 8.9; two
 // 128x128 per CU are never ahead, 6656x3456 12.7 / 14.3), but where its rounds of two workgroups per CU are twice as many as those of

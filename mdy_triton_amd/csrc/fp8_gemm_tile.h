@@ -30,6 +30,19 @@ __device__ __forceinline__ void fold(floatx4& acc, const floatx4& p, float sc) {
     acc[3] = __builtin_fmaf(p[3], sc, acc[3]);
 }
 
+// Products of row scales for four sub-tiles at a time, laid out like the results of four mfma_block: v_mfma_f32_16x16x1_4b, each product an
+// FMA onto zero and so rounded as v_mul_f32 rounds it.  Lane l holds the scale of row l of four sub-tiles.  ALL_WEIGHTS: the four weight
+// sub-tiles against activation sub-tile ONE of its four (blgp 4..7 broadcasts 16 lanes), otherwise weight sub-tile ONE (cbsz / abid) against
+// the four activation sub-tiles.  Eight of these per 128x64 wave tile and K block replace 128 multiplies (32 clocks of a SIMD's matrix core, 8 passes, for
+// what takes its VALU 64) and 16 to 24 registers of scales; same bits.  4096x7168x512 25.3 -> 24.6 us, x1024 39.7 -> 37.5, x4096 120.6 -> 115.0,
+// 2048x2048x2048 15.2 -> 14.0; 200 drawn shapes 3.5 % less time in the mean, none more beyond 2 %.  An MFMA between the products and their
+// first use, in place of the wait states there, is slower (4096x7168x1024 37.9).
+template <bool ALL_WEIGHTS, int ONE>
+__device__ __forceinline__ floatx16 scale_products(float weight_scales, float act_scales) {
+    const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    return __builtin_amdgcn_mfma_f32_16x16x1f32(weight_scales, act_scales, zero, ALL_WEIGHTS ? 0 : 2, ALL_WEIGHTS ? 0 : ONE, ALL_WEIGHTS ? 4 + ONE : 0);
+}
+
 template <typename OUT>
 __device__ __forceinline__ void store4(OUT* c, int64_t ldc, int m, int n, int M, int N, const float (&v)[4], bool vec_ok) {
     if (m >= M || n >= N) return;
@@ -292,8 +305,8 @@ struct OneTile {};
 // pipe instead of in front of the first MFMA of the next K block.
 // BROW_: the weight operand carries one scale per ROW and K block (b_s[n * bs_rs + kb * bs_cs], bs_bytes long) instead of
 // one per 128x128 block: the scales of the tile's BN rows travel through LDS per K block like the activation scales
-// (copied by the waves behind the activation-scale waves), a lane keeps the four scales of its four columns of every
-// sub-tile, and the fold multiplies them in: 4 multiplies + 4 FMAs per MFMA instead of 4 FMAs.
+// (copied by the waves behind the activation-scale waves), and scale_products multiplies the two for a streamed fragment behind the
+// last MFMA of it, when the products of the fragment before have been folded.
 //
 // NEXT: a workgroup that walks its tiles passes next(m0, n0, duty) -> bool, which moves on to its next tile.  The copies of that
 // tile's first two K blocks are then issued BEFORE the results of this one are stored (through LDS beside the ring).  Loads
@@ -349,6 +362,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
     // means "block kb+1 has landed")
     constexpr int YOUNGER = (STAGES - 2) * NDMA + STAGES - 1;
     static_assert(STAGES >= 2 && YOUNGER <= 63, "vmcnt is a 6-bit counter");
+    static_assert(!BROW_ || (NH == 4 && DEPTH == 4 && TJ == 4 && WM % 64 == 0), "scale products of four sub-tiles at a time");
     static_assert(NS % 2 == 0 && NS >= 2, "the first streamed fragment of the next K block reuses queue slot 0");
     static_assert(TOUCH < TB, "not enough slots in front of the barrier");
 
@@ -488,16 +502,20 @@ __device__ __forceinline__ void fp8_gemm_tile(
     __syncthreads();
     intx8 fh[NH], fx[2];
     float sc[TI], sc_hi[STRADDLE ? TI : 1];
-    floatx4 sbv[BROW_ ? TJ : 1];                 // BROW_: the weight-row scales of this lane's four columns of every sub-tile
-    const float* sbr_lane = lds_sbr + wn * WN + 4 * fk;
+    // BROW_: the scales of the wave's 64 weight rows and of its activation rows, one a lane
+    constexpr int SAV = BROW_ ? TI / 4 : 1;
+    const float* sbr_lane = lds_sbr + wn * WN + lane;
+    const int sar_lane = wm * WM + lane;
+    float sb_row = 1.0f, sa_row[SAV];
     if (BROW_) {
+        sb_row = sbr_lane[0];
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) sbv[j] = *reinterpret_cast<const floatx4*>(sbr_lane + j * 16);
+        for (int v = 0; v < SAV; ++v) sa_row[v] = lds_s[0][sar_lane + v * 64];
     }
 #pragma unroll
     for (int h = 0; h < NH; ++h) fh[h] = read_frag(HOLD_A ? lds_a[0] : lds_b[0], h0, h1, h);
-    {
-        const float sb = BROW_ ? 1.0f : my_bs[kb0], sb_hi = BROW_ ? 1.0f : my_bs_hi[kb0];
+    if (!BROW_) {
+        const float sb = my_bs[kb0], sb_hi = my_bs_hi[kb0];
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
             const float sa = lds_s[0][s_rd + i * 16];
@@ -519,6 +537,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
         const float* ls_n = lds_s[nxt];
         float sa_n[TI], sb_n = 1.0f, sb_hi_n = 1.0f;         // scales of the next K block
         floatx4 p[DEPTH + 1];
+        floatx16 sp;                                         // BROW_: scale products of the streamed fragment that is folded
 #pragma unroll
         for (int t = 0; t < NT + DEPTH; ++t) {
             if (t < NT) {
@@ -542,11 +561,12 @@ __device__ __forceinline__ void fp8_gemm_tile(
                     __syncthreads();
                     if (!NO_LDS) {
                         fx[0] = read_frag(lx_n, x0, x1, 0);      // queue slot 0 was last used by streamed fragment NS-2
-                        const float sb = BROW_ ? 1.0f : my_bs[min(kb + 1, KB - 1)], sb_hi = BROW_ ? 1.0f : my_bs_hi[min(kb + 1, KB - 1)];
+                        if (!BROW_) {
+                            sb_n = my_bs[min(kb + 1, KB - 1)];
+                            sb_hi_n = my_bs_hi[min(kb + 1, KB - 1)];
 #pragma unroll
-                        for (int i = 0; i < TI; ++i) sa_n[i] = ls_n[s_rd + i * 16];      // combined at the end of the block: nothing waits here
-                        sb_n = sb;
-                        sb_hi_n = sb_hi;
+                            for (int i = 0; i < TI; ++i) sa_n[i] = ls_n[s_rd + i * 16];      // combined at the end of the block: nothing waits here
+                        }
                     } else {
                         asm volatile("" : "+v"(fx[0]));
                     }
@@ -561,13 +581,20 @@ __device__ __forceinline__ void fp8_gemm_tile(
                 const int i = HOLD_A ? h : si, j = HOLD_A ? si : h;
                 const floatx4 q = p[u % (DEPTH + 1)];
                 if (BROW_) {
-                    acc[i][j][0] = __builtin_fmaf(q[0], sc[i] * sbv[j][0], acc[i][j][0]);
-                    acc[i][j][1] = __builtin_fmaf(q[1], sc[i] * sbv[j][1], acc[i][j][1]);
-                    acc[i][j][2] = __builtin_fmaf(q[2], sc[i] * sbv[j][2], acc[i][j][2]);
-                    acc[i][j][3] = __builtin_fmaf(q[3], sc[i] * sbv[j][3], acc[i][j][3]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_fmaf(q[e], sp[h * 4 + e], acc[i][j][e]);
                 } else {
                     fold(acc[i][j], q, (STRADDLE && j >= jsplit) ? sc_hi[i] : sc[i]);
                 }
+                if (FRESH) asm volatile("" : "+v"(acc[i][j]));      // here, not behind the branch around the wait below
+            }
+            if (BROW_ && t < NT && t % NH == NH - 1) {
+                // the fragment before has just been folded: its products make room
+                constexpr bool W = !HOLD_A;
+                const int si = t / NH;
+                const float sa = sa_row[W ? si / 4 : 0];
+                sp = si % 4 == 0 ? scale_products<W, 0>(sb_row, sa) : si % 4 == 1 ? scale_products<W, 1>(sb_row, sa)
+                     : si % 4 == 2 ? scale_products<W, 2>(sb_row, sa) : scale_products<W, 3>(sb_row, sa);
             }
             if (!NO_COPY) {
 #pragma unroll
@@ -579,17 +606,16 @@ __device__ __forceinline__ void fp8_gemm_tile(
             }
             if (t == TOUCH && !NO_TOUCH) touch(me, kb + TD);
             if (BROW_ && t == NT + DEPTH - 1) {
-                // the block's last fold is done: its weight-row scales make room for the next block's, which are first used
-                // DEPTH MFMAs from here (a second set of registers would not fit the 256x256 tile)
+                sb_row = sbr_lane[nxt * BN];      // first used NH - 1 MFMAs from here
 #pragma unroll
-                for (int j = 0; j < TJ; ++j) sbv[j] = *reinterpret_cast<const floatx4*>(sbr_lane + nxt * BN + j * 16);
+                for (int v = 0; v < SAV; ++v) sa_row[v] = ls_n[sar_lane + v * 64];
             }
             __builtin_amdgcn_sched_barrier(0);  // keep the MFMA / FMA / ds_read / copy interleaving as written
         }
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
-            if (NO_LDS) continue;
-            sc[i] = BROW_ ? sa_n[i] : sa_n[i] * sb_n;
+            if (NO_LDS || BROW_) continue;
+            sc[i] = sa_n[i] * sb_n;
             if (STRADDLE) sc_hi[i] = sa_n[i] * sb_hi_n;
         }
         cur = nxt;

@@ -80,3 +80,31 @@ def test_exact_integer_fp32(M, N, K, form):
     rc = lib.mdy_fp8_gemm_nt_rowscaled_ws(a.data_ptr(), sa.data_ptr(), K // 128, 1, b.data_ptr(), sb.data_ptr(), K // 128, 1, c.data_ptr(), M, N, K, 0, 1,
                                           0, 0, torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and torch.equal(c.double(), 4 * (ai.double().to(DEV) @ bi.double().to(DEV).t()))
+
+
+@pytest.mark.parametrize("M,N,K,form", [(890, 1028, 3072, RING3), (300, 700, 512, TWO), (644, 5433, 640, T128X256), (4090, 3336, 384, T256X256)])
+def test_scale_products_are_rounded_once_and_keep_special_values(M, N, K, form):
+    """One product per result, 1 * 1, in the second of the K blocks: the result is the fp32 product of the two scales to the bit, among them
+    denormal products, zeros, infinities and NaN (the matrix instruction that multiplies scales rounds and propagates as v_mul_f32)."""
+    lib = _lib.load()
+    runs(M, N, K, form, workspace=0)
+    g = torch.Generator().manual_seed(K)
+    a, b = (torch.zeros(r, K) for r in (M, N))
+    a[:, 200] = b[:, 200] = 1.0
+    a, b = (v.to(torch.float8_e4m3fn).to(DEV) for v in (a, b))
+
+    def scales(r):
+        s = torch.ones(r, K // 128)
+        v = torch.rand(r, generator=g) + 0.5
+        v[: r // 2] *= torch.exp2(torch.randint(-75, -60, (r // 2,), generator=g).float())      # products from 2^-152 to 2^-118
+        v[r - 40:r - 32], v[r - 20], v[r - 10], v[r - 5] = 0.0, float("inf"), float("nan"), 2.0 ** -140
+        s[:, 1] = v
+        return s, v
+
+    (sa, va), (sb, vb) = scales(M), scales(N)
+    c = torch.full((M, N), 7.0, device=DEV)
+    sa, sb = sa.to(DEV), sb.to(DEV)
+    rc = lib.mdy_fp8_gemm_nt_rowscaled_ws(a.data_ptr(), sa.data_ptr(), K // 128, 1, b.data_ptr(), sb.data_ptr(), K // 128, 1, c.data_ptr(), M, N, K, 0, 1,
+                                          0, 0, torch.cuda.current_stream().cuda_stream)
+    ref = va[:, None] * vb[None, :]
+    assert rc == 0 and torch.equal(c.cpu().nan_to_num(nan=-1.0), ref.nan_to_num(nan=-1.0))
