@@ -242,8 +242,9 @@ __global__ __launch_bounds__(2048 / RPT, 32 / RPT) void quant_transpose_kernel(c
                                                                int PK, int64_t s_kb_stride, int64_t s_m_stride,
                                                                int64_t st_a_stride, int64_t st_k_stride,
                                                                float* __restrict__ col_sum) {
-    const int bm = block_row(), bk = blockIdx.x;
+    int bm = block_row(), bk = blockIdx.x;
     if (bm >= (PM >> 7)) return;
+    xcd_patch(bm, bk, gridDim.x, PM >> 7);
     quant_transpose_tile<MODE, TMODE, VEC, XT, CSUM>(bm, bk, x, y, s, y_t + (int64_t)bm * 128, PM, TMODE == 0 ? s_t + bm * st_a_stride : s_t, M, K,
                                                      x_row_stride, x_col_stride, PM, PK, s_kb_stride, s_m_stride, st_k_stride, col_sum);
 }
@@ -264,8 +265,9 @@ __global__ __launch_bounds__(2048 / RPT, 16 / RPT) void swiglu_bwd_quant_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ d, uint8_t* __restrict__ act_t, float* __restrict__ act_ts, uint8_t* __restrict__ y,
     float* __restrict__ s, uint8_t* __restrict__ y_t, float* __restrict__ s_t, int M, int I, int up_off, int gate_off, int PM) {
     constexpr bool DEEP = MODE == 1;
-    const int bm = block_row(), bi = blockIdx.x;
+    int bm = block_row(), bi = blockIdx.x;
     if (bm >= (PM >> 7)) return;
+    xcd_patch(bm, bi, gridDim.x, PM >> 7);
     __shared__ QtLds<false> lds;
     const int row0 = bm * 128 + (threadIdx.x >> 4) * RPT, c0 = bi * 128 + (threadIdx.x & 15) * 8;
     const bool inside = bi * 128 < I;             // beyond: the zero rows that complete act_t to PI (uniform)
@@ -348,8 +350,9 @@ template <bool VEC, int XT>
 __global__ __launch_bounds__(2048 / RPT, 32 / RPT) void quant_transpose_grouped_kernel(const void* __restrict__ x, uint8_t* __restrict__ y,
                                                                              float* __restrict__ s, int M, int K, int64_t x_row_stride,
                                                                              int64_t x_col_stride, int64_t s_kb_stride, const QtGroups groups) {
-    const int bm = block_row(), bk = blockIdx.x;
+    int bm = block_row(), bk = blockIdx.x;
     if (bm >= (M >> 7)) return;
+    xcd_patch(bm, bk, gridDim.x, M >> 7);
     int lo = 0, hi = groups.n - 1;                       // the last group that starts at or before the tile (empty ones skipped)
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;

@@ -99,9 +99,10 @@ __global__ __launch_bounds__(512) void weight_quant_kernel(const void* __restric
                                                             float* __restrict__ s, uint8_t* __restrict__ y_t,
                                                             float* __restrict__ s_t, int N, int K, int64_t w_row_stride,
                                                             int64_t w_col_stride, int PN, int PK) {
-    const int bn = block_row();  // block row (along N)
-    const int bk = blockIdx.x;   // block column (along K)
+    int bn = block_row();  // block row (along N)
+    int bk = blockIdx.x;   // block column (along K)
     if (bn >= (PN >> 7)) return;
+    if (y_t) xcd_patch(bn, bk, gridDim.x, PN >> 7);
     weight_quant_tile<MODE, VEC, XT>(bn, bk, w, y, s, y_t, s_t, N, K, w_row_stride, w_col_stride, PN, PK);
 }
 
@@ -116,9 +117,11 @@ template <int MODE, bool VEC, int XT>
 __global__ __launch_bounds__(512) void weight_quant_group_kernel(const WeightList list, int G, uint8_t* __restrict__ y, float* __restrict__ s,
                                                             uint8_t* __restrict__ y_t, float* __restrict__ s_t, int N, int K,
                                                             int64_t w_row_stride, int64_t w_col_stride, int PN, int PK) {
-    const int rows = PN >> 7, row = block_row();      // block rows of one weight, of all of them
-    const int g = row / rows, bn = row - g * rows, bk = blockIdx.x;
-    if (g >= G) return;
+    const int rows = PN >> 7;                         // block rows of one weight
+    int row = block_row(), bk = blockIdx.x;           // of all of them
+    if (row >= rows * G) return;
+    if (y_t) xcd_patch(row, bk, gridDim.x, rows * G);
+    const int g = row / rows, bn = row - g * rows;
     const int64_t bytes = (int64_t)PN * PK, scales = (int64_t)rows * (PK >> 7);
     weight_quant_tile<MODE, VEC, XT>(bn, bk, list.w[g], y ? y + g * bytes : nullptr, s ? s + g * scales : nullptr, y_t ? y_t + g * bytes : nullptr,
                                      s_t ? s_t + g * scales : nullptr, N, K, w_row_stride, w_col_stride, PN, PK);
