@@ -233,7 +233,7 @@ int launch_act_quant_typed(const void* x, int x_dtype, int block_size, void* y, 
     if (!grid_rows((PK + 511) / 512, (PM + kAqRowsPerBlock - 1) / kAqRowsPerBlock, grid)) return kErrTooManyBlocks;
     uint8_t* yp = static_cast<uint8_t*>(y);
 #define MDY_AQT(MODE, XT, VEC)                                                                                         \
-    hipLaunchKernelGGL((act_quant_typed_kernel<MODE, XT, VEC>), grid, dim3(256), 0, stream, x, yp, s, (int)M, (int)K, \
+    launch_kernel((act_quant_typed_kernel<MODE, XT, VEC>), grid, dim3(256), 0, stream, x, yp, s, (int)M, (int)K, \
                        x_row_stride, (int)PM, (int)PK, s_row_stride, s_col_stride, lanes, shift)
 #define MDY_AQT_V(MODE, XT) do { if (vec) MDY_AQT(MODE, XT, true); else MDY_AQT(MODE, XT, false); } while (0)
 #define MDY_AQT_X(MODE) do { if (x_dtype == 0) MDY_AQT_V(MODE, 0); else if (x_dtype == 1) MDY_AQT_V(MODE, 1); else MDY_AQT_V(MODE, 2); } while (0)
@@ -256,7 +256,7 @@ int launch_act_quant(const void* x, void* y, float* s, int64_t M, int64_t K, int
         const uint16_t* xp = static_cast<const uint16_t*>(x);
         uint8_t* yp = static_cast<uint8_t*>(y);
 #define MDY_CM(MODE, VEC)                                                                                          \
-    hipLaunchKernelGGL((act_quant_cm_kernel<MODE, VEC>), grid, block, 0, stream, xp, yp, s, (int)M, (int)K, x_row_stride, \
+    launch_kernel((act_quant_cm_kernel<MODE, VEC>), grid, block, 0, stream, xp, yp, s, (int)M, (int)K, x_row_stride, \
                        (int)PM, (int)PK, s_col_stride)
         if (mode == 0) {
             if (vec) MDY_CM(0, true); else MDY_CM(0, false);
@@ -282,7 +282,7 @@ int launch_act_quant(const void* x, void* y, float* s, int64_t M, int64_t K, int
         uint8_t* yp = static_cast<uint8_t*>(y) + r0 * PK;
         float* sp = s + r0 * s_row_stride;
 #define MDY_AQ(MODE, VEC)                                                                                       \
-    hipLaunchKernelGGL((act_quant_kernel<MODE, VEC>), grid, block, 0, stream, xp, yp, sp, (int)m, (int)K,       \
+    launch_kernel((act_quant_kernel<MODE, VEC>), grid, block, 0, stream, xp, yp, sp, (int)m, (int)K,       \
                        x_row_stride, (int)pm, (int)PK, s_row_stride, s_col_stride, by_xcd)
         if (mode == 0) {
             if (vec) MDY_AQ(0, true); else MDY_AQ(0, false);
@@ -318,14 +318,14 @@ __global__ void cast_f32_to_e5m2_kernel(const float* __restrict__ x, uint8_t* __
 
 int launch_cast_f32_to_e5m2(const float* x, void* y, int64_t n, hipStream_t stream) {
     if (n == 0) return 0;
-    hipLaunchKernelGGL(cast_f32_to_e5m2_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, x,
+    launch_kernel(cast_f32_to_e5m2_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, x,
                        static_cast<uint8_t*>(y), n);
     return (int)hipGetLastError();
 }
 
 int launch_cast_f32_to_e4m3(const float* x, void* y, int64_t n, int saturate, hipStream_t stream) {
     if (n == 0) return 0;
-    hipLaunchKernelGGL(cast_f32_to_e4m3_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, x,
+    launch_kernel(cast_f32_to_e4m3_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, x,
                        static_cast<uint8_t*>(y), n, saturate);
     return (int)hipGetLastError();
 }
@@ -367,13 +367,13 @@ __global__ void zero4_kernel(unsigned long long* out) {
 
 int launch_quotient_selfcheck(uint64_t* out, int amax_lo, int amax_hi, int mode, hipStream_t stream) {
     unsigned long long* o = reinterpret_cast<unsigned long long*>(out);
-    hipLaunchKernelGGL(zero4_kernel, dim3(1), dim3(64), 0, stream, o);
+    launch_kernel(zero4_kernel, dim3(1), dim3(64), 0, stream, o);
     if (amax_hi <= amax_lo) return (int)hipGetLastError();
     dim3 grid((unsigned)(amax_hi - amax_lo)), block(256);
     if (mode == 0)
-        hipLaunchKernelGGL(quotient_selfcheck_kernel<0>, grid, block, 0, stream, o, amax_lo);
+        launch_kernel(quotient_selfcheck_kernel<0>, grid, block, 0, stream, o, amax_lo);
     else
-        hipLaunchKernelGGL(quotient_selfcheck_kernel<1>, grid, block, 0, stream, o, amax_lo);
+        launch_kernel(quotient_selfcheck_kernel<1>, grid, block, 0, stream, o, amax_lo);
     return (int)hipGetLastError();
 }
 

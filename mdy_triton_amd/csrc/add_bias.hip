@@ -53,7 +53,7 @@ int launch_add_bias(void* x, const void* b, int b_dtype, int64_t M, int64_t N, h
     const bool vec = (N % 8 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0) &&
                      ((reinterpret_cast<uintptr_t>(b) & 15) == 0);
     uint16_t* xp = static_cast<uint16_t*>(x);
-#define MDY_AB(VEC, BT) hipLaunchKernelGGL((add_bias_kernel<VEC, BT>), grid, dim3(256), 0, stream, xp, b, (int)M, (int)N)
+#define MDY_AB(VEC, BT) launch_kernel((add_bias_kernel<VEC, BT>), grid, dim3(256), 0, stream, xp, b, (int)M, (int)N)
     if (b_dtype == 0) { if (vec) MDY_AB(true, 0); else MDY_AB(false, 0); }
     else if (b_dtype == 1) { if (vec) MDY_AB(true, 1); else MDY_AB(false, 1); }
     else { if (vec) MDY_AB(true, 2); else MDY_AB(false, 2); }
@@ -90,13 +90,13 @@ int launch_add_grad(void* x, const void* y, int64_t n, int x_dtype, int y_dtype,
     if (blocks > 0x7FFFFFFF) return kErrTooManyBlocks;
     dim3 grid((unsigned)blocks), block(256);
     if (x_dtype == 1 && y_dtype == 0)
-        hipLaunchKernelGGL((add_grad_kernel<float, uint16_t>), grid, block, 0, stream, static_cast<float*>(x), static_cast<const uint16_t*>(y), n);
+        launch_kernel((add_grad_kernel<float, uint16_t>), grid, block, 0, stream, static_cast<float*>(x), static_cast<const uint16_t*>(y), n);
     else if (x_dtype == 1)
-        hipLaunchKernelGGL((add_grad_kernel<float, float>), grid, block, 0, stream, static_cast<float*>(x), static_cast<const float*>(y), n);
+        launch_kernel((add_grad_kernel<float, float>), grid, block, 0, stream, static_cast<float*>(x), static_cast<const float*>(y), n);
     else if (y_dtype == 0)
-        hipLaunchKernelGGL((add_grad_kernel<uint16_t, uint16_t>), grid, block, 0, stream, static_cast<uint16_t*>(x), static_cast<const uint16_t*>(y), n);
+        launch_kernel((add_grad_kernel<uint16_t, uint16_t>), grid, block, 0, stream, static_cast<uint16_t*>(x), static_cast<const uint16_t*>(y), n);
     else
-        hipLaunchKernelGGL((add_grad_kernel<uint16_t, float>), grid, block, 0, stream, static_cast<uint16_t*>(x), static_cast<const float*>(y), n);
+        launch_kernel((add_grad_kernel<uint16_t, float>), grid, block, 0, stream, static_cast<uint16_t*>(x), static_cast<const float*>(y), n);
     return (int)hipGetLastError();
 }
 

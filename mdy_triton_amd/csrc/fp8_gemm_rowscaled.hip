@@ -278,7 +278,7 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
         const int tm = (int)((M + 127) / 128), tn = (int)((N + 255) / 256);
         float* ws = static_cast<float*>(workspace);
 #define MDY_RSS(FMT, EPI)                                                                                                \
-    hipLaunchKernelGGL((fp8_gemm_rowscaled_split_kernel<FMT, EPI>), dim3((unsigned)(tm * tn * sp.slabs)), dim3(512), 0, stream, \
+    launch_kernel((fp8_gemm_rowscaled_split_kernel<FMT, EPI>), dim3((unsigned)(tm * tn * sp.slabs)), dim3(512), 0, stream, \
                        static_cast<const uint8_t*>(a), a_s, (int)as_rs, (int)as_cs, (uint32_t)a_ext, static_cast<const uint8_t*>(b), b_s, \
                        (int)bs_rs, (int)bs_cs, (uint32_t)b_ext, ws, (int)M, (int)N, (int)K, tm, tn, sp.slabs, sp.kb_per)
         if (epilogue_kind(ws, N, N, 4, false, true) == kEpiRows) {
@@ -298,7 +298,7 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
         if (tm * tn > 0x7FFFFFFF) return kErrTooManyBlocks;
         const dim3 grid((unsigned)(cfg == kTiles256x256 && tm * tn > cus ? cus : tm * tn));      // 256x256: a workgroup per CU walks its tiles
 #define MDY_RST(BM, ST, OUT_T, FMT, EPI)                                                                                 \
-    hipLaunchKernelGGL((fp8_gemm_rowscaled_tile_kernel<BM, 256, ST, OUT_T, FMT, EPI>), grid, dim3(512), 0, stream,            \
+    launch_kernel((fp8_gemm_rowscaled_tile_kernel<BM, 256, ST, OUT_T, FMT, EPI>), grid, dim3(512), 0, stream,            \
                        static_cast<const uint8_t*>(a), a_s, (int)as_rs, (int)as_cs, (uint32_t)a_ext,                      \
                        static_cast<const uint8_t*>(b), b_s, (int)bs_rs, (int)bs_cs, (uint32_t)b_ext, static_cast<OUT_T*>(c), \
                        (int)M, (int)N, (int)K, (int)tm, (int)tn)
@@ -320,9 +320,9 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
         (int)bs_rs, (int)bs_cs, (uint32_t)b_ext, static_cast<OUT_T*>(c), (int)M, (int)N, (int)K
 #define MDY_RS(OUT_T, FMT, EPI)                                                                                                                     \
     do {                                                                                                                                            \
-        if (cfg == kTiles128Ring3) hipLaunchKernelGGL((fp8_gemm_rowscaled_small_kernel<3, OUT_T, FMT, EPI>), MDY_RS_ARGS(OUT_T), tiles_m, tiles_n); \
-        else if (cfg == kTiles128Two) hipLaunchKernelGGL((fp8_gemm_rowscaled_small_kernel<2, OUT_T, FMT, EPI>), MDY_RS_ARGS(OUT_T), tiles_m, tiles_n); \
-        else hipLaunchKernelGGL((fp8_gemm_rowscaled_kernel<OUT_T, FMT, EPI>), MDY_RS_ARGS(OUT_T), tiles_n);                                          \
+        if (cfg == kTiles128Ring3) launch_kernel((fp8_gemm_rowscaled_small_kernel<3, OUT_T, FMT, EPI>), MDY_RS_ARGS(OUT_T), tiles_m, tiles_n); \
+        else if (cfg == kTiles128Two) launch_kernel((fp8_gemm_rowscaled_small_kernel<2, OUT_T, FMT, EPI>), MDY_RS_ARGS(OUT_T), tiles_m, tiles_n); \
+        else launch_kernel((fp8_gemm_rowscaled_kernel<OUT_T, FMT, EPI>), MDY_RS_ARGS(OUT_T), tiles_n);                                          \
     } while (0)
     const int epi = epilogue_kind(c, N, N, out_dtype == 0 ? 2 : 4, false, out_dtype == 0);
     if (out_dtype != 0) { if (fmt == 0) MDY_RS(float, 0, kEpiDirect); else MDY_RS(float, 1, kEpiDirect); }

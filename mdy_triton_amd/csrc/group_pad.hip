@@ -98,7 +98,7 @@ int launch_group_pad(const void* x, void* y, const int64_t* m_splits, int64_t G,
         if (!grid_rows((row_bytes + 64 * pieces * vec - 1) / (64 * pieces * vec), (rows + 3) / 4, grid)) return kErrTooManyBlocks;
         const uint8_t* xp = static_cast<const uint8_t*>(x) + src0 * row_bytes;
         uint8_t* yp = static_cast<uint8_t*>(y) + dst0 * row_bytes;
-#define MDY_PAD(VEC, PIECES) hipLaunchKernelGGL((group_pad_kernel<VEC, PIECES>), grid, dim3(256), 0, stream, xp, yp, row_bytes, rows, tbl)
+#define MDY_PAD(VEC, PIECES) launch_kernel((group_pad_kernel<VEC, PIECES>), grid, dim3(256), 0, stream, xp, yp, row_bytes, rows, tbl)
 #define MDY_PAD_P(VEC) do { if (unpad) MDY_PAD(VEC, kUnpadPieces); else MDY_PAD(VEC, kPadPieces); } while (0)
         if (vec == 16) MDY_PAD_P(16);
         else if (vec == 2) MDY_PAD_P(2);

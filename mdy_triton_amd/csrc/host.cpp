@@ -11,13 +11,19 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <algorithm>
+#include <cstdlib>
+#include <cstring>
+
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DefaultDtype.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Device.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/variable.h>
@@ -73,6 +79,17 @@ Tensor make_strided(at::IntArrayRef sizes, at::IntArrayRef strides, ScalarType d
     return Tensor(at::detail::empty_strided_cuda(sizes, strides, dtype, dev));
 }
 
+// Memory on the current stream for what no caller sees, from the same allocator (0.2 us; a tensor around it takes another 0.25).  It may go as soon as the
+// launches that use it are enqueued: the allocator hands it out again in stream order only.
+struct Scratch {
+    c10::DataPtr p;
+    explicit Scratch(int64_t bytes) {
+        if (bytes > 0) p = c10::hip::HIPCachingAllocator::get()->allocate((size_t)bytes);
+    }
+    uint8_t* at(int64_t offset) const { return p.get() == nullptr ? nullptr : static_cast<uint8_t*>(p.get()) + offset; }
+};
+int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
+
 PyObject* tuple2(Tensor&& a, Tensor&& b) {
     PyObject* r = PyTuple_New(2);
     if (r == nullptr) return nullptr;
@@ -99,12 +116,10 @@ bool bias_arg(PyObject* o, int64_t N, int& device, const void*& p) {
 
 // c[M, N] = a . b^T with block scales; false when the library rejects the call
 bool gemm(const void* a, const float* a_s, int64_t rs, int64_t cs, const void* b, const float* b_s, void* c, const void* bias, int bias_mode,
-          int64_t M, int64_t N, int64_t K, int fmt, int out_code, const at::Device& dev, void* stream) {
+          int64_t M, int64_t N, int64_t K, int fmt, int out_code, void* stream) {
     const int64_t bytes = mdy_fp8_gemm_workspace_bytes(M, N, K);
-    Tensor ws;      // handed back as soon as the launch is enqueued: the allocator reuses it in stream order only
-    if (bytes > 0) ws = make({bytes}, ScalarType::Byte, dev);
-    return mdy_fp8_gemm_nt_ex(a, a_s, rs, cs, b, b_s, c, bias, bias_mode, M, N, K, fmt, out_code, bytes > 0 ? ws.data_ptr() : nullptr,
-                              bytes > 0 ? bytes : 0, stream) == 0;
+    const Scratch ws(bytes);
+    return mdy_fp8_gemm_nt_ex(a, a_s, rs, cs, b, b_s, c, bias, bias_mode, M, N, K, fmt, out_code, ws.at(0), bytes > 0 ? bytes : 0, stream) == 0;
 }
 // What the MFMA kernels need of a GEMM (anything else may run the scalar kernel, about which the wrapper warns)
 bool gemm_shape_ok(int64_t M, int64_t N, int64_t K, int64_t rs, int64_t cs) {
@@ -168,7 +183,7 @@ PyObject* fp8_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
         sizes.back() = N;
         c = make(sizes, out, a->device());
         return gemm(a->data_ptr(), (const float*)as->data_ptr(), KB, 1, b->data_ptr(), (const float*)bs->data_ptr(), c.data_ptr(), bias, MDY_BIAS_IN_SUM,
-                    M, N, K, fmt, code, a->device(), stream_of(device));
+                    M, N, K, fmt, code, stream_of(device));
     });
     if (!ok) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(c));
@@ -217,7 +232,7 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const bool ok = unlocked([&] {
         c = make({M, N}, ScalarType::BFloat16, a->device());
         return gemm(a->data_ptr(), (const float*)as->data_ptr(), rs, cs, b->data_ptr(), (const float*)bs->data_ptr(), c.data_ptr(), bias, mode, M, N, K,
-                    MDY_FMT_E4M3, MDY_DT_BF16, a->device(), stream_of(device));
+                    MDY_FMT_E4M3, MDY_DT_BF16, stream_of(device));
     });
     if (!ok) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(c));
@@ -282,16 +297,44 @@ PyObject* deep_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Tensor c;
     const bool ok = unlocked([&] {
         void* stream = stream_of(device);
-        Tensor y, s;
-        if (!quantize_rows(r, y, s, stream)) return false;
+        // the quantized rows, their scales and the product's workspace
+        const int64_t s_at = round_up(PM * PK, 512), ws_at = round_up(s_at + PM * KB * 4, 512), bytes = mdy_fp8_gemm_workspace_bytes(r.M, N, PK);
+        const Scratch room(ws_at + std::max<int64_t>(bytes, 0));
+        if (mdy_act_quant_typed(r.t->data_ptr(), r.xt, 128, room.at(0), (float*)room.at(s_at), r.M, r.K, r.stride, PM, PK, 1, PM, MDY_QUANT_DEEPLINEAR,
+                                stream) != 0)
+            return false;
         auto sizes = r.t->sizes().vec();
         sizes.back() = N;
         c = make(sizes, ScalarType::BFloat16, r.t->device());
-        return gemm(y.data_ptr(), (const float*)s.data_ptr(), 1, PM, b->data_ptr(), (const float*)bs->data_ptr(), c.data_ptr(), bias, mode, r.M, N, PK,
-                    MDY_FMT_E4M3, MDY_DT_BF16, r.t->device(), stream);
+        return mdy_fp8_gemm_nt_ex(room.at(0), (const float*)room.at(s_at), 1, PM, b->data_ptr(), (const float*)bs->data_ptr(), c.data_ptr(), bias, mode, r.M,
+                                  N, PK, MDY_FMT_E4M3, MDY_DT_BF16, bytes > 0 ? room.at(ws_at) : nullptr, bytes > 0 ? bytes : 0, stream) == 0;
     });
     if (!ok) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(c));
+}
+
+// cached_weight(weight, cache, with_transpose) -> the quantized copies (y, s, yt, st) that DeepLinear keeps, if they are the weight's: cache is
+// ((data_ptr, version, shape, device), copies, fingerprint).  None where that has to be looked at more closely, and where
+// MDY_FP8_CHECK_WEIGHT_CACHE asks for it.
+PyObject* cached_weight(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    int device = -1;
+    if (n != 3 || !PyTuple_CheckExact(args[1]) || PyTuple_GET_SIZE(args[1]) != 3) Py_RETURN_NONE;
+    const Tensor* w = plain(args[0], device);
+    PyObject *key = PyTuple_GET_ITEM(args[1], 0), *copies = PyTuple_GET_ITEM(args[1], 1);
+    if (w == nullptr || w->is_inference() || !PyTuple_CheckExact(key) || PyTuple_GET_SIZE(key) != 4 || !PyTuple_CheckExact(copies) || PyTuple_GET_SIZE(copies) != 4)
+        Py_RETURN_NONE;
+    PyObject *ptr = PyTuple_GET_ITEM(key, 0), *version = PyTuple_GET_ITEM(key, 1), *shape = PyTuple_GET_ITEM(key, 2), *dev = PyTuple_GET_ITEM(key, 3);
+    if (!PyLong_CheckExact(ptr) || !PyLong_CheckExact(version) || !PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != w->dim() || !THPDevice_Check(dev)) Py_RETURN_NONE;
+    if (PyLong_AsUnsignedLongLong(ptr) != (unsigned long long)(uintptr_t)w->const_data_ptr() || PyLong_AsLongLong(version) != (long long)w->_version() ||
+        reinterpret_cast<THPDevice*>(dev)->device != w->device())
+        Py_RETURN_NONE;
+    for (int64_t d = 0; d < w->dim(); ++d)
+        if (!PyLong_CheckExact(PyTuple_GET_ITEM(shape, d)) || PyLong_AsLongLong(PyTuple_GET_ITEM(shape, d)) != w->size(d)) Py_RETURN_NONE;
+    if (flag(args[2]) && PyTuple_GET_ITEM(copies, 2) == Py_None) Py_RETURN_NONE;
+    const char* check = std::getenv("MDY_FP8_CHECK_WEIGHT_CACHE");
+    if (check != nullptr && check[0] != 0 && std::strcmp(check, "0") != 0) Py_RETURN_NONE;
+    Py_INCREF(copies);
+    return copies;
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -396,9 +439,8 @@ Tensor product(const Tensor& a, const Tensor& a_s, int64_t rs, int64_t cs, const
                int64_t M, int64_t N, int64_t K, int fmt, at::IntArrayRef sizes, void* stream) {
     Tensor c = make(sizes, ScalarType::BFloat16, a.device());
     const int64_t bytes = mdy_fp8_gemm_workspace_bytes(M, N, K);
-    Tensor ws;
-    if (bytes > 0) ws = make({bytes}, ScalarType::Byte, a.device());
-    done(mdy_fp8_gemm_nt_ex(raw(a), f32(a_s), rs, cs, raw(b), f32(b_s), raw(c), bias, bias_mode, M, N, K, fmt, MDY_DT_BF16, raw(ws), bytes > 0 ? bytes : 0,
+    const Scratch ws(bytes);
+    done(mdy_fp8_gemm_nt_ex(raw(a), f32(a_s), rs, cs, raw(b), f32(b_s), raw(c), bias, bias_mode, M, N, K, fmt, MDY_DT_BF16, ws.at(0), bytes > 0 ? bytes : 0,
                             stream));
     return c;
 }
@@ -407,10 +449,9 @@ Tensor product(const Tensor& a, const Tensor& a_s, int64_t rs, int64_t cs, const
 Tensor row_scaled(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, int64_t M, int64_t N, int64_t K, int fmt, void* stream) {
     Tensor c = make({M, N}, ScalarType::BFloat16, a.device());
     const int64_t bytes = mdy_fp8_gemm_rowscaled_workspace_bytes(M, N, K);
-    Tensor ws;
-    if (bytes > 0) ws = make({bytes}, ScalarType::Byte, a.device());
+    const Scratch ws(bytes);
     done(mdy_fp8_gemm_nt_rowscaled_ws(raw(a), f32(a_s), a_s.stride(0), a_s.stride(1), raw(b), f32(b_s), b_s.stride(0), b_s.stride(1), raw(c), M, N, K, fmt,
-                                      MDY_DT_BF16, raw(ws), bytes > 0 ? bytes : 0, stream));
+                                      MDY_DT_BF16, ws.at(0), bytes > 0 ? bytes : 0, stream));
     return c;
 }
 
@@ -875,15 +916,19 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return THPVariable_Wrap(unlocked([&] {
         const at::Device dev = r.t->device();
         void* stream = stream_of(device);
-        Tensor y = make({PM, K}, kE4m3, dev), s = make({PM * (K / 128)}, ScalarType::Float, dev);
-        done(mdy_act_quant_typed(r.t->data_ptr(), r.xt, 128, raw(y), f32(s), M, r.K, r.stride, PM, K, rs, cs, mode, stream));
-        const Tensor act = make({PM, PI}, kE4m3, dev), act_s = make({PM, PI / 128}, ScalarType::Float, dev);      // written [PI / 128, PM] with deep
-        const int64_t bytes = mdy_fp8_gemm_swiglu_workspace_bytes(M, N2, K);
-        Tensor ws = make({bytes}, ScalarType::Byte, dev);
-        done(mdy_fp8_gemm_swiglu(raw(y), f32(s), rs, cs, raw(*qwu), f32(*swu), M, N2, K, gate_first, raw(act), f32(act_s), PM, PI, act_rs, cs, mode, raw(ws),
-                                 bytes, stream));
-        y.reset(), s.reset(), ws.reset();      // the down projection finds room where these were
-        return product(act, act_s, act_rs, cs, *qwd, *swd, nullptr, 0, M, N, PI, MDY_FMT_E4M3, sizes, stream);
+        const int64_t bytes = mdy_fp8_gemm_swiglu_workspace_bytes(M, N2, K), s_at = round_up(PM * K, 512), ws_at = round_up(s_at + PM * (K / 128) * 4, 512),
+                      act_s_at = round_up(PM * PI, 512);
+        const Scratch act(act_s_at + PM * (PI / 128) * 4);      // quantized activation and its scales, written [PI / 128, PM] with deep
+        {
+            const Scratch room(ws_at + std::max<int64_t>(bytes, 0));      // quantized x, its scales, workspace: the down projection finds room where these were
+            done(mdy_act_quant_typed(r.t->data_ptr(), r.xt, 128, room.at(0), (float*)room.at(s_at), M, r.K, r.stride, PM, K, rs, cs, mode, stream));
+            done(mdy_fp8_gemm_swiglu(room.at(0), (float*)room.at(s_at), rs, cs, raw(*qwu), f32(*swu), M, N2, K, gate_first, act.at(0), (float*)act.at(act_s_at), PM,
+                                     PI, act_rs, cs, mode, bytes > 0 ? room.at(ws_at) : nullptr, bytes > 0 ? bytes : 0, stream));
+        }
+        Tensor c = make(sizes, ScalarType::BFloat16, dev);
+        if (!gemm(act.at(0), (const float*)act.at(act_s_at), act_rs, cs, raw(*qwd), f32(*swd), raw(c), nullptr, 0, M, N, PI, MDY_FMT_E4M3, MDY_DT_BF16, stream))
+            throw Rejected();
+        return c;
     }));
 }
 
@@ -958,7 +1003,7 @@ PyObject* guarded(PyObject* self, PyObject* const* args, Py_ssize_t n) {
 
 #define MDY_METHOD(F) {#F, (PyCFunction)(void (*)(void))guarded<F>, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {MDY_METHOD(act_quant), MDY_METHOD(fp8_gemm), MDY_METHOD(weight_dequant), MDY_METHOD(matmul), MDY_METHOD(quant_input),
-                         MDY_METHOD(deep_linear), MDY_METHOD(silu_act_quant), MDY_METHOD(deep_forward), MDY_METHOD(deep_backward),
+                         MDY_METHOD(deep_linear), MDY_METHOD(cached_weight), MDY_METHOD(silu_act_quant), MDY_METHOD(deep_forward), MDY_METHOD(deep_backward),
                          MDY_METHOD(official_forward), MDY_METHOD(ordinary), MDY_METHOD(version_guard), MDY_METHOD(official_backward), MDY_METHOD(act_copies), MDY_METHOD(block_copies),
                          MDY_METHOD(quant_weight), MDY_METHOD(quant_transposed), MDY_METHOD(row_scaled_product), MDY_METHOD(silu_fwd),
                          MDY_METHOD(silu_bwd), MDY_METHOD(mlp), MDY_METHOD(mlp_backward), MDY_METHOD(group_cast), MDY_METHOD(grouped_matmul), MDY_METHOD(move_rows),

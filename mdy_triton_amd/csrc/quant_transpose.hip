@@ -328,7 +328,7 @@ int launch_swiglu_bwd_quant(const void* x, const void* d, void* act_t, float* ac
     if (!grid_rows(PI / 128, PM / 128, grid)) return kErrTooManyBlocks;
     const int up_off = gate_first ? (int)I : 0, gate_off = gate_first ? 0 : (int)I;
 #define MDY_SBQ(MODE)                                                                                                                         \
-    hipLaunchKernelGGL((swiglu_bwd_quant_kernel<MODE>), grid, dim3(2048 / RPT), 0, stream, static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(d), \
+    launch_kernel((swiglu_bwd_quant_kernel<MODE>), grid, dim3(2048 / RPT), 0, stream, static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(d), \
                        static_cast<uint8_t*>(act_t), act_ts, static_cast<uint8_t*>(y), s, static_cast<uint8_t*>(y_t), s_t, (int)M, (int)I, up_off, gate_off, \
                        (int)PM)
     if (mode == 0) MDY_SBQ(0); else if (mode == 1) MDY_SBQ(1); else MDY_SBQ(2);
@@ -377,7 +377,7 @@ static int launch_qt(int mode, const void* x, int x_dtype, void* y, float* s, vo
     uint8_t* yp = static_cast<uint8_t*>(y);
     uint8_t* ytp = static_cast<uint8_t*>(y_t);
 #define MDY_QT(MODE, TM, VEC, XT)                                                                                        \
-    hipLaunchKernelGGL((quant_transpose_kernel<MODE, TM, VEC, XT>), grid, block, 0, stream, x, yp, s, ytp, s_t,          \
+    launch_kernel((quant_transpose_kernel<MODE, TM, VEC, XT>), grid, block, 0, stream, x, yp, s, ytp, s_t,          \
                        (int)M, (int)K, x_row_stride, x_col_stride, (int)PM, (int)PK, s_kb_stride, s_m_stride,           \
                        st_a_stride, st_k_stride, static_cast<float*>(nullptr))
 #define MDY_QT_V(MODE, TM, XT) do { if (vec) MDY_QT(MODE, TM, true, XT); else MDY_QT(MODE, TM, false, XT); } while (0)
@@ -429,7 +429,7 @@ int launch_quant_transpose_grouped(const void* x, int x_dtype, void* y, float* s
         uint8_t* yg = static_cast<uint8_t*>(y) + row0 * K;
         float* sg = s + row0;
 #define MDY_QTG(VEC, XT)                                                                                                        \
-    hipLaunchKernelGGL((quant_transpose_grouped_kernel<VEC, XT>), grid, dim3(2048 / RPT), 0, stream, xg, yg, sg, rows, (int)K, x_row_stride, \
+    launch_kernel((quant_transpose_grouped_kernel<VEC, XT>), grid, dim3(2048 / RPT), 0, stream, xg, yg, sg, rows, (int)K, x_row_stride, \
                        x_col_stride, M, groups)
 #define MDY_QTG_V(XT) do { if (vec) MDY_QTG(true, XT); else MDY_QTG(false, XT); } while (0)
         if (x_dtype == 0) MDY_QTG_V(0); else if (x_dtype == 1) MDY_QTG_V(1); else MDY_QTG_V(2);
@@ -476,7 +476,7 @@ int launch_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, f
     const bool deep = mode == 1;
     const int64_t s_kb = deep ? s_kb_stride : 1, s_m = deep ? 1 : PK / 128, st_a = deep ? PK : 1, st_k = deep ? 1 : PM / 128;
 #define MDY_QTC(MODE, VEC)                                                                                                        \
-    hipLaunchKernelGGL((quant_transpose_kernel<MODE, 0, VEC, 0, true>), grid, dim3(2048 / RPT), 0, stream, x, static_cast<uint8_t*>(y), s, \
+    launch_kernel((quant_transpose_kernel<MODE, 0, VEC, 0, true>), grid, dim3(2048 / RPT), 0, stream, x, static_cast<uint8_t*>(y), s, \
                        static_cast<uint8_t*>(y_t), s_t, (int)M, (int)K, x_row_stride, x_col_stride, (int)PM, (int)PK, s_kb, s_m, st_a, st_k, part)
 #define MDY_QTC_V(MODE) do { if (vec) MDY_QTC(MODE, true); else MDY_QTC(MODE, false); } while (0)
     if (PM > 0) {
@@ -486,7 +486,7 @@ int launch_quant_transpose_colsum(const void* x, void* y, float* s, void* y_t, f
 #undef MDY_QTC
     const int rc = (int)hipGetLastError();
     if (rc != 0 || K == 0) return rc;
-    hipLaunchKernelGGL(col_sum_reduce_kernel, dim3((unsigned)((K + 31) / 32)), dim3(256), 0, stream, part, static_cast<uint16_t*>(col_sum),
+    launch_kernel(col_sum_reduce_kernel, dim3((unsigned)((K + 31) / 32)), dim3(256), 0, stream, part, static_cast<uint16_t*>(col_sum),
                        (int)(PM / 128), (int)K, (int)PK);
     return (int)hipGetLastError();
 }

@@ -154,7 +154,7 @@ int launch_swiglu_slabs(const float* ws, void* y, float* s, int64_t M, int64_t N
     dim3 grid;
     if (!grid_rows((PN + 511) / 512, (PM + kSgWaves - 1) / kSgWaves, grid)) return kErrTooManyBlocks;
 #define MDY_SS(MODE, KS)                                                                                                                  \
-    hipLaunchKernelGGL((swiglu_slabs_kernel<MODE, KS>), grid, dim3(256), 0, stream, ws, static_cast<uint8_t*>(y), s, (int)M, (int)N, 2 * M * N, \
+    launch_kernel((swiglu_slabs_kernel<MODE, KS>), grid, dim3(256), 0, stream, ws, static_cast<uint8_t*>(y), s, (int)M, (int)N, 2 * M * N, \
                        up_off, gate_off, (int)PM, (int)PN, s_row_stride, s_col_stride, ksplit)
 #define MDY_SS_K(MODE) do { if (ksplit == 2) MDY_SS(MODE, 2); else if (ksplit == 3) MDY_SS(MODE, 3); else if (ksplit == 4) MDY_SS(MODE, 4); else MDY_SS(MODE, 0); } while (0)
     if (mode == 0) MDY_SS_K(0); else MDY_SS_K(1);
@@ -223,7 +223,7 @@ int launch_swiglu(const void* x, void* act, void* y, float* s, int64_t M, int64_
         float* sp = quant ? s + r0 * s_row_stride : nullptr;
         const int pm = quant ? (int)n_rows : 0;
 #define MDY_SG(MODE, QUANT, VEC)                                                                                     \
-    hipLaunchKernelGGL((swiglu_kernel<MODE, QUANT, VEC>), grid, block, 0, stream, xp, ap, yp, sp, (int)m, (int)N,      \
+    launch_kernel((swiglu_kernel<MODE, QUANT, VEC>), grid, block, 0, stream, xp, ap, yp, sp, (int)m, (int)N,      \
                        x_row_stride, up_off, gate_off, pm, (int)PN, s_row_stride, s_col_stride, by_xcd)
         if (!quant) {
             if (vec) MDY_SG(0, false, true); else MDY_SG(0, false, false);
@@ -249,9 +249,9 @@ int launch_swiglu_bwd(const void* x, const void* dy, void* dx, int64_t M, int64_
     const uint16_t* dyp = static_cast<const uint16_t*>(dy);
     uint16_t* dxp = static_cast<uint16_t*>(dx);
     if (vec)
-        hipLaunchKernelGGL((swiglu_bwd_kernel<true>), grid, dim3(256), 0, stream, xp, dyp, dxp, (int)M, (int)N, x_row_stride, up_off, gate_off);
+        launch_kernel((swiglu_bwd_kernel<true>), grid, dim3(256), 0, stream, xp, dyp, dxp, (int)M, (int)N, x_row_stride, up_off, gate_off);
     else
-        hipLaunchKernelGGL((swiglu_bwd_kernel<false>), grid, dim3(256), 0, stream, xp, dyp, dxp, (int)M, (int)N, x_row_stride, up_off, gate_off);
+        launch_kernel((swiglu_bwd_kernel<false>), grid, dim3(256), 0, stream, xp, dyp, dxp, (int)M, (int)N, x_row_stride, up_off, gate_off);
     return (int)hipGetLastError();
 }
 

@@ -101,15 +101,15 @@ int launch_weight_dequant(const void* x, const float* s, void* y, int64_t N, int
     if (out_dtype == 0) {
         uint16_t* yp = static_cast<uint16_t*>(y);
         if (vec)
-            hipLaunchKernelGGL((weight_dequant_kernel<uint16_t, true>), grid, block, 0, stream, xp, s, yp, (int)N, (int)K, sK, bshift);
+            launch_kernel((weight_dequant_kernel<uint16_t, true>), grid, block, 0, stream, xp, s, yp, (int)N, (int)K, sK, bshift);
         else
-            hipLaunchKernelGGL((weight_dequant_kernel<uint16_t, false>), grid, block, 0, stream, xp, s, yp, (int)N, (int)K, sK, bshift);
+            launch_kernel((weight_dequant_kernel<uint16_t, false>), grid, block, 0, stream, xp, s, yp, (int)N, (int)K, sK, bshift);
     } else {
         float* yp = static_cast<float*>(y);
         if (vec)
-            hipLaunchKernelGGL((weight_dequant_kernel<float, true>), grid, block, 0, stream, xp, s, yp, (int)N, (int)K, sK, bshift);
+            launch_kernel((weight_dequant_kernel<float, true>), grid, block, 0, stream, xp, s, yp, (int)N, (int)K, sK, bshift);
         else
-            hipLaunchKernelGGL((weight_dequant_kernel<float, false>), grid, block, 0, stream, xp, s, yp, (int)N, (int)K, sK, bshift);
+            launch_kernel((weight_dequant_kernel<float, false>), grid, block, 0, stream, xp, s, yp, (int)N, (int)K, sK, bshift);
     }
     return (int)hipGetLastError();
 }

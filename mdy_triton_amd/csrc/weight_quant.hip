@@ -151,10 +151,10 @@ int launch_weight_quant(const void* const* w, int64_t G, int w_dtype, void* y, f
 #define MDY_WQ(MODE, VEC, XT)                                                                                            \
     do {                                                                                                                 \
         if (n == 1)                                                                                                      \
-            hipLaunchKernelGGL((weight_quant_kernel<MODE, VEC, XT>), grid, block, 0, stream, list.w[0], yp, sp, ytp, stp, (int)N, (int)K, \
+            launch_kernel((weight_quant_kernel<MODE, VEC, XT>), grid, block, 0, stream, list.w[0], yp, sp, ytp, stp, (int)N, (int)K, \
                                w_row_stride, w_col_stride, (int)PN, (int)PK);                                            \
         else                                                                                                             \
-            hipLaunchKernelGGL((weight_quant_group_kernel<MODE, VEC, XT>), grid, block, 0, stream, list, n, yp, sp, ytp, stp, (int)N, (int)K, \
+            launch_kernel((weight_quant_group_kernel<MODE, VEC, XT>), grid, block, 0, stream, list, n, yp, sp, ytp, stp, (int)N, (int)K, \
                                w_row_stride, w_col_stride, (int)PN, (int)PK);                                            \
     } while (0)
 #define MDY_WQ_V(MODE, XT) do { if (vec) MDY_WQ(MODE, true, XT); else MDY_WQ(MODE, false, XT); } while (0)

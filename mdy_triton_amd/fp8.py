@@ -11,7 +11,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from ._torch_glue import FP8, check, gemm_workspace, host, lib, on_device, ptr, require_gpu, stream_ptr, warn_if_scalar_gemm, xt_code
+from ._torch_glue import FP8, check, gemm_workspace, host, lib, on_device, parameter_of, ptr, require_gpu, stream_ptr, warn_if_scalar_gemm, xt_code
 
 
 def _cdiv(a: int, b: int) -> int:
@@ -307,11 +307,15 @@ class DeepLinear(torch.nn.Linear):
         if flag:
             self.invalidate_weight_cache()
 
-    def _quantized_weight(self, with_transpose: bool):
-        w = self.weight
+    def _quantized_weight(self, with_transpose: bool, w=None):
+        w = self.weight if w is None else w
+        cached = getattr(self, "_wq_cache", None)
+        if not self.check_weight_cache:
+            hit = host().cached_weight(w, cached, with_transpose)
+            if hit is not None:
+                return hit
         key = (w.data_ptr(), w._version, w.shape, w.device)
         checking = self.check_weight_cache or os.environ.get("MDY_FP8_CHECK_WEIGHT_CACHE", "0") not in ("", "0")
-        cached = getattr(self, "_wq_cache", None)
         if cached is not None and cached[0] == key and (cached[1][2] is not None or not with_transpose):
             if checking and cached[2] is not None and cached[2] != self._fingerprint(w):
                 raise RuntimeError(
@@ -324,17 +328,16 @@ class DeepLinear(torch.nn.Linear):
 
     def forward(self, input):
         grad = torch.is_grad_enabled()
-        bias = self.bias
+        w, bias = parameter_of(self, "weight"), parameter_of(self, "bias")
         if not grad and (bias is None or bias.dtype == torch.bfloat16):
             # nothing to keep for a backward pass: both launches by one native call
-            weight = self._quantized_weight(False) if self.cache_weight else quant_weight(self.weight)
-            done = host().deep_linear(input, weight[0], weight[1], self.weight.size(0), bias,
-                                      BIAS_IN_SUM if self.fuse_bias else BIAS_AFTER_ROUNDING)
+            weight = self._quantized_weight(False, w) if self.cache_weight else quant_weight(w)
+            done = host().deep_linear(input, weight[0], weight[1], w.size(0), bias, BIAS_IN_SUM if self.fuse_bias else BIAS_AFTER_ROUNDING)
             if done is not None:
                 return done
             # something else than a plain call: the function gets the arguments it always got where it is traced or transformed
-            if not self.cache_weight and not host().ordinary(self.weight):
+            if not self.cache_weight and not host().ordinary(w):
                 weight = None
-            return _DeepLinear.apply(input, self.weight, bias, False, weight, self.fuse_bias)
-        cache = self._quantized_weight(grad and input.requires_grad) if self.cache_weight else None
-        return _DeepLinear.apply(input, self.weight, bias, grad, cache, self.fuse_bias)
+            return _DeepLinear.apply(input, w, bias, False, weight, self.fuse_bias)
+        cache = self._quantized_weight(grad and input.requires_grad, w) if self.cache_weight else None
+        return _DeepLinear.apply(input, w, bias, grad, cache, self.fuse_bias)

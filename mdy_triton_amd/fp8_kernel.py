@@ -15,7 +15,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from ._torch_glue import FP8, check, gemm_workspace, host, lib, on_device, ptr, require_gpu, rowscaled_workspace, stream_ptr, xt_code
+from ._torch_glue import FP8, check, gemm_workspace, host, lib, on_device, parameter_of, ptr, require_gpu, rowscaled_workspace, stream_ptr, xt_code
 
 _ORDERS = ("up-gate", "gate-up")
 
@@ -668,21 +668,21 @@ class Fp8MLP(torch.nn.Module):
 
     def forward(self, hidden_states, low_memory=False):
         up, down = self.up_gate_proj, self.down_proj
-        needs_grad = torch.is_grad_enabled() and (hidden_states.requires_grad or up.weight.requires_grad or
-                                                  down.weight.requires_grad)
-        if not needs_grad and host().ordinary(hidden_states, up.weight, down.weight):
+        w_up, w_down = parameter_of(up, "weight"), parameter_of(down, "weight")
+        needs_grad = torch.is_grad_enabled() and (hidden_states.requires_grad or w_up.requires_grad or w_down.requires_grad)
+        if not needs_grad and host().ordinary(hidden_states, w_up, w_down):
             # nothing to differentiate and nothing that traces or transforms the call: no autograd function around it
             if self.dialect == "official":
-                y = _official_mlp(hidden_states.reshape(-1, hidden_states.size(-1)), up.weight, down.weight, self.fp8_dtype, self.order)
-                return y.view(*hidden_states.shape[:-1], down.weight.size(0))
-            return _deep_mlp(hidden_states, up.weight, down.weight, self.order,
-                             up._quantized_weight(False) if up.cache_weight else None,
-                             down._quantized_weight(False) if down.cache_weight else None)
+                y = _official_mlp(hidden_states.reshape(-1, hidden_states.size(-1)), w_up, w_down, self.fp8_dtype, self.order)
+                return y.view(*hidden_states.shape[:-1], w_down.size(0))
+            return _deep_mlp(hidden_states, w_up, w_down, self.order,
+                             up._quantized_weight(False, w_up) if up.cache_weight else None,
+                             down._quantized_weight(False, w_down) if down.cache_weight else None)
         if not needs_grad or low_memory or self.low_memory:
             if self.dialect == "official":
-                return _Fp8MlpCkptOfficial.apply(hidden_states, up.weight, down.weight, self.fp8_dtype, self.order)
+                return _Fp8MlpCkptOfficial.apply(hidden_states, w_up, w_down, self.fp8_dtype, self.order)
             # cached quantized weights (when the projections cache); the forward needs no transposed copies
-            return _Fp8MlpCkptOps.apply(hidden_states, up.weight, down.weight, self.fp8_dtype, self.order,
-                                        up._quantized_weight(False) if up.cache_weight else None,
-                                        down._quantized_weight(False) if down.cache_weight else None)
+            return _Fp8MlpCkptOps.apply(hidden_states, w_up, w_down, self.fp8_dtype, self.order,
+                                        up._quantized_weight(False, w_up) if up.cache_weight else None,
+                                        down._quantized_weight(False, w_down) if down.cache_weight else None)
         return down(triton_silu(up(hidden_states), self.order))
