@@ -10,7 +10,8 @@
 // fold would be 4 multiplies + 4 FMAs per MFMA instead of 4 FMAs, as much work as the matrix cores have; the scheduled tile body of fp8_gemm_tile.h
 // forms the products on the matrix cores instead (scale_products there).  It takes 256x256 tiles where their rounds come out ahead (a
 // quarter fewer LDS reads and a third fewer copies per MFMA than 128x256: 4096x7168x4096 154 -> 130 us, 4096x4096x8192 159 -> 136 us; with the
-// products on the matrix cores 120.6 -> 115.0 and 129.1 -> 122.9 us = 2.09 and 2.24 PFLOP/s), 128x256 and 128x128 tiles otherwise; a plain
+// products on the matrix cores 120.6 -> 115.0 and 129.1 -> 122.9 us = 2.09 and 2.24 PFLOP/s; row-major scales, copied in chunks of four K blocks,
+// no longer cost more than column-major ones, 131 -> 120 us), 128x256 and 128x128 tiles otherwise; a plain
 // loop (128x128 tile, four waves of 64x64, the K block's two panels and two scale vectors copied global -> LDS by `buffer_load
 // ... lds`, double buffered, one barrier per K block: short ends, but 0.93 us per K block against 0.72) runs what has few K blocks.
 // K % 128 == 0 (the callers contract over a padded token count).
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_tile_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, int bs_rs, int bs_cs, uint32_t bs_bytes,
     OUT* __restrict__ c, int M, int N, int K, int tiles_m, int tiles_n) {
-    using L = TileLds<BM, BN, 8, STAGES>;
+    using L = TileLds<BM, BN, 8, STAGES, true>;
     constexpr bool WALK = walks(BM, BN, STAGES, (int)sizeof(OUT), EPI);
     __shared__ __attribute__((aligned(1024))) uint8_t pool[WALK ? L::walk_bytes : L::bytes];
     const int ntiles = tiles_m * tiles_n;
@@ -166,7 +167,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_rowscaled_small_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, int bs_rs, int bs_cs, uint32_t bs_bytes,
     OUT* __restrict__ c, int M, int N, int K, int tiles_m, int tiles_n) {
-    __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<128, 128, 4, STAGES>::bytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<128, 128, 4, STAGES, true>::bytes];
     int tm, tn;
     const Duty duty = tile_of(xcd_contiguous(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
     fp8_gemm_tile<128, 128, 2, 2, STAGES, OUT, 0, 0, 0, FMT, true, EPI>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, Bias{}, tm * 128, M, M, tn * 128, N,
@@ -180,7 +181,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, int bs_rs, int bs_cs, uint32_t bs_bytes,
     float* __restrict__ ws, int M, int N, int K, int tiles_m, int tiles_n, int slabs, int kb_per) {
-    __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<128, 256, 8, 3>::bytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<128, 256, 8, 3, true>::bytes];
     const int ntiles = tiles_m * tiles_n;
     // runs per XCD from 13 K blocks per slab on, against K > 8192 from 10 (runs against plain order, warm / cold: 768x512x11648, slabs of 7,
     // 21.9 -> 23.5 / 23.7 -> 26.2 us, 512x1152x10368 (9) 24.0 -> 24.8 / 26.0 -> 27.1, 2304x512x3712 (10) 22.0 -> 23.5 / 24.8 -> 27.0; 640x768x15232

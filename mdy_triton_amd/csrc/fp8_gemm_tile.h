@@ -254,29 +254,45 @@ struct Duty {
 
 // LDS of one tile workgroup, carved out of a pool that the kernel declares: the ring of A and B panels, the ring of activation scales, the tile's weight
 // scales for all K blocks, and a dummy area for copies that must go nowhere.
-template <int BM, int BN, int WAVES, int STAGES>
+//
+// CHUNKED: row scales (of the activations, with BROW of the weight rows behind them) come in chunks of 4 K blocks, [group of 16 rows][row]
+// [K block % 4]: a copy of a wave takes 16 rows x 4 K blocks, which with row-major scales, the official dialect's, is 16 lines; one K block of 64
+// rows is 64.  Part r of a chunk (groups r * WAVES ..) goes out with the copies of the K block PARTS - 1 - r in front of the chunk.  With row scales on
+// both sides, 16 lines a copy of the 32 that a chunk takes instead of 64 of 32: 8192x4096x4096 row-major 138 -> 129 us, column-major as before
+// (128).  Against one operand's it pays with 128x256 tiles and row-major scales (1500x4096x4096 33.8 -> 32.3, column-major 30.8 -> 32.4), not with
+// 256x256 (2048x18432x2048 82.9 -> 85.9 row-major, 81.8 -> 85.9) or 64x64 (65x1024x4096 8.83 -> 8.88, 8.4 -> 8.9): those copy a K block at a time.
+template <int BM, int BN, int WAVES, int STAGES, bool BROW = false, bool CHUNKED = BROW>
 struct TileLds {
     static constexpr int NBS = (BN + 127) / 128;
+    static constexpr int GROUPS = BM / 16 + (BROW ? BN / 16 : 0), PARTS = CHUNKED ? (GROUPS + WAVES - 1) / WAVES : 1;
+    // Part 0 of chunk c + 1 is copied behind the barrier of K block 4 c + 5 - PARTS - STAGES, when the scales of the next one are read: the chunks
+    // from that one's to c + 1 have a buffer each.
+    static constexpr int CHUNKS = PARTS + STAGES <= 6 ? 2 : 2 + (PARTS + STAGES - 6 + 3) / 4;
     static constexpr int a_off = 0;
     static constexpr int b_off = a_off + STAGES * BM * 128;
     static constexpr int s_off = b_off + STAGES * BN * 128;
-    static constexpr int bs_off = s_off + (STAGES * BM * 4 + 255) / 256 * 256;
-    static constexpr int dummy_off = bs_off + NBS * 512 * 4;
+    static constexpr int bs_off = s_off + (CHUNKED ? CHUNKS * GROUPS * 256 : (STAGES * BM * 4 + 255) / 256 * 256);
+    static constexpr int dummy_off = bs_off + (BROW ? 0 : NBS * 512 * 4);
     static constexpr int bytes = dummy_off + WAVES * 512;
-    // a workgroup that walks its tiles: 16 rows of results of every wave on their way to memory, beside a ring that already
-    // receives the next tile
-    static constexpr int rows_off = bytes, walk_bytes = bytes + WAVES * 2048;
+    // A workgroup that walks its tiles: 16 rows of results of every wave on their way to memory, beside a ring that already
+    // receives the next tile.  256x256 tiles with row scales on both sides fill the CU's LDS without a dummy area: a wave's touches go where its
+    // rows of results go later.
+    static constexpr bool no_dummy = BROW && bytes + WAVES * 2048 > 160 * 1024;
+    static constexpr int rows_off = no_dummy ? dummy_off : bytes, walk_bytes = rows_off + WAVES * 2048;
 };
 
-// LDS of a wave-specialized tile workgroup: separate ring depths for the a panels, the b panels and the activation scales.
-template <int BM, int BN, int WAVES, int SA, int SB, int SS>
+// K blocks whose activation scales a wave-specialized tile can hold at once (PRE_ of fp8_gemm_tile_ws).
+constexpr int kPreBlocks = 64;
+// LDS of a wave-specialized tile workgroup: separate ring depths for the a panels, the b panels and the activation scales (PRE: no ring
+// but those of all K blocks).
+template <int BM, int BN, int WAVES, int SA, int SB, int SS, bool PRE = false>
 struct TileLdsWs {
     static constexpr int NBS = (BN + 127) / 128;
     static constexpr int BSROW = 512;
     static constexpr int a_off = 0;
     static constexpr int b_off = a_off + SA * BM * 128;
     static constexpr int s_off = b_off + SB * BN * 128;
-    static constexpr int bs_off = s_off + (SS * BM * 4 + 255) / 256 * 256;
+    static constexpr int bs_off = s_off + ((PRE ? kPreBlocks : SS) * BM * 4 + 255) / 256 * 256;
     static constexpr int dummy_off = bs_off + NBS * BSROW * 4;
     static constexpr int bytes = dummy_off + WAVES * 512;
 };
@@ -317,7 +333,7 @@ struct OneTile {};
 // (Those without a bias.  With one its loads complete behind the copies that went out in front of them, and the stores wait for
 // both: 0 to 4 us more, 3752x15224x768 64.5 -> 68.6 us, 16384x4096x1024 78.1 -> 79.4, none from K = 4096 on.)
 template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ = 0, int TD_ = 0, int ABL_ = 0, int FMT_ = 0,
-          bool BROW_ = false, int EPI_ = kEpiDirect, typename NEXT = OneTile>
+          bool BROW_ = false, int EPI_ = kEpiDirect, bool CHUNKED_ = BROW_, typename NEXT = OneTile>
 __device__ __forceinline__ void fp8_gemm_tile(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
@@ -333,14 +349,13 @@ __device__ __forceinline__ void fp8_gemm_tile(
     constexpr int WM = BM / WGM, WN = BN / WGN, TI = WM / 16, TJ = WN / 16;
     constexpr int PASS_ROWS = WAVES * 8;  // rows copied by one DMA instruction of every wave
     constexpr int A_PASSES = BM / PASS_ROWS, B_PASSES = BN / PASS_ROWS;
-    constexpr int S_WAVES = BM / 64;      // waves that also copy the activation scales
     constexpr int DEPTH = 4;              // MFMAs in flight before their results are folded
     static_assert(BM % PASS_ROWS == 0 && BN % PASS_ROWS == 0 && PASS_ROWS % 16 == 0, "tile/threads mismatch");
     // A wave's WN columns lie in one 128-column weight-scale block when WN divides 128 (tiles then start on multiples
     // of WN); the 192-wide tile (WN = 48, tiles start on multiples of 64) can straddle two: its 16-column sub-tiles never
     // do, so such a wave keeps two combined scales per row and each sub-tile takes the one of its block.
     constexpr bool STRADDLE = (128 % WN) != 0;
-    static_assert(WN <= 128 && (!STRADDLE || BN == 192) && S_WAVES <= WAVES && WAVES >= 2, "weight-scale blocks per wave column");
+    static_assert(WN <= 128 && (!STRADDLE || BN == 192) && WAVES >= 2, "weight-scale blocks per wave column");
     constexpr bool HOLD_A = TI <= TJ;
     constexpr int NH = HOLD_A ? TI : TJ, NS = HOLD_A ? TJ : TI;
     constexpr int NT = TI * TJ;
@@ -366,44 +381,43 @@ __device__ __forceinline__ void fp8_gemm_tile(
     static_assert(NS % 2 == 0 && NS >= 2, "the first streamed fragment of the next K block reuses queue slot 0");
     static_assert(TOUCH < TB, "not enough slots in front of the barrier");
 
-    using L = TileLds<BM, BN, WAVES, STAGES>;
-    constexpr int NBS = L::NBS;
+    using L = TileLds<BM, BN, WAVES, STAGES, BROW_, CHUNKED_>;
+    constexpr int NBS = L::NBS, PARTS = L::PARTS, PARTS_A = BM / 16 / WAVES, CHUNKS = L::CHUNKS, CHUNK = L::GROUPS * 64;      // (floats)
+    constexpr int S_WAVES = BM / 64;      // !CHUNKED_: waves that also copy 64 activation scales of the K block each
+    constexpr bool NO_DUMMY = WALK && L::no_dummy;
+    static_assert(CHUNKED_ ? BM / 16 % WAVES == 0 && PARTS <= 4 && (!BROW_ || BN / 16 % WAVES == 0) : !BROW_ && S_WAVES <= WAVES,
+                  "a part of a chunk is a group of 16 rows for every wave, a K block has one part");
+    static_assert(!NO_DUMMY || L::GROUPS == 4 * WAVES, "every scale copy has a part to go to");
     uint8_t(*lds_a)[BM * 128] = reinterpret_cast<uint8_t(*)[BM * 128]>(pool + L::a_off);     // [STAGES]
     uint8_t(*lds_b)[BN * 128] = reinterpret_cast<uint8_t(*)[BN * 128]>(pool + L::b_off);     // [STAGES]
-    float(*lds_s)[BM] = reinterpret_cast<float(*)[BM]>(pool + L::s_off);                      // [STAGES]
+    const float* lds_s = reinterpret_cast<const float*>(pool + L::s_off);                     // [CHUNKS][GROUPS][16][4]; !CHUNKED_: [STAGES][BM]
     float(*lds_bs)[512] = reinterpret_cast<float(*)[512]>(pool + L::bs_off);                  // [NBS] weight scales, all K blocks
-    uint8_t* lds_dummy = pool + L::dummy_off;                                                 // target of copies that must go nowhere
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
+    const uint32_t dummy = lds_addr(pool + (NO_DUMMY ? L::rows_off : L::dummy_off)) + wave * (NO_DUMMY ? 2048 : 512);      // target of copies that must go nowhere
     const int M = m_end;
     const int KB = K >> 7;
 
     // ---- DMA.  What depends on the tile: the descriptors (limited to the rows of the tile, so that the M and N
-    // tails read 0), the rows whose scales a lane copies, and the share of the panels this workgroup pre-touches.
+    // tails read 0), its place, and the share of the panels this workgroup pre-touches.
     struct TileAddr {
         intx4 ra, rb, rt;
-        int s_voff, touch_off, n0;
+        int s_voff, touch_off, m0, n0;
     };
     const int prow = wave * 8 + (lane >> 3);                          // row inside a pass
     const int voff = prow * K + (((lane & 7) ^ swz(prow)) << 4);      // permuted chunk of that row
-    // scale copies: waves 0 .. S_WAVES-1 copy 64 activation scales of the K block each; with BROW_ the next BN / 64 waves
-    // copy 64 weight-row scales each (into the area that otherwise holds the weight's block scales); the rest copy nothing
-    constexpr int SB_WAVES = BROW_ ? BN / 64 : 0;
-    static_assert(S_WAVES + SB_WAVES <= WAVES && (!BROW_ || STAGES * BN * 4 <= L::NBS * 512 * 4), "waves / LDS for the weight-row scales");
-    const bool sb_wave = BROW_ && wave >= S_WAVES && wave < S_WAVES + SB_WAVES;
-    float* lds_sbr = reinterpret_cast<float*>(pool + L::bs_off);     // BROW_: [STAGES][BN] weight-row scales
-    intx4 rs = sb_wave ? make_rsrc(b_s, bs_bytes) : make_rsrc(a_s, as_bytes);
-    if (wave >= S_WAVES && !sb_wave) rs[2] = 0;                       // these waves copy no scales: always out of range
-    const int sc_cs = sb_wave ? bs_cs : as_cs;
-    const uint32_t sc_bytes = sb_wave ? bs_bytes : as_bytes;
-    const uint32_t ld_base = lds_addr(&lds_dummy[0]) + wave * 512;
+    // scale copies: lane -> row lane / 4 of the wave's group, K block lane % 4 of the chunk.  Rows beyond the matrix read what lies there, or
+    // zeros beyond the array: nothing they scale is stored.
+    const bool s_none = !CHUNKED_ && wave >= S_WAVES;                 // this wave copies no scales: always out of range
+    const intx4 rsa = make_rsrc(a_s, s_none ? 0u : as_bytes), rsb = make_rsrc(BROW_ ? b_s : a_s, BROW_ ? bs_bytes : 0u);
+    const int srow = wave * 16 + (lane >> 2);
+    const auto scale_offset = [](int row, int rs, int kb, int cs) { return (int)(((uint32_t)row * (uint32_t)rs + (uint32_t)kb * (uint32_t)cs) * 4u); };
+    const int sa_voff = scale_offset(srow, as_rs, lane & 3, as_cs), sb_voff = BROW_ ? scale_offset(srow, bs_rs, lane & 3, bs_cs) : 0;
+    const uint32_t ls_base = s_none ? dummy : lds_addr(pool + L::s_off) + wave * 256, ls_buf = s_none ? 0 : BM * 4;
     const uint32_t la_base = lds_addr(&lds_a[0][0]) + wave * 1024;
     const uint32_t lb_base = lds_addr(&lds_b[0][0]) + wave * 1024;
-    const uint32_t ls_base = wave < S_WAVES ? lds_addr(&lds_s[0][0]) + wave * 256
-                             : sb_wave ? lds_addr(lds_sbr) + (wave - S_WAVES) * 256 : ld_base;
-    const uint32_t ls_buf = wave < S_WAVES ? BM * 4 : sb_wave ? BN * 4 : 0;
     // duty touch: the even waves load one dword of every line of this workgroup's share of the B panel (64
     // rows per wave), the odd waves of the A panel, TD K blocks ahead, into the dummy area: the lines are in L2
     // when this workgroup and its neighbours copy them.  Waves beyond the share run the same instruction on an
@@ -414,13 +428,13 @@ __device__ __forceinline__ void fp8_gemm_tile(
         TileAddr t;
         t.ra = make_rsrc(a + (size_t)tm0 * K, (uint32_t)min(BM, M - tm0) * (uint32_t)K);
         t.rb = make_rsrc(b + (size_t)tn0 * K, (uint32_t)min(BN, N - tn0) * (uint32_t)K);
-        t.s_voff = sb_wave ? min(tn0 + (wave - S_WAVES) * 64 + lane, N - 1) * bs_rs * 4
-                           : min(tm0 + (wave % S_WAVES) * 64 + lane, m_total - 1) * as_rs * 4;
         const int share = touch_b ? (BN >> d.b_sh) : (BM >> d.a_sh);      // rows of the share
         t.rt = touch_b ? t.rb : t.ra;
         // nobody to share with: touching one's own lines ahead of the copy only adds requests (measured)
         if ((wave >> 1) * 64 >= share || (touch_b ? d.b_sh : d.a_sh) == 0) t.rt[2] = 0;
         t.touch_off = ((touch_b ? d.b_duty : d.a_duty) * share + t_idx % share) * K;
+        t.s_voff = CHUNKED_ ? 0 : min(tm0 + (wave % S_WAVES) * 64 + lane, m_total - 1) * as_rs * 4;
+        t.m0 = tm0;
         t.n0 = tn0;
         return t;
     };
@@ -428,17 +442,31 @@ __device__ __forceinline__ void fp8_gemm_tile(
 
     // copy i (0: scales, then the A passes, then the B passes) of K block kb into buffer buf.  Past the last K
     // block the offsets run beyond the descriptors: no memory access, zeros into a buffer nobody reads any more.
+    auto scale_part = [&](const TileAddr& t, int part, int chunk, bool on) {
+        const bool weight = BROW_ && part >= PARTS_A;
+        const int rs = weight ? bs_rs : as_rs, cs = weight ? bs_cs : as_cs;
+        const int row0 = weight ? t.n0 + (part - PARTS_A) * (WAVES * 16) : t.m0 + part * (WAVES * 16);
+        const int slot = CHUNKS == 2 ? chunk & 1 : chunk % CHUNKS;
+        dma4(weight ? rsb : rsa, weight ? sb_voff : sa_voff, on ? scale_offset(row0, rs, kb0 + 4 * chunk, cs) : (int)(weight ? bs_bytes : as_bytes),
+             on || NO_DUMMY ? ls_base + slot * (CHUNK * 4) + part * (WAVES * 256) : dummy);
+    };
     auto issue = [&](const TileAddr& t, int i, int kb, int buf) {
         const bool more = kb < kb1;
-        if (i == 0)
-            dma4(rs, t.s_voff, more ? kb * sc_cs * 4 : (int)sc_bytes, ls_base + buf * ls_buf);
-        else if (i <= A_PASSES)
+        if (i == 0 && !CHUNKED_) {
+            dma4(rsa, t.s_voff, more ? kb * as_cs * 4 : (int)as_bytes, ls_base + buf * ls_buf);
+        } else if (i == 0) {
+            const int u = kb - kb0 + PARTS - 1;
+            scale_part(t, u & 3, u >> 2, more && (PARTS == 4 || (u & 3) < PARTS));
+        } else if (i <= A_PASSES)
             dma16(t.ra, voff, (i - 1) * PASS_ROWS * K + (more ? kb * 128 : t.ra[2]), la_base + buf * (BM * 128) + (i - 1) * PASS_ROWS * 128);
         else
             dma16(t.rb, voff, (i - 1 - A_PASSES) * PASS_ROWS * K + (more ? kb * 128 : t.rb[2]),
                   lb_base + buf * (BN * 128) + (i - 1 - A_PASSES) * PASS_ROWS * 128);
     };
-    auto touch = [&](const TileAddr& t, int kb) { dma4(t.rt, t.touch_off, kb < kb1 ? kb * 128 : t.rt[2], ld_base + 256); };
+    // to: where the touch of a tile's start goes without a dummy area, while the last tile's results lie in the rows: a part of the second chunk that
+    // this wave itself copies later (loads complete in order)
+    const uint32_t touch_to = NO_DUMMY ? dummy : dummy + 256, first_touch_to = NO_DUMMY ? ls_base + CHUNK * 4 + (PARTS - 1) * (WAVES * 256) : touch_to;
+    auto touch = [&](const TileAddr& t, int kb, uint32_t to) { dma4(t.rt, t.touch_off, kb < kb1 ? kb * 128 : t.rt[2], to); };
     // The start of a tile: its weight scales, then the copies in the order the K loop keeps up: for every K block its
     // first FIRST copies, the rest, one touch; K blocks 0 .. STAGES-2 whole and the first copies of block STAGES-1.
     auto prologue = [&](const TileAddr& t) {
@@ -448,11 +476,13 @@ __device__ __forceinline__ void fp8_gemm_tile(
             for (int cc = 0; cc < KB; cc += 64) dma4(rbs, lane * 4, cc * 4, lds_addr(&lds_bs[wave][cc]));
         }
 #pragma unroll
+        for (int part = 0; part < (CHUNKED_ ? PARTS - 1 : 0); ++part) scale_part(t, part, 0, true);      // the first chunk; its last part comes with the first K block
+#pragma unroll
         for (int blk = 0; blk < STAGES - 1; ++blk) {
 #pragma unroll
             for (int i = 0; i < NDMA; ++i) issue(t, i, kb0 + blk, blk);
-            if (!NO_TOUCH) touch(t, kb0 + blk + 1 + TD - STAGES);
-            else touch(t, 1 << 20);      // same load count for the waits below: a copy of nothing
+            if (!NO_TOUCH) touch(t, kb0 + blk + 1 + TD - STAGES, first_touch_to);
+            else touch(t, 1 << 20, first_touch_to);      // same load count for the waits below: a copy of nothing
         }
 #pragma unroll
         for (int i = 0; i < (WALK ? NDMA : FIRST); ++i) issue(t, i, kb0 + STAGES - 1, STAGES - 1);
@@ -471,6 +501,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
     const int h0 = HOLD_A ? a_rd0 : b_rd0, h1 = HOLD_A ? a_rd1 : b_rd1;   // held operand
     const int x0 = HOLD_A ? b_rd0 : a_rd0, x1 = HOLD_A ? b_rd1 : a_rd1;   // streamed operand
     const int s_rd = wm * WM + frow;
+    constexpr int S_STRIDE = CHUNKED_ ? 4 : 1;
     const int bs_col = (n0 & 127) + wn * WN;                        // first column of the wave inside the tile's first scale block
     const float* my_bs = lds_bs[bs_col >> 7];
     const float* my_bs_hi = lds_bs[(bs_col + WN - 1) >> 7];         // STRADDLE: the block of the wave's last columns
@@ -504,13 +535,12 @@ __device__ __forceinline__ void fp8_gemm_tile(
     float sc[TI], sc_hi[STRADDLE ? TI : 1];
     // BROW_: the scales of the wave's 64 weight rows and of its activation rows, one a lane
     constexpr int SAV = BROW_ ? TI / 4 : 1;
-    const float* sbr_lane = lds_sbr + wn * WN + lane;
-    const int sar_lane = wm * WM + lane;
+    const int sbr_lane = (BM + wn * WN + lane) * 4, sar_lane = (wm * WM + lane) * 4;
     float sb_row = 1.0f, sa_row[SAV];
     if (BROW_) {
-        sb_row = sbr_lane[0];
+        sb_row = lds_s[sbr_lane];
 #pragma unroll
-        for (int v = 0; v < SAV; ++v) sa_row[v] = lds_s[0][sar_lane + v * 64];
+        for (int v = 0; v < SAV; ++v) sa_row[v] = lds_s[sar_lane + v * 256];
     }
 #pragma unroll
     for (int h = 0; h < NH; ++h) fh[h] = read_frag(HOLD_A ? lds_a[0] : lds_b[0], h0, h1, h);
@@ -518,7 +548,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
         const float sb = my_bs[kb0], sb_hi = my_bs_hi[kb0];
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
-            const float sa = lds_s[0][s_rd + i * 16];
+            const float sa = lds_s[(s_rd + i * 16) * S_STRIDE];
             sc[i] = sa * sb;
             if (STRADDLE) sc_hi[i] = sa * sb_hi;
         }
@@ -534,7 +564,8 @@ __device__ __forceinline__ void fp8_gemm_tile(
         const uint8_t* lx = HOLD_A ? lds_b[cur] : lds_a[cur];            // streamed operand of this K block
         const uint8_t* lh_n = HOLD_A ? lds_a[nxt] : lds_b[nxt];          // operands and scales of the next one
         const uint8_t* lx_n = HOLD_A ? lds_b[nxt] : lds_a[nxt];
-        const float* ls_n = lds_s[nxt];
+        const int bn = kb + 1 - kb0, cn = bn >> 2;
+        const float* ls_n = CHUNKED_ ? lds_s + (CHUNKS == 2 ? cn & 1 : cn % CHUNKS) * CHUNK + (bn & 3) : lds_s + nxt * BM;
         float sa_n[TI], sb_n = 1.0f, sb_hi_n = 1.0f;         // scales of the next K block
         floatx4 p[DEPTH + 1];
         floatx16 sp;                                         // BROW_: scale products of the streamed fragment that is folded
@@ -565,7 +596,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
                             sb_n = my_bs[min(kb + 1, KB - 1)];
                             sb_hi_n = my_bs_hi[min(kb + 1, KB - 1)];
 #pragma unroll
-                            for (int i = 0; i < TI; ++i) sa_n[i] = ls_n[s_rd + i * 16];      // combined at the end of the block: nothing waits here
+                            for (int i = 0; i < TI; ++i) sa_n[i] = ls_n[(s_rd + i * 16) * S_STRIDE];      // combined at the end of the block: nothing waits here
                         }
                     } else {
                         asm volatile("" : "+v"(fx[0]));
@@ -604,11 +635,11 @@ __device__ __forceinline__ void fp8_gemm_tile(
                     if (!FRESH && v >= NSLOT && v - NSLOT == t) issue(me, j, kb + STAGES - 1, last);      // the rest of the block started in kb-1
                 }
             }
-            if (t == TOUCH && !NO_TOUCH) touch(me, kb + TD);
+            if (t == TOUCH && !NO_TOUCH) touch(me, kb + TD, touch_to);
             if (BROW_ && t == NT + DEPTH - 1) {
-                sb_row = sbr_lane[nxt * BN];      // first used NH - 1 MFMAs from here
+                sb_row = ls_n[sbr_lane];      // first used NH - 1 MFMAs from here
 #pragma unroll
-                for (int v = 0; v < SAV; ++v) sa_row[v] = ls_n[sar_lane + v * 64];
+                for (int v = 0; v < SAV; ++v) sa_row[v] = ls_n[sar_lane + v * 256];
             }
             __builtin_amdgcn_sched_barrier(0);  // keep the MFMA / FMA / ds_read / copy interleaving as written
         }
@@ -720,7 +751,11 @@ __device__ __forceinline__ Duty tile_of(int local, int tiles_m, int tiles_n, int
 //   * on the 192-wide tile a wave's columns can straddle two 128-column blocks of weight scales: the combined scale is
 //     kept per row and 32-column group (multiplies once per block instead of a select per MFMA).
 // Swizzle, fragment layout, fold, epilogue and pre-touch shares are fp8_gemm_tile's.
-template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, int FMT_ = 0, int EPI_ = kEpiDirect, int E_ = 2>
+// PRE_: the activation scales of all K blocks (up to kPreBlocks) are copied at the start, 16 rows x 4 K blocks a copy, instead of 64 rows of one K
+// block with every block's panels: with row-major scales, the official dialect's, those were 64 lines of 4 bytes for 128 of panels.  Row-major
+// 777x2112x7168 27.4 -> 25.4 us, 1024x4096x7168 39.4 -> 35.2, 2048x2048x7168 39.2 -> 34.8, 300x7168x4096 23.9 -> 21.2, 128x7168x7168
+// 24.4 -> 22.8, 200x7168x2048 10.4 -> 10.1; column-major 35.6 -> 35.2, 35.2 -> 34.9, the others even.
+template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, int FMT_ = 0, int EPI_ = kEpiDirect, int E_ = 2, bool PRE_ = false>
 __device__ __forceinline__ void fp8_gemm_tile_ws(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
@@ -738,7 +773,7 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
     constexpr bool HOLD_A = TI <= TJ;
     constexpr int NH = HOLD_A ? TI : TJ, NS = HOLD_A ? TJ : TI;
     constexpr int NT = TI * TJ;
-    constexpr int SC = 1;                               // scale copies per K block and producer
+    constexpr int SC = PRE_ ? 0 : 1;                    // scale copies per K block and producer
     constexpr int NDMA = SC + A_PASSES + B_PASSES;
     constexpr int E = E_;
     constexpr int TDA = 2;
@@ -752,11 +787,13 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
     constexpr int PWIN = NT - 2 - (E + 1);
     static_assert(E >= 0 && E < NT - NH && PWIN >= NH, "barrier slot");
 
-    using L = TileLdsWs<BM, BN, CW + PW, SA, SB, SS>;
+    using L = TileLdsWs<BM, BN, CW + PW, SA, SB, SS, PRE_>;
+    static_assert(L::bytes <= 160 * 1024 && (!PRE_ || (BM / 16) % PW == 0), "LDS of a CU; groups of 16 rows per producer");
     constexpr int NBS = L::NBS;
     uint8_t(*lds_a)[BM * 128] = reinterpret_cast<uint8_t(*)[BM * 128]>(pool + L::a_off);
     uint8_t(*lds_b)[BN * 128] = reinterpret_cast<uint8_t(*)[BN * 128]>(pool + L::b_off);
     float(*lds_s)[BM] = reinterpret_cast<float(*)[BM]>(pool + L::s_off);
+    const float* lds_pre = reinterpret_cast<const float*>(pool + L::s_off);      // PRE_: [K block / 4][row][K block % 4]
     float(*lds_bs)[L::BSROW] = reinterpret_cast<float(*)[L::BSROW]>(pool + L::bs_off);
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -809,6 +846,18 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
             const int nb = min((n0 >> 7) + pw, ((N + 127) >> 7) - 1);
             const intx4 rbs = make_rsrc(b_s + (size_t)nb * KB, (uint32_t)KB * 4u);
             for (int cc = 0; cc < KB; cc += 64) dma4(rbs, lane * 4, cc * 4, pool_addr + L::bs_off + (pw * L::BSROW + cc) * 4);
+        }
+        if constexpr (PRE_) {
+            // 16 rows x 4 consecutive K blocks a copy: 16 lines instead of 64
+            constexpr int RG = BM / 16 / PW;
+            int row_off[RG];
+#pragma unroll
+            for (int r = 0; r < RG; ++r) row_off[r] = (min(m0 + (r * PW + pw) * 16 + (lane >> 2), m_total - 1) * as_rs + (kb0 + (lane & 3)) * as_cs) * 4;
+            const intx4 rsp = make_rsrc(a_s, as_bytes);
+            for (int q = 0; q < (kb1 - kb0 + 3) >> 2; ++q) {
+#pragma unroll
+                for (int r = 0; r < RG; ++r) dma4(rsp, row_off[r], q * 16 * as_cs, pool_addr + L::s_off + q * (BM * 16) + (r * PW + pw) * 256);
+            }
         }
 #pragma unroll
         for (int blk = 0; blk < STAGES - 1; ++blk) {
@@ -878,7 +927,7 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
     for (int h = 0; h < NH; ++h) fh_a[h] = read_frag(HOLD_A ? lds_a[0] : lds_b[0], h0, h1, h);
 #pragma unroll
     for (int i = 0; i < TI; ++i) {
-        const float sa = lds_s[0][s_rd + i * 16];
+        const float sa = PRE_ ? lds_pre[(s_rd + i * 16) * 4] : lds_s[0][s_rd + i * 16];
 #pragma unroll
         for (int g = 0; g < NG; ++g) sc_a[i][g] = sa * my_bs[g][kb0];
     }
@@ -906,11 +955,13 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
                 if (t == E) __syncthreads();
                 if (t == E + 1) {
                     float sbg[NG];
+                    const int nb = min(kb + 1, kb1 - 1) - kb0;
+                    const float* ls_pre = lds_pre + (nb >> 2) * (BM * 4) + (nb & 3) + s_rd * 4;
 #pragma unroll
                     for (int g = 0; g < NG; ++g) sbg[g] = my_bs[g][min(kb + 1, KB - 1)];
 #pragma unroll
                     for (int i = 0; i < TI; ++i) {
-                        const float sa = ls_n[s_rd + i * 16];
+                        const float sa = PRE_ ? ls_pre[i * 64] : ls_n[s_rd + i * 16];
 #pragma unroll
                         for (int g = 0; g < NG; ++g) scn[i][g] = sa * sbg[g];
                     }
@@ -962,20 +1013,20 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
 }
 
 // the wave-specialized tile as a kernel: one workgroup of WGM*WGN + PW waves per tile (or per several, walked in turn)
-template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, int FMT_ = 0, int EPI_ = kEpiDirect, int E_ = 2>
+template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, int FMT_ = 0, int EPI_ = kEpiDirect, bool PRE_ = false>
 __global__ __launch_bounds__((WGM * WGN + PW) * 64) void fp8_gemm_ws_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
     const Bias bias, int M, int N, int K, int ldc, int tiles_m, int tiles_n, int pretouch) {
     constexpr bool HOLD_A = BM / WGM <= BN / WGN;
     __shared__ __attribute__((aligned(1024)))
-    uint8_t pool[TileLdsWs<BM, BN, WGM * WGN + PW, HOLD_A ? STAGES - 1 : STAGES, HOLD_A ? STAGES : STAGES - 1, STAGES - 1>::bytes];
+    uint8_t pool[TileLdsWs<BM, BN, WGM * WGN + PW, HOLD_A ? STAGES - 1 : STAGES, HOLD_A ? STAGES : STAGES - 1, STAGES - 1, PRE_>::bytes];
     const int ntiles = tiles_m * tiles_n;
     for (int pid = blockIdx.x; pid < ntiles; pid += gridDim.x) {
         int tm, tn;
         Duty duty = tile_of(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
         if (!pretouch) duty.a_sh = duty.b_sh = 0;
-        fp8_gemm_tile_ws<BM, BN, WGM, WGN, PW, STAGES, OUT, FMT_, EPI_, E_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M, M,
+        fp8_gemm_tile_ws<BM, BN, WGM, WGN, PW, STAGES, OUT, FMT_, EPI_, 2, PRE_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M, M,
                                                                             tn * BN, N, K, ldc, duty, 0, K >> 7, pool);
         __syncthreads();
     }
@@ -1001,7 +1052,7 @@ struct Walk {
 constexpr bool walks(int BM, int BN, int STAGES, int esz, int EPI) { return BM == 256 && BN == 256 && STAGES == 2 && esz == 2 && EPI != kEpiDirect; }
 
 template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ = 0, int TD_ = 0, int ABL_ = 0, int FMT_ = 0, int GM_ = 4,
-          int EPI_ = kEpiDirect>
+          int EPI_ = kEpiDirect, bool CHUNKED_ = false>
 __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
@@ -1010,7 +1061,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
     // then walks tiles blockIdx.x, blockIdx.x + gridDim.x, ... itself, which saves the ~4.5 us that pass between
     // the end of a workgroup and the start of its successor on the same CU.  Workgroup ids keep their XCD
     // (id % 8) from tile to tile when gridDim.x is a multiple of 8.
-    using L = TileLds<BM, BN, WGM * WGN, STAGES>;
+    using L = TileLds<BM, BN, WGM * WGN, STAGES, false, CHUNKED_>;
     constexpr bool WALK = walks(BM, BN, STAGES, (int)sizeof(OUT), EPI_) && ABL_ == 0;
     __shared__ __attribute__((aligned(1024))) uint8_t pool[WALK ? L::walk_bytes : L::bytes];
     const int ntiles = tiles_m * tiles_n;
@@ -1019,7 +1070,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
         int m0, n0;
         Duty duty;
         if (!walk(m0, n0, duty)) return;
-        fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, OUT, GAP_, TD_, ABL_, FMT_, false, EPI_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, m0, M, M, n0,
+        fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, OUT, GAP_, TD_, ABL_, FMT_, false, EPI_, CHUNKED_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, m0, M, M, n0,
                                                                                          N, K, ldc, duty, 0, K >> 7, pool, 0, 0, 0, walk);
         return;
     }
@@ -1027,7 +1078,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
         int tm, tn;
         Duty duty = tile_of<GM_>(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
         if (!pretouch) duty.a_sh = duty.b_sh = 0;
-        fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, OUT, GAP_, TD_, ABL_, FMT_, false, EPI_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M,
+        fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, OUT, GAP_, TD_, ABL_, FMT_, false, EPI_, CHUNKED_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M,
                                                                             M, tn * BN, N, K, ldc, duty, 0, K >> 7, pool);
         __syncthreads();   // every wave has left the tile's LDS buffers before the next tile's copies land in them
     }
