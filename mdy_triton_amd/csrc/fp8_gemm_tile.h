@@ -281,20 +281,30 @@ struct TileLds {
     static constexpr int rows_off = no_dummy ? dummy_off : bytes, walk_bytes = rows_off + WAVES * 2048;
 };
 
-// K blocks whose activation scales a wave-specialized tile can hold at once (PRE_ of fp8_gemm_tile_ws).
-constexpr int kPreBlocks = 64;
-// LDS of a wave-specialized tile workgroup: separate ring depths for the a panels, the b panels and the activation scales (PRE: no ring
-// but those of all K blocks).
-template <int BM, int BN, int WAVES, int SA, int SB, int SS, bool PRE = false>
+// LDS of a wave-specialized tile workgroup: separate ring depths for the a panels and the b panels, and a ring of kScaleChunks chunks of activation
+// scales, 4 K blocks each.
+constexpr int kScaleChunks = 4;
+template <int BM, int BN, int WAVES, int SA, int SB>
 struct TileLdsWs {
     static constexpr int NBS = (BN + 127) / 128;
     static constexpr int BSROW = 512;
     static constexpr int a_off = 0;
     static constexpr int b_off = a_off + SA * BM * 128;
     static constexpr int s_off = b_off + SB * BN * 128;
-    static constexpr int bs_off = s_off + ((PRE ? kPreBlocks : SS) * BM * 4 + 255) / 256 * 256;
+    static constexpr int bs_off = s_off + kScaleChunks * BM * 16;
     static constexpr int dummy_off = bs_off + NBS * BSROW * 4;
     static constexpr int bytes = dummy_off + WAVES * 512;
+};
+// Ring depths: of the operand that a consumer streams through registers during a K block, and of the one it holds, read a block earlier.  4 K blocks, as the
+// K loop is unrolled by 4 and the buffers' addresses are then part of the LDS instructions; 3 where LDS has no room for more (the held operand's buffer is
+// free a block earlier).  Deeper rings, 5 K blocks streamed, put one more block in flight and lose (128x128: 0 to 5 % more time, 300x7168x4096 18.0 -> 18.6
+// us, 2048x2048x512 6.6 -> 6.9) or tie (128x64, 64x128).
+template <int BM, int BN>
+struct WsRings {
+    static constexpr bool HOLD_A = BM / 2 <= BN / 2;      // 2 x 2 consumers
+    static constexpr int STREAM = 4, HOLD = BM * BN > 128 * 128 ? 3 : 4;
+    static constexpr int SA = HOLD_A ? HOLD : STREAM, SB = HOLD_A ? STREAM : HOLD;
+    using L = TileLdsWs<BM, BN, 8, SA, SB>;
 };
 
 // the `next` of a workgroup that computes one tile
@@ -743,58 +753,68 @@ __device__ __forceinline__ Duty tile_of(int local, int tiles_m, int tiles_n, int
 //   * the barrier of block kb is at slot E, a few MFMAs into the block.  For a consumer it says "I have left block kb-1";
 //     a producer first waits for its own copies of block kb+1.  Behind it the consumers read block kb+1's held fragments,
 //     first streamed fragment and scales from LDS into a SECOND set of registers, spread over the slots (block kb+1 then
-//     starts on registers loaded a dozen slots earlier; the K loop is unrolled by two so that the sets swap without
-//     moves), and the producers copy block kb+STAGES-1 and touch the lines of a later block;
+//     starts on registers loaded a dozen slots earlier; an even number of unrolled blocks lets the sets swap without
+//     moves), and the producers copy block kb+3 and touch the lines of a later block;
 //   * the held operand of block kb is read during block kb-1, the streamed operand during block kb itself: the held
-//     operand's buffer is free one block earlier, so its ring is one buffer shorter (STAGES-1) than the streamed operand's
-//     (STAGES) for the same STAGES-2 blocks in flight.  The activation scales follow the held operand;
+//     operand's buffer is free one block earlier, and a ring of 3 serves it where the streamed operand needs 4 (WsRings);
 //   * on the 192-wide tile a wave's columns can straddle two 128-column blocks of weight scales: the combined scale is
-//     kept per row and 32-column group (multiplies once per block instead of a select per MFMA).
+//     kept per row and 32-column group (multiplies once per block instead of a select per MFMA);
+//   * a consumer alone on its SIMD is bound by the issue of its instructions: an MFMA holds the wave for 16 clocks and any other instruction,
+//     scalar ones too, for 4, so with the 4 FMAs of the fold (16 + 16 of the MFMA's 32 clocks) nothing is free.  A K block of 64x64 needs 512 + 64 for
+//     its 16 LDS reads; ring positions, addresses and scales used to take 160 more and waits another 100.  Unrolled by 4 K blocks, with rings of 4, the
+//     addresses of the buffers are constants in the LDS instructions, and a lane's scales of the next 4 K blocks come as one read per row, 16 bytes:
+//     838 -> 690 clocks a K block (64 tiles of 128x128; 861 -> 755 with 256, which also wait for copies).  With the chunks of scales below, rotating
+//     operands: 4096x1536x7168 47.7 -> 45.1 us, 2048x2048x16384 74.1 -> 67.7, 900x4096x9216 44.5 -> 40.1, 700x7168x7168 45.4 -> 41.7,
+//     1300x4096x4096 29.2 -> 27.1, 200x7168x2048 10.0 -> 9.5, 1000x1090x1664 10.3 -> 9.9, 777x2112x7168 24.6 -> 24.4.
 // Swizzle, fragment layout, fold, epilogue and pre-touch shares are fp8_gemm_tile's.
-// PRE_: the activation scales of all K blocks (up to kPreBlocks) are copied at the start, 16 rows x 4 K blocks a copy, instead of 64 rows of one K
-// block with every block's panels: with row-major scales, the official dialect's, those were 64 lines of 4 bytes for 128 of panels.  Row-major
+// The activation scales come in chunks of 4 K blocks, 16 rows x 4 K blocks a copy, the first three with the tile's start and one more with every 4th
+// K block: with row-major scales, the official dialect's, 64 rows of one K block at a time are 64 lines of 4 bytes for 128 of panels.  Row-major
 // 777x2112x7168 27.4 -> 25.4 us, 1024x4096x7168 39.4 -> 35.2, 2048x2048x7168 39.2 -> 34.8, 300x7168x4096 23.9 -> 21.2, 128x7168x7168
-// 24.4 -> 22.8, 200x7168x2048 10.4 -> 10.1; column-major 35.6 -> 35.2, 35.2 -> 34.9, the others even.
-template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, int FMT_ = 0, int EPI_ = kEpiDirect, int E_ = 2, bool PRE_ = false>
+// 24.4 -> 22.8, 200x7168x2048 10.4 -> 10.1; column-major 35.6 -> 35.2, 35.2 -> 34.9, the others even (measured with all of a tile's chunks at its start).
+template <int BM, int BN, typename OUT, int FMT_ = 0, int EPI_ = kEpiDirect>
 __device__ __forceinline__ void fp8_gemm_tile_ws(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
     const Bias bias, int m0, int m_end, int m_total, int n0, int N, int K, int ldc, const Duty duty,
     int kb0, int kb1, uint8_t* __restrict__ pool) {
+    constexpr int WGM = 2, WGN = 2, PW = 4;
     constexpr int CW = WGM * WGN;                       // consumer waves
     constexpr int WM = BM / WGM, WN = BN / WGN, TI = WM / 16, TJ = WN / 16;
     constexpr int PASS_ROWS = PW * 8;                   // rows copied by one instruction of every producer
     constexpr int A_PASSES = BM / PASS_ROWS, B_PASSES = BN / PASS_ROWS;
-    constexpr int S_WAVES = BM / 64;                    // producers that also copy the activation scales
     constexpr int DEPTH = 4;
     static_assert(BM % PASS_ROWS == 0 && BN % PASS_ROWS == 0 && PASS_ROWS % 16 == 0, "tile/threads mismatch");
     constexpr bool STRADDLE = (128 % WN) != 0;
-    static_assert(WN <= 128 && (!STRADDLE || BN == 192) && S_WAVES <= PW && PW >= 2, "weight-scale blocks per wave column");
-    constexpr bool HOLD_A = TI <= TJ;
+    static_assert(WN <= 128 && (!STRADDLE || BN == 192), "weight-scale blocks per wave column");
+    using R = WsRings<BM, BN>;
+    constexpr bool HOLD_A = R::HOLD_A;
     constexpr int NH = HOLD_A ? TI : TJ, NS = HOLD_A ? TJ : TI;
     constexpr int NT = TI * TJ;
-    constexpr int SC = PRE_ ? 0 : 1;                    // scale copies per K block and producer
-    constexpr int NDMA = SC + A_PASSES + B_PASSES;
-    constexpr int E = E_;
+    constexpr int NDMA = A_PASSES + B_PASSES;           // panel copies per K block and producer
+    constexpr int E = 2;                                // slot of the barrier
     constexpr int TDA = 2;
-    static_assert(STAGES >= 4 && (STAGES - 2) * (NDMA + 1) + 1 <= 63, "streamed ring of at least 4 K blocks; vmcnt is a 6-bit counter");
-    constexpr int SA = HOLD_A ? STAGES - 1 : STAGES, SB = HOLD_A ? STAGES : STAGES - 1;   // ring depths of a and b
-    constexpr int SS = STAGES - 1;                                                        // ring depth of the activation scales
+    constexpr int SA = R::SA, SB = R::SB, STREAM = R::STREAM, HOLD = R::HOLD;
+    // A K block's panels go out this many blocks ahead: behind the barrier of a block, the streamed operand of the one before is free and the held
+    // operand of the block itself.
+    constexpr int AHEAD = 3;
+    static_assert(STREAM == 4 && HOLD >= AHEAD && (AHEAD - 1) * (NDMA + 1) + 1 <= 63, "two K blocks in flight; vmcnt is a 6-bit counter");
     // loads younger than the last copy of block kb+1 at the barrier of block kb: the touch behind those copies and the
-    // copies + touches of blocks kb+2 .. kb+STAGES-2
-    constexpr int YOUNGER = (STAGES - 3) * (NDMA + 1) + 1;
-    static_assert(NS % 2 == 0 && NS >= 2, "the first streamed fragment of the next K block reuses queue slot 0");
+    // copies + touches of blocks kb+2 .. kb+AHEAD-1 (and chunks of scales, for which a wait may then wait as well)
+    constexpr int YOUNGER = (AHEAD - 2) * (NDMA + 1) + 1;
+    // streamed fragments are read PF in front of the one in use, at least 4 MFMAs
+    constexpr int PF = NH >= 4 ? 1 : 2, FX = NH >= 4 ? 2 : 4;
+    static_assert(NS % FX == 0 && NH * (NS - PF) > E && DEPTH <= NT, "the next K block's first fragments are read behind the barrier");
     constexpr int PWIN = NT - 2 - (E + 1);
     static_assert(E >= 0 && E < NT - NH && PWIN >= NH, "barrier slot");
 
-    using L = TileLdsWs<BM, BN, CW + PW, SA, SB, SS, PRE_>;
-    static_assert(L::bytes <= 160 * 1024 && (!PRE_ || (BM / 16) % PW == 0), "LDS of a CU; groups of 16 rows per producer");
+    using L = typename R::L;
+    constexpr int RG = BM / 16 / PW;                    // groups of 16 rows per producer in a chunk of scales
+    static_assert(L::bytes <= 160 * 1024 && (BM / 16) % PW == 0, "LDS of a CU; groups of 16 rows per producer");
     constexpr int NBS = L::NBS;
     uint8_t(*lds_a)[BM * 128] = reinterpret_cast<uint8_t(*)[BM * 128]>(pool + L::a_off);
     uint8_t(*lds_b)[BN * 128] = reinterpret_cast<uint8_t(*)[BN * 128]>(pool + L::b_off);
-    float(*lds_s)[BM] = reinterpret_cast<float(*)[BM]>(pool + L::s_off);
-    const float* lds_pre = reinterpret_cast<const float*>(pool + L::s_off);      // PRE_: [K block / 4][row][K block % 4]
-    float(*lds_bs)[L::BSROW] = reinterpret_cast<float(*)[L::BSROW]>(pool + L::bs_off);
+    const float* lds_s = reinterpret_cast<const float*>(pool + L::s_off);                       // [chunk % kScaleChunks][row][K block % 4]
+    float(*lds_bs)[L::BSROW] = reinterpret_cast<float(*)[L::BSROW]>(pool + L::bs_off);          // of the tile's K blocks, from kb0 on
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -808,16 +828,11 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
         const int pw = wave - CW;
         const int prow = pw * 8 + (lane >> 3);
         const int voff = prow * K + (((lane & 7) ^ swz(prow)) << 4);
-        intx4 rs = make_rsrc(a_s, as_bytes);
-        if (pw >= S_WAVES) rs[2] = 0;
         const uint32_t pool_addr = lds_addr(pool), ld_base = pool_addr + L::dummy_off + wave * 512;
         const uint32_t la_base = pool_addr + L::a_off + pw * 1024;
         const uint32_t lb_base = pool_addr + L::b_off + pw * 1024;
-        const uint32_t ls_base = pw < S_WAVES ? pool_addr + L::s_off + pw * 256 : ld_base;
-        const uint32_t ls_buf = pw < S_WAVES ? BM * 4 : 0;
         const intx4 ra = make_rsrc(a + (size_t)m0 * K, (uint32_t)min(BM, M - m0) * (uint32_t)K);
         const intx4 rb = make_rsrc(b + (size_t)n0 * K, (uint32_t)min(BN, N - n0) * (uint32_t)K);
-        const int s_voff = min(m0 + (pw % S_WAVES) * 64 + lane, m_total - 1) * as_rs * 4;
         const bool touch_b = (pw & 1) == 0;
         const int t_idx = (pw >> 1) * 64 + lane;
         const int share = touch_b ? (BN >> duty.b_sh) : (BM >> duty.a_sh);
@@ -825,15 +840,12 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
         if ((touch_b ? duty.b_sh : duty.a_sh) == 0) rt[2] = 0;
         const int touch_row0 = (touch_b ? duty.b_duty : duty.a_duty) * share;
         constexpr int TOUCH_LANES = (PW / 2) * 64;
-        auto issue = [&](int i, int kb, int bufa, int bufb, int bufs) {
+        auto issue = [&](int i, int kb, int bufa, int bufb) {
             const bool more = kb < kb1;
-            if (i < SC)
-                dma4(rs, s_voff, more ? kb * as_cs * 4 : (int)as_bytes, ls_base + bufs * ls_buf);
-            else if (i < SC + A_PASSES)
-                dma16(ra, voff, (i - SC) * PASS_ROWS * K + (more ? kb * 128 : ra[2]), la_base + bufa * (BM * 128) + (i - SC) * PASS_ROWS * 128);
+            if (i < A_PASSES)
+                dma16(ra, voff, i * PASS_ROWS * K + (more ? kb * 128 : ra[2]), la_base + bufa * (BM * 128) + i * PASS_ROWS * 128);
             else
-                dma16(rb, voff, (i - SC - A_PASSES) * PASS_ROWS * K + (more ? kb * 128 : rb[2]),
-                      lb_base + bufb * (BN * 128) + (i - SC - A_PASSES) * PASS_ROWS * 128);
+                dma16(rb, voff, (i - A_PASSES) * PASS_ROWS * K + (more ? kb * 128 : rb[2]), lb_base + bufb * (BN * 128) + (i - A_PASSES) * PASS_ROWS * 128);
         };
         auto touch = [&](int kbp) {      // kTouchBurst consecutive lines of a row at a time (see kTouchBurst)
             const int j = kbp & (kTouchBurst - 1), base = kbp - j;
@@ -841,48 +853,50 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
             const bool ok = row < share && base + line < kb1;
             dma4(rt, ok ? (touch_row0 + row) * K + (base + line) * 128 : kOutOfRange, 0, ld_base + 256);
         };
+        // scales of K blocks kb0 + 4 * chunk ..: rows beyond the matrix read its last one's, K blocks beyond it what lies there or zeros; nothing uses them
+        const intx4 rs = make_rsrc(a_s, as_bytes);
+        int s_voff[RG];
+#pragma unroll
+        for (int r = 0; r < RG; ++r) s_voff[r] = (min(m0 + (r * PW + pw) * 16 + (lane >> 2), m_total - 1) * as_rs + (kb0 + (lane & 3)) * as_cs) * 4;
+        auto scales = [&](int chunk) {
+#pragma unroll
+            for (int r = 0; r < RG; ++r)
+                dma4(rs, s_voff[r], chunk * 16 * as_cs, pool_addr + L::s_off + (chunk & (kScaleChunks - 1)) * (BM * 16) + (r * PW + pw) * 256);
+        };
+        const int chunks = (kb1 - kb0 + 3) >> 2;
 
         if (pw < NBS) {
             const int nb = min((n0 >> 7) + pw, ((N + 127) >> 7) - 1);
             const intx4 rbs = make_rsrc(b_s + (size_t)nb * KB, (uint32_t)KB * 4u);
-            for (int cc = 0; cc < KB; cc += 64) dma4(rbs, lane * 4, cc * 4, pool_addr + L::bs_off + (pw * L::BSROW + cc) * 4);
+            for (int cc = 0; cc < kb1 - kb0; cc += 64) dma4(rbs, lane * 4, (kb0 + cc) * 4, pool_addr + L::bs_off + (pw * L::BSROW + cc) * 4);
         }
-        if constexpr (PRE_) {
-            // 16 rows x 4 consecutive K blocks a copy: 16 lines instead of 64
-            constexpr int RG = BM / 16 / PW;
-            int row_off[RG];
+        for (int q = 0; q < min(chunks, kScaleChunks - 1); ++q) scales(q);
 #pragma unroll
-            for (int r = 0; r < RG; ++r) row_off[r] = (min(m0 + (r * PW + pw) * 16 + (lane >> 2), m_total - 1) * as_rs + (kb0 + (lane & 3)) * as_cs) * 4;
-            const intx4 rsp = make_rsrc(a_s, as_bytes);
-            for (int q = 0; q < (kb1 - kb0 + 3) >> 2; ++q) {
+        for (int blk = 0; blk < AHEAD; ++blk) {
 #pragma unroll
-                for (int r = 0; r < RG; ++r) dma4(rsp, row_off[r], q * 16 * as_cs, pool_addr + L::s_off + q * (BM * 16) + (r * PW + pw) * 256);
-            }
+            for (int i = 0; i < NDMA; ++i) issue(i, kb0 + blk, blk % SA, blk % SB);
+            touch(kb0 + blk);                  // groups 0 .. AHEAD-1 of the first burst
         }
-#pragma unroll
-        for (int blk = 0; blk < STAGES - 1; ++blk) {
-#pragma unroll
-            for (int i = 0; i < NDMA; ++i) issue(i, kb0 + blk, blk % SA, blk % SB, blk % SS);
-            touch(kb0 + blk);                  // groups 0 .. STAGES-2 of the first burst
-        }
-        // the loop's first touch is of block kb0 + STAGES - 1 + TDA: the blocks in between are touched here, behind the copies,
+        // the loop's first touch is of block kb0 + AHEAD + TDA: the blocks in between are touched here, behind the copies,
         // so that the waits below only wait for more than they need (4096x1536x7168 after a cache flush 57.4 -> 56.1 us,
         // 2048x2048x7168 44.0 -> 43.0 us, 2048x1024x7168 34.6 -> 33.5 us)
 #pragma unroll
-        for (int t = 0; t < TDA; ++t) touch(kb0 + STAGES - 1 + t);
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * (NDMA + 1) + 1) : "memory");    // block kb0 has landed
+        for (int t = 0; t < TDA; ++t) touch(kb0 + AHEAD + t);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 1) * (NDMA + 1) + 1) : "memory");    // block kb0 has landed
         __syncthreads();
-        // buffers of block kb+STAGES-1 in the three rings (kb = kb0: block index STAGES-1)
-        int fa = (STAGES - 1) % SA, fb = (STAGES - 1) % SB, fs = (STAGES - 1) % SS;
+        int fa = AHEAD % SA, fb = AHEAD % SB;      // buffers of block kb + AHEAD
         for (int kb = kb0; kb < kb1; ++kb) {
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER) : "memory");   // this wave's copies of block kb+1 have landed
             __syncthreads();                                                   // every consumer has left block kb-1
+            if (((kb - kb0) & 3) == 0) {      // every consumer has read the chunk before this block's: it makes room
+                const int next = ((kb - kb0) >> 2) + kScaleChunks - 1;
+                if (next < chunks) scales(next);
+            }
 #pragma unroll
-            for (int i = 0; i < NDMA; ++i) issue(i, kb + STAGES - 1, fa, fb, fs);
-            touch(kb + STAGES - 1 + TDA);
+            for (int i = 0; i < NDMA; ++i) issue(i, kb + AHEAD, fa, fb);
+            touch(kb + AHEAD + TDA);
             fa = fa + 1 == SA ? 0 : fa + 1;
             fb = fb + 1 == SB ? 0 : fb + 1;
-            fs = fs + 1 == SS ? 0 : fs + 1;
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing may still be writing LDS when the wave ends
         if (through_lds) __syncthreads();                  // the consumers' epilogue goes through the pool
@@ -898,10 +912,9 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
     const int b_rd1 = (wn * WN + frow) * 128 + (((2 * fk + 1) ^ swz(frow)) << 4);
     const int h0 = HOLD_A ? a_rd0 : b_rd0, h1 = HOLD_A ? a_rd1 : b_rd1;
     const int x0 = HOLD_A ? b_rd0 : a_rd0, x1 = HOLD_A ? b_rd1 : a_rd1;
-    const int s_rd = wm * WM + frow;
     const int bs_col = (n0 & 127) + wn * WN;
-    // A wave's columns lie in one 128-column block of weight scales, except on the 192-wide tile (WN = 96 or 48): there
-    // every group of GW columns does (GW = 32 or 16 divides the possible offsets), so the combined scale is kept per row
+    // A wave's columns lie in one 128-column block of weight scales, except on the 192-wide tile (WN = 96): there
+    // every group of GW columns does (GW = 32 divides the possible offsets), so the combined scale is kept per row
     // and column group: NG multiplies per row and K block instead of one select per MFMA.
     constexpr int GW = STRADDLE ? ((WN % 32 == 0) ? 32 : 16) : WN, NG = WN / GW, JPG = GW / 16;
     const float* my_bs[NG];
@@ -920,52 +933,54 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
         return intx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     };
 
-    __syncthreads();                                     // block kb0, the weight scales have landed
-    intx8 fh_a[NH], fh_b[NH], fx[2];
+    // Scales of the next K block(s): a chunk's in one read per row where registers allow (not with the 24 sub-tiles of 128x192), else a K block's.
+    constexpr bool BY_CHUNK = NT <= 16;
+    constexpr int SV = BY_CHUNK ? 4 : 1;
+    typedef float scale_t __attribute__((ext_vector_type(SV)));
+    scale_t sa_n[TI], sb_n[NG];
+    auto read_scales = [&](int chunk, int at) {
+        const float* p = lds_s + (chunk & (kScaleChunks - 1)) * (BM * 4) + (wm * WM + frow) * 4 + (BY_CHUNK ? 0 : at);
+#pragma unroll
+        for (int i = 0; i < TI; ++i) sa_n[i] = *reinterpret_cast<const scale_t*>(p + i * 64);
+#pragma unroll
+        for (int g = 0; g < NG; ++g) sb_n[g] = *reinterpret_cast<const scale_t*>(my_bs[g] + 4 * chunk + (BY_CHUNK ? 0 : at));
+    };
+    auto combine = [&](float(&sc)[TI][NG], int at) {
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int g = 0; g < NG; ++g) sc[i][g] = sa_n[i][BY_CHUNK ? at : 0] * sb_n[g][BY_CHUNK ? at : 0];
+    };
+
+    __syncthreads();                                     // block kb0, the first scales have landed
+    intx8 fh_a[NH], fh_b[NH], fx[FX];
     float sc_a[TI][NG], sc_b[TI][NG];
 #pragma unroll
     for (int h = 0; h < NH; ++h) fh_a[h] = read_frag(HOLD_A ? lds_a[0] : lds_b[0], h0, h1, h);
+    read_scales(0, 0);
+    combine(sc_a, 0);
 #pragma unroll
-    for (int i = 0; i < TI; ++i) {
-        const float sa = PRE_ ? lds_pre[(s_rd + i * 16) * 4] : lds_s[0][s_rd + i * 16];
-#pragma unroll
-        for (int g = 0; g < NG; ++g) sc_a[i][g] = sa * my_bs[g][kb0];
-    }
-    fx[0] = read_frag(HOLD_A ? lds_b[0] : lds_a[0], x0, x1, 0);
+    for (int f = 0; f < PF; ++f) fx[f] = read_frag(HOLD_A ? lds_b[0] : lds_a[0], x0, x1, f);
 
-    // buffers of K block kb in the ring of the held operand (and of the scales) / of the streamed operand
-    int ch = 0, cx = 0;
-    auto block = [&](intx8(&fh)[NH], intx8(&fhn)[NH], float(&sc)[TI][NG], float(&scn)[TI][NG], int kb) {
-        const int nh = ch + 1 == STAGES - 1 ? 0 : ch + 1;     // block kb+1, held ring
-        const int nx = cx + 1 == STAGES ? 0 : cx + 1;         // block kb+1, streamed ring
-        const uint8_t* lx = HOLD_A ? lds_b[cx] : lds_a[cx];
+    // K block kb0 + 4 * chunk + AT, in buffer AT of a ring of 4; ch: its buffer in a held ring of 3
+    int ch = 0, chunk = 0;
+    auto block = [&](auto at_, intx8(&fh)[NH], intx8(&fhn)[NH], float(&sc)[TI][NG], float(&scn)[TI][NG]) __attribute__((always_inline)) {
+        constexpr int AT = decltype(at_)::value, NEXT = (AT + 1) & 3;
+        const int nh = HOLD == 4 ? NEXT : ch + 1 == HOLD ? 0 : ch + 1;      // block kb+1, held ring
+        const uint8_t* lx = HOLD_A ? lds_b[AT] : lds_a[AT];
         const uint8_t* lh_n = HOLD_A ? lds_a[nh] : lds_b[nh];
-        const uint8_t* lx_n = HOLD_A ? lds_b[nx] : lds_a[nx];
-        const float* ls_n = lds_s[nh];
+        const uint8_t* lx_n = HOLD_A ? lds_b[NEXT] : lds_a[NEXT];
         floatx4 p[DEPTH + 1];
 #pragma unroll
         for (int t = 0; t < NT + DEPTH; ++t) {
             if (t < NT) {
                 const int si = t / NH, h = t % NH;
-                if (h == 0 && si + 1 < NS) fx[(si + 1) & 1] = read_frag(lx, x0, x1, si + 1);
-                if (h == 0 && si + 1 == NS) fx[0] = read_frag(lx_n, x0, x1, 0);      // first streamed fragment of block kb+1
-                const intx8 fa_ = HOLD_A ? fh[h] : fx[si & 1];
-                const intx8 fb_ = HOLD_A ? fx[si & 1] : fh[h];
+                const intx8 fa_ = HOLD_A ? fh[h] : fx[si % FX];
+                const intx8 fb_ = HOLD_A ? fx[si % FX] : fh[h];
                 p[t % (DEPTH + 1)] = mfma_block<FMT_>(fb_, fa_);
                 if (t == E) __syncthreads();
-                if (t == E + 1) {
-                    float sbg[NG];
-                    const int nb = min(kb + 1, kb1 - 1) - kb0;
-                    const float* ls_pre = lds_pre + (nb >> 2) * (BM * 4) + (nb & 3) + s_rd * 4;
-#pragma unroll
-                    for (int g = 0; g < NG; ++g) sbg[g] = my_bs[g][min(kb + 1, KB - 1)];
-#pragma unroll
-                    for (int i = 0; i < TI; ++i) {
-                        const float sa = PRE_ ? ls_pre[i * 64] : ls_n[s_rd + i * 16];
-#pragma unroll
-                        for (int g = 0; g < NG; ++g) scn[i][g] = sa * sbg[g];
-                    }
-                }
+                if (h == 0) fx[(si + PF) % FX] = si + PF < NS ? read_frag(lx, x0, x1, si + PF) : read_frag(lx_n, x0, x1, si + PF - NS);
+                if (t == E + 1 && (!BY_CHUNK || AT == 3)) read_scales(AT == 3 ? chunk + 1 : chunk, NEXT);
 #pragma unroll
                 for (int hh = 0; hh < NH; ++hh)
                     if (t == E + 1 + (hh * PWIN) / NH) fhn[hh] = read_frag(lh_n, h0, h1, hh);
@@ -975,18 +990,27 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
                 const int i = HOLD_A ? h : si, j = HOLD_A ? si : h;
                 fold(acc[i][j], p[u % (DEPTH + 1)], sc[i][j / JPG]);
             }
+            if (t == NT + DEPTH - 1) combine(scn, NEXT);
             __builtin_amdgcn_sched_barrier(0);
         }
         ch = nh;
-        cx = nx;
     };
     {
-        int kb = kb0;
-        for (; kb + 1 < kb1; kb += 2) {
-            block(fh_a, fh_b, sc_a, sc_b, kb);
-            block(fh_b, fh_a, sc_b, sc_a, kb + 1);
+        constexpr std::integral_constant<int, 0> k0{};
+        constexpr std::integral_constant<int, 1> k1{};
+        constexpr std::integral_constant<int, 2> k2{};
+        constexpr std::integral_constant<int, 3> k3{};
+        int left = kb1 - kb0;
+        for (; left >= 4; left -= 4) {
+            block(k0, fh_a, fh_b, sc_a, sc_b);
+            block(k1, fh_b, fh_a, sc_b, sc_a);
+            block(k2, fh_a, fh_b, sc_a, sc_b);
+            block(k3, fh_b, fh_a, sc_b, sc_a);
+            ++chunk;
         }
-        if (kb < kb1) block(fh_a, fh_b, sc_a, sc_b, kb);     // odd number of K blocks
+        if (left > 0) block(k0, fh_a, fh_b, sc_a, sc_b);
+        if (left > 1) block(k1, fh_b, fh_a, sc_b, sc_a);
+        if (left > 2) block(k2, fh_a, fh_b, sc_a, sc_b);
     }
 
     if constexpr (through_lds) {
@@ -1012,22 +1036,19 @@ __device__ __forceinline__ void fp8_gemm_tile_ws(
     }
 }
 
-// the wave-specialized tile as a kernel: one workgroup of WGM*WGN + PW waves per tile (or per several, walked in turn)
-template <int BM, int BN, int WGM, int WGN, int PW, int STAGES, typename OUT, int FMT_ = 0, int EPI_ = kEpiDirect, bool PRE_ = false>
-__global__ __launch_bounds__((WGM * WGN + PW) * 64) void fp8_gemm_ws_kernel(
+// the wave-specialized tile as a kernel: one workgroup of 4 + 4 waves per tile (or per several, walked in turn)
+template <int BM, int BN, typename OUT, int FMT_ = 0, int EPI_ = kEpiDirect>
+__global__ __launch_bounds__(512) void fp8_gemm_ws_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
     const Bias bias, int M, int N, int K, int ldc, int tiles_m, int tiles_n, int pretouch) {
-    constexpr bool HOLD_A = BM / WGM <= BN / WGN;
-    __shared__ __attribute__((aligned(1024)))
-    uint8_t pool[TileLdsWs<BM, BN, WGM * WGN + PW, HOLD_A ? STAGES - 1 : STAGES, HOLD_A ? STAGES : STAGES - 1, STAGES - 1, PRE_>::bytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t pool[WsRings<BM, BN>::L::bytes];
     const int ntiles = tiles_m * tiles_n;
     for (int pid = blockIdx.x; pid < ntiles; pid += gridDim.x) {
         int tm, tn;
         Duty duty = tile_of(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
         if (!pretouch) duty.a_sh = duty.b_sh = 0;
-        fp8_gemm_tile_ws<BM, BN, WGM, WGN, PW, STAGES, OUT, FMT_, EPI_, 2, PRE_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M, M,
-                                                                            tn * BN, N, K, ldc, duty, 0, K >> 7, pool);
+        fp8_gemm_tile_ws<BM, BN, OUT, FMT_, EPI_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M, M, tn * BN, N, K, ldc, duty, 0, K >> 7, pool);
         __syncthreads();
     }
 }

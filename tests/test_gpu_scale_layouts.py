@@ -52,6 +52,28 @@ def test_block_scaled(M, N, K, layout):
     assert rc == 0 and torch.equal(c, ref)
 
 
+# the producer / consumer tiles in one launch: K blocks in every remainder of the four that their loop takes at a time, and on either side of the
+# twelve whose scales come with a tile's start
+@pytest.mark.parametrize("KB", [*range(1, 10), 11, 12, 13, 15, 16, 17, 18, 33])
+@pytest.mark.parametrize("M,N,form", [(900, 2100, 5), (2000, 1000, 6), (2030, 1900, 7), (3000, 1500, 9)])
+def test_chunks_of_scales(M, N, form, KB):
+    lib, K = _lib.load(), KB * 128
+    if form == 9 and KB < 3 or lib.mdy_fp8_gemm_form(M, N, K, 0) != form:
+        pytest.skip("another form")
+    g = torch.Generator(device=DEV).manual_seed(M + KB)
+    a, sa = _operand(M, K, g)
+    b = torch.randint(-2, 3, (N, K), generator=g, device=DEV).float()
+    sb = torch.exp2(torch.randint(-2, 3, (-(-N // 128), KB), generator=g, device=DEV).float())
+    qa, qb = a.to(torch.float8_e4m3fn), b.to(torch.float8_e4m3fn)
+    ref = (a * sa.repeat_interleave(128, 1)) @ (b * sb.repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)).t()
+    for layout in ("rows", "columns", "inside"):
+        s, rs, cs = _laid_out(sa, layout)
+        c = torch.full((M, N), float("nan"), device=DEV)
+        rc = lib.mdy_fp8_gemm_nt_ws(qa.data_ptr(), s.data_ptr(), rs, cs, qb.data_ptr(), sb.data_ptr(), c.data_ptr(), None, M, N, K, 1, None, 0,
+                                    torch.cuda.current_stream().cuda_stream)
+        assert rc == 0 and torch.equal(c, ref)
+
+
 # plain loop, 128x128 tiles alone and two per CU, 128x256 (also slabs), 256x256 (also walked), K blocks 1 to 37
 ROWS = [(250, 1036, 256), (890, 1028, 3072), (250, 1036, 1664), (1000, 2301, 896), (300, 700, 512), (2550, 3190, 1024), (770, 260, 384), (7290, 2170, 640), (644, 5433, 640),
         (3074, 4879, 640), (512, 512, 4096), (1530, 640, 4736), (4090, 3336, 384), (4352, 4104, 640), (4352, 4104, 256), (4097, 4160, 1152), (5504, 4735, 128)]
