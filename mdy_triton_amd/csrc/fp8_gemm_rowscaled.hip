@@ -10,8 +10,8 @@
 // fold would be 4 multiplies + 4 FMAs per MFMA instead of 4 FMAs, as much work as the matrix cores have; the scheduled tile body of fp8_gemm_tile.h
 // forms the products on the matrix cores instead (scale_products there).  It takes 256x256 tiles where their rounds come out ahead (a
 // quarter fewer LDS reads and a third fewer copies per MFMA than 128x256: 4096x7168x4096 154 -> 130 us, 4096x4096x8192 159 -> 136 us; with the
-// products on the matrix cores 120.6 -> 115.0 and 129.1 -> 122.9 us = 2.09 and 2.24 PFLOP/s; row-major scales, copied in chunks of four K blocks,
-// no longer cost more than column-major ones, 131 -> 120 us), 128x256 and 128x128 tiles otherwise; a plain
+// products on the matrix cores 120.6 -> 115.0 and 129.1 -> 122.9 us = 2.09 and 2.24 PFLOP/s; with row-major scales, copied in chunks of four K
+// blocks where K is long, 131 -> 122 us), 128x256 and 128x128 tiles otherwise; a plain
 // loop (128x128 tile, four waves of 64x64, the K block's two panels and two scale vectors copied global -> LDS by `buffer_load
 // ... lds`, double buffered, one barrier per K block: short ends, but 0.93 us per K block against 0.72) runs what has few K blocks.
 // K % 128 == 0 (the callers contract over a padded token count).
@@ -131,12 +131,12 @@ __global__ __launch_bounds__(256) void fp8_gemm_rowscaled_kernel(
 }
 
 // The scheduled tile body of fp8_gemm_tile.h in its row-scaled-weight form; a grid smaller than the number of tiles walks them.
-template <int BM, int BN, int STAGES, typename OUT, int FMT, int EPI>
+template <int BM, int BN, int STAGES, typename OUT, int FMT, int EPI, bool CHUNKED>
 __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_tile_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, int bs_rs, int bs_cs, uint32_t bs_bytes,
     OUT* __restrict__ c, int M, int N, int K, int tiles_m, int tiles_n) {
-    using L = TileLds<BM, BN, 8, STAGES, true>;
+    using L = TileLds<BM, BN, 8, STAGES, true, CHUNKED>;
     constexpr bool WALK = walks(BM, BN, STAGES, (int)sizeof(OUT), EPI);
     __shared__ __attribute__((aligned(1024))) uint8_t pool[WALK ? L::walk_bytes : L::bytes];
     const int ntiles = tiles_m * tiles_n;
@@ -145,14 +145,14 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_tile_kernel(
         int m0, n0;
         Duty duty;
         if (!walk(m0, n0, duty)) return;
-        fp8_gemm_tile<BM, BN, 2, 4, STAGES, OUT, 0, 0, 0, FMT, true, EPI>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, Bias{}, m0, M, M, n0, N, K, N,
+        fp8_gemm_tile<BM, BN, 2, 4, STAGES, OUT, 0, 0, 0, FMT, true, EPI, CHUNKED>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, Bias{}, m0, M, M, n0, N, K, N,
                                                                           duty, 0, K >> 7, pool, bs_rs, bs_cs, bs_bytes, walk);
         return;
     }
     for (int pid = blockIdx.x; pid < ntiles; pid += gridDim.x) {
         int tm, tn;
         const Duty duty = tile_of(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
-        fp8_gemm_tile<BM, BN, 2, 4, STAGES, OUT, 0, 0, 0, FMT, true, EPI>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, Bias{}, tm * BM, M, M,
+        fp8_gemm_tile<BM, BN, 2, 4, STAGES, OUT, 0, 0, 0, FMT, true, EPI, CHUNKED>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, Bias{}, tm * BM, M, M,
                                                                      tn * BN, N, K, N, duty, 0, K >> 7, pool, bs_rs, bs_cs, bs_bytes);
         __syncthreads();
     }
@@ -176,12 +176,12 @@ __global__ __launch_bounds__(256) void fp8_gemm_rowscaled_small_kernel(
 
 // The 128x256 tiles cut along K: workgroup (slab, tile) writes the fp32 partial sums of K blocks slab * kb_per .. of its tile into a
 // workspace [slabs][M][N]; splitk_reduce_kernel adds the slabs in order.
-template <int FMT, int EPI>
+template <int FMT, int EPI, bool CHUNKED>
 __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, int bs_rs, int bs_cs, uint32_t bs_bytes,
     float* __restrict__ ws, int M, int N, int K, int tiles_m, int tiles_n, int slabs, int kb_per) {
-    __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<128, 256, 8, 3, true>::bytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t pool[TileLds<128, 256, 8, 3, true, CHUNKED>::bytes];
     const int ntiles = tiles_m * tiles_n;
     // runs per XCD from 13 K blocks per slab on, against K > 8192 from 10 (runs against plain order, warm / cold: 768x512x11648, slabs of 7,
     // 21.9 -> 23.5 / 23.7 -> 26.2 us, 512x1152x10368 (9) 24.0 -> 24.8 / 26.0 -> 27.1, 2304x512x3712 (10) 22.0 -> 23.5 / 24.8 -> 27.0; 640x768x15232
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_rowscaled_split_kernel(
     int tm, tn;
     const Duty duty = tile_of(pid - ks * ntiles, tiles_m, tiles_n, tm, tn);
     const int kb0 = ks * kb_per, kb1 = min(K >> 7, kb0 + kb_per);
-    fp8_gemm_tile<128, 256, 2, 4, 3, float, 0, 0, 0, FMT, true, EPI>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, Bias{},
+    fp8_gemm_tile<128, 256, 2, 4, 3, float, 0, 0, 0, FMT, true, EPI, CHUNKED>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, ws + (size_t)ks * M * N, Bias{},
                                                                 tm * 128, M, M, tn * 256, N, K, N, duty, kb0, kb1, pool, bs_rs, bs_cs,
                                                                 bs_bytes);
 }
@@ -275,11 +275,17 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
         128 * K >= ((int64_t)1 << 31))
         return -1;
     RowscaledPlan sp = plan_rowscaled(M, N, K, true);
+    // Scales that lie K block after K block (row-major) in chunks of four of them (CHUNKED of TileLds), with tiles of 256 columns, from 12 K blocks on.
+    // A K block at a time -> in chunks, row-major: 8192x4096x4096 137 -> 131 us, 7168x2048x4096 67.6 -> 62.9, 1792x4096x4096 39.7 -> 36.9, 4096x7168 with
+    // 12 / 16 blocks 52.5 -> 50.7 / 65.2 -> 64.5, but with 2 to 8 blocks +1 % (the first chunk comes before the first K block), 128x128 tiles +2 to 5 % (2048x2048x2048 14.9 ->
+    // 15.3); column-major +1 % (4096x7168x1024 38.8 -> 39.4), 128x128 tiles +4 to 8 % (1024x3072x2048 13.5 -> 14.6).
+    const bool chunked = KB >= 12 && (as_cs < as_rs || bs_cs < bs_rs);
     if (sp.slabs > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && workspace_bytes >= (int64_t)sp.slabs * M * N * 4) {
         const int tm = (int)((M + 127) / 128), tn = (int)((N + 255) / 256);
         float* ws = static_cast<float*>(workspace);
-#define MDY_RSS(FMT, EPI)                                                                                                \
-    launch_kernel((fp8_gemm_rowscaled_split_kernel<FMT, EPI>), dim3((unsigned)(tm * tn * sp.slabs)), dim3(512), 0, stream, \
+#define MDY_RSS(FMT, EPI) do { if (chunked) MDY_RSS_C(FMT, EPI, true); else MDY_RSS_C(FMT, EPI, false); } while (0)
+#define MDY_RSS_C(FMT, EPI, CHUNKED)                                                                                     \
+    launch_kernel((fp8_gemm_rowscaled_split_kernel<FMT, EPI, CHUNKED>), dim3((unsigned)(tm * tn * sp.slabs)), dim3(512), 0, stream, \
                        static_cast<const uint8_t*>(a), a_s, (int)as_rs, (int)as_cs, (uint32_t)a_ext, static_cast<const uint8_t*>(b), b_s, \
                        (int)bs_rs, (int)bs_cs, (uint32_t)b_ext, ws, (int)M, (int)N, (int)K, tm, tn, sp.slabs, sp.kb_per)
         if (epilogue_kind(ws, N, N, 4, false, true) == kEpiRows) {
@@ -288,6 +294,7 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
             if (fmt == 0) MDY_RSS(0, kEpiDirect); else MDY_RSS(1, kEpiDirect);
         }
 #undef MDY_RSS
+#undef MDY_RSS_C
         const int rc = (int)hipGetLastError();
         return rc != 0 ? rc : launch_splitk_reduce(ws, c, out_dtype, Bias{}, M, N, sp.slabs, stream);
     }
@@ -298,8 +305,9 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
         const int64_t tm = (M + bm - 1) / bm, tn = (N + 255) / 256, cus = cu_count();
         if (tm * tn > 0x7FFFFFFF) return kErrTooManyBlocks;
         const dim3 grid((unsigned)(cfg == kTiles256x256 && tm * tn > cus ? cus : tm * tn));      // 256x256: a workgroup per CU walks its tiles
-#define MDY_RST(BM, ST, OUT_T, FMT, EPI)                                                                                 \
-    launch_kernel((fp8_gemm_rowscaled_tile_kernel<BM, 256, ST, OUT_T, FMT, EPI>), grid, dim3(512), 0, stream,            \
+#define MDY_RST(BM, ST, OUT_T, FMT, EPI) do { if (chunked) MDY_RST_K(BM, ST, OUT_T, FMT, EPI, true); else MDY_RST_K(BM, ST, OUT_T, FMT, EPI, false); } while (0)
+#define MDY_RST_K(BM, ST, OUT_T, FMT, EPI, CHUNKED)                                                                      \
+    launch_kernel((fp8_gemm_rowscaled_tile_kernel<BM, 256, ST, OUT_T, FMT, EPI, CHUNKED>), grid, dim3(512), 0, stream,            \
                        static_cast<const uint8_t*>(a), a_s, (int)as_rs, (int)as_cs, (uint32_t)a_ext,                      \
                        static_cast<const uint8_t*>(b), b_s, (int)bs_rs, (int)bs_cs, (uint32_t)b_ext, static_cast<OUT_T*>(c), \
                        (int)M, (int)N, (int)K, (int)tm, (int)tn)
@@ -310,6 +318,7 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
         else if (epi == kEpiRows) { if (fmt == 0) MDY_RST(256, 2, uint16_t, 0, kEpiRows); else MDY_RST(256, 2, uint16_t, 1, kEpiRows); }
         else { if (fmt == 0) MDY_RST_C(uint16_t, 0, kEpiDirect); else MDY_RST_C(uint16_t, 1, kEpiDirect); }
 #undef MDY_RST_C
+#undef MDY_RST_K
 #undef MDY_RST
         return (int)hipGetLastError();
     }

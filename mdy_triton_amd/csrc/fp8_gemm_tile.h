@@ -258,10 +258,11 @@ struct Duty {
 // CHUNKED: row scales (of the activations, with BROW of the weight rows behind them) come in chunks of 4 K blocks, [group of 16 rows][row]
 // [K block % 4]: a copy of a wave takes 16 rows x 4 K blocks, which with row-major scales, the official dialect's, is 16 lines; one K block of 64
 // rows is 64.  Part r of a chunk (groups r * WAVES ..) goes out with the copies of the K block PARTS - 1 - r in front of the chunk.  With row scales on
-// both sides, 16 lines a copy of the 32 that a chunk takes instead of 64 of 32: 8192x4096x4096 row-major 138 -> 129 us, column-major as before
-// (128).  Against one operand's it pays with 128x256 tiles and row-major scales (1500x4096x4096 33.8 -> 32.3, column-major 30.8 -> 32.4), not with
+// both sides, 16 lines a copy of the 32 that a chunk takes instead of 64 of 32: 8192x4096x4096 row-major 138 -> 129 us; column-major ones lie together
+// anyway and lose 1 to 2 % with 256x256 tiles, 2 to 8 % with 128x128 (launch_fp8_gemm_nt_rowscaled says when).  Against one operand's it pays with 128x256 tiles and row-major scales (1500x4096x4096 33.8 -> 32.3, column-major 30.8 -> 32.4), not with
 // 256x256 (2048x18432x2048 82.9 -> 85.9 row-major, 81.8 -> 85.9) or 64x64 (65x1024x4096 8.83 -> 8.88, 8.4 -> 8.9): those copy a K block at a time.
-template <int BM, int BN, int WAVES, int STAGES, bool BROW = false, bool CHUNKED = BROW>
+// Without chunks, the weight rows' scales of STAGES K blocks lie where the weight's block scales would.
+template <int BM, int BN, int WAVES, int STAGES, bool BROW = false, bool CHUNKED = false>
 struct TileLds {
     static constexpr int NBS = (BN + 127) / 128;
     static constexpr int GROUPS = BM / 16 + (BROW ? BN / 16 : 0), PARTS = CHUNKED ? (GROUPS + WAVES - 1) / WAVES : 1;
@@ -272,12 +273,12 @@ struct TileLds {
     static constexpr int b_off = a_off + STAGES * BM * 128;
     static constexpr int s_off = b_off + STAGES * BN * 128;
     static constexpr int bs_off = s_off + (CHUNKED ? CHUNKS * GROUPS * 256 : (STAGES * BM * 4 + 255) / 256 * 256);
-    static constexpr int dummy_off = bs_off + (BROW ? 0 : NBS * 512 * 4);
+    static constexpr int dummy_off = bs_off + (!BROW ? NBS * 512 * 4 : CHUNKED ? 0 : STAGES * BN * 4);
     static constexpr int bytes = dummy_off + WAVES * 512;
     // A workgroup that walks its tiles: 16 rows of results of every wave on their way to memory, beside a ring that already
     // receives the next tile.  256x256 tiles with row scales on both sides fill the CU's LDS without a dummy area: a wave's touches go where its
     // rows of results go later.
-    static constexpr bool no_dummy = BROW && bytes + WAVES * 2048 > 160 * 1024;
+    static constexpr bool no_dummy = CHUNKED && bytes + WAVES * 2048 > 160 * 1024;
     static constexpr int rows_off = no_dummy ? dummy_off : bytes, walk_bytes = rows_off + WAVES * 2048;
 };
 
@@ -343,7 +344,7 @@ struct OneTile {};
 // (Those without a bias.  With one its loads complete behind the copies that went out in front of them, and the stores wait for
 // both: 0 to 4 us more, 3752x15224x768 64.5 -> 68.6 us, 16384x4096x1024 78.1 -> 79.4, none from K = 4096 on.)
 template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ = 0, int TD_ = 0, int ABL_ = 0, int FMT_ = 0,
-          bool BROW_ = false, int EPI_ = kEpiDirect, bool CHUNKED_ = BROW_, typename NEXT = OneTile>
+          bool BROW_ = false, int EPI_ = kEpiDirect, bool CHUNKED_ = false, typename NEXT = OneTile>
 __device__ __forceinline__ void fp8_gemm_tile(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
@@ -393,9 +394,10 @@ __device__ __forceinline__ void fp8_gemm_tile(
 
     using L = TileLds<BM, BN, WAVES, STAGES, BROW_, CHUNKED_>;
     constexpr int NBS = L::NBS, PARTS = L::PARTS, PARTS_A = BM / 16 / WAVES, CHUNKS = L::CHUNKS, CHUNK = L::GROUPS * 64;      // (floats)
-    constexpr int S_WAVES = BM / 64;      // !CHUNKED_: waves that also copy 64 activation scales of the K block each
+    // !CHUNKED_: waves that also copy 64 activation scales of the K block each, and behind them those that copy 64 weight rows' scales
+    constexpr int S_WAVES = BM / 64, SB_WAVES = BROW_ && !CHUNKED_ ? BN / 64 : 0;
     constexpr bool NO_DUMMY = WALK && L::no_dummy;
-    static_assert(CHUNKED_ ? BM / 16 % WAVES == 0 && PARTS <= 4 && (!BROW_ || BN / 16 % WAVES == 0) : !BROW_ && S_WAVES <= WAVES,
+    static_assert(CHUNKED_ ? BM / 16 % WAVES == 0 && PARTS <= 4 && (!BROW_ || BN / 16 % WAVES == 0) : S_WAVES + SB_WAVES <= WAVES,
                   "a part of a chunk is a group of 16 rows for every wave, a K block has one part");
     static_assert(!NO_DUMMY || L::GROUPS == 4 * WAVES, "every scale copy has a part to go to");
     uint8_t(*lds_a)[BM * 128] = reinterpret_cast<uint8_t(*)[BM * 128]>(pool + L::a_off);     // [STAGES]
@@ -420,12 +422,16 @@ __device__ __forceinline__ void fp8_gemm_tile(
     const int voff = prow * K + (((lane & 7) ^ swz(prow)) << 4);      // permuted chunk of that row
     // scale copies: lane -> row lane / 4 of the wave's group, K block lane % 4 of the chunk.  Rows beyond the matrix read what lies there, or
     // zeros beyond the array: nothing they scale is stored.
-    const bool s_none = !CHUNKED_ && wave >= S_WAVES;                 // this wave copies no scales: always out of range
+    const bool s_none = !CHUNKED_ && wave >= S_WAVES + SB_WAVES;      // this wave copies no scales: always out of range
+    const bool sb_wave = SB_WAVES > 0 && wave >= S_WAVES && !s_none;
     const intx4 rsa = make_rsrc(a_s, s_none ? 0u : as_bytes), rsb = make_rsrc(BROW_ ? b_s : a_s, BROW_ ? bs_bytes : 0u);
     const int srow = wave * 16 + (lane >> 2);
     const auto scale_offset = [](int row, int rs, int kb, int cs) { return (int)(((uint32_t)row * (uint32_t)rs + (uint32_t)kb * (uint32_t)cs) * 4u); };
     const int sa_voff = scale_offset(srow, as_rs, lane & 3, as_cs), sb_voff = BROW_ ? scale_offset(srow, bs_rs, lane & 3, bs_cs) : 0;
-    const uint32_t ls_base = s_none ? dummy : lds_addr(pool + L::s_off) + wave * 256, ls_buf = s_none ? 0 : BM * 4;
+    const uint32_t ls_base = s_none ? dummy : sb_wave ? lds_addr(pool + L::bs_off) + (wave - S_WAVES) * 256 : lds_addr(pool + L::s_off) + wave * 256;
+    const uint32_t ls_buf = s_none ? 0 : sb_wave ? BN * 4 : BM * 4;
+    const intx4 rs = sb_wave ? rsb : rsa;
+    const int sc_cs = sb_wave ? bs_cs : as_cs;
     const uint32_t la_base = lds_addr(&lds_a[0][0]) + wave * 1024;
     const uint32_t lb_base = lds_addr(&lds_b[0][0]) + wave * 1024;
     // duty touch: the even waves load one dword of every line of this workgroup's share of the B panel (64
@@ -443,7 +449,8 @@ __device__ __forceinline__ void fp8_gemm_tile(
         // nobody to share with: touching one's own lines ahead of the copy only adds requests (measured)
         if ((wave >> 1) * 64 >= share || (touch_b ? d.b_sh : d.a_sh) == 0) t.rt[2] = 0;
         t.touch_off = ((touch_b ? d.b_duty : d.a_duty) * share + t_idx % share) * K;
-        t.s_voff = CHUNKED_ ? 0 : min(tm0 + (wave % S_WAVES) * 64 + lane, m_total - 1) * as_rs * 4;
+        t.s_voff = CHUNKED_ ? 0 : sb_wave ? min(tn0 + (wave - S_WAVES) * 64 + lane, N - 1) * bs_rs * 4
+                                          : min(tm0 + (wave % S_WAVES) * 64 + lane, m_total - 1) * as_rs * 4;
         t.m0 = tm0;
         t.n0 = tn0;
         return t;
@@ -463,7 +470,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
     auto issue = [&](const TileAddr& t, int i, int kb, int buf) {
         const bool more = kb < kb1;
         if (i == 0 && !CHUNKED_) {
-            dma4(rsa, t.s_voff, more ? kb * as_cs * 4 : (int)as_bytes, ls_base + buf * ls_buf);
+            dma4(rs, t.s_voff, more ? kb * sc_cs * 4 : (int)(sb_wave ? bs_bytes : as_bytes), ls_base + buf * ls_buf);
         } else if (i == 0) {
             const int u = kb - kb0 + PARTS - 1;
             scale_part(t, u & 3, u >> 2, more && (PARTS == 4 || (u & 3) < PARTS));
@@ -545,12 +552,13 @@ __device__ __forceinline__ void fp8_gemm_tile(
     float sc[TI], sc_hi[STRADDLE ? TI : 1];
     // BROW_: the scales of the wave's 64 weight rows and of its activation rows, one a lane
     constexpr int SAV = BROW_ ? TI / 4 : 1;
-    const int sbr_lane = (BM + wn * WN + lane) * 4, sar_lane = (wm * WM + lane) * 4;
+    const float* lds_sbr = reinterpret_cast<const float*>(pool + L::bs_off);      // !CHUNKED_: [STAGES][BN]
+    const int sbr_lane = CHUNKED_ ? (BM + wn * WN + lane) * 4 : wn * WN + lane, sar_lane = (wm * WM + lane) * S_STRIDE;
     float sb_row = 1.0f, sa_row[SAV];
     if (BROW_) {
-        sb_row = lds_s[sbr_lane];
+        sb_row = CHUNKED_ ? lds_s[sbr_lane] : lds_sbr[sbr_lane];
 #pragma unroll
-        for (int v = 0; v < SAV; ++v) sa_row[v] = lds_s[sar_lane + v * 256];
+        for (int v = 0; v < SAV; ++v) sa_row[v] = lds_s[sar_lane + v * 64 * S_STRIDE];
     }
 #pragma unroll
     for (int h = 0; h < NH; ++h) fh[h] = read_frag(HOLD_A ? lds_a[0] : lds_b[0], h0, h1, h);
@@ -647,9 +655,9 @@ __device__ __forceinline__ void fp8_gemm_tile(
             }
             if (t == TOUCH && !NO_TOUCH) touch(me, kb + TD, touch_to);
             if (BROW_ && t == NT + DEPTH - 1) {
-                sb_row = ls_n[sbr_lane];      // first used NH - 1 MFMAs from here
+                sb_row = CHUNKED_ ? ls_n[sbr_lane] : lds_sbr[nxt * BN + sbr_lane];      // first used NH - 1 MFMAs from here
 #pragma unroll
-                for (int v = 0; v < SAV; ++v) sa_row[v] = ls_n[sar_lane + v * 256];
+                for (int v = 0; v < SAV; ++v) sa_row[v] = ls_n[sar_lane + v * 64 * S_STRIDE];
             }
             __builtin_amdgcn_sched_barrier(0);  // keep the MFMA / FMA / ds_read / copy interleaving as written
         }

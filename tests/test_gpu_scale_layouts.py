@@ -76,7 +76,9 @@ def test_chunks_of_scales(M, N, form, KB):
 
 # plain loop, 128x128 tiles alone and two per CU, 128x256 (also slabs), 256x256 (also walked), K blocks 1 to 37
 ROWS = [(250, 1036, 256), (890, 1028, 3072), (250, 1036, 1664), (1000, 2301, 896), (300, 700, 512), (2550, 3190, 1024), (770, 260, 384), (7290, 2170, 640), (644, 5433, 640),
-        (3074, 4879, 640), (512, 512, 4096), (1530, 640, 4736), (4090, 3336, 384), (4352, 4104, 640), (4352, 4104, 256), (4097, 4160, 1152), (5504, 4735, 128)]
+        (3074, 4879, 640), (512, 512, 4096), (1530, 640, 4736), (4090, 3336, 384), (4352, 4104, 640), (4352, 4104, 256), (4097, 4160, 1152), (5504, 4735, 128),
+        # on either side of the 12 K blocks from which row-major scales come in chunks
+        (4000, 7100, 1408), (4000, 7096, 1536), (4000, 4090, 1920), (4352, 4104, 1664), (3074, 4879, 1920), (1790, 4097, 1792), (2305, 512, 3712)]
 
 
 @pytest.mark.parametrize("layout", [("rows", "rows"), ("columns", "columns"), ("inside", "columns"), ("columns", "inside")])
