@@ -255,17 +255,18 @@ struct Duty {
 // LDS of one tile workgroup, carved out of a pool that the kernel declares: the ring of A and B panels, the ring of activation scales, the tile's weight
 // scales for all K blocks, and a dummy area for copies that must go nowhere.
 //
-// CHUNKED: row scales (of the activations, with BROW of the weight rows behind them) come in chunks of 4 K blocks, [group of 16 rows][row]
+// CHUNKED (with BROW): row scales, of the activations and behind them of the weight rows, come in chunks of 4 K blocks, [group of 16 rows][row]
 // [K block % 4]: a copy of a wave takes 16 rows x 4 K blocks, which with row-major scales, the official dialect's, is 16 lines; one K block of 64
 // rows is 64.  Part r of a chunk (groups r * WAVES ..) goes out with the copies of the K block PARTS - 1 - r in front of the chunk.  With row scales on
 // both sides, 16 lines a copy of the 32 that a chunk takes instead of 64 of 32: 8192x4096x4096 row-major 138 -> 129 us; column-major ones lie together
-// anyway and lose 1 to 2 % with 256x256 tiles, 2 to 8 % with 128x128 (launch_fp8_gemm_nt_rowscaled says when).  Against one operand's it pays with 128x256 tiles and row-major scales (1500x4096x4096 33.8 -> 32.3, column-major 30.8 -> 32.4), not with
-// 256x256 (2048x18432x2048 82.9 -> 85.9 row-major, 81.8 -> 85.9) or 64x64 (65x1024x4096 8.83 -> 8.88, 8.4 -> 8.9): those copy a K block at a time.
+// anyway and lose 1 to 2 % with 256x256 tiles, 2 to 8 % with 128x128 (launch_fp8_gemm_nt_rowscaled says when).  One operand's row scales are copied a
+// K block at a time: in chunks 128x256 tiles tie right behind the quantizer and lose otherwise (1500x4096x4096 34.1 -> 35.9 us, 2048x4096x3072
+// 27.5 -> 28.1, a weight's rotating copies), 256x256 lose (2048x18432x2048 82.9 -> 85.9), 64x64 tie.
 // Without chunks, the weight rows' scales of STAGES K blocks lie where the weight's block scales would.
 template <int BM, int BN, int WAVES, int STAGES, bool BROW = false, bool CHUNKED = false>
 struct TileLds {
     static constexpr int NBS = (BN + 127) / 128;
-    static constexpr int GROUPS = BM / 16 + (BROW ? BN / 16 : 0), PARTS = CHUNKED ? (GROUPS + WAVES - 1) / WAVES : 1;
+    static constexpr int GROUPS = BM / 16 + BN / 16, PARTS = CHUNKED ? (GROUPS + WAVES - 1) / WAVES : 1;
     // Part 0 of chunk c + 1 is copied behind the barrier of K block 4 c + 5 - PARTS - STAGES, when the scales of the next one are read: the chunks
     // from that one's to c + 1 have a buffer each.
     static constexpr int CHUNKS = PARTS + STAGES <= 6 ? 2 : 2 + (PARTS + STAGES - 6 + 3) / 4;
@@ -397,7 +398,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
     // !CHUNKED_: waves that also copy 64 activation scales of the K block each, and behind them those that copy 64 weight rows' scales
     constexpr int S_WAVES = BM / 64, SB_WAVES = BROW_ && !CHUNKED_ ? BN / 64 : 0;
     constexpr bool NO_DUMMY = WALK && L::no_dummy;
-    static_assert(CHUNKED_ ? BM / 16 % WAVES == 0 && PARTS <= 4 && (!BROW_ || BN / 16 % WAVES == 0) : S_WAVES + SB_WAVES <= WAVES,
+    static_assert(CHUNKED_ ? BROW_ && BM / 16 % WAVES == 0 && PARTS <= 4 && BN / 16 % WAVES == 0 : S_WAVES + SB_WAVES <= WAVES,
                   "a part of a chunk is a group of 16 rows for every wave, a K block has one part");
     static_assert(!NO_DUMMY || L::GROUPS == 4 * WAVES, "every scale copy has a part to go to");
     uint8_t(*lds_a)[BM * 128] = reinterpret_cast<uint8_t(*)[BM * 128]>(pool + L::a_off);     // [STAGES]
@@ -566,7 +567,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
         const float sb = my_bs[kb0], sb_hi = my_bs_hi[kb0];
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
-            const float sa = lds_s[(s_rd + i * 16) * S_STRIDE];
+            const float sa = lds_s[s_rd + i * 16];
             sc[i] = sa * sb;
             if (STRADDLE) sc_hi[i] = sa * sb_hi;
         }
@@ -614,7 +615,7 @@ __device__ __forceinline__ void fp8_gemm_tile(
                             sb_n = my_bs[min(kb + 1, KB - 1)];
                             sb_hi_n = my_bs_hi[min(kb + 1, KB - 1)];
 #pragma unroll
-                            for (int i = 0; i < TI; ++i) sa_n[i] = ls_n[(s_rd + i * 16) * S_STRIDE];      // combined at the end of the block: nothing waits here
+                            for (int i = 0; i < TI; ++i) sa_n[i] = ls_n[s_rd + i * 16];      // combined at the end of the block: nothing waits here
                         }
                     } else {
                         asm volatile("" : "+v"(fx[0]));
@@ -1081,7 +1082,7 @@ struct Walk {
 constexpr bool walks(int BM, int BN, int STAGES, int esz, int EPI) { return BM == 256 && BN == 256 && STAGES == 2 && esz == 2 && EPI != kEpiDirect; }
 
 template <int BM, int BN, int WGM, int WGN, int STAGES, typename OUT, int GAP_ = 0, int TD_ = 0, int ABL_ = 0, int FMT_ = 0, int GM_ = 4,
-          int EPI_ = kEpiDirect, bool CHUNKED_ = false>
+          int EPI_ = kEpiDirect>
 __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
     const uint8_t* __restrict__ b, const float* __restrict__ b_s, OUT* __restrict__ c,
@@ -1090,7 +1091,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
     // then walks tiles blockIdx.x, blockIdx.x + gridDim.x, ... itself, which saves the ~4.5 us that pass between
     // the end of a workgroup and the start of its successor on the same CU.  Workgroup ids keep their XCD
     // (id % 8) from tile to tile when gridDim.x is a multiple of 8.
-    using L = TileLds<BM, BN, WGM * WGN, STAGES, false, CHUNKED_>;
+    using L = TileLds<BM, BN, WGM * WGN, STAGES>;
     constexpr bool WALK = walks(BM, BN, STAGES, (int)sizeof(OUT), EPI_) && ABL_ == 0;
     __shared__ __attribute__((aligned(1024))) uint8_t pool[WALK ? L::walk_bytes : L::bytes];
     const int ntiles = tiles_m * tiles_n;
@@ -1099,7 +1100,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
         int m0, n0;
         Duty duty;
         if (!walk(m0, n0, duty)) return;
-        fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, OUT, GAP_, TD_, ABL_, FMT_, false, EPI_, CHUNKED_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, m0, M, M, n0,
+        fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, OUT, GAP_, TD_, ABL_, FMT_, false, EPI_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, m0, M, M, n0,
                                                                                          N, K, ldc, duty, 0, K >> 7, pool, 0, 0, 0, walk);
         return;
     }
@@ -1107,7 +1108,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void fp8_gemm_mfma_kernel(
         int tm, tn;
         Duty duty = tile_of<GM_>(xcd_contiguous(pid, ntiles), tiles_m, tiles_n, tm, tn);
         if (!pretouch) duty.a_sh = duty.b_sh = 0;
-        fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, OUT, GAP_, TD_, ABL_, FMT_, false, EPI_, CHUNKED_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M,
+        fp8_gemm_tile<BM, BN, WGM, WGN, STAGES, OUT, GAP_, TD_, ABL_, FMT_, false, EPI_>(a, a_s, as_rs, as_cs, as_bytes, b, b_s, c, bias, tm * BM, M,
                                                                             M, tn * BN, N, K, ldc, duty, 0, K >> 7, pool);
         __syncthreads();   // every wave has left the tile's LDS buffers before the next tile's copies land in them
     }
