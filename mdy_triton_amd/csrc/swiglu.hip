@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const uint16_t* __restrict_
 // and rounded to bf16 as splitk_reduce_kernel does, and the activation is formed and quantized from the rounded values: the bytes
 // and scales of the two kernels in turn, without the bf16 projection's way through memory and without a launch: both kernels
 // were bound by their ends, 4 us each (the MLP of 7168 -> 2x2048 -> 7168 at 200 tokens, 4 slabs: 34.3 -> 31.4 us).  One row per wave (the loads of all slabs of a row are in flight together: 2 * ksplit * 32 bytes a lane).
-// KS: number of slabs, 0: `ksplit` of them.
+// KS: number of slabs, 0: `ksplit` of them, four at a time.
 template <int MODE, int KS>
 __global__ __launch_bounds__(256) void swiglu_slabs_kernel(const float* __restrict__ ws, uint8_t* __restrict__ y, float* __restrict__ s, int M, int N,
                                                            int64_t slab, int up_off, int gate_off, int PM, int PN, int64_t s_row_stride,
@@ -156,8 +156,18 @@ int launch_swiglu_slabs(const float* ws, void* y, float* s, int64_t M, int64_t N
 #define MDY_SS(MODE, KS)                                                                                                                  \
     launch_kernel((swiglu_slabs_kernel<MODE, KS>), grid, dim3(256), 0, stream, ws, static_cast<uint8_t*>(y), s, (int)M, (int)N, 2 * M * N, \
                        up_off, gate_off, (int)PM, (int)PN, s_row_stride, s_col_stride, ksplit)
-#define MDY_SS_K(MODE) do { if (ksplit == 2) MDY_SS(MODE, 2); else if (ksplit == 3) MDY_SS(MODE, 3); else if (ksplit == 4) MDY_SS(MODE, 4); else MDY_SS(MODE, 0); } while (0)
-    if (mode == 0) MDY_SS_K(0); else MDY_SS_K(1);
+#define MDY_SS_K(MODE)                          \
+    switch (ksplit) {                           \
+        case 2: MDY_SS(MODE, 2); break;         \
+        case 3: MDY_SS(MODE, 3); break;         \
+        case 4: MDY_SS(MODE, 4); break;         \
+        case 5: MDY_SS(MODE, 5); break;         \
+        case 6: MDY_SS(MODE, 6); break;         \
+        case 7: MDY_SS(MODE, 7); break;         \
+        case 8: MDY_SS(MODE, 8); break;         \
+        default: MDY_SS(MODE, 0);               \
+    }
+    if (mode == 0) MDY_SS_K(0) else MDY_SS_K(1)
 #undef MDY_SS_K
 #undef MDY_SS
     return (int)hipGetLastError();

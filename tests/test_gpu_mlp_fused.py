@@ -12,7 +12,8 @@ E4M3 = torch.float8_e4m3fn
 
 # slabs: 4, 2, 3, many, the whole-line kernel's, none; ragged rows; halves of 8 k and of odd columns
 @pytest.mark.parametrize("M,H,I", [(200, 7168, 2048), (300, 7168, 2048), (197, 7168, 1024), (100, 16384, 256), (61, 7168, 768), (40, 4096, 512),
-                                   (777, 7168, 1056), (333, 7168, 1000), (250, 4096, 517), (5, 2048, 768), (2048, 2048, 512)])
+                                   (777, 7168, 1056), (333, 7168, 1000), (250, 4096, 517), (5, 2048, 768), (2048, 2048, 512),
+                                   (130, 6528, 352), (211, 4224, 320), (110, 11136, 2240)])
 @pytest.mark.parametrize("order", ["up-gate", "gate-up"])
 @pytest.mark.parametrize("dialect", ["deeplinear", "official"])
 def test_same_bits_as_the_operators_in_turn(M, H, I, order, dialect):

@@ -34,3 +34,26 @@ def test_reduction(M, N, K, biased):
     bias = torch.randn(N, generator=torch.Generator(device="cuda").manual_seed(1), device="cuda").bfloat16() if biased else None
     out = [m.fp8_gemm(q, s, w.contiguous(), ws, out_dtype=dt, bias=bias) for dt in (torch.bfloat16, torch.float32)]
     assert torch.equal(out[0], out[1].bfloat16())
+
+
+@pytest.mark.parametrize("M,N,K,slabs", [(161, 1536, 3712, 5), (441, 1472, 17408, 5), (82, 2432, 6016, 6), (97, 1536, 3968, 7), (441, 1470, 17408, 5), (213, 576, 8832, 8),
+                                         (123, 574, 7040, 8)])
+def test_counts_of_slabs(M, N, K, slabs):
+    """Whole numbers: exact in any order, over however many slabs (5 to 8 all in flight at once)."""
+    g = torch.Generator(device="cuda").manual_seed(slabs)
+    a, b = (torch.randint(-2, 3, (r, K), generator=g, device="cuda").float() for r in (M, N))
+    s, ws = torch.ones(M, K // 128, device="cuda"), torch.ones(-(-N // 128), K // 128, device="cuda")
+    bias = torch.randint(-9, 10, (N,), generator=g, device="cuda").bfloat16()
+    ref = a @ b.t() + bias.float()
+    for dtype in (torch.float32, torch.bfloat16):
+        assert torch.equal(m.fp8_gemm(a.to(torch.float8_e4m3fn), s, b.to(torch.float8_e4m3fn), ws, out_dtype=dtype, bias=bias), ref.to(dtype))
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 2432, 2688), (384, 3584, 9344), (128, 1536, 3968), (256, 3456, 15104), (256, 1920, 5760), (384, 832, 9216), (256, 960, 14208)])
+def test_counts_of_row_scaled_slabs(M, N, K):      # 5 to 9, 12 and 16
+    from mdy_triton_amd import fp8_kernel
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = (torch.randint(-2, 3, (r, K), generator=g, device="cuda").float() for r in (M, N))
+    sa, sb = (torch.ones(r, K // 128, device="cuda") for r in (M, N))
+    got = fp8_kernel.fp8_matmul(a.to(torch.float8_e4m3fn), b.to(torch.float8_e4m3fn), sa, sb, have_w=False)
+    assert torch.equal(got, (a @ b.t()).to(got.dtype))
