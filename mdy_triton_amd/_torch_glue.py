@@ -79,6 +79,10 @@ class _NoHost:
     """Stands in for the native host side where there is neither a GPU nor a build: every call goes the Python way, which
     raises what it raises there."""
 
+    @staticmethod
+    def parameter(module, name, _):
+        return getattr(module, name)
+
     def __getattr__(self, name):
         return lambda *args: None
 
@@ -101,11 +105,13 @@ def host():
     return _host
 
 
+_MODULE_GETATTR = torch.nn.Module.__getattr__
+
+
 def parameter_of(module, name):
-    """module.<name>, without the failed attribute lookup that comes before torch.nn.Module finds a parameter (0.25 us); what a
-    parametrization or a replica put in a parameter's place is an attribute."""
-    parameters = module._parameters
-    return parameters[name] if name in parameters else getattr(module, name)
+    """module.<name>, without the failed attribute lookup that comes before torch.nn.Module finds a parameter (0.25 us); a property, an
+    attribute of the instance or whatever else module.<name> means is what it means here."""
+    return host().parameter(module, name, _MODULE_GETATTR)
 
 
 _WS_BYTES = {}

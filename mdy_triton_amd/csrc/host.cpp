@@ -313,6 +313,28 @@ PyObject* deep_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return THPVariable_Wrap(std::move(c));
 }
 
+// parameter(module, name, getattr) -> module.<name>.  What torch.nn.Module keeps under that name is taken without the failed lookup that comes in front of
+// it (0.25 us), but only where nothing comes in front of it: not an attribute of the type (a subclass's property) or of the instance, not a lookup of the
+// type's own; getattr is torch.nn.Module's.  The type is asked on each call (by the interpreter's own cache): a class may change.
+PyObject* parameter(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    static PyObject *const lookup = PyUnicode_InternFromString("__getattribute__"), *const missing = PyUnicode_InternFromString("__getattr__"),
+                    *const parameters = PyUnicode_InternFromString("_parameters");
+    if (n != 3 || lookup == nullptr || missing == nullptr || parameters == nullptr) Py_RETURN_NONE;
+    PyObject *module = args[0], *name = args[1];
+    PyTypeObject* type = Py_TYPE(module);
+    PyObject** dict = _PyObject_GetDictPtr(module);
+    if (dict != nullptr && *dict != nullptr && PyUnicode_CheckExact(name) && _PyType_Lookup(type, name) == nullptr && _PyType_Lookup(type, missing) == args[2] &&
+        _PyType_Lookup(type, lookup) == _PyType_Lookup(&PyBaseObject_Type, lookup) && PyDict_GetItemWithError(*dict, name) == nullptr) {
+        PyObject* kept = PyDict_GetItemWithError(*dict, parameters);
+        PyObject* found = kept != nullptr && PyDict_CheckExact(kept) ? PyDict_GetItemWithError(kept, name) : nullptr;
+        if (found != nullptr) {
+            Py_INCREF(found);
+            return found;
+        }
+    }
+    return PyErr_Occurred() ? nullptr : PyObject_GetAttr(module, name);
+}
+
 // cached_weight(weight, cache, with_transpose) -> the quantized copies (y, s, yt, st) that DeepLinear keeps, if they are the weight's: cache is
 // ((data_ptr, version, shape, device), copies, fingerprint).  None where that has to be looked at more closely, and where
 // MDY_FP8_CHECK_WEIGHT_CACHE asks for it.
@@ -1003,7 +1025,7 @@ PyObject* guarded(PyObject* self, PyObject* const* args, Py_ssize_t n) {
 
 #define MDY_METHOD(F) {#F, (PyCFunction)(void (*)(void))guarded<F>, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {MDY_METHOD(act_quant), MDY_METHOD(fp8_gemm), MDY_METHOD(weight_dequant), MDY_METHOD(matmul), MDY_METHOD(quant_input),
-                         MDY_METHOD(deep_linear), MDY_METHOD(cached_weight), MDY_METHOD(silu_act_quant), MDY_METHOD(deep_forward), MDY_METHOD(deep_backward),
+                         MDY_METHOD(deep_linear), MDY_METHOD(parameter), MDY_METHOD(cached_weight), MDY_METHOD(silu_act_quant), MDY_METHOD(deep_forward), MDY_METHOD(deep_backward),
                          MDY_METHOD(official_forward), MDY_METHOD(ordinary), MDY_METHOD(version_guard), MDY_METHOD(official_backward), MDY_METHOD(act_copies), MDY_METHOD(block_copies),
                          MDY_METHOD(quant_weight), MDY_METHOD(quant_transposed), MDY_METHOD(row_scaled_product), MDY_METHOD(silu_fwd),
                          MDY_METHOD(silu_bwd), MDY_METHOD(mlp), MDY_METHOD(mlp_backward), MDY_METHOD(group_cast), MDY_METHOD(grouped_matmul), MDY_METHOD(move_rows),
