@@ -239,3 +239,11 @@ def test_large_tiles_that_just_miss_a_round(lib):
     assert lib.mdy_fp8_gemm_form(2383, 6656, 2176, 0) == lib.mdy_fp8_gemm_form(2841, 5632, 128, 0) == 10
     assert lib.mdy_fp8_gemm_form(7172, 3264, 128, 0) == lib.mdy_fp8_gemm_form(1854, 12480, 1920, 0) != 10
     assert lib.mdy_fp8_gemm_form(1854, 12480, 2048, 0) == 10
+
+
+def test_one_tile_row_keeps_the_slabs_of_a_weight_from_memory(lib):
+    """65 to 128 rows: 128x64 tiles in one launch, or in fewer slabs, are faster with the operands in the caches and up to 15 % slower without (256 CUs)."""
+    for shape, form in (((107, 8576, 4736), 7 | 3 << 8), ((66, 12032, 6784), 9 | 4 << 8), ((115, 6208, 6912), 7 | 5 << 8), ((104, 6080, 5248), 7 | 5 << 8)):
+        assert lib.mdy_fp8_gemm_form(*shape, 1) == form, shape
+    assert lib.mdy_fp8_gemm_form(123, 1088, 1152, 1) == lib.mdy_fp8_gemm_form(120, 2112, 1280, 1) == 4
+    assert lib.mdy_fp8_gemm_form(777, 2112, 7168, 1) == 6      # seven tile rows: as before
