@@ -288,11 +288,13 @@ __device__ __forceinline__ int block_row() { return (int)(blockIdx.y + blockIdx.
 // an eighth of the columns in 8 rows of tiles.  A tile's pieces of the transposed rows are 128 bytes and its row-major scales 4 bytes each: those of neighbours
 // now meet in one L2 before they go to memory (scales and copies of 8192x4096 29.9 -> 27.6 us, with column sums 32.8 -> 30.3, block scales
 // 27.1 -> 25.6, 4096x7168 27.1 -> 26.0, 16384x8192 101 -> 96, eight weights of 4096x7168 138.3 -> 135.4).  Patches of 2, 4 and 16 rows tie.  Where the
-// 1024 workgroups that run at once have all tiles, or nearly so, it has nothing to gather: 4096x4096 16.6 -> 16.6, 5120x4096 20.0 -> 20.2, 2048x4096 9.7 -> 9.9.
-constexpr unsigned kPatchMinTiles = 1280;
-__device__ __forceinline__ void xcd_patch(int& row, int& col, int cols, int rows) {
+// 1024 workgroups that run at once have all tiles, or nearly so, it has nothing to gather: 4096x4096 16.6 -> 16.6, 2048x4096 9.7 -> 9.9.  Of 1280 tiles, plain
+// order / patches: row scales and copies of 10240x2048 20.4 / 21.1, 5120x4096 21.1 / 21.1, block scales 18.5 / 18.9, 4096x5120 19.1 / 19.7, weights alone gain
+// (5120x4096 18.1 / 17.4, 8192x2560 17.7 / 17.9); of 1344 (5376x4096) all do: 22.4 / 21.9, 20.6 / 19.8, weights 18.7 / 18.0.
+constexpr unsigned kPatchAbove = 1280;
+__host__ __device__ __forceinline__ void xcd_patch(int& row, int& col, int cols, int rows) {
     const int r0 = row & ~7;
-    if ((unsigned)cols * (unsigned)rows < kPatchMinTiles || r0 + 8 > rows) return;      // also the last rows that are no 8
+    if ((unsigned)cols * (unsigned)rows <= kPatchAbove || r0 + 8 > rows) return;      // also the last rows that are no 8
     const int p = (row - r0) * cols + col, i = (p & 7) * cols + (p >> 3);      // r0 * cols is a multiple of 8
     row = r0 + (i & 7);
     col = i >> 3;

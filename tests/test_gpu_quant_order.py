@@ -1,4 +1,4 @@
-"""Quantizers with a transposed copy deal their tiles out to the XCDs in patches from 1280 tiles on: every tile once, the same bytes and scales as
+"""Quantizers with a transposed copy deal their tiles out to the XCDs in patches beyond 1280 tiles: every tile once, the same bytes and scales as
 slabs of the rows, which stay below that and run in plain order."""
 import ctypes
 
@@ -10,7 +10,7 @@ from mdy_triton_amd import _lib
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
-# tiles: 22 x 59 (the last 6 rows are no patch), 8 x 161, 9 x 143, 160 x 8, 161 x 8, 1 x 1300 (no patch at all), 80 x 16 = 1280, 1264 (below)
+# tiles: 22 x 59 (the last 6 rows are no patch), 8 x 161, 9 x 143, 160 x 8 = 1280 (in plain order), 161 x 8, 1 x 1300 (no patch at all), 80 x 16 = 1280, 1264
 SIZES = [(2816, 7552), (1024, 20608), (1152, 18304), (20480, 1024), (20608, 1024), (128, 166400), (10240, 2048), (10112, 2048)]
 
 
