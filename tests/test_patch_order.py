@@ -29,9 +29,9 @@ int main(int argc, char** argv) {
     }
 }
 """
-# columns x rows of tiles and whether they are dealt out in patches
+# columns x rows of tiles and whether their order changes (an eighth of 8 columns is one: plain order)
 CASES = [((1, 1), False), ((32, 32), False), ((32, 40), False), ((40, 32), False), ((16, 80), False), ((160, 8), False), ((8, 160), False), ((1280, 1), False),
-         ((183, 7), False), ((1300, 1), False), ((1, 2000), False), ((161, 8), True), ((8, 161), True), ((143, 9), True), ((59, 22), True), ((427, 3), False),
+         ((183, 7), False), ((1300, 1), False), ((1, 2000), False), ((161, 8), True), ((8, 161), False), ((9, 161), True), ((143, 9), True), ((59, 22), True), ((427, 3), False),
          ((61, 21), True), ((32, 42), True), ((56, 64), True), ((7, 1001), True)]
 
 
