@@ -10,15 +10,19 @@ pytestmark = pytest.mark.gpu
 E4M3 = torch.float8_e4m3fn
 
 
-# slabs: 4, 2, 3, many, the whole-line kernel's, none; ragged rows; halves of 8 k and of odd columns
-@pytest.mark.parametrize("M,H,I", [(200, 7168, 2048), (300, 7168, 2048), (197, 7168, 1024), (100, 16384, 256), (61, 7168, 768), (40, 4096, 512),
-                                   (777, 7168, 1056), (333, 7168, 1000), (250, 4096, 517), (5, 2048, 768), (2048, 2048, 512),
-                                   (130, 6528, 352), (211, 4224, 320), (110, 11136, 2240)])
+# slabs of the up/gate projection (0: one launch) with the sizes of either dialect; tiles and the whole-line kernel's; ragged rows; halves of 8 k and of odd columns
+@pytest.mark.parametrize("M,H,I,slabs", [(200, 7168, 2048, (4, 4)), (300, 7168, 2048, (2, 2)), (197, 7168, 1024, (4, 4)), (100, 16384, 256, (16, 16)),
+                                         (61, 7168, 768, (5, 5)), (40, 4096, 512, (4, 4)), (777, 7168, 1056, (0, 0)), (333, 7168, 1000, (5, 3)),
+                                         (250, 4096, 517, (4, 4)), (5, 2048, 768, (0, 0)), (2048, 2048, 512, (0, 0)), (130, 6528, 352, (8, 8)),
+                                         (211, 4224, 320, (7, 7)), (110, 11136, 2240, (7, 7)), (185, 7552, 2312, (3, 3)), (326, 7040, 400, (6, 6)),
+                                         (83, 3840, 568, (6, 6)), (104, 9344, 336, (9, 9)), (169, 12544, 280, (11, 11))])
 @pytest.mark.parametrize("order", ["up-gate", "gate-up"])
 @pytest.mark.parametrize("dialect", ["deeplinear", "official"])
-def test_same_bits_as_the_operators_in_turn(M, H, I, order, dialect):
+def test_same_bits_as_the_operators_in_turn(M, H, I, slabs, order, dialect):
     if dialect == "official" and I % 128:
         I = I // 128 * 128
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert lib().mdy_fp8_gemm_form(M, 2 * I, H, 1) >> 8 == slabs[dialect == "official"]
     g = torch.Generator(device="cuda").manual_seed(M + H + I)
     x = torch.randn(M, H, generator=g, device="cuda").bfloat16()
     wu, wd = ((torch.randn(*s, generator=g, device="cuda") * 0.02).bfloat16() for s in ((2 * I, H), (H, I)))
