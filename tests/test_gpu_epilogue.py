@@ -22,10 +22,20 @@ def _gemm(a, a_s, b, b_s, bias, dtype):
     return out[:M]
 
 
-# 256x256 tiles with a 128x256 remainder, 128x256, 256x128, 128x192, 128x128, 128x64 and 64x64 tiles; ragged rows and columns
-# that are and are not a multiple of 8
-@pytest.mark.parametrize("M,N,K", [(4100, 5000, 256), (3590, 4612, 128), (1100, 6008, 1024), (12700, 392, 1024), (4090, 1544, 1024),
-                                   (2040, 2056, 256), (2040, 1036, 384), (1000, 1096, 256), (65, 136, 128), (300, 520, 384), (200, 7168, 256)])
+# ragged rows and columns that are and are not a multiple of 8
+SIZES = [(4100, 5000, 256), (3590, 4612, 128), (1100, 6008, 1024), (12700, 392, 1024), (4090, 1544, 1024), (2040, 2056, 256), (2040, 1036, 384), (1000, 1096, 256),
+         (65, 136, 128), (300, 520, 384), (200, 7168, 256), (33000, 120, 1024), (33000, 100, 1024), (1348, 3564, 1280), (1348, 3560, 1280), (1055, 424, 1408),
+         (1055, 420, 1408), (680, 2712, 1024), (822, 2380, 1024)]
+
+
+def test_sizes_take_every_tile():
+    """64x64, 64x128, 128x64, 128x128 one and two per CU, 128x192, 128x256, 256x128 and 256x256 tiles with a 128x256 remainder."""
+    got = {_lib.load().mdy_fp8_gemm_form(*size, 0) for size in SIZES}
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert got == {4, 5, 6, 7, 8, 9, 10, 11, 13}
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
 @pytest.mark.parametrize("with_bias", [False, True])
 def test_bf16_rows_equal_rounded_fp32(M, N, K, with_bias):
     g = torch.Generator().manual_seed(M + N + K)

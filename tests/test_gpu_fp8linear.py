@@ -433,14 +433,14 @@ E5M2_SMALL = [(1, 512, 256), (5, 512, 384), (16, 520, 256), (17, 512, 256), (33,
               (48, 3600, 256), (64, 3200, 128), (48, 6400, 256), (64, 6404, 128),                                   # the same with 4 row tiles against a middling N
               (5, 16384, 256), (17, 9216, 256), (31, 9216, 128), (5, 25600, 256), (16, 25600, 128),                # 32 columns per workgroup
               (20, 25600, 256), (33, 25616, 256), (64, 25600, 128),                                                # strip kernel
-              (48, 16384, 256), (33, 16400, 128),                                                                  # 128x128 tiles
+              (48, 16384, 256), (33, 16400, 128),                                                                  # 64x64 and 64x128 tiles
               (48, 12800, 256), (64, 12804, 128)]                                                                  # 64x64 tiles
 
 
 @pytest.mark.parametrize("M,N,K", E5M2_SMALL)
 def test_e5m2_small_m_exact_integer(M, N, K):
     """e5m2 operands, up to 64 rows: every branch of the small-M dispatch (the whole-line kernel with 16 and 32 columns per
-    workgroup and 1, 2 or 4 row tiles, the strip kernel, 128x128 and 64x64 tiles against a wide weight), exact on integer
+    workgroup and 1, 2 or 4 row tiles, the strip kernel, 64x128 and 64x64 tiles against a wide weight), exact on integer
     operands with power-of-two scales; fp32 and bf16 output, bias in the epilogue, through the C entry point and through
     fp8_matmul."""
     from mdy_triton_amd import _lib

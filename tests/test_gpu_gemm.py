@@ -73,20 +73,26 @@ def test_gemm_exact_integer_cases_all_kernels(M, N, K):
     assert torch.equal(got.cpu().double(), c)
 
 
-@pytest.mark.parametrize("M,N,K", [(896, 9300, 256), (880, 9344, 640),         # 128x128 tiles, 2 K blocks in LDS
-                                   (2000, 2304, 256), (2048, 2200, 512),          # the same for a short K
-                                   (2000, 2304, 1024), (4096, 1536, 1152), (1300, 5800, 2304),   # 128x256 tiles, ring of 3
-                                   (4096, 1100, 1024), (4000, 1530, 1280), (3000, 1700, 1152), (3072, 1536, 2048),   # 128x192 tiles (wave columns straddle weight-scale blocks)
-                                   (12800, 384, 1024),                                              # 128x256 tiles although they pad more
-                                   (38400, 128, 1024), (36000, 100, 1280),       # 256x128 tiles, ring of 3
-                                   (1536, 2048, 128), (1500, 2000, 1280),      # 128x128 tiles, ring of 4 K blocks
-                                   (1024, 1100, 128), (1000, 1090, 1664),      # 128x64 tiles, ring of 6
-                                   (200, 300, 128), (130, 70, 2304), (520, 776, 1024),    # 64x64 tiles, ring of 8
-                                   (40, 16400, 256), (64, 6500, 384), (33, 7168, 1280)])  # 32..64 rows, wide weight
-def test_gemm_exact_integer_few_tiles_configs(M, N, K):
+# MDY_FORM_... of each size
+FEW_TILES = [*[(v, 8) for v in ((896, 9300, 256), (880, 9344, 640), (2000, 2304, 256))],      # 128x128 tiles, two per CU
+             *[(v, 9) for v in ((2048, 2200, 512), (2000, 2304, 1024), (4096, 1536, 1152), (4096, 1100, 1024), (4000, 1530, 1280), (3000, 1700, 1152),
+                                (3072, 1536, 2048), (12800, 384, 1024))],      # 128x192 (wave columns straddle weight-scale blocks)
+             ((1300, 5800, 2304), 10),      # 128x256, ring of 3
+             *[(v, 11) for v in ((38400, 128, 1024), (36000, 100, 1280))],      # 256x128, ring of 3
+             *[(v, 7) for v in ((1536, 2048, 128), (1500, 2000, 1280))],      # 128x128
+             *[(v, 6) for v in ((1024, 1100, 128), (1000, 1090, 1664), (200, 300, 128), (130, 70, 2304), (520, 776, 1024))],      # 128x64, once over slabs
+             *[(v, 4) for v in ((1055, 422, 1408), (128, 3433, 1280))],      # 64x64, ring of 8
+             *[(v, 5) for v in ((40, 16400, 256), (680, 2712, 1024))],      # 64x128
+             *[(v, 1) for v in ((64, 6500, 384), (33, 7168, 1280))]]      # the whole-line kernel: 33 to 64 rows, wide weight
+
+
+@pytest.mark.parametrize("size,form", FEW_TILES)
+def test_gemm_exact_integer_few_tiles_configs(size, form):
     """Shapes with fewer than 200 tiles of 256x256 pick tile size and LDS ring depth by tile count; K runs
     from one K block (shorter than every ring) to more K blocks than the deepest ring, M and N ragged."""
-    test_gemm_exact_integer_cases_all_kernels(M, N, K)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert _lib.load().mdy_fp8_gemm_form(*size, 1) & 255 == form
+    test_gemm_exact_integer_cases_all_kernels(*size)
 
 
 @pytest.mark.parametrize("M,N,K", [(4096, 1536, 7168), (4000, 1531, 1152), (2048, 3000, 1408), (3900, 1345, 1024)])
@@ -136,7 +142,7 @@ def test_gemm_exact_integer_random_mid_shapes(M, N, K):
 
 
 SPLIT_SHAPES = [(128, 1536, 4096), (100, 777, 4224), (256, 2304, 4096), (130, 1100, 5120),
-                (130, 520, 6528), (300, 1536, 4480), (1000, 640, 8192),             # slabs of 9 / 12 and 11 / 11 K blocks, 3 and 8 tile rows
+                (130, 520, 6528), (300, 1536, 4480), (1000, 640, 8192),             # slabs of 7, 12 and 22 K blocks, 2, 3 and 8 tile rows
                 (64, 2304, 4352), (48, 4096, 7168), (64, 2048, 4352),               # 33..64 rows on 64x64 tiles
                 # the whole-line kernel over slabs of K (one or two K blocks per wave and pass, several passes, ragged N with the
                 # scalar reduction, a slab count that does not divide K)

@@ -35,11 +35,15 @@ def _call(a, a_s, b, b_s, bias, mode, fmt):
     return c
 
 
+CUT = [(64, 1024, 4224), (128, 1030, 4224), (70, 600, 8320), (637, 1252, 7552), (662, 833, 9984)]      # split along K
+
+
 @pytest.mark.parametrize("fmt", [0, 1])
 @pytest.mark.parametrize("M,N,K", [(1, 1000, 4224), (16, 2050, 1024), (20, 26000, 256), (48, 16640, 256), (40, 6500, 384),      # up to 64 rows
-                                   (64, 1024, 4224), (128, 1030, 4224), (777, 2112, 4096), (70, 600, 8320),                      # split along K
-                                   (100, 264, 384), (2050, 1032, 384), (4100, 4620, 256), (5300, 18440, 2176)])                 # tiles
+                                   *CUT, (777, 2112, 4096), (100, 264, 384), (2050, 1032, 384), (4100, 4620, 256), (5300, 18440, 2176)])                 # tiles
 def test_bias_after_rounding_and_formats(M, N, K, fmt):
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert (_lib.load().mdy_fp8_gemm_form(M, N, K, 1) >> 8 > 1) == ((M, N, K) in CUT)
     a, a_s, b, b_s, bias, ref = _operands(M, N, K, fmt)
     plain = _call(a, a_s, b, b_s, None, 0, fmt)
     assert torch.equal(plain, ref.bfloat16())

@@ -61,7 +61,7 @@ def test_e5m2_and_bias(M, N, K):
     assert torch.equal(got.cpu(), want)
 
 
-# more than 64 rows where an estimate overrides the line between sizes: 64x128 and 128x192 tiles, in one launch and over slabs
+# more than 64 rows where the estimates of one fit or another override the line between sizes: among them 64x128 tiles in one launch and over slabs, 128x192 over slabs
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(113, 11451, 8576), (354, 3968, 12032), (123, 17920, 1152), (65, 961, 3584), (163, 1725, 3584), (294, 960, 12928),
                                    (150, 8897, 2304), (256, 4096, 4096), (255, 4090, 4224), (142, 8960, 896), (129, 3000, 4608), (900, 960, 6400)])
