@@ -278,7 +278,11 @@ int launch_fp8_gemm_nt_rowscaled(const void* a, const float* a_s, int64_t as_rs,
     // Scales that lie K block after K block (row-major) in chunks of four of them (CHUNKED of TileLds), with tiles of 256 columns, from 12 K blocks on.
     // A K block at a time -> in chunks, row-major: 8192x4096x4096 137 -> 131 us, 7168x2048x4096 67.6 -> 62.9, 1792x4096x4096 39.7 -> 36.9, 4096x7168 with
     // 12 / 16 blocks 52.5 -> 50.7 / 65.2 -> 64.5, but with 2 to 8 blocks +1 % (the first chunk comes before the first K block), 128x128 tiles +2 to 5 % (2048x2048x2048 14.9 ->
-    // 15.3); column-major +1 % (4096x7168x1024 38.8 -> 39.4), 128x128 tiles +4 to 8 % (1024x3072x2048 13.5 -> 14.6).
+    // 15.3); column-major +1 % (4096x7168x1024 38.8 -> 39.4), 128x128 tiles +4 to 8 % (1024x3072x2048 13.5 -> 14.6).  It is all of K that counts, not a slab's
+    // part: row-major slabs gain down to 4 blocks, in the caches / out of them 512x512x4096 (8 slabs of 4) 15.7 -> 15.5 / 18.3 -> 17.8, 256x1280x6400 (5) 19.8 ->
+    // 19.2 / 21.6 -> 20.6, 2305x512x3712 (6) 20.7 -> 19.9 / 22.0 -> 21.0, 1530x640x4736 (8) 22.7 -> 20.9 / 23.6 -> 21.8; the shortest, 4 slabs of 5,
+    // 384x576x2176 13.0 -> 13.5 / 15.9 -> 15.3.  One operand row-major is enough: a weight's 3 % less in the mean of 43 shapes in the caches and 4.5 % out
+    // of them, the activations' even (in one launch -7.5 to +3.6 %) and 1 to 3 % less.
     const bool chunked = KB >= 12 && (as_cs < as_rs || bs_cs < bs_rs);
     if (sp.slabs > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && workspace_bytes >= (int64_t)sp.slabs * M * N * 4) {
         const int tm = (int)((M + 127) / 128), tn = (int)((N + 255) / 256);

@@ -777,9 +777,10 @@ __device__ __forceinline__ Duty tile_of(int local, int tiles_m, int tiles_n, int
 //     1300x4096x4096 29.2 -> 27.1, 200x7168x2048 10.0 -> 9.5, 1000x1090x1664 10.3 -> 9.9, 777x2112x7168 24.6 -> 24.4.
 // Swizzle, fragment layout, fold, epilogue and pre-touch shares are fp8_gemm_tile's.
 // The activation scales come in chunks of 4 K blocks, 16 rows x 4 K blocks a copy, the first three with the tile's start and one more with every 4th
-// K block: with row-major scales, the official dialect's, 64 rows of one K block at a time are 64 lines of 4 bytes for 128 of panels.  Row-major
-// 777x2112x7168 27.4 -> 25.4 us, 1024x4096x7168 39.4 -> 35.2, 2048x2048x7168 39.2 -> 34.8, 300x7168x4096 23.9 -> 21.2, 128x7168x7168
-// 24.4 -> 22.8, 200x7168x2048 10.4 -> 10.1; column-major 35.6 -> 35.2, 35.2 -> 34.9, the others even (measured with all of a tile's chunks at its start).
+// K block: with row-major scales, the official dialect's, 64 rows of one K block at a time are 64 lines of 4 bytes for 128 of panels.  What row-major
+// scales take over column-major ones, a K block at a time and the longer loop -> now: 1024x4096x7168 41.5 / 37.0 -> 36.6 / 36.2 us, 2048x2048x7168 40.1 / 36.7
+// -> 36.2 / 35.6, 300x7168x4096 24.4 / 21.8 -> 21.7 / 21.5, 128x7168x7168 23.4 / 21.7 -> 21.3 / 21.3, 200x7168x2048 11.5 / 10.9 -> 10.5 / 10.4, 4096x1536x7168
+// 51.5 / 48.8 -> 49.1 / 48.3 (out of the caches).
 template <int BM, int BN, typename OUT, int FMT_ = 0, int EPI_ = kEpiDirect>
 __device__ __forceinline__ void fp8_gemm_tile_ws(
     const uint8_t* __restrict__ a, const float* __restrict__ a_s, int as_rs, int as_cs, uint32_t as_bytes,
